@@ -159,6 +159,41 @@ def test_strided_field(torch_cuda):
     assert np.all(o == -7.0)   # nothing outside the field was touched
 
 
+@pytest.mark.parametrize("nx,ny,nz", [(2, 2, 300), (3, 5, 90), (5, 4, 4), (6, 3, 129), (7, 7, 70), (35, 6, 9), (261, 2, 5),
+                                      (12, 9, 10), (1, 7, 9), (4, 1, 1)])
+@pytest.mark.parametrize("shift,gap", [(0, 0), (1, 0), (3, 5), (0, 4)])
+def test_rows_at_any_element(torch_cuda, nx, ny, nz, shift, gap, zfp_form):
+    """Contiguous rows that start at any element and end inside a block: the 16-byte row path
+    reads a cut-off row to its fourth element (the next row, the gap between rows) and must drop
+    what it finds there, and must store nothing outside the field.  NaNs all around it."""
+    torch = torch_cuda
+    import oracle
+    from cswap_amd._lib import check, lib
+
+    rng = np.random.default_rng(nx * 1009 + ny * 31 + nz + shift)
+    f = rng.standard_normal((nz, ny, nx)).astype(np.float32)
+    big = np.full((nz, ny, nx + gap), np.nan, dtype=np.float32)
+    big[:, :, :nx] = f
+    flat = np.concatenate([np.full(shift, np.nan, np.float32), big.ravel(), np.full(8, np.nan, np.float32)])
+    tb = torch.from_numpy(flat).cuda()
+    sy, sz = nx + gap, ny * (nx + gap)
+    for maxbits in (256, 520, 1024):
+        s = torch.zeros(lib().cswap_zfp_stream_capacity(nx, ny, nz, maxbits), dtype=torch.uint8, device="cuda")
+        check(lib().cswap_zfp_compress_f32(tb.data_ptr() + 4 * shift, nx, ny, nz, 1, sy, sz, maxbits, s.data_ptr(), None),
+              "compress")
+        out = torch.full(tb.shape, -7.0, dtype=torch.float32, device="cuda")
+        check(lib().cswap_zfp_decompress_f32(s.data_ptr(), nx, ny, nz, 1, sy, sz, maxbits, out.data_ptr() + 4 * shift,
+                                             None), "decompress")
+        torch.cuda.synchronize()
+        want = oracle.zfp_encode3(f, maxbits)
+        assert np.array_equal(s.cpu().numpy().view(np.uint64), want), maxbits
+        o = out.cpu().numpy()
+        inside = o[shift:shift + big.size].reshape(big.shape)
+        assert np.array_equal(inside[:, :, :nx].view(np.uint32), oracle.zfp_decode3(want, f.shape, maxbits).view(np.uint32))
+        inside[:, :, :nx] = -7.0
+        assert np.all(o == -7.0), maxbits   # nothing outside the field was touched
+
+
 @pytest.mark.parametrize("case", ["padded_rows_and_planes", "one_block_per_slab", "slab_crossing", "planes_before_rows",
                                   "big_offsets"])
 def test_aligned_strided_fields(torch_cuda, case, zfp_form):

@@ -40,12 +40,41 @@ __device__ __forceinline__ int wave_sum(int v)
   return v;
 }
 
+// Inclusive prefix sum over the 64 lanes of a wavefront with data-parallel-primitive
+// moves (row shifts inside rows of 16 lanes, then the row broadcasts): six additions, no
+// trip through the LDS crossbar that a shuffle takes.
+__device__ __forceinline__ unsigned wave_inclusive_scan(unsigned v)
+{
+  v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);  // row_shr:2
+  v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);  // row_shr:4
+  v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);  // row_shr:8
+  v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1, 3
+  v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2, 3
+  return v;
+}
+
 // 16-byte store with the nontemporal hint, for output that is written once in whole lines
 typedef float stream_f4 __attribute__((ext_vector_type(4)));
+// 16 bytes at any element: chunks of a length that is no multiple of four start on no 16-byte boundary
+typedef float any_f4 __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ void st_stream4(float4* p, float4 v)
 {
   stream_f4 t = {v.x, v.y, v.z, v.w};
   __builtin_nontemporal_store(t, reinterpret_cast<stream_f4*>(p));
+}
+
+// the same where the address may be any element's: partial lines at both ends of what the
+// wavefront writes, so without the hint
+template <bool ALIGNED>
+__device__ __forceinline__ void st_row4(float* p, float4 v)
+{
+  if (ALIGNED) {
+    st_stream4(reinterpret_cast<float4*>(p), v);
+  } else {
+    any_f4 t = {v.x, v.y, v.z, v.w};
+    *reinterpret_cast<any_f4*>(p) = t;
+  }
 }
 
 struct Geometry {
@@ -68,17 +97,13 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_count_kernel(const fl
   const int len = (int)min((long long)g.E, (long long)g.n - b);
   const float* p = in + b;
   int acc = 0;
-  if ((((uintptr_t)p) & 15u) == 0) {
-    const float4* p4 = reinterpret_cast<const float4*>(p);
-    const int n4 = len >> 2;
-    for (int i = lane; i < n4; i += 64) {
-      float4 v = p4[i];
-      acc += (v.x != 0.0f) + (v.y != 0.0f) + (v.z != 0.0f) + (v.w != 0.0f);
-    }
-    for (int i = (n4 << 2) + lane; i < len; i += 64) acc += (p[i] != 0.0f);
-  } else {
-    for (int i = lane; i < len; i += 64) acc += (p[i] != 0.0f);
+  const any_f4* p4 = reinterpret_cast<const any_f4*>(p);
+  const int n4 = len >> 2;
+  for (int i = lane; i < n4; i += 64) {
+    const any_f4 v = p4[i];
+    acc += (v.x != 0.0f) + (v.y != 0.0f) + (v.z != 0.0f) + (v.w != 0.0f);
   }
+  for (int i = (n4 << 2) + lane; i < len; i += 64) acc += (p[i] != 0.0f);
   acc = wave_sum(acc);
   if (lane == 0) count[c] = acc;
 }
@@ -316,47 +341,6 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_compact_rows_kernel(
 }
 
 // ------------------------------------------------------------------ expand
-__global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand_kernel(
-    const float* __restrict__ values, const uint32_t* __restrict__ mask, const int* __restrict__ begin,
-    Geometry g, float* __restrict__ out)
-{
-  const int c = blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6);
-  if (c >= g.active) return;
-  const unsigned lane = lane_id();
-  const long long b = (long long)g.E * c;
-  const int len = (int)min((long long)g.E, (long long)g.n - b);
-  const uint32_t* mrow = mask + (size_t)c * g.W;
-  float* q = out + b;
-  unsigned off = (unsigned)begin[c];
-  const int iters = (len + 63) >> 6;
-  uint32_t held = 0;
-  for (int t0 = 0; t0 < iters; t0 += kUnroll) {
-    if ((t0 & 31) == 0) {  // refill: lane l takes mask word 64*(t0/32)+l of this chunk
-      const int w = (t0 >> 5) * 64 + (int)lane;
-      held = w < g.W ? mrow[w] : 0u;
-    }
-    float x[kUnroll];
-#pragma unroll
-    for (int j = 0; j < kUnroll; j++) {
-      const int t = t0 + j;
-      const int slot = (2 * t) & 63;
-      const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)held, slot);
-      const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)held, slot + 1);
-      unsigned long long m = ((unsigned long long)hi << 32) | lo;
-      const int rem = len - t * 64;  // bits past the end of the chunk carry no data
-      if (rem < 64) m = rem > 0 ? (m & ((1ull << rem) - 1ull)) : 0ull;
-      const bool nz = (m >> lane) & 1ull;
-      x[j] = nz ? values[off + rank_below(m)] : 0.0f;
-      off += popc64(m);
-    }
-#pragma unroll
-    for (int j = 0; j < kUnroll; j++) {
-      const int k = (t0 + j) * 64 + (int)lane;
-      if (k < len) q[k] = x[j];
-    }
-  }
-}
-
 // Same expansion with one lane = four consecutive elements and 16-byte stores
 // (with the nontemporal hint: 256 MiB expand in 63 instead of 88 us, 32 MiB in
 // 10.9 instead of 12.3 us, a reader of the result right after it no slower;
@@ -366,10 +350,16 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand_kernel(
 // lane l keeps mask word 64*(row/8) + l of the chunk, together with the number
 // of set bits in the words before it inside its row, so a lane finds its nibble
 // and the rank of its first element with two cross-lane reads.
-// Needs E % 4 == 0 and a 16-byte aligned destination (every chunk then starts
-// on a 16-byte boundary); the caller checks.
+// ALIGNED: E % 4 == 0 and a 16-byte aligned destination, so every chunk starts on a
+// 16-byte boundary.  Otherwise the same 16-byte stores at any element, without the hint:
+// 60 MB in chunks of 1838 elements 16.3 us, against 18.6 us with a 4-byte store per element.
+// Chunks of at most so many mask words share a wavefront (zvc_expand_packed_kernel) where there are
+// more than so many of them: three or more to a wavefront.  Two to a wavefront measure the same as one
+// each, and few chunks are all in flight at once either way.
+constexpr int kPackedWords = 21, kPackedFrom = 2048;
 constexpr int kRowsInFlight = 8;  // divides the 8 rows one refill covers
 
+template <bool ALIGNED>
 __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand4_kernel(
     const float* __restrict__ values, const uint32_t* __restrict__ mask, const int* __restrict__ begin,
     Geometry g, float* __restrict__ out)
@@ -425,12 +415,84 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand4_kernel(
     for (int j = 0; j < kRowsInFlight; j++) {
       const int k = (r0 + j) * 256 + 4 * (int)lane;
       if (k + 4 <= len) {
-        st_stream4(reinterpret_cast<float4*>(q + k), x[j]);
+        st_row4<ALIGNED>(q + k, x[j]);
       } else {  // ragged end of the last chunk
         if (k < len) q[k] = x[j].x;
         if (k + 1 < len) q[k + 1] = x[j].y;
         if (k + 2 < len) q[k + 2] = x[j].z;
       }
+    }
+  }
+}
+
+// Short chunks.  A wavefront per chunk is bound by the wavefronts there are to start: 16384 of
+// them take 8.8 us with three elements each.  Here one wavefront takes as many of them as 64 words hold.  Lane l
+// keeps one word together with where its values start and where its elements go, so a word
+// finds its chunk's end and offset by itself and the eight rows of a refill are full.
+// 16384 chunks, one wavefront per chunk -> this: 7 MB 11.3 -> 5.9 us, 25.7 MB 11.1 -> 8.4,
+// 33.6 MB (512 elements per chunk) 11.0 -> 8.7.
+template <bool ALIGNED>
+__global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand_packed_kernel(
+    const float* __restrict__ values, const uint32_t* __restrict__ mask, const int* __restrict__ begin,
+    Geometry g, int per, float* __restrict__ out)
+{
+  const int c0 = (int)(blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6)) * per;
+  if (c0 >= g.active) return;
+  const unsigned lane = lane_id();
+  const unsigned W = (unsigned)g.W;
+  const unsigned cl = lane * ((65536u + W - 1) / W) >> 16;  // lane / W
+  const unsigned k = lane - cl * W, c = (unsigned)c0 + cl;
+  const bool live = (int)cl < per && c < (unsigned)g.active;
+  uint32_t held = 0;
+  unsigned first = 0, dst = 0;
+  int valid = 0;  // elements of my word that exist
+  if (live) {
+    held = mask[(size_t)c0 * W + lane];
+    first = (unsigned)begin[c];
+    dst = (unsigned)g.E * c + 32u * k;
+    const int len = (int)min((unsigned)g.E, (unsigned)g.n - (unsigned)g.E * c);
+    valid = min(max(len - 32 * (int)k, 0), 32);
+    if (valid < 32) held &= (1u << valid) - 1u;  // bits past the end of the chunk carry no data
+  }
+  const unsigned cnt = (unsigned)__popc(held);
+  const unsigned before = wave_inclusive_scan(cnt) - cnt;
+  const unsigned rank = first + before - (unsigned)__shfl((int)before, (int)(cl * W), 64);
+  const unsigned sub = lane & 7u;
+  const uint32_t below = (1u << (4u * sub)) - 1u;
+  const int rows = ((int)W * per + 7) >> 3;
+  float4 x[8];
+  unsigned to[8];
+  int left[8];
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    if (j >= rows) break;
+    const int src = (j << 3) + (int)(lane >> 3);
+    const uint32_t w = (uint32_t)__shfl((int)held, src, 64);
+    unsigned rk = (unsigned)__shfl((int)rank, src, 64);
+    to[j] = (unsigned)__shfl((int)dst, src, 64) + 4u * sub;
+    left[j] = __shfl(valid, src, 64) - 4 * (int)sub;
+    const uint32_t nib = (w >> (4u * sub)) & 15u;
+    rk += (unsigned)__popc(w & below);
+    float4 v;
+    v.x = (nib & 1u) ? values[rk] : 0.0f;
+    rk += nib & 1u;
+    v.y = (nib & 2u) ? values[rk] : 0.0f;
+    rk += (nib >> 1) & 1u;
+    v.z = (nib & 4u) ? values[rk] : 0.0f;
+    rk += (nib >> 2) & 1u;
+    v.w = (nib & 8u) ? values[rk] : 0.0f;
+    x[j] = v;
+  }
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    if (j >= rows) break;
+    float* q = out + to[j];
+    if (left[j] >= 4) {
+      st_row4<ALIGNED>(q, x[j]);
+    } else {
+      if (left[j] > 0) q[0] = x[j].x;
+      if (left[j] > 1) q[1] = x[j].y;
+      if (left[j] > 2) q[2] = x[j].z;
     }
   }
 }
@@ -448,6 +510,7 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand4_kernel(
 // the kernel above.
 constexpr int kRowsStaged = 4;  // divides kRowsInFlight
 
+template <bool ALIGNED>
 __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand4_staged_kernel(
     const float* __restrict__ values, const uint32_t* __restrict__ mask, const int* __restrict__ begin,
     Geometry g, float* __restrict__ out)
@@ -528,7 +591,7 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand4_staged_kernel
       for (int j = 0; j < kRowsStaged; j++) {
         const int k = (r0 + h + j) * 256 + 4 * (int)lane;
         if (k + 4 <= len) {
-          st_stream4(reinterpret_cast<float4*>(q + k), x[j]);
+          st_row4<ALIGNED>(q + k, x[j]);
         } else {  // ragged end of the last chunk
           if (k < len) q[k] = x[j].x;
           if (k + 1 < len) q[k + 1] = x[j].y;
@@ -624,25 +687,11 @@ constexpr int kSAhead = kSSlots - 1;  // the loads run this many tiles ahead of 
 constexpr uint32_t kTileReady = 1u << 31;
 
 struct StreamGeometry {
-  int n, E, process, active;
-  int rows;    // rows that exist in the mask layout: process * E / 64 rounded up
+  int n, E, W, process, active;
+  int rows;    // rows that exist in the mask layout: process * W / 2 rounded up
   int tiles;   // ceil(rows / 256)
   int mask_words;
 };
-
-// Inclusive prefix sum over the 64 lanes of a wavefront with data-parallel-primitive
-// moves (row shifts inside rows of 16 lanes, then the row broadcasts): six additions, no
-// trip through the LDS crossbar that a shuffle takes.
-__device__ __forceinline__ unsigned wave_inclusive_scan(unsigned v)
-{
-  v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr:1
-  v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);  // row_shr:2
-  v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);  // row_shr:4
-  v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);  // row_shr:8
-  v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1, 3
-  v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2, 3
-  return v;
-}
 
 // The scanner: one wavefront turns counts into offsets, 256 tiles at a time, in tile order.
 __device__ void zvc_stream_scanner(uint32_t* ws, int tiles, int step, int* nnz, unsigned spin_limit)
@@ -733,7 +782,7 @@ __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
   uint32_t* offset = ws + 16 + g.tiles;
   const int iters = (g.tiles - w + G - 1) / G;  // >= 1: the grid has no more data workgroups than there are tiles
   // chunk index = half row / W by multiply and shift (exact while half rows * W < 2^40)
-  const unsigned long long w_magic = ((1ull << 40) + (unsigned)g.E / 32u - 1) / ((unsigned)g.E / 32u);
+  const unsigned long long w_magic = ((1ull << 40) + (unsigned)g.W - 1) / (unsigned)g.W;
 
   float x[kSSlots][kSRows];
   unsigned woff[kSSlots];   // non-zeros of the workgroup's tile in the wavefronts before mine
@@ -917,7 +966,7 @@ __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
         const unsigned before = wave_inclusive_scan(in_word) - in_word;
         const unsigned half = 2u * (unsigned)r0 + lane;
         const unsigned c = (unsigned)(((unsigned long long)half * w_magic) >> 40);
-        const bool starts = lane < 2u * kSRows && c * ((unsigned)g.E / 32u) == half && (int)c < g.active;
+        const bool starts = lane < 2u * kSRows && c * (unsigned)g.W == half && (int)c < g.active;
         out_begin_idx = starts ? (int)c : -1;
         out_begin_val = (int)(out_prefix - (out_prefix & 3u) + at0 + before);
         out_held = held;
@@ -943,16 +992,24 @@ __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
 }
 
 // ------------------------------------------------------------------ one kernel for small tensors
-// Up to 32 MiB the whole tensor fits in the registers of one grid: every workgroup (one per
+// Up to 64 MiB the whole tensor fits in the registers of one grid: every workgroup (one per
 // compute unit, sixteen wavefronts) loads its share once -- wavefront v of workgroup w owns R
-// consecutive rows of 64 elements --, counts it, writes its mask words, and publishes its count.
-// There is no scanner: every workgroup reads the counts of the workgroups before it itself, one
-// trip through memory instead of two, takes their sum as its offset, and stores its non-zeros
-// straight from the registers (at these sizes the values array stays in the memory-side cache,
-// where whole-line stores through an LDS stage gain nothing).  The last workgroup, which has
-// read every count but its own, writes the total.  Nobody waits for a workgroup with a higher
-// number than its own, so the grid makes progress however few of its workgroups the hardware
-// runs at a time (they are started in order).
+// consecutive rows of 64 elements of the mask layout --, counts it, writes its mask words, and
+// publishes its count.  There is no scanner: every workgroup reads the counts of the workgroups
+// before it itself, one trip through memory instead of two, takes their sum as its offset, and
+// stores its non-zeros straight from the registers (at these sizes the values array stays in the
+// memory-side cache, where whole-line stores through an LDS stage gain nothing).  The last
+// workgroup, which has read every count but its own, writes the total.  Nobody waits for a
+// workgroup with a higher number than its own, so the grid makes progress however few of its
+// workgroups the hardware runs at a time (they are started in order).
+//
+// RAGGED: chunks of any length.  A half row of the mask layout is then up to 32 elements of one
+// chunk, at any element of the tensor, and a lane works out place and existence of its element
+// row by row (about 12 instructions a row, behind the loads that are already on their way).
+// Measured, three kernels -> this one: 60 MB in 8192 chunks of 1838 elements 35 -> 25.3 us (30.5
+// with the counting pass's 16-byte loads at any element), 30 MB 17.3 -> 14.6, 7 MB 12.3 -> 8.4,
+// 1.6 MB in 16384 chunks 14.4 -> 8.2.  64 rows per wavefront instead of the three kernels
+// (33.6 to 67 MB): 63.7 MB 31 -> 25.
 //
 // The counts live in two arrays of 256 words at the end of the workspace, used in turns: run
 // k publishes into array k & 1 and every workgroup clears its word of the other one, which
@@ -960,12 +1017,15 @@ __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
 // size, so every word is cleared every time.  Failure works as in the pipeline kernel: a wait
 // that runs out raises the sticky flag, the offsets are kept inside the tensor, and the
 // wavefront that gave up writes -1 after the last workgroup has stepped the run counter.
+// The variants that took over shapes of the three kernels (RAGGED, 64 rows) must not fail where
+// those did not: a workgroup that finds the workspace unusable or whose wait runs out counts the
+// elements before its own by itself, which costs time and nothing else.
 constexpr int kQWaves = 16;
 constexpr int kQGroupsMax = 256;
 constexpr int kWsSmallRuns = 4;
 constexpr int kSmallWords = 2 * kQGroupsMax;  // taken from the end of the workspace's status words
 
-template <int R>
+template <int R, bool RAGGED>
 __global__ __launch_bounds__(64 * kQWaves) void zvc_small_kernel(
     const float* __restrict__ in, StreamGeometry g, uint32_t* __restrict__ ws, uint32_t* __restrict__ counts,
     int* __restrict__ begin, int* __restrict__ nnz, float* __restrict__ values, uint32_t* __restrict__ mask,
@@ -973,22 +1033,51 @@ __global__ __launch_bounds__(64 * kQWaves) void zvc_small_kernel(
 {
   constexpr int kHeld = (R + 31) / 32;  // registers of mask words: lane l of register h holds half row 64h + l
   __shared__ unsigned s_cnt[kQWaves];
-  __shared__ unsigned s_head[4];        // refused, parity, my offset, total
+  __shared__ unsigned s_head[5];        // refused, parity, my offset, total, count for myself
   const int G = (int)gridDim.x, w = (int)blockIdx.x;
   const unsigned lane = lane_id();
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int r0 = (w * kQWaves + wv) * R;  // my first row
 
-  // ---- my rows; rows that do not exist are read from the start of the tensor and ignored
-  const long long first = (long long)r0 * 64;
-  long long left_ll = (long long)g.n - first;
-  left_ll = left_ll < 0 ? 0 : (left_ll > R * 64 ? R * 64 : left_ll);
-  const int left = (int)left_ll;
-  const float* base = in + (left > 0 ? first : 0);
-  const unsigned last = (unsigned)max(left - 1, 0);
+  constexpr bool kCountsItself = RAGGED || R > 32;
+  const unsigned long long w_magic = ((1ull << 40) + (unsigned)g.W - 1) / (unsigned)g.W;
+
+  // ---- my rows; what does not exist is read from an element that does and ignored
   float x[R];
+  int left = 0;             // !RAGGED: elements that exist from my first row on
+  uint32_t exists[kHeld];   // RAGGED: bit j % 32 of register j / 32: my element of row j exists
+  if (RAGGED) {
+    const unsigned half = 2u * (unsigned)r0 + (lane >> 5);
+    const unsigned c = (unsigned)(((unsigned long long)half * w_magic) >> 40);
+    const unsigned row_elems = 32u * (unsigned)g.W, E = (unsigned)g.E;  // a chunk's elements in the mask layout, and in the tensor
+    unsigned e = 32u * (half - c * (unsigned)g.W) + (lane & 31u);       // place in the chunk
+    unsigned idx = E * c + e;
+    const unsigned chunks = 64u / row_elems, rest = 64u - chunks * row_elems;  // one row further
+    const unsigned step = chunks * E + rest, wrapped = step + E - row_elems, last = (unsigned)g.n - 1u;
 #pragma unroll
-  for (int j = 0; j < R; j++) x[j] = base[min(lane + 64u * j, last)];
+    for (int h = 0; h < kHeld; h++) exists[h] = 0;
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      x[j] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(in) + (size_t)(4u * min(idx, last)));
+      exists[j / 32] |= (e < E && idx <= last ? 1u : 0u) << (j % 32);
+      e += rest;
+      const bool wraps = e >= row_elems;
+      e -= wraps ? row_elems : 0u;
+      idx += wraps ? wrapped : step;
+      // row after row, and the bits in a register: not a pair of scalars per row
+      asm volatile("" : "+v"(exists[j / 32]), "+v"(e), "+v"(idx));
+    }
+  } else {
+    const long long first = (long long)r0 * 64;
+    long long left_ll = (long long)g.n - first;
+    left_ll = left_ll < 0 ? 0 : (left_ll > R * 64 ? R * 64 : left_ll);
+    left = (int)left_ll;
+    const float* base = in + (left > 0 ? first : 0);
+    const unsigned last = (unsigned)max(left - 1, 0);
+#pragma unroll
+    for (int j = 0; j < R; j++)
+      x[j] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + (size_t)(4u * min(lane + 64u * j, last)));
+  }
   if (threadIdx.x == 0) {  // together with the data: is the workspace usable, and which count array is this run's
     const uint32_t magic = ld_status(&ws[0]), flag = ld_status(&ws[kWsFlag]), runs = ld_status(&ws[kWsSmallRuns]);
     s_head[0] = (magic != kWsMagic || flag != 0u) ? 1u : 0u;
@@ -1002,10 +1091,16 @@ __global__ __launch_bounds__(64 * kQWaves) void zvc_small_kernel(
   for (int h = 0; h < kHeld; h++) held[h] = 0;
 #pragma unroll
   for (int j = 0; j < R; j++) {
-    const unsigned long long m = __ballot(x[j] != 0.0f && (int)lane < left - 64 * j);
+    // an element that does not exist is a zero from here on
+    if (RAGGED) x[j] = __uint_as_float(__float_as_uint(x[j]) & (0u - ((exists[j / 32] >> (j % 32)) & 1u)));
+    else x[j] = (int)lane < left - 64 * j ? x[j] : 0.0f;
+    asm volatile("" : "+v"(x[j]));
+    const unsigned long long m = __ballot(x[j] != 0.0f);
     cnt += popc64(m);
-    if (lane == 2u * (j % 32)) held[j / 32] = (uint32_t)m;
-    if (lane == 2u * (j % 32) + 1u) held[j / 32] = (uint32_t)(m >> 32);
+    unsigned me = lane;
+    asm volatile("" : "+v"(me));  // compared afresh for every row: kept, the conditions would not last in scalars either
+    if (me == 2u * (j % 32)) held[j / 32] = (uint32_t)m;
+    if (me == 2u * (j % 32) + 1u) held[j / 32] = (uint32_t)(m >> 32);
   }
 #pragma unroll
   for (int h = 0; h < kHeld; h++) {
@@ -1014,7 +1109,8 @@ __global__ __launch_bounds__(64 * kQWaves) void zvc_small_kernel(
   }
   if (lane == 0) s_cnt[wv] = cnt;
   __syncthreads();
-  if (s_head[0] != 0u) {  // refused: nothing is published, nothing written but the result
+  const bool refused = s_head[0] != 0u;
+  if (!kCountsItself && refused) {  // nothing is published, nothing written but the result
     if (w == 0 && threadIdx.x == 0) *nnz = -1;
     return;
   }
@@ -1024,7 +1120,7 @@ __global__ __launch_bounds__(64 * kQWaves) void zvc_small_kernel(
   const unsigned wave_incl = wave_inclusive_scan(wave_cnt);
   const unsigned group_total = (unsigned)__builtin_amdgcn_readlane((int)wave_incl, kQWaves - 1);
   const unsigned woff = (unsigned)__builtin_amdgcn_readlane((int)(wave_incl - wave_cnt), wv);
-  if (threadIdx.x == 0) {
+  if (!refused && threadIdx.x == 0) {
     st_status(&counts[((runs0 & 1u) ^ 1u) * kQGroupsMax + w], 0u);
     if (!(skip_first && w == 0)) st_status(&mine_arr[w], kTileReady | group_total);
   }
@@ -1042,9 +1138,9 @@ __global__ __launch_bounds__(64 * kQWaves) void zvc_small_kernel(
         v[r] = k < w ? ld_status(&mine_arr[k]) : kTileReady;
         missing |= (v[r] & kTileReady) == 0u;
       }
-      if (__ballot(missing) == 0ull) break;
-      if (++spins > spin_limit) {
-        if (lane == 0) atomicOr(&ws[kWsFlag], 1u);
+      if (__ballot(missing) == 0ull && !refused) break;
+      if (refused || ++spins > spin_limit) {
+        if (!kCountsItself && lane == 0) atomicOr(&ws[kWsFlag], 1u);
         gave_up = true;
         break;
       }
@@ -1067,27 +1163,48 @@ __global__ __launch_bounds__(64 * kQWaves) void zvc_small_kernel(
       // whatever the words held: what this workgroup writes stays inside the tensor
       s_head[2] = min(before_me, (unsigned)g.n - group_total);
       s_head[3] = total;
+      s_head[4] = gave_up ? 1u : 0u;
     }
   }
   __syncthreads();
+  if (kCountsItself && s_head[4] != 0u) {
+    const unsigned half = 2u * (unsigned)(w * kQWaves * R);  // my workgroup's first half row
+    const unsigned c = (unsigned)(((unsigned long long)half * w_magic) >> 40);
+    const unsigned long long from = (unsigned long long)(unsigned)g.E * c + min(32u * (half - c * (unsigned)g.W), (unsigned)g.E);
+    const unsigned end = (unsigned)(from < (unsigned long long)g.n ? from : (unsigned long long)g.n);
+    int before = 0;
+    for (unsigned i = threadIdx.x; i < end; i += 64 * kQWaves) before += in[i] != 0.0f;
+    before = wave_sum(before);
+    if (lane == 0) s_cnt[wv] = (unsigned)before;  // woff and group_total have been taken out of it
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      unsigned sum = 0;
+      for (int v = 0; v < kQWaves; v++) sum += s_cnt[v];
+      s_head[2] = sum;
+      s_head[3] = sum + group_total;
+    }
+    __syncthreads();
+    gave_up = false;
+  }
   uint32_t flag_late = 0;
-  if (w == G - 1 && threadIdx.x == 0) flag_late = ld_status(&ws[kWsFlag]);  // asked for now, looked at when the rows are out
+  if (!kCountsItself && w == G - 1 && threadIdx.x == 0) flag_late = ld_status(&ws[kWsFlag]);  // asked for now, looked at when the rows are out
 
   // ---- my non-zeros, row by row, straight from the lanes that hold them; chunk starts on the way
   unsigned at = s_head[2] + woff;
-  const unsigned long long w_magic = ((1ull << 40) + (unsigned)g.E / 32u - 1) / ((unsigned)g.E / 32u);
+#pragma unroll
+  for (int j = 0; j < R; j++) asm volatile("" : "+v"(x[j]));  // the ballots below are made again: two scalars per row would not last
 #pragma unroll
   for (int h = 0; h < kHeld; h++) {
     const unsigned in_word = (unsigned)__popc(held[h]);
     const unsigned before = wave_inclusive_scan(in_word) - in_word;
     const unsigned half = 2u * ((unsigned)r0 + 32u * h) + lane;
     const unsigned c = (unsigned)(((unsigned long long)half * w_magic) >> 40);
-    if ((int)lane < 2 * (R - 32 * h) && c * ((unsigned)g.E / 32u) == half && (int)c < g.active)
+    if ((int)lane < 2 * (R - 32 * h) && c * (unsigned)g.W == half && (int)c < g.active)
       begin[c] = (int)(at + before);
 #pragma unroll
     for (int j = 32 * h; j < R && j < 32 * h + 32; j++) {
       const float v = x[j];
-      const bool nz = v != 0.0f && (int)lane < left - 64 * j;
+      const bool nz = v != 0.0f;
       const unsigned long long m = __ballot(nz);
       if (nz) values[at + rank_below(m)] = v;
       at += popc64(m);
@@ -1098,7 +1215,7 @@ __global__ __launch_bounds__(64 * kQWaves) void zvc_small_kernel(
   if (w == G - 1 && threadIdx.x == 0) {
     *nnz = (gave_up || flag_late != 0u) ? -1 : (int)s_head[3];
     __threadfence();
-    __hip_atomic_fetch_add(&ws[kWsSmallRuns], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!refused) __hip_atomic_fetch_add(&ws[kWsSmallRuns], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   } else if (gave_up && w != G - 1) {  // (wavefront 0 of another workgroup) after the last workgroup has spoken
     for (unsigned spins = 0; ld_status(&ws[kWsSmallRuns]) == runs0 && spins < spin_limit; spins++)
       __builtin_amdgcn_s_sleep(2);
@@ -1233,17 +1350,27 @@ extern "C" int cswap_zvc_expand(const float* d_values, const uint32_t* d_mask, c
   int rc = make_geometry(g, n, process);
   if (rc) return rc;
   unsigned grid = (g.active + kWavesPerGroup - 1) / kWavesPerGroup;
-  const bool quads = g.E % 4 == 0 && (reinterpret_cast<uintptr_t>(d_out) & 15u) == 0;
-  if (quads && (reinterpret_cast<uintptr_t>(d_values) & 15u) == 0 &&
-      4ull * (unsigned long long)n >= g_staged_compact_bytes)
-    hipLaunchKernelGGL(zvc_expand4_staged_kernel, dim3(grid), dim3(64 * kWavesPerGroup), 0, (hipStream_t)stream,
-                       d_values, d_mask, d_begin, g, d_out);
-  else if (quads)
-    hipLaunchKernelGGL(zvc_expand4_kernel, dim3(grid), dim3(64 * kWavesPerGroup), 0, (hipStream_t)stream,
-                       d_values, d_mask, d_begin, g, d_out);
-  else
-    hipLaunchKernelGGL(zvc_expand_kernel, dim3(grid), dim3(64 * kWavesPerGroup), 0, (hipStream_t)stream,
-                       d_values, d_mask, d_begin, g, d_out);
+  const bool aligned = g.E % 4 == 0 && (reinterpret_cast<uintptr_t>(d_out) & 15u) == 0;
+  const bool staged = (reinterpret_cast<uintptr_t>(d_values) & 15u) == 0 &&
+                      4ull * (unsigned long long)n >= g_staged_compact_bytes;
+#define CSWAP_EXPAND(KERNEL_)                                                                                     \
+  hipLaunchKernelGGL(KERNEL_, dim3(grid), dim3(64 * kWavesPerGroup), 0, (hipStream_t)stream, d_values, d_mask, d_begin, \
+                     g, d_out)
+  if (!staged && g.W <= kPackedWords && g.active > kPackedFrom) {
+    const int per = 64 / g.W;
+    const unsigned waves = (unsigned)((g.active + per - 1) / per);
+    const dim3 packed_grid((waves + kWavesPerGroup - 1) / kWavesPerGroup);
+    if (aligned)
+      hipLaunchKernelGGL(zvc_expand_packed_kernel<true>, packed_grid, dim3(64 * kWavesPerGroup), 0, (hipStream_t)stream,
+                         d_values, d_mask, d_begin, g, per, d_out);
+    else
+      hipLaunchKernelGGL(zvc_expand_packed_kernel<false>, packed_grid, dim3(64 * kWavesPerGroup), 0, (hipStream_t)stream,
+                         d_values, d_mask, d_begin, g, per, d_out);
+  } else if (staged && aligned) CSWAP_EXPAND(zvc_expand4_staged_kernel<true>);
+  else if (staged) CSWAP_EXPAND(zvc_expand4_staged_kernel<false>);
+  else if (aligned) CSWAP_EXPAND(zvc_expand4_kernel<true>);
+  else CSWAP_EXPAND(zvc_expand4_kernel<false>);
+#undef CSWAP_EXPAND
   return check_launch();
 }
 
@@ -1315,7 +1442,7 @@ extern "C" int cswap_test_zvc_stream_groups(int tiles, int compute_units) { retu
 // whether the single pass takes a tensor of this shape; fills its geometry
 static bool single_pass_shape(const Geometry& g, int n, int process, StreamGeometry& sg)
 {
-  sg.n = n; sg.E = g.E; sg.process = process; sg.active = g.active;
+  sg.n = n; sg.E = g.E; sg.W = g.W; sg.process = process; sg.active = g.active;
   const long long mask_words = (long long)g.W * process;
   sg.mask_words = (int)mask_words;
   sg.rows = (int)((mask_words + 1) / 2);
@@ -1329,9 +1456,13 @@ static bool single_pass_shape(const Geometry& g, int n, int process, StreamGeome
 // Whether the one-kernel form for small tensors takes this shape (a tensor below the size from
 // which the pipeline kernel runs, whole half rows per chunk, the whole tensor in the registers
 // of one grid); fills the geometry, the grid and the rows per wavefront.
-static bool small_pass_shape(const Geometry& g, int n, int process, StreamGeometry& sg, int* groups, int* rows_per_wave)
+// `any`: also the shapes of the form's variants that cannot fail (zvc_small_kernel: kCountsItself),
+// chunks of any length and up to 64 rows per wavefront; a caller that has to know beforehand
+// whether the workspace decides about success (cswap_zvc_takes_single_pass) leaves those out.
+static bool small_pass_shape(const Geometry& g, int n, int process, StreamGeometry& sg, int* groups, int* rows_per_wave,
+                             bool any)
 {
-  sg.n = n; sg.E = g.E; sg.process = process; sg.active = g.active;
+  sg.n = n; sg.E = g.E; sg.W = g.W; sg.process = process; sg.active = g.active;
   const long long mask_words = (long long)g.W * process;
   sg.mask_words = (int)mask_words;
   sg.rows = (int)((mask_words + 1) / 2);
@@ -1339,11 +1470,12 @@ static bool small_pass_shape(const Geometry& g, int n, int process, StreamGeomet
   const int cus = device_compute_units();
   const int G = cus < kQGroupsMax ? cus : kQGroupsMax;
   const unsigned long long single_from = g_single_pass_bytes.load();
-  if (G < 1 || g.E % 32 != 0 || single_from == ~0ull || 4ull * (unsigned long long)n >= single_from) return false;
+  if (G < 1 || (!any && g.E % 32 != 0) || mask_words >= (1ll << 31) - 64 || single_from == ~0ull || 4ull * (unsigned long long)n >= single_from) return false;
   // every row of the mask layout has an owner, also the rows of chunks that hold no data (their words are zero)
-  int R = 8;  // 8, 16 or 32 rows per wavefront (64 would need more registers than a wavefront of sixteen has)
-  while (R <= 32 && (long long)G * kQWaves * R < (long long)sg.rows) R *= 2;
-  if (R > 32) return false;
+  const int most = any ? 64 : 32;
+  int R = 8;
+  while (R <= most && (long long)G * kQWaves * R < (long long)sg.rows) R *= 2;
+  if (R > most) return false;
   *groups = G;
   *rows_per_wave = R;
   return true;
@@ -1356,7 +1488,7 @@ extern "C" int cswap_zvc_takes_single_pass(int n, int process)
   int groups, rows;
   if (make_geometry(g, n, process) != CSWAP_OK) return 0;
   if (single_pass_shape(g, n, process, sg)) return 1;
-  return small_pass_shape(g, n, process, sg, &groups, &rows) ? 2 : 0;
+  return small_pass_shape(g, n, process, sg, &groups, &rows, false) ? 2 : 0;
 }
 
 extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, void* d_ws, int* d_begin,
@@ -1372,14 +1504,16 @@ extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, v
   // anything the single pass does not take, or an output that is not 16-byte aligned, runs the three kernels
   const bool single_pass = single_pass_shape(g, n, process, sg) && (reinterpret_cast<uintptr_t>(d_values) & 15u) == 0;
   int groups = 0, rows = 0;
-  if (!single_pass && small_pass_shape(g, n, process, sg, &groups, &rows)) {
+  if (!single_pass && small_pass_shape(g, n, process, sg, &groups, &rows, true)) {
     uint32_t* counts = ws + 16 + status_words(process) - kSmallWords;
-#define CSWAP_SMALL(R)                                                                                              \
-  hipLaunchKernelGGL(zvc_small_kernel<R>, dim3(groups), dim3(64 * kQWaves), 0, (hipStream_t)stream, d_in, sg, ws, \
-                     counts, d_begin, d_nnz, d_values, d_mask, g_spin_limit.load(), g_skip_first.load())
-    if (rows == 8) CSWAP_SMALL(8);
-    else if (rows == 16) CSWAP_SMALL(16);
-    else CSWAP_SMALL(32);
+#define CSWAP_SMALL(R, RAGGED)                                                                                     \
+  hipLaunchKernelGGL((zvc_small_kernel<R, RAGGED>), dim3(groups), dim3(64 * kQWaves), 0, (hipStream_t)stream, d_in, \
+                     sg, ws, counts, d_begin, d_nnz, d_values, d_mask, g_spin_limit.load(), g_skip_first.load())
+    const bool ragged = g.E % 32 != 0;
+    if (rows == 8) { if (ragged) CSWAP_SMALL(8, true); else CSWAP_SMALL(8, false); }
+    else if (rows == 16) { if (ragged) CSWAP_SMALL(16, true); else CSWAP_SMALL(16, false); }
+    else if (rows == 32) { if (ragged) CSWAP_SMALL(32, true); else CSWAP_SMALL(32, false); }
+    else { if (ragged) CSWAP_SMALL(64, true); else CSWAP_SMALL(64, false); }
 #undef CSWAP_SMALL
     return check_launch();
   }

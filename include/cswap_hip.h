@@ -179,16 +179,16 @@ int cswap_zvc_compress(const float* d_in, int n, int process, int* d_begin, int*
  * scanner workgroup has turned the published tile counts into offsets, and then
  * write mask, offsets and packed values, so HBM traffic is the algorithmic
  * 4 + 1/8 + 4*density bytes per element.  Smaller tensors than
- * cswap_zvc_set_single_pass_bytes says (64 MiB) do not fill that pipeline; of those,
- * tensors whose mask layout has at most 131072 rows of 64 elements (32 MiB) run
+ * cswap_zvc_set_single_pass_bytes says (64 MiB) do not fill that pipeline; they run
  * another one-kernel form -- the whole tensor in the registers of one grid, every
- * workgroup reads the counts of the workgroups before it -- and the rest the three kernels.  d_ws is a
+ * workgroup reads the counts of the workgroups before it -- while their mask layout
+ * has at most 262144 rows of 64 elements (64 MiB).  d_ws is a
  * workspace of cswap_zvc_workspace_bytes(process) bytes (at least 256 KiB) that
  * cswap_zvc_workspace_clear has prepared once, after it was allocated; every call
  * that succeeds leaves it ready for the next one (the kernel clears each status
  * word as it consumes it, so no launch is spent on clearing); calls that share a
- * workspace must not overlap.  Shapes the one-kernel forms do not take -- a chunk
- * length that is not a multiple of 32, for the pipeline d_values not 16-byte
+ * workspace must not overlap.  Shapes the one-kernel forms do not take -- for the
+ * pipeline a chunk length that is not a multiple of 32, d_values not 16-byte
  * aligned or more than 32512 tiles of 12288 elements -- run the three kernels instead.  The workgroups
  * wait for each other's counts; that wait is bounded, and if it ever runs out (for
  * example because the pipeline kernel, whose 256 workgroups all have to run at the
@@ -197,7 +197,9 @@ int cswap_zvc_compress(const float* d_in, int n, int process, int* d_begin, int*
  * negative count as failure (the return value cannot tell, the call does not
  * synchronise).  A workspace that was never prepared is reported the same way, and
  * so is every later call on a workspace after a failure, until
- * cswap_zvc_workspace_clear has been called on it again. */
+ * cswap_zvc_workspace_clear has been called on it again.  Shapes for which
+ * cswap_zvc_takes_single_pass is 0 never fail: whatever the workspace holds, their
+ * result is right. */
 size_t cswap_zvc_workspace_bytes(int process);
 int cswap_zvc_compress_fused(const float* d_in, int n, int process, void* d_ws, int* d_begin,
                              int* d_nnz, float* d_values, uint32_t* d_mask, cswap_stream_t stream);
@@ -209,8 +211,11 @@ int cswap_zvc_compress_fused(const float* d_in, int n, int process, void* d_ws, 
  * `process` is ignored). */
 int cswap_zvc_workspace_clear(void* d_ws, int process, cswap_stream_t stream);
 /* What cswap_zvc_compress_fused would run for this shape (given a 16-byte aligned
- * d_values): 1 the pipeline kernel, 2 the one-kernel form for small tensors, 0 the
- * three kernels.  Host only. */
+ * d_values): 1 the pipeline kernel, 2 the one-kernel form for small tensors (chunk
+ * lengths that are multiples of 32, at most 131072 rows of 64 elements, 32 MiB), 0 a
+ * form that does not need the workspace to succeed: the three kernels, or the small
+ * form of tensors of other chunk lengths and of up to 262144 rows, whose workgroups
+ * count for themselves where the workspace fails them.  Host only. */
 int cswap_zvc_takes_single_pass(int n, int process);
 /* No counterpart in the reference: the tensor size in bytes from which
  * cswap_zvc_compress_fused runs the pipeline kernel (default 64 MiB; 0 = whenever

@@ -466,3 +466,66 @@ def test_staged_threshold_is_reported_and_restored(torch_cuda):
     default = L.cswap_zvc_set_staged_compact_bytes(12345)
     assert default == 192 << 20
     assert L.cswap_zvc_set_staged_compact_bytes(default) == 12345
+
+
+RAGGED = [(33, 1), (31 * 5, 5), (7, 7), (63 * 64, 64), (1000, 1024), (16384 * 16 - 5, 16384), (100_003, 16384), (1024 * 33, 1024),
+          (P * 90 + 7, P), (1 << 20, 1023), (256 * 16 * 8 * 64 + 1, 4096), (P * 511 - 3, P), (P * 700 + 11, P),
+          (256 * 16 * 64 * 64 - 8192, 8192), (P * 513, P), (P * 1024 - 32, P)]
+
+
+@pytest.mark.parametrize("n,process", RAGGED)
+@pytest.mark.parametrize("workspace", ["prepared", "never_prepared", "wait_runs_out"])
+def test_one_kernel_form_of_any_chunk_length(torch_cuda, n, process, workspace):
+    """Chunks that are no whole half rows, and tensors of up to 64 rows per wavefront, in the
+    one-kernel form: chunk ends inside a row, chunks shorter than a row, several of them in a
+    row, idle chunks.  These shapes do not depend on the workspace's state: a workgroup that
+    gets no counts from it counts for itself."""
+    import oracle
+    from cswap_amd import api
+    from cswap_amd._lib import check, lib
+
+    torch = torch_cuda
+    L = lib()
+    before = L.cswap_zvc_set_single_pass_bytes(64 << 20)
+    try:
+        assert L.cswap_zvc_takes_single_pass(n, process) in (0, 2)
+        rng = np.random.default_rng(n % 9973 + process)
+        x = (rng.standard_normal(n, dtype=np.float32) * (rng.random(n, dtype=np.float32) < 0.5)).astype(np.float32)
+        if n > 16:
+            x[[0, 3, n - 1]] = [np.nan, -0.0, 1e-45]
+        E, W, active = oracle.zvc_geometry(n, process)
+        may_fail = L.cswap_zvc_takes_single_pass(n, process) == 2
+        ws = api.zvc_workspace(process)
+        if workspace == "never_prepared":
+            ws = torch.full_like(ws, 0xa5)
+        t = torch.from_numpy(x).cuda()
+        for shift in (0, 1):
+            values = torch.empty(n + 1, device="cuda")[shift:]
+            mask = torch.full((W * process,), -1, dtype=torch.int32, device="cuda")
+            begin = torch.full((process,), -5, dtype=torch.int32, device="cuda")
+            nnz = torch.zeros(1, dtype=torch.int32, device="cuda")
+            out = torch.full((n + 1,), 3.0, device="cuda")[shift:]
+            if workspace == "wait_runs_out":
+                L.cswap_zvc_debug_set_lookback(4, 1)
+            try:
+                check(L.cswap_zvc_compress_fused(t.data_ptr(), n, process, ws.data_ptr(), begin.data_ptr(), nnz.data_ptr(),
+                                                 values.data_ptr(), mask.data_ptr(), None), "fused")
+                torch.cuda.synchronize()
+            finally:
+                L.cswap_zvc_debug_set_lookback(0, 0)
+            if may_fail and workspace != "prepared":
+                assert int(nnz.item()) == -1
+                return
+            ov, om, ob, on = oracle.zvc_compress(x, process)
+            assert int(nnz.item()) == on
+            assert np.array_equal(values[:on].cpu().numpy().view(np.uint32), ov[:on].view(np.uint32))
+            assert np.array_equal(mask.cpu().numpy().view(np.uint32), om)
+            assert np.array_equal(begin[:active].cpu().numpy(), ob[:active])
+            check(L.cswap_zvc_expand(values.data_ptr(), mask.data_ptr(), begin.data_ptr(), n, process, out.data_ptr(), None),
+                  "expand")
+            torch.cuda.synchronize()
+            want = x.copy()
+            want[x == 0] = 0.0
+            assert np.array_equal(out[:n].cpu().numpy().view(np.uint32), want.view(np.uint32))
+    finally:
+        L.cswap_zvc_set_single_pass_bytes(before)

@@ -301,8 +301,8 @@ CSWAP_HD uint32_t vector_const()
 }
 
 // VM: the stage's mask in a vector register (one more register while the stage runs)
-template <int J, int R0, int R1, int NB = kPlain, bool VM = false>
-CSWAP_HD void tr_stage(uint32_t (&a)[32])
+template <int J, int R0, int R1, int NB = kPlain, bool VM = false, int ROWS = 32>
+CSWAP_HD void tr_stage(uint32_t (&a)[ROWS])
 {
   static_assert(NB == kPlain || J == 1, "only the stage that pairs neighbouring planes can complement them");
   constexpr uint32_t mc = J == 16 ? 0x0000ffffu : J == 8 ? 0x00ff00ffu : J == 4 ? 0x0f0f0f0fu
@@ -949,6 +949,78 @@ CSWAP_HD void pair_encode_half(const float (&p)[16], const float (&q)[16], bool 
     pair_code16<H>(x, enc, acc, false);
     ex.done();
   }
+}
+
+// ---------------------------------------------------------------- one block, four lanes
+// The bit side of the quad form (zfp_kernels.hip), where lane q of four holds the coefficients
+// 16q .. 16q+15 of a block in coding order.  Planes of 16 coefficients, two to a word: word j
+// has plane P + j in its low half and plane P + 8 + j in its high half (P = 16 or 0).  A byte
+// permute brings four 8x8 bit tiles into the bytes of eight words (it is the stages 16 and 8 of
+// the butterfly at once), three stages transpose all four of them.
+CSWAP_HD uint32_t byte_perm(uint32_t hi, uint32_t lo, uint32_t sel)  // byte k of the result: byte sel.k of {hi, lo}
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_perm(hi, lo, sel);
+#else
+  const uint64_t v = ((uint64_t)hi << 32) | lo;
+  uint32_t r = 0;
+  for (int k = 0; k < 4; k++) r |= (uint32_t)((v >> (8 * ((sel >> (8 * k)) & 7u))) & 0xffu) << (8 * k);
+  return r;
+#endif
+}
+
+// a: coefficients with the negabinary constant added; TOP: planes 31..16, else 15..0
+template <bool TOP>
+CSWAP_HD void quad_planes(const uint32_t (&a)[16], uint32_t (&t)[8])
+{
+#pragma unroll
+  for (int i = 0; i < 8; i++) t[i] = byte_perm(a[i + 8], a[i], TOP ? 0x07030602u : 0x05010400u);
+  tr_stage<4, 0, 8>(t);
+  tr_stage<2, 0, 8>(t);
+  tr_stage<1, 0, 8, kNotOut>(t);
+}
+
+// the way back: t (top) and l (low planes) to coefficients that still carry the negabinary constant
+CSWAP_HD void quad_coefficients(uint32_t (&t)[8], const uint32_t (&l)[8], uint32_t (&a)[16])
+{
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    a[i] = byte_perm(t[i], l[i], 0x06040200u);
+    a[i + 8] = byte_perm(t[i], l[i], 0x07050301u);
+  }
+}
+CSWAP_HD void quad_untranspose(uint32_t (&t)[8])
+{
+  tr_stage<1, 0, 8, kNotIn>(t);
+  tr_stage<2, 0, 8>(t);
+  tr_stage<4, 0, 8>(t);
+}
+
+// What a plane of the block costs, in closed form (BlockEncoder::skip_plane): before / upto are
+// the OR of the planes above it, without and with it.
+CSWAP_HD unsigned known_after(uint64_t upto) { return upto ? 64u - (unsigned)__builtin_clzll(upto) : 0u; }
+CSWAP_HD unsigned plane_bits(uint64_t x, unsigned n, unsigned n_new)
+{
+  const uint64_t rest = n < 64 ? x >> n : 0;
+  return n_new + (unsigned)__builtin_popcountll(rest) + (n_new < 64 ? 1u : (n < 64 ? ~0u : 0u));
+}
+
+// Byte offsets in an array of 64 words by which the four lanes change between the order of the
+// coefficients in space and in coding: to_seq[y] has, byte x + 4z, the place in coding order of
+// (x, y, z); to_xyz[q] has, byte j, the place x + 4y + 16z of the coefficient 16q + j.
+struct QuadOrder {
+  uint32_t to_seq[4][4], to_xyz[4][4];
+};
+constexpr QuadOrder make_quad_order()
+{
+  QuadOrder o = {};
+  for (int q = 0; q < 4; q++)
+    for (int i = 0; i < 16; i++) {
+      const int x = i & 3, z = i >> 2;
+      o.to_seq[q][i >> 2] |= (uint32_t)(4 * kSeqOf.v[x + 4 * q + 16 * z]) << (8 * (i & 3));
+      o.to_xyz[q][i >> 2] |= (uint32_t)(4 * kPerm3.v[16 * q + i]) << (8 * (i & 3));
+    }
+  return o;
 }
 
 // ---------------------------------------------------------------- decoder

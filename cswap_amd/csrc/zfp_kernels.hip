@@ -709,6 +709,335 @@ __global__ __launch_bounds__(128) void zfp_decode3_f32_pair_kernel(const uint64_
   else pair_decode_body<1>(fd, maxbits, lds, lane, first, out);
 }
 
+// ------------------------------------------------------------- the quad form: four lanes per block
+// For the smallest fields.  A wavefront codes 16 blocks: lane 4 * block + q holds z-slice q, so
+// a lane's share of every phase but the coder is a quarter of a block's, and a field keeps four
+// times as many wavefronts in flight as with one lane per block.  Through LDS the lanes of a
+// block turn its values (along z the lines y = q), put the coefficients in coding order and
+// hand out the bit planes.
+//   encoder  lane q codes every fourth plane, q first: where a plane starts is a prefix over the
+//            planes before it (plane_bits), a quad of lanes at a time with data-parallel-primitive
+//            moves, so four planes are coded at once and nobody steps through a plane twice
+//   decoder  where a plane starts is only known when the one before is decoded: all four lanes
+//            decode every plane, each keeps its quarter, and the exchange that the encoder needs falls away
+// A lane's rows are loaded by the padding rule's addresses, so the form takes every field of
+// floats at a whole-word rate.  What bounds it is the chain left in a wavefront: the encoder's
+// four rounds of planes, the decoder's 13 to 16 planes one after the other.  4.2 MB at 8 bits
+// per value: encode 8.4 (pair form) -> 6.7 us, decode 12.8 -> 10.6; the rule is at quad_pays.
+constexpr unsigned kQuadBlocks = 16;   // blocks of a wavefront
+constexpr unsigned kQuadStride = 68;   // dwords of a block's exchange area: 64 and four to spread the banks
+__host__ __device__ inline unsigned quad_region_dwords(unsigned slot) { return (kQuadBlocks * slot / 32 + 4u + 3u) & ~3u; }
+__host__ __device__ inline unsigned quad_lds_dwords(unsigned slot) { return quad_region_dwords(slot) + kQuadBlocks * kQuadStride; }
+
+__constant__ const QuadOrder kQuadOrder = make_quad_order();
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t quad_move(uint32_t v)  // value of the quad's lane that CTRL names for mine
+{
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false);
+}
+constexpr int kQuadXor1 = 0xb1, kQuadXor2 = 0x4e, kQuadDown1 = 0x90, kQuadDown2 = 0x44, kQuadLast = 0xff;
+template <int CTRL>
+__device__ __forceinline__ uint64_t quad_move64(uint64_t v)
+{
+  return ((uint64_t)quad_move<CTRL>((uint32_t)(v >> 32)) << 32) | quad_move<CTRL>((uint32_t)v);
+}
+
+// index inside a block of n elements along an axis that the padding rule (pad4) puts at i
+__device__ __forceinline__ uint32_t padded_index(uint32_t n, uint32_t i)
+{
+  return i < n ? i : (n == 2 && i == 2 ? 1u : 0u);
+}
+
+// the four rows of z-slice q of block b
+__device__ __forceinline__ void quad_load(const float* __restrict__ in, const Field3& fd, uint32_t b, uint32_t q,
+                                          float (&f)[16])
+{
+  uint32_t x0, y0, z0;
+  block_origin(fd, b, x0, y0, z0);
+  const float* p = in + ((long long)x0 * fd.sx + (long long)y0 * fd.sy + (long long)z0 * fd.sz);
+  if (fd.full) {
+#pragma unroll
+    for (int y = 0; y < 4; y++) {
+      const row_f4 v = *reinterpret_cast<const row_f4*>(p + ((long long)q * fd.sz + y * fd.sy));
+      f[4 * y] = v.x; f[4 * y + 1] = v.y; f[4 * y + 2] = v.z; f[4 * y + 3] = v.w;
+    }
+    return;
+  }
+  const uint32_t bx = min(4u, fd.nx - x0), by = min(4u, fd.ny - y0), bz = min(4u, fd.nz - z0);
+  const bool leaves = bx < 4 && y0 + by == fd.ny && z0 + bz == fd.nz;  // as in load_block
+  p += (long long)padded_index(bz, q) * fd.sz;
+  if (fd.rows4 && !leaves) {
+#pragma unroll
+    for (int y = 0; y < 4; y++) {
+      const row_f4 v = *reinterpret_cast<const row_f4*>(p + (long long)padded_index(by, y) * fd.sy);
+      f[4 * y] = v.x;
+      f[4 * y + 1] = bx >= 2 ? v.y : v.x;
+      f[4 * y + 2] = bx >= 3 ? v.z : f[4 * y + 1];
+      f[4 * y + 3] = bx >= 4 ? v.w : v.x;
+    }
+  } else {
+#pragma unroll
+    for (int y = 0; y < 4; y++)
+#pragma unroll
+      for (int x = 0; x < 4; x++)
+        f[4 * y + x] = p[(long long)padded_index(bx, x) * fd.sx + (long long)padded_index(by, y) * fd.sy];
+  }
+}
+
+// One round of the coder: four planes, lane q's is x; acc and base (the OR of the planes so far
+// and the bit position behind them) are the same in the four lanes.
+__device__ __forceinline__ void quad_round(BlockEncoder<LdsBits, false>& enc, uint64_t x, uint32_t q, uint64_t& acc,
+                                           unsigned& base)
+{
+  const uint32_t from1 = q >= 1 ? ~0u : 0u, from2 = q >= 2 ? ~0u : 0u;
+  const uint64_t from1w = ((uint64_t)from1 << 32) | from1, from2w = ((uint64_t)from2 << 32) | from2;
+  uint64_t all = x | (quad_move64<kQuadDown1>(x) & from1w);
+  all |= quad_move64<kQuadDown2>(all) & from2w;  // planes of the lanes up to mine
+  const uint64_t before = acc | (quad_move64<kQuadDown1>(all) & from1w);
+  const unsigned n = known_after(before);
+  const unsigned bits = plane_bits(x, n, known_after(acc | all));
+  unsigned sum = bits + (quad_move<kQuadDown1>(bits) & from1);
+  sum += quad_move<kQuadDown2>(sum) & from2;
+  enc.pos = base + sum - bits;
+  enc.n = n;
+  acc |= quad_move64<kQuadLast>(all);
+  base += quad_move<kQuadLast>(sum);
+  if (CSWAP_ANY(x != 0 || n != 0)) enc.plane(x);  // an empty plane of a block without known coefficients is one zero bit
+}
+
+// 16 planes: t as quad_planes leaves it, exchange: the block's exchange area
+__device__ __forceinline__ void quad_code16(const uint32_t (&t)[8], uint32_t* exchange, uint32_t q,
+                                            BlockEncoder<LdsBits, false>& enc, uint64_t& acc, unsigned& base)
+{
+#pragma unroll
+  for (int j = 0; j < 8; j++) exchange[4 * j + q] = t[j];
+  __syncthreads();
+  const uint4 u = *reinterpret_cast<const uint4*>(exchange + 4 * (7 - q));
+  const uint4 v = *reinterpret_cast<const uint4*>(exchange + 4 * (3 - q));
+  constexpr uint32_t kHigh = 0x07060302u, kLow = 0x05040100u;  // the high / low halves of two words
+  const uint64_t r0 = ((uint64_t)byte_perm(u.w, u.z, kHigh) << 32) | byte_perm(u.y, u.x, kHigh);
+  const uint64_t r1 = ((uint64_t)byte_perm(v.w, v.z, kHigh) << 32) | byte_perm(v.y, v.x, kHigh);
+  const uint64_t r2 = ((uint64_t)byte_perm(u.w, u.z, kLow) << 32) | byte_perm(u.y, u.x, kLow);
+  const uint64_t r3 = ((uint64_t)byte_perm(v.w, v.z, kLow) << 32) | byte_perm(v.y, v.x, kLow);
+  quad_round(enc, r0, q, acc, base);
+  if (CSWAP_ANY(base < enc.limit)) quad_round(enc, r1, q, acc, base);
+  if (CSWAP_ANY(base < enc.limit)) quad_round(enc, r2, q, acc, base);
+  if (CSWAP_ANY(base < enc.limit)) quad_round(enc, r3, q, acc, base);
+}
+
+__global__ __launch_bounds__(64) void zfp_encode3_f32_quad_kernel(const float* __restrict__ in, Field3 fd,
+                                                                  unsigned maxbits, uint64_t* __restrict__ stream)
+{
+  extern __shared__ uint4 lds_raw[];
+  uint32_t* lds = reinterpret_cast<uint32_t*>(lds_raw);
+  const unsigned lane = threadIdx.x, bl = lane >> 2, q = lane & 3u;
+  const uint32_t b = blockIdx.x * kQuadBlocks + bl;
+  const bool live = b < fd.nblocks;
+  const unsigned slot = slot_bits(maxbits);
+  uint32_t* ex = lds + quad_region_dwords(slot) + bl * kQuadStride;
+
+  float f[16];
+  quad_load(in, fd, live ? b : fd.nblocks - 1, q, f);
+  uint32_t to_seq[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) to_seq[i] = kQuadOrder.to_seq[q][i];
+  {
+    const unsigned n16 = quad_region_dwords(slot) / 4;
+    for (unsigned i = lane; i < n16; i += 64) lds_raw[i] = make_uint4(0, 0, 0, 0);
+  }
+  float m = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 16; i++) m = fmaxf(m, fabsf(f[i]));
+  m = fmaxf(m, f32_from_bits(quad_move<kQuadXor1>(f32_bits(m))));
+  m = fmaxf(m, f32_from_bits(quad_move<kQuadXor2>(f32_bits(m))));
+  const uint32_t mb = f32_bits(m);
+  const uint32_t e = (live && mb) ? (mb >> 23) + 1 : 0;  // as block_header_e
+  const float s = e ? pow2f(30 - ((int)e - 127)) : 0.0f;
+
+  int32_t c[16];  // x + 4y of slice q, then x + 4z of the plane y = q
+#pragma unroll
+  for (int i = 0; i < 16; i++) c[i] = (int32_t)(s * f[i]);
+#pragma unroll
+  for (int y = 0; y < 4; y++) fwd_lift4(c[4 * y], c[4 * y + 1], c[4 * y + 2], c[4 * y + 3]);
+#pragma unroll
+  for (int x = 0; x < 4; x++) fwd_lift4(c[x], c[x + 4], c[x + 8], c[x + 12]);
+#pragma unroll
+  for (int y = 0; y < 4; y++)
+    *reinterpret_cast<int4*>(ex + 16 * q + 4 * y) = make_int4(c[4 * y], c[4 * y + 1], c[4 * y + 2], c[4 * y + 3]);
+  __syncthreads();
+#pragma unroll
+  for (int z = 0; z < 4; z++) {
+    const int4 v = *reinterpret_cast<const int4*>(ex + 16 * z + 4 * q);
+    c[4 * z] = v.x; c[4 * z + 1] = v.y; c[4 * z + 2] = v.z; c[4 * z + 3] = v.w;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int x = 0; x < 4; x++) fwd_lift4(c[x], c[x + 4], c[x + 8], c[x + 12]);
+#pragma unroll
+  for (int i = 0; i < 16; i++)  // negabinary: the add here, the xor inside the transpose
+    *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(ex) + ((to_seq[i / 4] >> (8 * (i % 4))) & 0xffu)) =
+        (uint32_t)c[i] + kNegabinary;
+  __syncthreads();
+  uint32_t a[16];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const uint4 v = *reinterpret_cast<const uint4*>(ex + 16 * q + 4 * i);
+    a[4 * i] = v.x; a[4 * i + 1] = v.y; a[4 * i + 2] = v.z; a[4 * i + 3] = v.w;
+  }
+  __syncthreads();
+
+  LdsBits mem(lds);
+  BlockEncoder<LdsBits, false> enc(mem, mem.bit0 + bl * slot, maxbits);
+  unsigned base = e ? enc.pos + 9 : enc.limit;  // an all-zero block or one past the end: nothing is written
+  if (e && q == 0) enc.put(2 * e + 1, 9);
+  uint64_t acc = 0;
+  uint32_t t[8];
+  quad_planes<true>(a, t);
+  quad_code16(t, ex, q, enc, acc, base);
+  if (CSWAP_ANY(base < enc.limit)) {
+    quad_planes<false>(a, t);
+    __syncthreads();
+    quad_code16(t, ex, q, enc, acc, base);
+  }
+  __syncthreads();
+
+  if (live) {  // the four lanes of a block move its words
+    const unsigned W = maxbits >> 6;
+    const uint64_t* src = reinterpret_cast<const uint64_t*>(lds + bl * (slot / 32));
+    uint64_t* dst = stream + (size_t)b * W;
+    if ((W & 1u) == 0 && fd.stream16) {
+      for (unsigned j = 2 * q; j < W; j += 8)
+        *reinterpret_cast<ulonglong2*>(dst + j) = *reinterpret_cast<const ulonglong2*>(src + j);
+    } else {
+      for (unsigned j = q; j < W; j += 4) dst[j] = src[j];
+    }
+  }
+}
+
+__global__ __launch_bounds__(64) void zfp_decode3_f32_quad_kernel(const uint64_t* __restrict__ stream, Field3 fd,
+                                                                  unsigned maxbits, float* __restrict__ out)
+{
+  extern __shared__ uint4 lds_raw[];
+  uint32_t* lds = reinterpret_cast<uint32_t*>(lds_raw);
+  const unsigned lane = threadIdx.x, bl = lane >> 2, q = lane & 3u;
+  const uint32_t b = blockIdx.x * kQuadBlocks + bl;
+  const bool live = b < fd.nblocks;
+  const unsigned slot = dec_slot_bits(maxbits);
+  uint32_t* ex = lds + quad_region_dwords(slot) + bl * kQuadStride;
+  {  // the four lanes of a block bring its words; blocks past the end read as empty
+    const unsigned W = maxbits >> 6;
+    uint64_t* dst = reinterpret_cast<uint64_t*>(lds + bl * (slot / 32));
+    const uint64_t* src = stream + (size_t)b * W;
+    if (!live) {
+      for (unsigned j = q; j < W; j += 4) dst[j] = 0;
+    } else if ((W & 1u) == 0 && fd.stream16) {
+      for (unsigned j = 2 * q; j < W; j += 8) {
+        const ulonglong2 v = *reinterpret_cast<const ulonglong2*>(src + j);
+        dst[j] = v.x;
+        dst[j + 1] = v.y;
+      }
+    } else {
+      for (unsigned j = q; j < W; j += 4) dst[j] = src[j];
+    }
+    if (q == 0) dst[W] = ~0ull;
+  }
+  uint32_t to_xyz[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) to_xyz[i] = kQuadOrder.to_xyz[q][i];
+  __syncthreads();
+
+  LdsBits mem(lds);
+  BlockDecoder<LdsBits, 64, true> dec(mem, mem.bit0 + bl * slot, maxbits);
+  const uint32_t h = (uint32_t)dec.window(dec.pos);
+  const bool coded = (h & 1) != 0;
+  dec.pos = coded ? dec.pos + 9 : dec.limit;
+  const uint32_t mine = (q & 1u) ? 0x07060302u : 0x05040100u;  // my half of the word that has my quarter of a plane
+  uint32_t t[8], l[8];
+#pragma unroll
+  for (int k = 15; k >= 0; k--) {
+    uint64_t x = 0;
+    if (CSWAP_ANY(dec.active())) x = k >= 12 ? dec.leading_plane() : dec.plane();
+    const uint32_t word = (q & 2u) ? (uint32_t)(x >> 32) : (uint32_t)x;
+    if (k >= 8) t[k - 8] = word;
+    else t[k] = byte_perm(t[k], word, mine);
+  }
+  quad_untranspose(t);
+  uint32_t bias = kNegabinary;
+  if (CSWAP_ANY(dec.active())) {
+#pragma unroll
+    for (int k = 15; k >= 0; k--) {
+      const uint64_t x = dec.plane();
+      const uint32_t word = (q & 2u) ? (uint32_t)(x >> 32) : (uint32_t)x;
+      if (k >= 8) l[k - 8] = word;
+      else l[k] = byte_perm(l[k], word, mine);
+    }
+    quad_untranspose(l);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 8; k++) l[k] = 0;
+    bias = kNegabinary & 0xffff0000u;
+  }
+  uint32_t a[16];
+  quad_coefficients(t, l, a);
+#pragma unroll
+  for (int i = 0; i < 16; i++)
+    *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(ex) + ((to_xyz[i / 4] >> (8 * (i % 4))) & 0xffu)) = a[i];
+  __syncthreads();
+  int32_t c[16];  // x + 4z of the plane y = q, then x + 4y of slice q
+#pragma unroll
+  for (int z = 0; z < 4; z++) {
+    const int4 v = *reinterpret_cast<const int4*>(ex + 16 * z + 4 * q);
+    c[4 * z] = v.x; c[4 * z + 1] = v.y; c[4 * z + 2] = v.z; c[4 * z + 3] = v.w;
+  }
+#pragma unroll
+  for (int x = 0; x < 4; x++) inv_lift4_biased(c[x], c[x + 4], c[x + 8], c[x + 12], bias);
+#pragma unroll
+  for (int z = 0; z < 4; z++)
+    *reinterpret_cast<int4*>(ex + 16 * z + 4 * q) = make_int4(c[4 * z], c[4 * z + 1], c[4 * z + 2], c[4 * z + 3]);
+  __syncthreads();
+#pragma unroll
+  for (int y = 0; y < 4; y++) {
+    const int4 v = *reinterpret_cast<const int4*>(ex + 16 * q + 4 * y);
+    c[4 * y] = v.x; c[4 * y + 1] = v.y; c[4 * y + 2] = v.z; c[4 * y + 3] = v.w;
+  }
+#pragma unroll
+  for (int x = 0; x < 4; x++) inv_lift4(c[x], c[x + 4], c[x + 8], c[x + 12]);
+  const float w = coded ? decode_scale((h >> 1) & 0xffu) : 0.0f;
+  float r[16];
+#pragma unroll
+  for (int y = 0; y < 4; y++) {
+    inv_lift4(c[4 * y], c[4 * y + 1], c[4 * y + 2], c[4 * y + 3]);
+#pragma unroll
+    for (int x = 0; x < 4; x++) r[4 * y + x] = w * (float)c[4 * y + x];
+  }
+
+  uint32_t x0, y0, z0;
+  block_origin(fd, live ? b : 0u, x0, y0, z0);
+  const uint32_t bx = min(4u, fd.nx - x0), by = min(4u, fd.ny - y0), bz = min(4u, fd.nz - z0);
+  if (!live || q >= bz) return;
+  float* p = out + ((long long)x0 * fd.sx + (long long)y0 * fd.sy + (long long)(z0 + q) * fd.sz);
+  if (fd.full && fd.rows16) {
+#pragma unroll
+    for (int y = 0; y < 4; y++) {
+      const stream_f4 v = {r[4 * y], r[4 * y + 1], r[4 * y + 2], r[4 * y + 3]};
+      __builtin_nontemporal_store(v, reinterpret_cast<stream_f4*>(p + y * fd.sy));
+    }
+  } else if (fd.rows4 && bx == 4) {
+#pragma unroll
+    for (int y = 0; y < 4; y++) {
+      const row_f4 v = {r[4 * y], r[4 * y + 1], r[4 * y + 2], r[4 * y + 3]};
+      if ((uint32_t)y < by) *reinterpret_cast<row_f4*>(p + y * fd.sy) = v;
+    }
+  } else {
+#pragma unroll
+    for (int y = 0; y < 4; y++)
+#pragma unroll
+      for (int x = 0; x < 4; x++)
+        if ((uint32_t)x < bx && (uint32_t)y < by) p[x * fd.sx + y * fd.sy] = r[4 * y + x];
+  }
+}
+
 // ------------------------------------------------------------- 64-bit elements
 // Fields of doubles or int64 (zfp_type_double, zfp_type_int64): the same
 // decomposition, values moved as 64-bit patterns.  Fast path: full block whose
@@ -1115,6 +1444,23 @@ static bool pair_fits(unsigned grid, size_t lds_bytes, unsigned long long limit)
 // end weighs more.
 constexpr unsigned kPairDecodeFromBits = 1024;
 
+// The quad form pays while its wavefronts (16 blocks each) are few per compute unit: it trades
+// instructions (half as many again as the pair form's, for the same blocks) for short chains.
+// Microseconds, quad / pair / one lane per block at 8 bits per value by wavefronts per compute unit:
+//   encode  1 (1 MB) 6.1 / 7.9 / 10.7 · 4: 6.7 / 8.4 / 11.1 · 8: 8.1 / 9.6 / 11.7 · 12: 10.1 / 9.9 / 12.2 ·
+//           16: 11.1 / 10.2 / 12.6; where the pair form does not apply (odd planes): 8: 8.2 / - / 12.3 ·
+//           19: 14.9 / - / 17.7 · 30: 20.2 / - / 17.4
+//   decode  1: 9.2 / - / 11.8 · 4: 10.6 / - / 12.8 · 8: 11.2 / - / 12.4 · 12: 12.6 / - / 12.6 · 16: 13.9 / - / 13.4;
+//           odd planes 8: 11.6 / - / 14.2 · 10: 14.0 / - / 15.4 · 19: 21.0 / - / 18.3
+// 4 and 16 bits per value cross at the same places.
+constexpr unsigned kQuadWaves = 11;        // per compute unit
+constexpr unsigned kQuadWavesNoPair = 22;  // the encoder's where the pair form does not apply
+static bool quad_pays(uint32_t nblocks, unsigned waves, unsigned long long bytes, unsigned long long pair_below)
+{
+  return pair_below != ~0ull && bytes < pair_below &&
+         (unsigned long long)nblocks <= (unsigned long long)kQuadBlocks * waves * (unsigned)device_compute_units();
+}
+
 extern "C" void cswap_zfp_set_pair_bytes(size_t encode_below, size_t decode_below, size_t* previous)
 {
   const size_t e = (size_t)g_pair_encode_bytes.exchange(encode_below, std::memory_order_relaxed);
@@ -1150,6 +1496,13 @@ static int compress3(const void* d_in, Elem elem, size_t nx, size_t ny, size_t n
   const bool whole = (maxbits & 63u) == 0;
   const bool is_int = elem == kI32 || elem == kI64;
   const unsigned long long pair_below = g_pair_encode_bytes.load(std::memory_order_relaxed);
+  if (elem == kF32 && whole && quad_pays(fd.nblocks, pair_shape(fd, maxbits) ? kQuadWaves : kQuadWavesNoPair,
+                                          (unsigned long long)nx * ny * nz * 4ull, pair_below)) {
+    hipLaunchKernelGGL(zfp_encode3_f32_quad_kernel, dim3((fd.nblocks + kQuadBlocks - 1) / kQuadBlocks), dim3(64),
+                       (size_t)quad_lds_dwords(slot_bits(maxbits)) * 4, st, static_cast<const float*>(d_in), fd, maxbits,
+                       d_stream);
+    return check_launch();
+  }
   if (elem == kF32 && pair_shape(fd, maxbits) && (unsigned long long)nx * ny * nz * 4ull < pair_below &&
       pair_fits(grid, (size_t)pair_lds_dwords(maxbits) * 4, pair_below)) {
     hipLaunchKernelGGL(zfp_encode3_f32_pair_kernel, dim3(grid), dim3(128), (size_t)pair_lds_dwords(maxbits) * 4, st,
@@ -1200,6 +1553,12 @@ static int decompress3(const uint64_t* d_stream, Elem elem, size_t nx, size_t ny
   const bool whole = (maxbits & 63u) == 0;
   const bool is_int = elem == kI32 || elem == kI64;
   const unsigned long long pair_below = g_pair_decode_bytes.load(std::memory_order_relaxed);
+  if (elem == kF32 && whole && quad_pays(fd.nblocks, kQuadWaves, (unsigned long long)nx * ny * nz * 4ull, pair_below)) {
+    hipLaunchKernelGGL(zfp_decode3_f32_quad_kernel, dim3((fd.nblocks + kQuadBlocks - 1) / kQuadBlocks), dim3(64),
+                       (size_t)quad_lds_dwords(dec_slot_bits(maxbits)) * 4, st, d_stream, fd, maxbits,
+                       static_cast<float*>(d_out));
+    return check_launch();
+  }
   if (elem == kF32 && pair_shape(fd, maxbits) && (unsigned long long)nx * ny * nz * 4ull < pair_below &&
       (maxbits >= kPairDecodeFromBits || pair_below == ~0ull) &&
       pair_fits(grid, (size_t)pair_dec_lds_dwords(maxbits) * 4, pair_below)) {

@@ -118,8 +118,12 @@ int cswap_zfp_decompress_i64_nd(const uint64_t* d_stream, int dims, size_t nx, s
  * Below the limit the form is taken while all of the field's workgroups fit on the chip
  * at once (their LDS decides how many do: about 37 MB at 8 bits per value, 30 MB at 16,
  * 21 MB at 32), and by the decoder only from 16 bits per value on (at 8 it measured no
- * gain).  0 = never; SIZE_MAX = whenever the shape allows, whatever the size and rate
- * (tests and measurements).  Defaults: 40 MiB both.  `previous`, if not NULL, receives
+ * gain).  The smallest fields (below the same limits, up to 11 wavefronts of 16 blocks
+ * per compute unit: about 11 MB; 22 for an encoder of a shape that the pair form does not
+ * take) run a form with four lanes per block, at any shape and any maxbits that is a
+ * multiple of 64.  0 = neither form, one lane per block; SIZE_MAX = the pair form
+ * whenever the shape allows, whatever the size and rate, and never the one with four
+ * lanes (tests and measurements).  Defaults: 40 MiB both.  `previous`, if not NULL, receives
  * the two values that were in force.  Process-wide. */
 void cswap_zfp_set_pair_bytes(size_t encode_below, size_t decode_below, size_t* previous);
 

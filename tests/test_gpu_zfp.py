@@ -194,6 +194,51 @@ def test_rows_at_any_element(torch_cuda, nx, ny, nz, shift, gap, zfp_form):
         assert np.all(o == -7.0), maxbits   # nothing outside the field was touched
 
 
+@pytest.mark.parametrize("nx,ny,nz", [(1, 1, 1), (4, 4, 60), (4, 4, 64), (4, 4, 68), (13, 1, 2), (9, 10, 11), (64, 64, 4 * 45),
+                                      (64, 64, 4 * 46), (35, 35, 4 * 285)])
+@pytest.mark.parametrize("order", ["xyz", "zyx", "reversed"])
+def test_four_lanes_per_block(torch_cuda, nx, ny, nz, order):
+    """The form for the smallest fields: counts of blocks around a wavefront's 16 and around the
+    size rule's limits (11 wavefronts per compute unit; 22 for an encoder of odd planes), strides
+    in other orders and negative ones, streams of an odd number of words per block and at an odd
+    word, all bit planes.  Exact against the checker."""
+    torch = torch_cuda
+    import oracle
+    from cswap_amd._lib import check, lib
+
+    rng = np.random.default_rng(nx * 31 + ny * 7 + nz)
+    f = (rng.standard_normal((nz, ny, nx)) * np.exp(rng.standard_normal((nz, ny, nx)))).astype(np.float32)
+    if nz > 4:
+        f[:4] = 0                                   # an empty block
+    n = f.size
+    if order == "xyz":
+        mem, base, strides = f.ravel(), 0, (1, nx, nx * ny)
+    elif order == "zyx":
+        mem, base, strides = np.ascontiguousarray(f.transpose(2, 1, 0)).ravel(), 0, (nz * ny, nz, 1)
+    else:
+        mem, base, strides = f[::-1, ::-1, ::-1].ravel(), n - 1, (-1, -nx, -nx * ny)
+    t = torch.from_numpy(np.ascontiguousarray(mem)).cuda()
+    for maxbits in (64, 192, 256, 512, 1024, 2048, 4096):
+        if n > 1 << 18 and maxbits not in (192, 512):
+            continue
+        cap = lib().cswap_zfp_stream_capacity(nx, ny, nz, maxbits)
+        for shift in (0, 8):
+            s = torch.zeros(cap + 16, dtype=torch.uint8, device="cuda")
+            check(lib().cswap_zfp_compress_f32(t.data_ptr() + 4 * base, nx, ny, nz, *strides, maxbits, s.data_ptr() + shift, None),
+                  "compress")
+            o = torch.full_like(t, -7.0)
+            check(lib().cswap_zfp_decompress_f32(s.data_ptr() + shift, nx, ny, nz, *strides, maxbits, o.data_ptr() + 4 * base,
+                                                 None), "decompress")
+            torch.cuda.synchronize()
+            want = oracle.zfp_encode3(f, maxbits)
+            sb = s.cpu().numpy()
+            assert np.array_equal(sb[shift:shift + cap].view(np.uint64), want), (maxbits, shift)
+            assert not sb[:shift].any() and not sb[shift + cap:].any()
+            d = oracle.zfp_decode3(want, f.shape, maxbits)
+            d = {"xyz": d, "zyx": d.transpose(2, 1, 0), "reversed": d[::-1, ::-1, ::-1]}[order]
+            assert np.array_equal(o.cpu().numpy().view(np.uint32), np.ascontiguousarray(d).ravel().view(np.uint32)), (maxbits, shift)
+
+
 @pytest.mark.parametrize("case", ["padded_rows_and_planes", "one_block_per_slab", "slab_crossing", "planes_before_rows",
                                   "big_offsets"])
 def test_aligned_strided_fields(torch_cuda, case, zfp_form):

@@ -17,7 +17,9 @@ PROCESS = 512 * 32  # CSWAP+/Execution.h:50-52
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current device's current stream, as torch.cuda.current_stream().cuda_stream names it but
+    without the Stream object (0.2 instead of 2.8 us, where a call on a small tensor takes 10)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _need_f32_cuda(t: torch.Tensor) -> None:

@@ -12,6 +12,7 @@ import ctypes as C
 
 import torch
 
+from .api import _stream
 from ._lib import Choice, Costs, EngineConfig, TicketInfo, TicketTiming, check, lib
 from .workloads import field_dims
 
@@ -84,7 +85,7 @@ class SwapEngine:
         nx, ny, nz = field_dims(t.shape)
         ticket = C.c_int(-1)
         check(lib().cswap_swap_out(self._h, t.data_ptr(), nx, ny, nz, policy,
-                                   torch.cuda.current_stream().cuda_stream, C.byref(ticket)), "cswap_swap_out")
+                                   _stream(), C.byref(ticket)), "cswap_swap_out")
         return ticket.value
 
     # Execution::post
@@ -92,7 +93,7 @@ class SwapEngine:
         check(lib().cswap_swap_wait(self._h, ticket), "cswap_swap_wait")
 
     def swap_in(self, ticket: int, out: torch.Tensor) -> torch.Tensor:
-        check(lib().cswap_swap_in(self._h, ticket, out.data_ptr(), torch.cuda.current_stream().cuda_stream),
+        check(lib().cswap_swap_in(self._h, ticket, out.data_ptr(), _stream()),
               "cswap_swap_in")
         return out
 

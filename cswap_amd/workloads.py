@@ -28,7 +28,7 @@ def field_dims(shape):
     with B a multiple of 4 becomes (F, 4, B/4); a flat vector becomes 32x32 or
     4x4 rows when its length allows.  Any such view of contiguous memory is a
     valid field as long as both directions use the same one."""
-    shape = [int(d) for d in shape]
+    shape = tuple(map(int, shape))
     if len(shape) <= 1:
         n = shape[0] if shape else 1
         if n % 1024 == 0:
@@ -37,7 +37,7 @@ def field_dims(shape):
             return 4, 4, n // 16
         return n, 1, 1
     nx, ny = shape[-1], shape[-2]
-    nz = int(np.prod(shape[:-2])) if len(shape) > 2 else 1
+    nz = math.prod(shape[:-2])
     if nz < 4 and ny >= 16 and ny % 4 == 0:
         nz, ny = nz * (ny // 4), 4
     return nx, ny, nz

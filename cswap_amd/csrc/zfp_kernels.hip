@@ -138,6 +138,44 @@ __device__ __forceinline__ uint32_t lane_bytes(const Field3& fd, const WaveBase&
   return ((x0 - w.fx) + (y0 - w.fy) * (uint32_t)fd.sy + (z0 - w.fz) * (uint32_t)fd.sz) * 4u;  // mod 2^32
 }
 
+template <bool ONCE>
+__device__ __forceinline__ void load_block(const float* __restrict__ in, const Field3& fd, uint32_t first,
+                                           uint32_t b, float (&f)[64])
+{
+  uint32_t x0, y0, z0;
+  block_origin(fd, b, x0, y0, z0);
+  uint32_t bx = min(4u, fd.nx - x0), by = min(4u, fd.ny - y0), bz = min(4u, fd.nz - z0);
+  if (fd.rows16 && bx == 4 && by == 4 && bz == 4) {
+    const WaveBase w = wave_base(fd, first);
+    const char* base = reinterpret_cast<const char*>(in + w.origin);
+    const uint32_t mine = lane_bytes(fd, w, x0, y0, z0);
+    const uint32_t sy4 = (uint32_t)fd.sy * 4u, sz4 = (uint32_t)fd.sz * 4u;
+#pragma unroll
+    for (int z = 0; z < 4; z++)
+#pragma unroll
+      for (int y = 0; y < 4; y++) {
+        const stream_f4* src = reinterpret_cast<const stream_f4*>(base + (size_t)(mine + (y * sy4 + z * sz4)));
+        const stream_f4 v = ONCE ? __builtin_nontemporal_load(src) : *src;
+        f[16 * z + 4 * y + 0] = v.x;
+        f[16 * z + 4 * y + 1] = v.y;
+        f[16 * z + 4 * y + 2] = v.z;
+        f[16 * z + 4 * y + 3] = v.w;
+      }
+  } else {
+    const float* p = in + (long long)x0 * fd.sx + (long long)y0 * fd.sy + (long long)z0 * fd.sz;
+#pragma unroll
+    for (int z = 0; z < 4; z++)
+#pragma unroll
+      for (int y = 0; y < 4; y++)
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+          bool ok = (uint32_t)x < bx && (uint32_t)y < by && (uint32_t)z < bz;
+          f[16 * z + 4 * y + x] = ok ? p[x * fd.sx + y * fd.sy + z * fd.sz] : 0.0f;
+        }
+    if (bx < 4 || by < 4 || bz < 4) pad_block3(f, bx, by, bz);
+  }
+}
+
 // Where the four rows (planes) of a block that has only n of them along this axis are read
 // from, in bytes from the first one at a distance of s bytes: the padding rule (pad4) as
 // addresses.  n = 1: a,a,a,a; 2: a,b,b,a; 3: a,b,c,a.
@@ -156,71 +194,48 @@ __device__ __forceinline__ void padded_offsets(uint32_t n, uint32_t s, uint32_t 
 // -- its end is the start of the next row, or what lies between rows -- and the padding is
 // selected in registers.  Only blocks whose reads would leave the field (the last block along
 // all three axes) go element by element.  nx = 1 stays out: four elements are up to four rows
-// there, and other blocks than the last could leave the field.  Against one predicated 4-byte access per element with its own
-// 64-bit address, at 8 bits per value: 60 MB in 35x35 planes encoded in 26.8 instead of 27.6 us
-// and decoded in 26.0 instead of 39.4, 241 MB of them in 69 instead of 84 and 99 instead of 130;
-// 51 MB in 14x14 planes 25.7 / 28.0 and 27.1 / 43.1, 51 MB in 7x7 planes 25.5 / 29.3 and 42 / 54.
-template <bool ONCE>
+// there, and other blocks than the last could leave the field.  Against one predicated 4-byte
+// access per element with its own 64-bit address, at 8 bits per value: 60 MB in 35x35 planes
+// encoded in 26.2 instead of 28.1 us and decoded in 26.4 instead of 39.8, 321 MB of them in 90
+// instead of 108 and 119 instead of 166; 26 MB in 14x14 planes 16.9 / 19.6 and 18.7 / 26.5.
 __device__ __forceinline__ void load_row(const char* src, float (&f)[64], int row)
 {
   const row_f4* p = reinterpret_cast<const row_f4*>(src);
-  const row_f4 v = ONCE ? __builtin_nontemporal_load(p) : *p;
+  const row_f4 v = *p;
   f[4 * row + 0] = v.x;
   f[4 * row + 1] = v.y;
   f[4 * row + 2] = v.z;
   f[4 * row + 3] = v.w;
 }
 
-template <bool ONCE>
-__device__ __forceinline__ void load_block(const float* __restrict__ in, const Field3& fd, uint32_t first,
-                                           uint32_t b, float (&f)[64])
+__device__ __forceinline__ void load_block_rows(const float* __restrict__ in, const Field3& fd, uint32_t first, uint32_t b,
+                                                float (&f)[64])
 {
   uint32_t x0, y0, z0;
   block_origin(fd, b, x0, y0, z0);
-  if (fd.full) {
-    const WaveBase w = wave_base(fd, first);
-    const char* base = reinterpret_cast<const char*>(in + w.origin);
-    const uint32_t mine = lane_bytes(fd, w, x0, y0, z0);
-    const uint32_t sy4 = (uint32_t)fd.sy * 4u, sz4 = (uint32_t)fd.sz * 4u;
-#pragma unroll
-    for (int z = 0; z < 4; z++)
-#pragma unroll
-      for (int y = 0; y < 4; y++) load_row<ONCE>(base + (size_t)(mine + (y * sy4 + z * sz4)), f, y + 4 * z);
-    return;
-  }
   const uint32_t bx = min(4u, fd.nx - x0), by = min(4u, fd.ny - y0), bz = min(4u, fd.nz - z0);
   const bool leaves = bx < 4 && y0 + by == fd.ny && z0 + bz == fd.nz;  // its last row is the field's, and is cut off
-  if (fd.rows4 && !leaves) {
-    const WaveBase w = wave_base(fd, first);
-    const char* base = reinterpret_cast<const char*>(in + w.origin);
-    const uint32_t mine = lane_bytes(fd, w, x0, y0, z0);
-    uint32_t yo[4], zo[4];
-    padded_offsets(by, (uint32_t)fd.sy * 4u, yo);
-    padded_offsets(bz, (uint32_t)fd.sz * 4u, zo);
+  if (leaves) {
+    load_block<false>(in, fd, first, b, f);
+    return;
+  }
+  const WaveBase w = wave_base(fd, first);
+  const char* base = reinterpret_cast<const char*>(in + w.origin);
+  const uint32_t mine = lane_bytes(fd, w, x0, y0, z0);
+  uint32_t yo[4], zo[4];
+  padded_offsets(by, (uint32_t)fd.sy * 4u, yo);
+  padded_offsets(bz, (uint32_t)fd.sz * 4u, zo);
 #pragma unroll
-    for (int z = 0; z < 4; z++)
+  for (int z = 0; z < 4; z++)
 #pragma unroll
-      for (int y = 0; y < 4; y++) load_row<ONCE>(base + (size_t)(mine + yo[y] + zo[z]), f, y + 4 * z);
-    if (fd.nx & 3u) {
+    for (int y = 0; y < 4; y++) load_row(base + (size_t)(mine + yo[y] + zo[z]), f, y + 4 * z);
+  if (fd.nx & 3u) {
 #pragma unroll
-      for (int r = 0; r < 16; r++) {
-        f[4 * r + 1] = bx >= 2 ? f[4 * r + 1] : f[4 * r];
-        f[4 * r + 2] = bx >= 3 ? f[4 * r + 2] : f[4 * r + 1];
-        f[4 * r + 3] = bx >= 4 ? f[4 * r + 3] : f[4 * r];
-      }
+    for (int r = 0; r < 16; r++) {
+      f[4 * r + 1] = bx >= 2 ? f[4 * r + 1] : f[4 * r];
+      f[4 * r + 2] = bx >= 3 ? f[4 * r + 2] : f[4 * r + 1];
+      f[4 * r + 3] = bx >= 4 ? f[4 * r + 3] : f[4 * r];
     }
-  } else {
-    const float* p = in + (long long)x0 * fd.sx + (long long)y0 * fd.sy + (long long)z0 * fd.sz;
-#pragma unroll
-    for (int z = 0; z < 4; z++)
-#pragma unroll
-      for (int y = 0; y < 4; y++)
-#pragma unroll
-        for (int x = 0; x < 4; x++) {
-          bool ok = (uint32_t)x < bx && (uint32_t)y < by && (uint32_t)z < bz;
-          f[16 * z + 4 * y + x] = ok ? p[x * fd.sx + y * fd.sy + z * fd.sz] : 0.0f;
-        }
-    if (bx < 4 || by < 4 || bz < 4) pad_block3(f, bx, by, bz);
   }
 }
 
@@ -241,7 +256,8 @@ __device__ __forceinline__ void finish_and_store_block(float* __restrict__ out, 
 {
   uint32_t x0, y0, z0;
   block_origin(fd, b, x0, y0, z0);
-  if (fd.full && fd.rows16) {
+  uint32_t bx = min(4u, fd.nx - x0), by = min(4u, fd.ny - y0), bz = min(4u, fd.nz - z0);
+  if (fd.rows16 && bx == 4 && by == 4 && bz == 4) {
     const WaveBase wb = wave_base(fd, first);
     char* base = reinterpret_cast<char*>(out + wb.origin);
     const uint32_t mine = lane_bytes(fd, wb, x0, y0, z0);
@@ -255,35 +271,6 @@ __device__ __forceinline__ void finish_and_store_block(float* __restrict__ out, 
         else decode_row(ib, y + 4 * z, w, r);
         const stream_f4 v = {r[0], r[1], r[2], r[3]};
         __builtin_nontemporal_store(v, reinterpret_cast<stream_f4*>(base + (size_t)(mine + (y * sy4 + z * sz4))));
-      }
-    return;
-  }
-  const uint32_t bx = min(4u, fd.nx - x0), by = min(4u, fd.ny - y0), bz = min(4u, fd.nz - z0);
-  if (fd.rows4) {
-    const WaveBase wb = wave_base(fd, first);
-    char* base = reinterpret_cast<char*>(out + wb.origin);
-    const uint32_t mine = lane_bytes(fd, wb, x0, y0, z0);
-    const uint32_t sy4 = (uint32_t)fd.sy * 4u, sz4 = (uint32_t)fd.sz * 4u;
-#pragma unroll
-    for (int z = 0; z < 4; z++)
-#pragma unroll
-      for (int y = 0; y < 4; y++) {
-        float r[4];
-        if (INT) decode_row_i32(ib, y + 4 * z, r);
-        else decode_row(ib, y + 4 * z, w, r);
-        if ((uint32_t)y < by && (uint32_t)z < bz) {
-          float* dst = reinterpret_cast<float*>(base + (size_t)(mine + (y * sy4 + z * sz4)));
-          if (bx == 4) {
-            const row_f4 v = {r[0], r[1], r[2], r[3]};
-            *reinterpret_cast<row_f4*>(dst) = v;
-          } else if (fd.nx & 2u) {
-            const row_f2 v = {r[0], r[1]};
-            *reinterpret_cast<row_f2*>(dst) = v;
-            if (fd.nx & 1u) dst[2] = r[2];
-          } else {
-            dst[0] = r[0];
-          }
-        }
       }
   } else {
     float* p = out + (long long)x0 * fd.sx + (long long)y0 * fd.sy + (long long)z0 * fd.sz;
@@ -299,6 +286,43 @@ __device__ __forceinline__ void finish_and_store_block(float* __restrict__ out, 
           if ((uint32_t)x < bx && (uint32_t)y < by && (uint32_t)z < bz) p[x * fd.sx + y * fd.sy + z * fd.sz] = r[x];
       }
   }
+}
+
+// The same where rows start at any element or end inside a block.  The hint is for aligned rows:
+// elsewhere it leaves partial lines to memory (60 MB in 35x35 planes 27.9 us with it, 26.4 without; 321 MB 149 and 119).
+template <bool INT, bool HINT>
+__device__ __forceinline__ void finish_and_store_rows(float* __restrict__ out, const Field3& fd, uint32_t first, uint32_t b,
+                                                      int32_t (&ib)[64], float w)
+{
+  uint32_t x0, y0, z0;
+  block_origin(fd, b, x0, y0, z0);
+  const uint32_t bx = min(4u, fd.nx - x0), by = min(4u, fd.ny - y0), bz = min(4u, fd.nz - z0);
+  const WaveBase wb = wave_base(fd, first);
+  char* base = reinterpret_cast<char*>(out + wb.origin);
+  const uint32_t mine = lane_bytes(fd, wb, x0, y0, z0);
+  const uint32_t sy4 = (uint32_t)fd.sy * 4u, sz4 = (uint32_t)fd.sz * 4u;
+#pragma unroll
+  for (int z = 0; z < 4; z++)
+#pragma unroll
+    for (int y = 0; y < 4; y++) {
+      float r[4];
+      if (INT) decode_row_i32(ib, y + 4 * z, r);
+      else decode_row(ib, y + 4 * z, w, r);
+      if ((uint32_t)y < by && (uint32_t)z < bz) {
+        float* dst = reinterpret_cast<float*>(base + (size_t)(mine + (y * sy4 + z * sz4)));
+        if (bx == 4) {
+          const row_f4 v = {r[0], r[1], r[2], r[3]};
+          if (HINT) __builtin_nontemporal_store(v, reinterpret_cast<row_f4*>(dst));
+          else *reinterpret_cast<row_f4*>(dst) = v;
+        } else if (fd.nx & 2u) {
+          const row_f2 v = {r[0], r[1]};
+          *reinterpret_cast<row_f2*>(dst) = v;
+          if (fd.nx & 1u) dst[2] = r[2];
+        } else {
+          dst[0] = r[0];
+        }
+      }
+    }
 }
 
 // ------------------------------------------------------------- LDS region <-> stream
@@ -379,10 +403,10 @@ __device__ __forceinline__ void load_region(uint32_t* lds, unsigned lane, uint32
 // into a compute unit, unevenly over its SIMDs, and the encoder measured fastest with
 // three per SIMD (402.7 MB at 16 bits per value: 130-133 us against 139-140 us with four
 // or five), the decoder with four (137-140 us against 143-156 us).
-template <bool WHOLE, bool INT = false, bool ONCE = false, int WPE = 5>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void zfp_encode3_f32_kernel(const float* __restrict__ in, Field3 fd,
-                                                             unsigned maxbits,
-                                                             uint64_t* __restrict__ stream)
+// ROWS: a field for load_block_rows
+template <bool WHOLE, bool INT, bool ONCE, bool ROWS>
+__device__ __forceinline__ void encode3_f32(const float* __restrict__ in, const Field3& fd, unsigned maxbits,
+                                            uint64_t* __restrict__ stream)
 {
   extern __shared__ uint4 lds_raw[];
   uint32_t* lds = reinterpret_cast<uint32_t*>(lds_raw);
@@ -397,7 +421,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
   // 97 us at 8 bits per value, 129 -> 126 us at 16; the other way round 100 and 131 us).
   float f[64];
   __builtin_amdgcn_s_setprio(3);
-  if (lane < valid) load_block<ONCE>(in, fd, first, first + lane, f);  // in flight while the region is cleared
+  if (lane < valid) {  // in flight while the region is cleared
+    if (ROWS) load_block_rows(in, fd, first, first + lane, f);
+    else load_block<ONCE>(in, fd, first, first + lane, f);
+  }
   zero_region(lds_raw, lane, maxbits);
   __syncthreads();
   __builtin_amdgcn_s_setprio(0);
@@ -418,13 +445,28 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
   store_region<WHOLE>(lds, lane, first, valid, maxbits, fd.stream16, stream);
 }
 
+template <bool WHOLE, bool INT = false, bool ONCE = false, int WPE = 5>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void zfp_encode3_f32_kernel(
+    const float* __restrict__ in, Field3 fd, unsigned maxbits, uint64_t* __restrict__ stream)
+{
+  encode3_f32<WHOLE, INT, ONCE, false>(in, fd, maxbits, stream);
+}
+// Kernels of their own for these fields: one kernel with both kinds of rows decoded full fields 2-6 %
+// slower (100 MB 29.2 instead of 27.5 us, 403 MB 89.7 instead of 87.4).
+template <bool WHOLE, bool INT = false, int WPE = 5>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void zfp_encode3_rows_kernel(
+    const float* __restrict__ in, Field3 fd, unsigned maxbits, uint64_t* __restrict__ stream)
+{
+  encode3_f32<WHOLE, INT, false, true>(in, fd, maxbits, stream);
+}
+
 // Five wavefronts per SIMD (at most 96 registers, which the row-wise finish
 // and the late block coordinates below reach without spilling): measured
 // 2.5 % faster than the four that the unconstrained 105 registers allow; six
 // (80 registers) spills and is slower again.
-template <bool WHOLE, bool INT = false, int WPE = 5>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void zfp_decode3_f32_kernel(const uint64_t* __restrict__ stream, Field3 fd,
-                                                             unsigned maxbits, float* __restrict__ out)
+template <bool WHOLE, bool INT, bool ROWS>
+__device__ __forceinline__ void decode3_f32(const uint64_t* __restrict__ stream, const Field3& fd, unsigned maxbits,
+                                            float* __restrict__ out)
 {
   extern __shared__ uint4 lds_raw[];
   uint32_t* lds = reinterpret_cast<uint32_t*>(lds_raw);
@@ -461,8 +503,24 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
     asm volatile("" : "+v"(zero) : "v"(ib[0]));
     const uint32_t b = first + __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));  // lane id again
     __builtin_amdgcn_s_setprio(1);
-    finish_and_store_block<INT>(out, fd, first, b, ib, w);
+    // (as one variant with the hint decided row by row, the compiler finishes all rows ahead and spills)
+    if (ROWS && fd.rows16) finish_and_store_rows<INT, true>(out, fd, first, b, ib, w);
+    else if (ROWS) finish_and_store_rows<INT, false>(out, fd, first, b, ib, w);
+    else finish_and_store_block<INT>(out, fd, first, b, ib, w);
   }
+}
+
+template <bool WHOLE, bool INT = false, int WPE = 5>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void zfp_decode3_f32_kernel(
+    const uint64_t* __restrict__ stream, Field3 fd, unsigned maxbits, float* __restrict__ out)
+{
+  decode3_f32<WHOLE, INT, false>(stream, fd, maxbits, out);
+}
+template <bool WHOLE, bool INT = false, int WPE = 5>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void zfp_decode3_rows_kernel(
+    const uint64_t* __restrict__ stream, Field3 fd, unsigned maxbits, float* __restrict__ out)
+{
+  decode3_f32<WHOLE, INT, true>(stream, fd, maxbits, out);
 }
 
 // ------------------------------------------------------------- the pair form: two wavefronts per 64 blocks
@@ -1426,6 +1484,14 @@ static bool pair_shape(const Field3& fd, unsigned maxbits)
   return fd.rows16 && fd.stream16 && (maxbits & 255u) == 0 && ((fd.nx | fd.ny | fd.nz) & 3u) == 0;
 }
 
+// Which fields the kernels for contiguous rows at any element take.  The encoder's: all that are not
+// whole blocks of aligned rows.  The decoder's leave those whose rows are aligned and whole along x:
+// there only the last block rows are cut off, and the hint on the others' whole lines is worth more
+// (39 MB in 197 rows of 768: encode 20.8 us either way, decode 16.2 with the other kernel, 17.1 with
+// this; 57 MB in 197 rows of 196: encode 28.1 and 26.3, decode 28.3 both).
+static bool encode_rows(const Field3& fd) { return fd.rows4 && !(fd.full && fd.rows16); }
+static bool decode_rows(const Field3& fd) { return fd.rows4 && !(fd.rows16 && (fd.nx & 3u) == 0); }
+
 static std::atomic<unsigned long long> g_pair_decode_bytes{CSWAP_PAIR_DECODE_BYTES};
 
 // The pair form pays while all of a field's workgroups are on the chip at once (twice the
@@ -1512,7 +1578,16 @@ static int compress3(const void* d_in, Elem elem, size_t nx, size_t ny, size_t n
   if (elem_bytes(elem) == 4) {
     const float* in = static_cast<const float*>(d_in);
     const bool once = fd.read_once && fd.rows16;
-    if (whole && maxbits >= kFewerWavesFrom) {
+    if (encode_rows(fd)) {
+      if (whole && maxbits >= kFewerWavesFrom && !is_int)
+        hipLaunchKernelGGL((zfp_encode3_rows_kernel<true, false, 3>), dim3(grid), dim3(64), lds_bytes, st, in, fd, maxbits,
+                           d_stream);
+      else if (whole && maxbits >= kFewerWavesFrom)
+        hipLaunchKernelGGL((zfp_encode3_rows_kernel<true, true, 3>), dim3(grid), dim3(64), lds_bytes, st, in, fd, maxbits,
+                           d_stream);
+      else
+        CSWAP_LAUNCH3(zfp_encode3_rows_kernel, float, in, d_stream);
+    } else if (whole && maxbits >= kFewerWavesFrom) {
       if (once && !is_int)
         hipLaunchKernelGGL((zfp_encode3_f32_kernel<true, false, true, 3>), dim3(grid), dim3(64), lds_bytes, st, in,
                            fd, maxbits, d_stream);
@@ -1569,7 +1644,16 @@ static int decompress3(const uint64_t* d_stream, Elem elem, size_t nx, size_t ny
   if (elem_bytes(elem) == 4) {
     float* out = static_cast<float*>(d_out);
     lds_bytes = (size_t)dec_region_dwords(maxbits) * 4;
-    if (whole && maxbits >= kFewerWavesFrom && !is_int)
+    if (decode_rows(fd)) {
+      if (whole && maxbits >= kFewerWavesFrom && !is_int)
+        hipLaunchKernelGGL((zfp_decode3_rows_kernel<true, false, 4>), dim3(grid), dim3(64), lds_bytes, st, d_stream, fd,
+                           maxbits, out);
+      else if (whole && maxbits >= kFewerWavesFrom)
+        hipLaunchKernelGGL((zfp_decode3_rows_kernel<true, true, 4>), dim3(grid), dim3(64), lds_bytes, st, d_stream, fd,
+                           maxbits, out);
+      else
+        CSWAP_LAUNCH3(zfp_decode3_rows_kernel, float, d_stream, out);
+    } else if (whole && maxbits >= kFewerWavesFrom && !is_int)
       hipLaunchKernelGGL((zfp_decode3_f32_kernel<true, false, 4>), dim3(grid), dim3(64), lds_bytes, st, d_stream, fd,
                          maxbits, out);
     else if (whole && maxbits >= kFewerWavesFrom)

@@ -490,7 +490,7 @@ def zvc_extras(torch, api, dev, ex, config2_tensor, only_mib=0, cpu=False):
                                                           nnz.data_ptr(), values.data_ptr(), mask.data_ptr(), st), reps)
         ws = api.zvc_workspace(api.PROCESS, dev)
         # count + scan + compact as one operation, as the swap engine runs it for a ZVC request: the
-        # single pass from 64 MiB on, the three kernels below
+        # single pass from 64 MiB on, the one-kernel form for small tensors below
         full = ev_ms(torch, lambda: L.cswap_zvc_compress_fused(t.data_ptr(), n, api.PROCESS, ws.data_ptr(),
                                                                begin.data_ptr(), nnz.data_ptr(),
                                                                values.data_ptr(), mask.data_ptr(), st), reps)

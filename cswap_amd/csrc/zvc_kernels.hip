@@ -674,9 +674,10 @@ __device__ __forceinline__ void st_status(uint32_t* p, uint32_t v)
 // starts on a half row), two status words per tile in the workspace, a 16-byte aligned
 // values pointer, and all G+1 workgroups resident at once (the waits are bounded).
 // Workspace (prepared once by cswap_zvc_workspace_clear; a run leaves it as it found it):
-// ws[16 + t] = kTileReady | count of tile t, ws[16 + tiles + t] = kTileReady | number of
-// non-zeros before tile t; the scanner clears a count when it has read it, a workgroup the
-// offsets of its tiles when it is through, so no launch is spent on clearing.
+// ws[status_at + t] = kTileReady | count of tile t, ws[offset_at + t] = kTileReady | number of
+// non-zeros before tile t (place_status_words says where); the scanner clears a count when it
+// has read it, a workgroup the offsets of its tiles when it is through, so no launch is spent on
+// clearing.
 //
 // Measured on one MI355X, half of the elements zero (this kernel / count + scan + compact):
 // 512 MiB 0.161 / 0.240 ms, 256 MiB 0.082 / 0.115 ms, 128 MiB 0.046 / 0.056, 64 MiB 0.031 /
@@ -691,17 +692,19 @@ constexpr uint32_t kTileReady = 1u << 31;
 struct StreamGeometry {
   int n, E, W, process, active;
   int rows;    // rows that exist in the mask layout: process * W / 2 rounded up
-  int tiles;   // ceil(rows / 256)
+  int tiles;   // rows / 192 rounded up
   int mask_words;
+  int status_at, offset_at;  // pipeline kernel: where the counts and the offsets of the tiles start in the workspace
 };
 
 // The scanner: one wavefront turns counts into offsets, 256 tiles at a time, in tile order.
-__device__ void zvc_stream_scanner(uint32_t* ws, int tiles, int step, int* nnz, unsigned spin_limit)
+__device__ void zvc_stream_scanner(uint32_t* ws, const StreamGeometry& g, int step, int* nnz, unsigned spin_limit)
 {
+  const int tiles = g.tiles;
   if (threadIdx.x >= 64) return;
   const unsigned lane = lane_id();
-  uint32_t* status = ws + 16;
-  uint32_t* offset = ws + 16 + tiles;
+  uint32_t* status = ws + g.status_at;
+  uint32_t* offset = ws + g.offset_at;
   const uint32_t magic = ld_status(&ws[0]), flag0 = ld_status(&ws[kWsFlag]);
   const bool refused = magic != kWsMagic || flag0 != 0u;
   if (refused && lane == 0) *nnz = -1;
@@ -775,13 +778,13 @@ __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
   __shared__ unsigned s_cnt[kSSlots][kSWaves];
   const int G = (int)gridDim.x - 1, w = (int)blockIdx.x;
   if (w == G) {
-    zvc_stream_scanner(ws, g.tiles, G, nnz, spin_limit);
+    zvc_stream_scanner(ws, g, G, nnz, spin_limit);
     return;
   }
   const unsigned lane = lane_id();
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  uint32_t* status = ws + 16;
-  uint32_t* offset = ws + 16 + g.tiles;
+  uint32_t* status = ws + g.status_at;
+  uint32_t* offset = ws + g.offset_at;
   const int iters = (g.tiles - w + G - 1) / G;  // >= 1: the grid has no more data workgroups than there are tiles
   // chunk index = half row / W by multiply and shift (exact while half rows * W < 2^40)
   const unsigned long long w_magic = ((1ull << 40) + (unsigned)g.W - 1) / (unsigned)g.W;
@@ -1013,19 +1016,23 @@ __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
 // 1.6 MB in 16384 chunks 14.4 -> 8.2.  64 rows per wavefront instead of the three kernels
 // (33.6 to 67 MB): 63.7 MB 31 -> 25.
 //
-// The counts live in two arrays of 256 words at the end of the workspace, used in turns: run
-// k publishes into array k & 1 and every workgroup clears its word of the other one, which
-// nobody reads any more; ws[kWsSmallRuns] counts the runs.  The grid is the same for every
-// size, so every word is cleared every time.  Failure works as in the pipeline kernel: a wait
-// that runs out raises the sticky flag, the offsets are kept inside the tensor, and the
-// wavefront that gave up writes -1 after the last workgroup has stepped the run counter.
+// The counts live in two arrays of 256 words, used in turns: run k publishes into array k & 1 and
+// every workgroup clears its word of the other one, which nobody reads any more;
+// ws[kWsSmallRuns] counts the runs.  The grid is the same for every size and the arrays have one
+// place in every workspace (status words 65024 to 65535, which the pipeline kernel leaves out),
+// whatever chunk count a call comes with, so every word is cleared every time.  Failure works as
+// in the pipeline kernel: a wait that runs out raises the sticky flag, the offsets are kept inside
+// the tensor, and the wavefront that gave up writes -1 after the last workgroup has stepped the
+// run counter.
 // The variants that took over shapes of the three kernels (RAGGED, 64 rows) must not fail where
 // those did not: a workgroup that finds the workspace unusable or whose wait runs out counts the
 // elements before its own by itself, which costs time and nothing else.
 constexpr int kQWaves = 16;
 constexpr int kQGroupsMax = 256;
 constexpr int kWsSmallRuns = 4;
-constexpr int kSmallWords = 2 * kQGroupsMax;  // taken from the end of the workspace's status words
+constexpr int kStatusWordsMin = 65536;  // status words of the smallest workspace
+constexpr int kSmallWords = 2 * kQGroupsMax;
+constexpr int kSmallCounts = kStatusWordsMin - kSmallWords;  // status word at which the two arrays start
 
 template <int R, bool RAGGED>
 __global__ __launch_bounds__(64 * kQWaves) void zvc_small_kernel(
@@ -1402,9 +1409,7 @@ extern "C" int cswap_zvc_pick_process(size_t n)
   return p;
 }
 
-constexpr int kStatusWordsMin = 65536;
-// status words of a workspace for `process` chunks: one per chunk for the look-back kernel,
-// one per tile for the pipeline kernel, never fewer than 65536
+// status words of a workspace for `process` chunks
 static int status_words(int process) { return process > kStatusWordsMin ? process : kStatusWordsMin; }
 
 extern "C" size_t cswap_zvc_workspace_bytes(int process)
@@ -1418,7 +1423,6 @@ extern "C" void cswap_zvc_debug_set_lookback(unsigned spin_limit, unsigned skip_
   g_skip_first.store(skip_first);
 }
 
-static int status_words(int process);
 // Tensors of at least this many bytes take the single pass in cswap_zvc_compress_fused; smaller ones
 // finish sooner with the three kernels (a few rounds of the grid do not fill the pipeline).
 static std::atomic<unsigned long long> g_single_pass_bytes{64ull << 20};  // cswap_zvc_set_single_pass_bytes
@@ -1441,6 +1445,18 @@ static int stream_data_groups(int tiles, int compute_units)
 }
 extern "C" int cswap_test_zvc_stream_groups(int tiles, int compute_units) { return stream_data_groups(tiles, compute_units); }
 
+// Where the pipeline kernel's two arrays of one word per tile go: around the small form's words, which
+// hold the counts of its last run.  In front of them; with many tiles behind them, if the workspace is
+// one for enough chunks; or one array on either side.  False: no room.
+static bool place_status_words(StreamGeometry& sg, int process)
+{
+  const int behind = status_words(process) - kStatusWordsMin;
+  const bool front = 2 * sg.tiles <= kSmallCounts, back = 2 * sg.tiles <= behind;
+  sg.status_at = 16 + (!front && back ? kStatusWordsMin : 0);
+  sg.offset_at = front || back ? sg.status_at + sg.tiles : 16 + kStatusWordsMin;
+  return front || back || (sg.tiles <= kSmallCounts && sg.tiles <= behind);
+}
+
 // whether the single pass takes a tensor of this shape; fills its geometry
 static bool single_pass_shape(const Geometry& g, int n, int process, StreamGeometry& sg)
 {
@@ -1451,7 +1467,7 @@ static bool single_pass_shape(const Geometry& g, int n, int process, StreamGeome
   sg.tiles = (sg.rows + kSTileRows - 1) / kSTileRows;
   // whole half rows per chunk, two status words per tile in the workspace, a compute unit for
   // every workgroup, and a tensor large enough to fill the pipeline
-  return g.E % 32 == 0 && mask_words < (1ll << 31) - 64 && 2 * sg.tiles <= status_words(process) - kSmallWords &&
+  return g.E % 32 == 0 && mask_words < (1ll << 31) - 64 && place_status_words(sg, process) &&
          device_compute_units() > 1 && 4ull * (unsigned long long)n >= g_single_pass_bytes;
 }
 
@@ -1468,7 +1484,7 @@ static bool small_pass_shape(const Geometry& g, int n, int process, StreamGeomet
   const long long mask_words = (long long)g.W * process;
   sg.mask_words = (int)mask_words;
   sg.rows = (int)((mask_words + 1) / 2);
-  sg.tiles = 0;
+  sg.tiles = sg.status_at = sg.offset_at = 0;
   const int cus = device_compute_units();
   const int G = cus < kQGroupsMax ? cus : kQGroupsMax;
   const unsigned long long single_from = g_single_pass_bytes.load();
@@ -1507,7 +1523,7 @@ extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, v
   const bool single_pass = single_pass_shape(g, n, process, sg) && (reinterpret_cast<uintptr_t>(d_values) & 15u) == 0;
   int groups = 0, rows = 0;
   if (!single_pass && small_pass_shape(g, n, process, sg, &groups, &rows, true)) {
-    uint32_t* counts = ws + 16 + status_words(process) - kSmallWords;
+    uint32_t* counts = ws + 16 + kSmallCounts;
 #define CSWAP_SMALL(R, RAGGED)                                                                                     \
   hipLaunchKernelGGL((zvc_small_kernel<R, RAGGED>), dim3(groups), dim3(64 * kQWaves), 0, (hipStream_t)stream, d_in, \
                      sg, ws, counts, d_begin, d_nnz, d_values, d_mask, g_spin_limit.load(), g_skip_first.load())

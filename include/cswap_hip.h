@@ -190,10 +190,12 @@ int cswap_zvc_compress(const float* d_in, int n, int process, int* d_begin, int*
  * workspace of cswap_zvc_workspace_bytes(process) bytes (at least 256 KiB) that
  * cswap_zvc_workspace_clear has prepared once, after it was allocated; every call
  * that succeeds leaves it ready for the next one (the kernel clears each status
- * word as it consumes it, so no launch is spent on clearing); calls that share a
+ * word as it consumes it, so no launch is spent on clearing), also one with
+ * another chunk count, up to the `process` of the workspace; calls that share a
  * workspace must not overlap.  Shapes the one-kernel forms do not take -- for the
  * pipeline a chunk length that is not a multiple of 32, d_values not 16-byte
- * aligned or more than 32512 tiles of 12288 elements -- run the three kernels instead.  The workgroups
+ * aligned or more tiles of 12288 elements than the workspace has room for (32512, more with
+ * `process` above 65536) -- run the three kernels instead.  The workgroups
  * wait for each other's counts; that wait is bounded, and if it ever runs out (for
  * example because the pipeline kernel, whose 256 workgroups all have to run at the
  * same time, does not get the whole GPU) the kernel still finishes

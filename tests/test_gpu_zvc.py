@@ -529,3 +529,104 @@ def test_one_kernel_form_of_any_chunk_length(torch_cuda, n, process, workspace):
             assert np.array_equal(out[:n].cpu().numpy().view(np.uint32), want.view(np.uint32))
     finally:
         L.cswap_zvc_set_single_pass_bytes(before)
+
+
+def _fused(torch, L, ws, x, process):
+    """One cswap_zvc_compress_fused call on this workspace; its outputs on the host."""
+    from cswap_amd._lib import check
+
+    n, W = x.size, L.cswap_zvc_chunk_words(x.size, process)
+    t = torch.from_numpy(x).cuda()
+    values = torch.full((n,), 7.0, device="cuda")
+    mask = torch.full((W * process,), -1, dtype=torch.int32, device="cuda")
+    begin = torch.full((process,), -5, dtype=torch.int32, device="cuda")
+    nnz = torch.zeros(1, dtype=torch.int32, device="cuda")
+    check(L.cswap_zvc_compress_fused(t.data_ptr(), n, process, ws.data_ptr(), begin.data_ptr(), nnz.data_ptr(),
+                                     values.data_ptr(), mask.data_ptr(), None), "fused")
+    torch.cuda.synchronize()
+    return int(nnz.item()), values.cpu().numpy(), mask.cpu().numpy(), begin.cpu().numpy()
+
+
+def _equals_oracle(got, x, process):
+    import oracle
+
+    ov, om, ob, on = oracle.zvc_compress(x, process)
+    active = oracle.zvc_geometry(x.size, process)[2]
+    assert got[0] == on
+    assert np.array_equal(got[1][:on].view(np.uint32), ov[:on].view(np.uint32))
+    assert np.array_equal(got[2].view(np.uint32), om)
+    assert np.array_equal(got[3][:active], ob[:active])
+
+
+def test_one_workspace_for_chunk_counts_either_side_of_65536(torch_cuda):
+    """A workspace takes calls with any chunk count up to its own, in any order.  The counts that the
+    one-kernel form leaves behind for its next run are where that run looks, whatever its chunk
+    count, and where the pipeline kernel never does.  Other data in every run, so that stale counts
+    are not the right ones."""
+    from cswap_amd import api
+    from cswap_amd._lib import lib
+
+    torch = torch_cuda
+    L = lib()
+    most = 131072
+    ws = api.zvc_workspace(most)
+    words = ws.view(torch.int32)
+    rng = np.random.default_rng(11)
+    before = L.cswap_zvc_set_single_pass_bytes(64 << 20)
+    try:
+        runs = 0
+        for n, process in ((100_000 * 33, 100_000), (P * 64, P), (100_000 * 33, 100_000), (most * 64, most), (P * 128 - 5, P),
+                           (P * 1024, P), (most * 32 - 9, most), (65_537 * 32, 65_537), (P * 700 + 11, P), (100_000 * 33, 100_000)):
+            x = (rng.standard_normal(n, dtype=np.float32) * (rng.random(n, dtype=np.float32) < rng.uniform(0.2, 0.8))).astype(np.float32)
+            print("n", n, "process", process, flush=True)
+            _equals_oracle(_fused(torch, L, ws, x, process), x, process)
+            runs += n != P * 1024                                # that one is the pipeline kernel's
+            assert int(words[4].item()) == runs and int(words[1].item()) == 0
+            left = words[16:].clone()
+            last = 65024 + 256 * ((runs - 1) & 1)
+            assert int(left[last:last + 256].count_nonzero().item()) == 256
+            left[last:last + 256] = 0
+            assert int(left.count_nonzero().item()) == 0
+    finally:
+        L.cswap_zvc_set_single_pass_bytes(before)
+
+
+@pytest.mark.parametrize("process,n", [(131072, 131072 * 3840 - 6144), (1 << 20, (1 << 20) * 416 - 200)])
+def test_pipeline_words_leave_out_the_small_forms(torch_cuda, process, n):
+    """Tensors of more tiles than fit in front of the small form's counts: the pipeline's two arrays go
+    on either side of them (131072 chunks) or behind them (2^20 chunks), between runs of the small
+    form that find their words as they left them.  Against the three kernels."""
+    from cswap_amd import api
+    from cswap_amd._lib import lib
+
+    torch = torch_cuda
+    L = lib()
+    before = L.cswap_zvc_set_single_pass_bytes(64 << 20)
+    try:
+        assert n > 32512 * 12288
+        assert L.cswap_zvc_chunk_elems(n, process) % 32 == 0 and L.cswap_zvc_takes_single_pass(n, process) == 1
+        ws = api.zvc_workspace(process)
+        rng = np.random.default_rng(process)
+        small = [np.maximum(rng.standard_normal(P * 64 + k), 0).astype(np.float32) for k in (0, 3, 9)]
+        _equals_oracle(_fused(torch, L, ws, small[0], P), small[0], P)
+        g = torch.Generator(device="cuda"); g.manual_seed(process)
+        t = torch.empty(n, device="cuda").normal_(generator=g).clamp_(min=0.0)
+        print("pipeline", n, process, flush=True)
+        want = api.zvc_compress(t, process)
+        got = [torch.zeros_like(o) for o in want]
+        assert L.cswap_zvc_compress_fused(t.data_ptr(), n, process, ws.data_ptr(), got[2].data_ptr(), got[3].data_ptr(),
+                                          got[0].data_ptr(), got[1].data_ptr(), None) == 0
+        torch.cuda.synchronize()
+        k = int(want[3].item())
+        assert int(got[3].item()) == k
+        assert torch.equal(got[0][:k], want[0][:k]) and torch.equal(got[1], want[1])
+        active = L.cswap_zvc_active_chunks(n, process)
+        assert torch.equal(got[2][:active], want[2][:active])
+        left = ws.view(torch.int32)[16:].clone()
+        assert int(left[65024:65280].count_nonzero().item()) == 256    # the first small run's counts
+        left[65024:65280] = 0
+        assert int(left.count_nonzero().item()) == 0
+        for x in small[1:]:
+            _equals_oracle(_fused(torch, L, ws, x, P), x, P)
+    finally:
+        L.cswap_zvc_set_single_pass_bytes(before)

@@ -1026,7 +1026,11 @@ __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
 // run counter.
 // The variants that took over shapes of the three kernels (RAGGED, 64 rows) must not fail where
 // those did not: a workgroup that finds the workspace unusable or whose wait runs out counts the
-// elements before its own by itself, which costs time and nothing else.
+// elements before its own by itself, which costs time and nothing else.  The last workgroup alone
+// steps the run counter, and only when it has seen everybody's count, so that everybody has taken
+// the same array: had it stepped past a workgroup that is still to start, that one would publish
+// into the next run's array.  If its wait runs out it leaves the counter and raises the flag
+// instead, which keeps later runs away from the words until they are cleared.
 constexpr int kQWaves = 16;
 constexpr int kQGroupsMax = 256;
 constexpr int kWsSmallRuns = 4;
@@ -1149,7 +1153,7 @@ __global__ __launch_bounds__(64 * kQWaves) void zvc_small_kernel(
       }
       if (__ballot(missing) == 0ull && !refused) break;
       if (refused || ++spins > spin_limit) {
-        if (!kCountsItself && lane == 0) atomicOr(&ws[kWsFlag], 1u);
+        if (!refused && (!kCountsItself || w == G - 1) && lane == 0) atomicOr(&ws[kWsFlag], 1u);
         gave_up = true;
         break;
       }
@@ -1224,7 +1228,7 @@ __global__ __launch_bounds__(64 * kQWaves) void zvc_small_kernel(
   if (w == G - 1 && threadIdx.x == 0) {
     *nnz = (gave_up || flag_late != 0u) ? -1 : (int)s_head[3];
     __threadfence();
-    if (!refused) __hip_atomic_fetch_add(&ws[kWsSmallRuns], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!refused && !(kCountsItself && s_head[4] != 0u)) __hip_atomic_fetch_add(&ws[kWsSmallRuns], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   } else if (gave_up && w != G - 1) {  // (wavefront 0 of another workgroup) after the last workgroup has spoken
     for (unsigned spins = 0; ld_status(&ws[kWsSmallRuns]) == runs0 && spins < spin_limit; spins++)
       __builtin_amdgcn_s_sleep(2);

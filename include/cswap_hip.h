@@ -204,8 +204,11 @@ int cswap_zvc_compress(const float* d_in, int n, int process, int* d_begin, int*
  * synchronise).  A workspace that was never prepared is reported the same way, and
  * so is every later call on a workspace after a failure, until
  * cswap_zvc_workspace_clear has been called on it again.  Shapes for which
- * cswap_zvc_takes_single_pass is 0 never fail: whatever the workspace holds, their
- * result is right. */
+ * cswap_zvc_takes_single_pass is 0 never report failure: where the workspace was not
+ * prepared, or a failure has been left in it, or their own wait runs out (which leaves
+ * one for the calls of other shapes), they count again what they cannot read there, so
+ * their result is right and takes longer.  They use the workspace all the same while
+ * it is good: calls that overlap on one are wrong for them, too. */
 size_t cswap_zvc_workspace_bytes(int process);
 int cswap_zvc_compress_fused(const float* d_in, int n, int process, void* d_ws, int* d_begin,
                              int* d_nnz, float* d_values, uint32_t* d_mask, cswap_stream_t stream);

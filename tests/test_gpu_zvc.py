@@ -630,3 +630,51 @@ def test_pipeline_words_leave_out_the_small_forms(torch_cuda, process, n):
             _equals_oracle(_fused(torch, L, ws, x, P), x, P)
     finally:
         L.cswap_zvc_set_single_pass_bytes(before)
+
+
+@pytest.mark.parametrize("n,process", [(P * 64 - 5 * P + 7, P), (P * 700 + 11, P), (P * 1024 - 32, P), (100_003, 1024)])
+def test_workspace_after_a_wait_that_ran_out(torch_cuda, n, process):
+    """The shapes that cannot fail, when the counts they wait for never come: their result is right,
+    and what they leave in the workspace misleads nobody -- the failure flag is up, the run counter
+    has not moved on from workgroups that may not have read it, and without clearing the next calls
+    give the right result from other data (the shapes that cannot fail) or -1 (the one that
+    can).  Cleared, all of them are right again."""
+    from cswap_amd import api
+    from cswap_amd._lib import check, lib
+
+    torch = torch_cuda
+    L = lib()
+    before = L.cswap_zvc_set_single_pass_bytes(64 << 20)
+    try:
+        ws = api.zvc_workspace(P)
+        words = ws.view(torch.int32)
+        rng = np.random.default_rng(n)
+
+        def data(m):
+            return (rng.standard_normal(m, dtype=np.float32) * (rng.random(m, dtype=np.float32) < rng.uniform(0.2, 0.8))).astype(np.float32)
+
+        assert L.cswap_zvc_takes_single_pass(n, process) == 0 and L.cswap_zvc_takes_single_pass(P * 256, P) == 2
+        x = data(n)
+        _equals_oracle(_fused(torch, L, ws, x, process), x, process)
+        assert int(words[1].item()) == 0 and int(words[4].item()) == 1
+        x = data(n)
+        L.cswap_zvc_debug_set_lookback(4, 1)
+        try:
+            print("forced give-up", flush=True)
+            got = _fused(torch, L, ws, x, process)
+        finally:
+            L.cswap_zvc_debug_set_lookback(0, 0)
+        _equals_oracle(got, x, process)
+        assert int(words[1].item()) == 1 and int(words[4].item()) == 1
+        others = ((n, process), (P * 90 + 7, P), (P * 1024 - 64, P))
+        for m, k in others:
+            x = data(m)
+            _equals_oracle(_fused(torch, L, ws, x, k), x, k)
+        assert _fused(torch, L, ws, data(P * 256), P)[0] == -1
+        check(L.cswap_zvc_workspace_clear(ws.data_ptr(), P, None), "clear")
+        for m, k in others + ((P * 256, P), (n, process)):
+            x = data(m)
+            _equals_oracle(_fused(torch, L, ws, x, k), x, k)
+        assert int(words[1].item()) == 0 and int(words[4].item()) == 5
+    finally:
+        L.cswap_zvc_set_single_pass_bytes(before)

@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 #include <atomic>
 #include "../../include/cswap_hip.h"
+#include "../../include/cswap_test_hooks.h"
 #include "zfp_block.h"
 #include "common.h"
 
@@ -1484,12 +1485,24 @@ static bool pair_shape(const Field3& fd, unsigned maxbits)
   return fd.rows16 && fd.stream16 && (maxbits & 255u) == 0 && ((fd.nx | fd.ny | fd.nz) & 3u) == 0;
 }
 
+// Whether the encoder loads with the nontemporal hint (make_field: read_once); the variants that do are
+// those of whole-word rates.
+static bool load_hint(const Field3& fd, bool whole) { return fd.read_once && fd.rows16 && whole; }
+
 // Which fields the kernels for contiguous rows at any element take.  The encoder's: all that are not
-// whole blocks of aligned rows.  The decoder's leave those whose rows are aligned and whole along x:
-// there only the last block rows are cut off, and the hint on the others' whole lines is worth more
-// (39 MB in 197 rows of 768: encode 20.8 us either way, decode 16.2 with the other kernel, 17.1 with
-// this; 57 MB in 197 rows of 196: encode 28.1 and 26.3, decode 28.3 both).
-static bool encode_rows(const Field3& fd) { return fd.rows4 && !(fd.full && fd.rows16); }
+// whole blocks of aligned rows.  Both leave fields whose rows are aligned and whole along x to the other
+// kernel where that one has the hint: only the last block rows are cut off there, and the hint on the
+// others' whole lines is worth more.  The decoder's has it always (39 MB in 197 rows of 768: encode
+// 20.8 us either way, decode 16.2 with the other kernel, 17.1 with this; 57 MB in 197 rows of 196: encode
+// 28.1 and 26.3, decode 28.3 both), the encoder's on large fields (producer kernel + encoder, other kernel
+// / this, 197 rows of 768 or 3072: 201 MB at 8 bits per value 116 / 123 us, 290 MB 156 / 172, 402 MB
+// 220 / 232; the encoder by itself, over and over on what is cached, 59.9 / 58.8, 74.1 / 75.8 and 101.1 /
+// 100.7, at 16 bits 71.2 / 73.7, 96.0 / 103.9 and 127 / 140).  Cut off along x, the hint gains less
+// than the rows (203 MB in 197 rows of 771 at a pitch of 772: 130 / 124).
+static bool encode_rows(const Field3& fd, bool whole)
+{
+  return fd.rows4 && !(fd.full && fd.rows16) && !(load_hint(fd, whole) && (fd.nx & 3u) == 0);
+}
 static bool decode_rows(const Field3& fd) { return fd.rows4 && !(fd.rows16 && (fd.nx & 3u) == 0); }
 
 static std::atomic<unsigned long long> g_pair_decode_bytes{CSWAP_PAIR_DECODE_BYTES};
@@ -1537,6 +1550,18 @@ extern "C" void cswap_zfp_set_pair_bytes(size_t encode_below, size_t decode_belo
   }
 }
 
+extern "C" int cswap_test_zfp_encode_route(size_t nx, size_t ny, size_t nz, ptrdiff_t sy, ptrdiff_t sz, unsigned misaligned,
+                                           unsigned maxbits)
+{
+  Field3 fd;
+  const uintptr_t base = 4096 + 4 * (uintptr_t)misaligned;  // looked at for its alignment only
+  int rc = make_field(fd, reinterpret_cast<const void*>(base), reinterpret_cast<const void*>(4096), nx, ny, nz, 1, sy, sz,
+                      maxbits, 4);
+  if (rc) return rc;
+  const bool whole = (maxbits & 63u) == 0;
+  return encode_rows(fd, whole) ? 1 : load_hint(fd, whole) ? 2 : 0;
+}
+
 #define CSWAP_LAUNCH3(KERNEL_, T_, ARG0_, ARG3_)                                                                   \
   do {                                                                                                              \
     if (whole && !is_int)                                                                                           \
@@ -1577,8 +1602,8 @@ static int compress3(const void* d_in, Elem elem, size_t nx, size_t ny, size_t n
   }
   if (elem_bytes(elem) == 4) {
     const float* in = static_cast<const float*>(d_in);
-    const bool once = fd.read_once && fd.rows16;
-    if (encode_rows(fd)) {
+    const bool once = load_hint(fd, whole);
+    if (encode_rows(fd, whole)) {
       if (whole && maxbits >= kFewerWavesFrom && !is_int)
         hipLaunchKernelGGL((zfp_encode3_rows_kernel<true, false, 3>), dim3(grid), dim3(64), lds_bytes, st, in, fd, maxbits,
                            d_stream);
@@ -1600,10 +1625,10 @@ static int compress3(const void* d_in, Elem elem, size_t nx, size_t ny, size_t n
       else
         hipLaunchKernelGGL((zfp_encode3_f32_kernel<true, true, false, 3>), dim3(grid), dim3(64), lds_bytes, st, in,
                            fd, maxbits, d_stream);
-    } else if (fd.read_once && fd.rows16 && whole && !is_int)
+    } else if (once && !is_int)
       hipLaunchKernelGGL((zfp_encode3_f32_kernel<true, false, true>), dim3(grid), dim3(64), lds_bytes, st, in, fd,
                          maxbits, d_stream);
-    else if (fd.read_once && fd.rows16 && whole)
+    else if (once)
       hipLaunchKernelGGL((zfp_encode3_f32_kernel<true, true, true>), dim3(grid), dim3(64), lds_bytes, st, in, fd,
                          maxbits, d_stream);
     else

@@ -9,6 +9,8 @@
 #ifndef CSWAP_TEST_HOOKS_H
 #define CSWAP_TEST_HOOKS_H
 
+#include <stddef.h>
+
 #ifdef __cplusplus
 extern "C" {
 #endif
@@ -24,6 +26,13 @@ void cswap_zvc_debug_set_lookback(unsigned spin_limit, unsigned skip_first);
  * tensor of `tiles` tiles on a part with `compute_units` compute units (the scanner's
  * workgroup comes on top).  Host only. */
 int cswap_test_zvc_stream_groups(int tiles, int compute_units);
+
+/* Which of the encoder's one-lane-per-block kernels a 3-D field of 32-bit elements with contiguous
+ * x-rows runs where no other form takes it: 0 the general one, 1 the one for rows at any element,
+ * 2 the general one with the nontemporal load hint; or an error code.  sy, sz: strides in elements
+ * (0 = packed), misaligned: elements that the field starts past a 16-byte boundary.  Host only. */
+int cswap_test_zfp_encode_route(size_t nx, size_t ny, size_t nz, ptrdiff_t sy, ptrdiff_t sz, unsigned misaligned,
+                                unsigned maxbits);
 
 #ifdef __cplusplus
 }

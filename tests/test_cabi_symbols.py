@@ -77,3 +77,24 @@ def test_pipeline_kernel_grid_fits_its_scanner_on_any_part():
     assert f(100, 256) == 100            # fewer tiles than compute units
     assert f(5, 304) == 5
     assert f(10000, 2) == 1 and f(10000, 1) == 0
+
+
+def test_large_aligned_fields_keep_the_load_hint():
+    """The encoder's nontemporal loads are for fields of 128 MiB and more whose rows are aligned and
+    whole along x, also where blocks are cut off along y or z; every other field that is not all
+    whole blocks of aligned rows takes the kernel for rows at any element."""
+    from cswap_amd import _lib
+
+    route = _lib.lib().cswap_test_zfp_encode_route
+    general, rows, hint = 0, 1, 2
+    for maxbits in (256, 512, 1024):
+        assert route(768, 512, 128, 0, 0, 0, maxbits) == hint            # all whole blocks, 201 MB
+        assert route(768, 197, 332, 0, 0, 0, maxbits) == hint            # 197 rows: cut off along y
+        assert route(4096, 512, 30, 0, 0, 0, maxbits) == hint            # along z
+        assert route(768, 49, 1001, 772, 772 * 49, 0, maxbits) == hint   # along both, pitched
+    assert route(768, 197, 332, 0, 0, 0, 520) == rows                    # no hinted variant at this rate
+    assert route(771, 197, 332, 772, 772 * 197, 0, 512) == rows          # cut off along x
+    assert route(768, 197, 332, 0, 0, 1, 512) == rows                    # rows at any element
+    assert route(768, 197, 220, 0, 0, 0, 512) == rows                    # 133 MB: below the hint's size
+    assert route(768, 512, 64, 0, 0, 0, 512) == general
+    assert route(1, 512, 64, 0, 0, 0, 512) == general

@@ -194,6 +194,41 @@ def test_rows_at_any_element(torch_cuda, nx, ny, nz, shift, gap, zfp_form):
         assert np.all(o == -7.0), maxbits   # nothing outside the field was touched
 
 
+@pytest.mark.parametrize("nx,ny,nz", [(768, 197, 226), (4096, 513, 17)])
+def test_large_field_cut_off_along_y_or_z(torch_cuda, nx, ny, nz):
+    """Fields of 128 MiB and more in aligned rows, the last blocks cut off: the encoder loads them with
+    the nontemporal hint.  The same field one element further takes the kernel for rows at any
+    element: the streams must be the same, and so must the blocks at both ends be the checker's."""
+    torch = torch_cuda
+    import oracle
+    from cswap_amd._lib import check, lib
+
+    L = lib()
+    n = nx * ny * nz
+    assert L.cswap_test_zfp_encode_route(nx, ny, nz, 0, 0, 0, 512) == 2 and L.cswap_test_zfp_encode_route(nx, ny, nz, 0, 0, 1, 512) == 1
+    g = torch.Generator(device="cuda"); g.manual_seed(nx)
+    t = torch.randn(n + 4, generator=g, device="cuda")
+    for maxbits in (512, 1024):
+        out = []
+        for shift in (0, 1):
+            if shift:
+                t[1:n + 1] = t[:n].clone()
+            s = torch.zeros(L.cswap_zfp_stream_capacity(nx, ny, nz, maxbits), dtype=torch.uint8, device="cuda")
+            check(L.cswap_zfp_compress_f32(t.data_ptr() + 4 * shift, nx, ny, nz, 0, 0, 0, maxbits, s.data_ptr(), None), "compress")
+            out.append(s)
+        torch.cuda.synchronize()
+        assert torch.equal(out[0], out[1]), maxbits
+        slab = nx * ny
+        f = t[1:n + 1].view(nz, ny, nx)
+        t[:n] = f.reshape(-1).clone()
+        words = out[0].view(torch.int64)
+        per_slab = -(-nx // 4) * -(-ny // 4) * maxbits // 64
+        for z0 in (0, (nz - 1) // 4 * 4):
+            part = t[z0 * slab:min(nz, z0 + 4) * slab].view(-1, ny, nx).cpu().numpy()
+            got = words[z0 // 4 * per_slab:(z0 // 4 + 1) * per_slab].cpu().numpy().view(np.uint64)
+            assert np.array_equal(got, oracle.zfp_encode3(part, maxbits)), (maxbits, z0)
+
+
 @pytest.mark.parametrize("nx,ny,nz", [(1, 1, 1), (4, 4, 60), (4, 4, 64), (4, 4, 68), (13, 1, 2), (9, 10, 11), (64, 64, 4 * 45),
                                       (64, 64, 4 * 46), (35, 35, 4 * 285)])
 @pytest.mark.parametrize("order", ["xyz", "zyx", "reversed"])

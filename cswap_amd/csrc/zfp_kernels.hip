@@ -1531,13 +1531,25 @@ constexpr unsigned kPairDecodeFromBits = 1024;
 //           19: 14.9 / - / 17.7 · 30: 20.2 / - / 17.4
 //   decode  1: 9.2 / - / 11.8 · 4: 10.6 / - / 12.8 · 8: 11.2 / - / 12.4 · 12: 12.6 / - / 12.6 · 16: 13.9 / - / 13.4;
 //           odd planes 8: 11.6 / - / 14.2 · 10: 14.0 / - / 15.4 · 19: 21.0 / - / 18.3
-// 4 and 16 bits per value cross at the same places.
+// Other rates, quad / the better of the other two.  Against the pair form and in the decoder the quad form
+// is ahead or level at its last size, 11, at all of them (encode 2 bits per value 8.6 / 10.3 · 16: 11.2 / 11.7 ·
+// 32: 12.5 / 14.4 · 64: 13.6 / 18.2; decode 10.4 / 10.3 · 14.6 / 14.7 · 14.8 / 16.0 · 15.5 / 17.8).  The encoder
+// of odd planes, 35x35: 2 bits 21: 12.0 / 13.3 · 16 bits 20: 16.2 / 17.8 · 22: 18.7 / 18.1 · 24 bits 18: 17.2 / 18.7 ·
+// 20: 20.5 / 19.3 · 28 bits 18: 17.8 / 19.5 · 20: 20.8 / 20.2 · 32 bits 20: 21.3 / 21.3 · 22: 22.3 / 22.3 ·
+// 40 bits 22: 23.7 / 24.6 · 64 bits 21: 25.8 / 40.7.  The steps are where the wavefronts' LDS no longer lets all of
+// them onto the chip at once; from 30 bits per value on one lane per block meets that limit, too.
 constexpr unsigned kQuadWaves = 11;        // per compute unit
 constexpr unsigned kQuadWavesNoPair = 22;  // the encoder's where the pair form does not apply
-static bool quad_pays(uint32_t nblocks, unsigned waves, unsigned long long bytes, unsigned long long pair_below)
+constexpr unsigned kQuadOneRoundBelow = 1920;
+static double quad_waves_encode(const Field3& fd, unsigned maxbits)
 {
-  return pair_below != ~0ull && bytes < pair_below &&
-         (unsigned long long)nblocks <= (unsigned long long)kQuadBlocks * waves * (unsigned)device_compute_units();
+  if (pair_shape(fd, maxbits)) return kQuadWaves;
+  const double fit = 0.92 * 160.0 * 1024.0 / (4.0 * (double)quad_lds_dwords(slot_bits(maxbits)));
+  return maxbits < kQuadOneRoundBelow && fit < kQuadWavesNoPair ? fit : kQuadWavesNoPair;
+}
+static bool quad_pays(uint32_t nblocks, double waves, unsigned long long bytes, unsigned long long pair_below, int compute_units)
+{
+  return pair_below != ~0ull && bytes < pair_below && (double)nblocks <= (double)kQuadBlocks * waves * (double)compute_units;
 }
 
 extern "C" void cswap_zfp_set_pair_bytes(size_t encode_below, size_t decode_below, size_t* previous)
@@ -1551,7 +1563,7 @@ extern "C" void cswap_zfp_set_pair_bytes(size_t encode_below, size_t decode_belo
 }
 
 extern "C" int cswap_test_zfp_encode_route(size_t nx, size_t ny, size_t nz, ptrdiff_t sy, ptrdiff_t sz, unsigned misaligned,
-                                           unsigned maxbits)
+                                           unsigned maxbits, int compute_units)
 {
   Field3 fd;
   const uintptr_t base = 4096 + 4 * (uintptr_t)misaligned;  // looked at for its alignment only
@@ -1559,6 +1571,9 @@ extern "C" int cswap_test_zfp_encode_route(size_t nx, size_t ny, size_t nz, ptrd
                       maxbits, 4);
   if (rc) return rc;
   const bool whole = (maxbits & 63u) == 0;
+  if (compute_units > 0 && whole && quad_pays(fd.nblocks, quad_waves_encode(fd, maxbits), (unsigned long long)nx * ny * nz * 4ull,
+                                              CSWAP_PAIR_ENCODE_BYTES, compute_units))
+    return 3;
   return encode_rows(fd, whole) ? 1 : load_hint(fd, whole) ? 2 : 0;
 }
 
@@ -1587,8 +1602,8 @@ static int compress3(const void* d_in, Elem elem, size_t nx, size_t ny, size_t n
   const bool whole = (maxbits & 63u) == 0;
   const bool is_int = elem == kI32 || elem == kI64;
   const unsigned long long pair_below = g_pair_encode_bytes.load(std::memory_order_relaxed);
-  if (elem == kF32 && whole && quad_pays(fd.nblocks, pair_shape(fd, maxbits) ? kQuadWaves : kQuadWavesNoPair,
-                                          (unsigned long long)nx * ny * nz * 4ull, pair_below)) {
+  if (elem == kF32 && whole && quad_pays(fd.nblocks, quad_waves_encode(fd, maxbits),
+                                          (unsigned long long)nx * ny * nz * 4ull, pair_below, device_compute_units())) {
     hipLaunchKernelGGL(zfp_encode3_f32_quad_kernel, dim3((fd.nblocks + kQuadBlocks - 1) / kQuadBlocks), dim3(64),
                        (size_t)quad_lds_dwords(slot_bits(maxbits)) * 4, st, static_cast<const float*>(d_in), fd, maxbits,
                        d_stream);
@@ -1653,7 +1668,8 @@ static int decompress3(const uint64_t* d_stream, Elem elem, size_t nx, size_t ny
   const bool whole = (maxbits & 63u) == 0;
   const bool is_int = elem == kI32 || elem == kI64;
   const unsigned long long pair_below = g_pair_decode_bytes.load(std::memory_order_relaxed);
-  if (elem == kF32 && whole && quad_pays(fd.nblocks, kQuadWaves, (unsigned long long)nx * ny * nz * 4ull, pair_below)) {
+  if (elem == kF32 && whole && quad_pays(fd.nblocks, kQuadWaves, (unsigned long long)nx * ny * nz * 4ull, pair_below,
+                                          device_compute_units())) {
     hipLaunchKernelGGL(zfp_decode3_f32_quad_kernel, dim3((fd.nblocks + kQuadBlocks - 1) / kQuadBlocks), dim3(64),
                        (size_t)quad_lds_dwords(dec_slot_bits(maxbits)) * 4, st, d_stream, fd, maxbits,
                        static_cast<float*>(d_out));

@@ -30,9 +30,11 @@ int cswap_test_zvc_stream_groups(int tiles, int compute_units);
 /* Which of the encoder's one-lane-per-block kernels a 3-D field of 32-bit elements with contiguous
  * x-rows runs where no other form takes it: 0 the general one, 1 the one for rows at any element,
  * 2 the general one with the nontemporal load hint; or an error code.  sy, sz: strides in elements
- * (0 = packed), misaligned: elements that the field starts past a 16-byte boundary.  Host only. */
+ * (0 = packed), misaligned: elements that the field starts past a 16-byte boundary.  3: as floats it
+ * runs the form with four lanes per block on a part with `compute_units` of them (0: that form is not
+ * asked about).  Host only. */
 int cswap_test_zfp_encode_route(size_t nx, size_t ny, size_t nz, ptrdiff_t sy, ptrdiff_t sz, unsigned misaligned,
-                                unsigned maxbits);
+                                unsigned maxbits, int compute_units);
 
 #ifdef __cplusplus
 }

@@ -85,7 +85,7 @@ def test_large_aligned_fields_keep_the_load_hint():
     whole blocks of aligned rows takes the kernel for rows at any element."""
     from cswap_amd import _lib
 
-    route = _lib.lib().cswap_test_zfp_encode_route
+    route = lambda *a: _lib.lib().cswap_test_zfp_encode_route(*a, 0)
     general, rows, hint = 0, 1, 2
     for maxbits in (256, 512, 1024):
         assert route(768, 512, 128, 0, 0, 0, maxbits) == hint            # all whole blocks, 201 MB
@@ -98,3 +98,24 @@ def test_large_aligned_fields_keep_the_load_hint():
     assert route(768, 197, 220, 0, 0, 0, 512) == rows                    # 133 MB: below the hint's size
     assert route(768, 512, 64, 0, 0, 0, 512) == general
     assert route(1, 512, 64, 0, 0, 0, 512) == general
+
+
+def test_four_lanes_per_block_while_they_fit_at_once():
+    """The encoder's form for the smallest fields, where the pair form does not apply: up to 22 wavefronts
+    of 16 blocks per compute unit, fewer at the rates where their LDS lets fewer of them run at once
+    and one lane per block does not have that limit itself."""
+    from cswap_amd import _lib
+
+    def limit(maxbits, cus=256, plane=35):
+        """wavefronts per compute unit up to which a field of odd planes runs the form"""
+        per_slab = ((plane + 3) // 4) ** 2
+        slabs = 1
+        while _lib.lib().cswap_test_zfp_encode_route(plane, plane, 4 * slabs, 0, 0, 0, maxbits, cus) == 3:
+            slabs += 1
+        return (slabs - 1) * per_slab / 16 / cus
+
+    for maxbits in (128, 512, 768, 1920, 2048, 3072, 4096):
+        assert 21.5 < limit(maxbits) <= 22, maxbits
+    for maxbits, at_least, below in ((1024, 20, 23), (1280, 20, 22), (1536, 18, 20), (1792, 18, 20)):
+        assert at_least <= limit(maxbits) < below, maxbits
+        assert at_least <= limit(maxbits, cus=128) < below, maxbits

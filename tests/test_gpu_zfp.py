@@ -205,7 +205,8 @@ def test_large_field_cut_off_along_y_or_z(torch_cuda, nx, ny, nz):
 
     L = lib()
     n = nx * ny * nz
-    assert L.cswap_test_zfp_encode_route(nx, ny, nz, 0, 0, 0, 512) == 2 and L.cswap_test_zfp_encode_route(nx, ny, nz, 0, 0, 1, 512) == 1
+    assert L.cswap_test_zfp_encode_route(nx, ny, nz, 0, 0, 0, 512, 0) == 2
+    assert L.cswap_test_zfp_encode_route(nx, ny, nz, 0, 0, 1, 512, 0) == 1
     g = torch.Generator(device="cuda"); g.manual_seed(nx)
     t = torch.randn(n + 4, generator=g, device="cuda")
     for maxbits in (512, 1024):

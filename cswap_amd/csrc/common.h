@@ -17,6 +17,13 @@ inline int hip_fail(hipError_t e)
 // compute units of the current device (0 if the query fails), looked up once per device
 int device_compute_units();
 
+// cswap_zfp_compress_f32 / cswap_zfp_decompress_f32 of a packed field without the form for the smallest
+// fields (four lanes per block), whatever the size
+int zfp_compress_f32_no_quad(const float* d_in, size_t nx, size_t ny, size_t nz, unsigned maxbits, uint64_t* d_stream,
+                             hipStream_t stream);
+int zfp_decompress_f32_no_quad(const uint64_t* d_stream, size_t nx, size_t ny, size_t nz, unsigned maxbits, float* d_out,
+                               hipStream_t stream);
+
 // to be called right after a kernel launch: picks up launch-configuration errors
 inline int check_launch()
 {

@@ -973,10 +973,12 @@ extern "C" int cswap_engine_calibrate(cswap_engine* e, cswap_costs* out_costs)
     if ((rc = ms(fdc, 2, &t))) break;
     if ((rc = ms(fdc, 10, &t))) break;
     c.zfp_decompress_gbs = gb / (t * 1e-3);
-    {  // fixed cost of a ZFP kernel: a field of one wavefront per SIMD at most (64 x 64 x 16 = 1024 blocks)
+    {  // Fixed cost of a ZFP kernel: a field of one wavefront per SIMD at most (64 x 64 x 16 = 1024 blocks).  The
+       // model charges it to tensors of every size, so it is that of the forms they share; the one for the
+       // smallest fields is 2 us shorter, which would have the selector take the lossy codec too early.
       double tc = 0, td = 0;
-      auto sc = [&]() { return cswap_zfp_compress_f32(d_x, 64, 64, 16, 0, 0, 0, e->maxbits, (uint64_t*)d_tmp, s); };
-      auto sd = [&]() { return cswap_zfp_decompress_f32((const uint64_t*)d_tmp, 64, 64, 16, 0, 0, 0, e->maxbits, d_y, s); };
+      auto sc = [&]() { return cswap::zfp_compress_f32_no_quad(d_x, 64, 64, 16, e->maxbits, (uint64_t*)d_tmp, s); };
+      auto sd = [&]() { return cswap::zfp_decompress_f32_no_quad((const uint64_t*)d_tmp, 64, 64, 16, e->maxbits, d_y, s); };
       if ((rc = ms(sc, 2, &tc))) break;
       if ((rc = ms(sc, 20, &tc))) break;
       if ((rc = ms(sd, 2, &td))) break;

@@ -1589,8 +1589,9 @@ extern "C" int cswap_test_zfp_encode_route(size_t nx, size_t ny, size_t nz, ptrd
       hipLaunchKernelGGL((KERNEL_<false, true>), dim3(grid), dim3(64), lds_bytes, st, ARG0_, fd, maxbits, ARG3_);   \
   } while (0)
 
+// quad: false leaves out the form with four lanes per block
 static int compress3(const void* d_in, Elem elem, size_t nx, size_t ny, size_t nz, ptrdiff_t sx, ptrdiff_t sy,
-                     ptrdiff_t sz, unsigned maxbits, uint64_t* d_stream, cswap_stream_t stream)
+                     ptrdiff_t sz, unsigned maxbits, uint64_t* d_stream, cswap_stream_t stream, bool quad = true)
 {
   if (!d_in || !d_stream) return CSWAP_E_ARG;
   Field3 fd;
@@ -1602,7 +1603,7 @@ static int compress3(const void* d_in, Elem elem, size_t nx, size_t ny, size_t n
   const bool whole = (maxbits & 63u) == 0;
   const bool is_int = elem == kI32 || elem == kI64;
   const unsigned long long pair_below = g_pair_encode_bytes.load(std::memory_order_relaxed);
-  if (elem == kF32 && whole && quad_pays(fd.nblocks, quad_waves_encode(fd, maxbits),
+  if (quad && elem == kF32 && whole && quad_pays(fd.nblocks, quad_waves_encode(fd, maxbits),
                                           (unsigned long long)nx * ny * nz * 4ull, pair_below, device_compute_units())) {
     hipLaunchKernelGGL(zfp_encode3_f32_quad_kernel, dim3((fd.nblocks + kQuadBlocks - 1) / kQuadBlocks), dim3(64),
                        (size_t)quad_lds_dwords(slot_bits(maxbits)) * 4, st, static_cast<const float*>(d_in), fd, maxbits,
@@ -1656,7 +1657,8 @@ static int compress3(const void* d_in, Elem elem, size_t nx, size_t ny, size_t n
 }
 
 static int decompress3(const uint64_t* d_stream, Elem elem, size_t nx, size_t ny, size_t nz, ptrdiff_t sx,
-                       ptrdiff_t sy, ptrdiff_t sz, unsigned maxbits, void* d_out, cswap_stream_t stream)
+                       ptrdiff_t sy, ptrdiff_t sz, unsigned maxbits, void* d_out, cswap_stream_t stream,
+                       bool quad = true)
 {
   if (!d_out || !d_stream) return CSWAP_E_ARG;
   Field3 fd;
@@ -1668,7 +1670,7 @@ static int decompress3(const uint64_t* d_stream, Elem elem, size_t nx, size_t ny
   const bool whole = (maxbits & 63u) == 0;
   const bool is_int = elem == kI32 || elem == kI64;
   const unsigned long long pair_below = g_pair_decode_bytes.load(std::memory_order_relaxed);
-  if (elem == kF32 && whole && quad_pays(fd.nblocks, kQuadWaves, (unsigned long long)nx * ny * nz * 4ull, pair_below,
+  if (quad && elem == kF32 && whole && quad_pays(fd.nblocks, kQuadWaves, (unsigned long long)nx * ny * nz * 4ull, pair_below,
                                           device_compute_units())) {
     hipLaunchKernelGGL(zfp_decode3_f32_quad_kernel, dim3((fd.nblocks + kQuadBlocks - 1) / kQuadBlocks), dim3(64),
                        (size_t)quad_lds_dwords(dec_slot_bits(maxbits)) * 4, st, d_stream, fd, maxbits,
@@ -1729,6 +1731,18 @@ extern "C" int cswap_zfp_decompress_f32(const uint64_t* d_stream, size_t nx, siz
                                         float* d_out, cswap_stream_t stream)
 {
   return decompress3(d_stream, kF32, nx, ny, nz, sx, sy, sz, maxbits, d_out, stream);
+}
+
+// A packed field through the forms that fields of every size share (common.h).
+int cswap::zfp_compress_f32_no_quad(const float* d_in, size_t nx, size_t ny, size_t nz, unsigned maxbits, uint64_t* d_stream,
+                                    hipStream_t stream)
+{
+  return compress3(d_in, kF32, nx, ny, nz, 0, 0, 0, maxbits, d_stream, stream, false);
+}
+int cswap::zfp_decompress_f32_no_quad(const uint64_t* d_stream, size_t nx, size_t ny, size_t nz, unsigned maxbits, float* d_out,
+                                      hipStream_t stream)
+{
+  return decompress3(d_stream, kF32, nx, ny, nz, 0, 0, 0, maxbits, d_out, stream, false);
 }
 
 // ------------------------------------------------------------- any dimensionality

@@ -285,6 +285,53 @@ def test_calibration_gives_sane_costs(torch_cuda):
     assert c.zvc_compress_gbs > 50 and c.zvc_expand_gbs > 50
 
 
+def test_calibrated_fixed_cost_is_that_of_fields_of_every_size(torch_cuda):
+    """The selector charges the fixed cost of a ZFP kernel to tensors of every size, so calibration
+    measures it without the form that only the smallest fields run: the time of a 1024-block field in
+    the other forms, not its time in that one (the two are about 2 us apart)."""
+    torch = torch_cuda
+    from cswap_amd import swap
+    from cswap_amd._lib import check, lib
+
+    L = lib()
+    x = torch.relu(torch.randn(16, 64, 64, device="cuda"))
+    s = torch.zeros(L.cswap_zfp_stream_capacity(64, 64, 16, 512), dtype=torch.uint8, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+
+    def microseconds(f, reps=50):
+        best = 1e9
+        for _ in range(7):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            f()
+            a.record()
+            for _ in range(reps):
+                f()
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 1e3 / reps)
+        return best
+
+    def both():
+        return 0.5 * (microseconds(lambda: check(L.cswap_zfp_compress_f32(x.data_ptr(), 64, 64, 16, 0, 0, 0, 512, s.data_ptr(), st), "c")) +
+                      microseconds(lambda: check(L.cswap_zfp_decompress_f32(s.data_ptr(), 64, 64, 16, 0, 0, 0, 512, x.data_ptr(), st), "d")))
+
+    smallest = both()
+    before = (C.c_size_t * 2)()
+    # as cswap_zfp_compress_f32 ran them before there was that form: encoder in the pair form, decoder one lane per block
+    L.cswap_zfp_set_pair_bytes(2 ** 64 - 1, 0, before)
+    try:
+        shared = both()
+    finally:
+        L.cswap_zfp_set_pair_bytes(before[0], before[1], None)
+    eng = swap.SwapEngine(pinned_bytes=256 << 20, device_bytes=64 << 20)
+    got = sorted(eng.calibrate().zfp_latency_us for _ in range(3))[1]
+    eng.close()
+    print("smallest", smallest, "shared", shared, "calibrated", got, flush=True)
+    assert shared > smallest + 1.0
+    # the engine's loop, with no Python between its launches, reads about half a microsecond less than this one
+    assert got > smallest + 0.35 * (shared - smallest)
+
+
 def test_reference_named_entry_points(torch_cuda):
     """cuda_compress / cuda_decompress with the reference's struct layout and
     device pointers (CSWAP+/simple.c:26-74 with device memory), compress /

@@ -79,6 +79,23 @@ def test_pipeline_kernel_grid_fits_its_scanner_on_any_part():
     assert f(10000, 2) == 1 and f(10000, 1) == 0
 
 
+def test_stream_handle_without_the_private_short_cut(monkeypatch):
+    """The handle of the current stream comes from torch's public interface where the short cut is
+    missing, and from the short cut, asked for the current device, where it is there."""
+    torch = pytest.importorskip("torch")
+    from cswap_amd import api
+
+    class Stream:
+        cuda_stream = 1234
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: Stream)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(api, "_raw_stream", None)
+    assert api._stream() == 1234
+    monkeypatch.setattr(api, "_raw_stream", lambda device: 100 + device)
+    assert api._stream() == 103
+
+
 def test_large_aligned_fields_keep_the_load_hint():
     """The encoder's nontemporal loads are for fields of 128 MiB and more whose rows are aligned and
     whole along x, also where blocks are cut off along y or z; every other field that is not all

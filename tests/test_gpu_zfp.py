@@ -194,6 +194,57 @@ def test_rows_at_any_element(torch_cuda, nx, ny, nz, shift, gap, zfp_form):
         assert np.all(o == -7.0), maxbits   # nothing outside the field was touched
 
 
+@pytest.mark.parametrize("nx,ny,nz,gap", [(35, 6, 9, 1), (35, 35, 64, 1), (6, 3, 129, 2), (7, 4, 90, 1), (261, 2, 5, 3), (2, 9, 70, 2),
+                                          (3, 4, 4, 5)])
+@pytest.mark.parametrize("kind", ["f32", "i32"])
+def test_aligned_rows_that_end_inside_a_block(torch_cuda, nx, ny, nz, gap, kind):
+    """Rows of an odd width at a pitch that keeps every one of them on a 16-byte boundary, one lane per
+    block: the decoder's whole row pieces there take the nontemporal store, and what is cut off must
+    end with the field.  NaNs (or large numbers) between the rows and around the field."""
+    import ctypes as C
+
+    torch = torch_cuda
+    import oracle
+    from cswap_amd._lib import check, lib
+
+    L = lib()
+    assert nx % 4 != 0 and (nx + gap) % 4 == 0
+    rng = np.random.default_rng(nx * 31 + ny + nz)
+    f = rng.standard_normal((nz, ny, nx)).astype(np.float32)
+    hole, mark, dtype = np.float32(np.nan), -7.0, torch.float32
+    encode, decode = oracle.zfp_encode3, oracle.zfp_decode3
+    compress = lambda *a: L.cswap_zfp_compress_f32(*a)
+    decompress = lambda *a: L.cswap_zfp_decompress_f32(*a)
+    if kind == "i32":
+        f, hole, mark, dtype = (f * 2.0 ** 20).astype(np.int32), np.int32(0x3fffffff), -7, torch.int32
+        encode, decode = oracle.zfp_encode_i32, oracle.zfp_decode_i32
+        compress = lambda p, *a: L.cswap_zfp_compress_i32_nd(p, 3, *a)
+        decompress = lambda p, *a: L.cswap_zfp_decompress_i32_nd(p, 3, *a)
+    big = np.full((nz, ny, nx + gap), hole, dtype=f.dtype)
+    big[:, :, :nx] = f
+    t = torch.from_numpy(np.concatenate([big.ravel(), np.full(8, hole, f.dtype)])).cuda()
+    sy, sz = nx + gap, ny * (nx + gap)
+    before = (C.c_size_t * 2)()
+    L.cswap_zfp_set_pair_bytes(0, 0, before)
+    try:
+        for maxbits in (512, 520, 1024):
+            s = torch.zeros(L.cswap_zfp_stream_capacity(nx, ny, nz, maxbits), dtype=torch.uint8, device="cuda")
+            out = torch.full(t.shape, mark, dtype=dtype, device="cuda")
+            assert out.data_ptr() % 16 == 0 and t.data_ptr() % 16 == 0
+            check(compress(t.data_ptr(), nx, ny, nz, 1, sy, sz, maxbits, s.data_ptr(), None), "compress")
+            check(decompress(s.data_ptr(), nx, ny, nz, 1, sy, sz, maxbits, out.data_ptr(), None), "decompress")
+            torch.cuda.synchronize()
+            want = encode(f, maxbits)
+            assert np.array_equal(s.cpu().numpy().view(np.uint64), want), maxbits
+            o = out.cpu().numpy()
+            inside = o[:big.size].reshape(big.shape)
+            assert np.array_equal(inside[:, :, :nx].view(np.uint32), decode(want, f.shape, maxbits).view(np.uint32)), maxbits
+            inside[:, :, :nx] = mark
+            assert np.all(o == mark), maxbits   # nothing outside the field was touched
+    finally:
+        L.cswap_zfp_set_pair_bytes(before[0], before[1], None)
+
+
 @pytest.mark.parametrize("nx,ny,nz", [(768, 197, 226), (4096, 513, 17)])
 def test_large_field_cut_off_along_y_or_z(torch_cuda, nx, ny, nz):
     """Fields of 128 MiB and more in aligned rows, the last blocks cut off: the encoder loads them with

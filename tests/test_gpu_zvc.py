@@ -17,8 +17,8 @@ def torch_cuda():
 
 @pytest.fixture(scope="module", autouse=True)
 def single_pass_at_any_size():
-    """cswap_zvc_compress_fused runs its single pass only from 64 MiB on (the three
-    kernels finish sooner below); the tests here want it on small shapes too."""
+    """cswap_zvc_compress_fused runs its pipeline kernel only from 64 MiB on (the one-kernel form
+    for small tensors finishes sooner below); the tests here want it on small shapes too."""
     from cswap_amd._lib import lib
 
     before = lib().cswap_zvc_set_single_pass_bytes(0)
@@ -30,7 +30,7 @@ def single_pass_at_any_size():
 def fused_form(request):
     """The two single-kernel forms behind cswap_zvc_compress_fused: the pipeline kernel, forced
     on at any size (what the module-wide fixture sets), and the one-kernel form that the size
-    rule picks for tensors of up to 32 MiB (the pipeline kernel takes over at 64 MiB)."""
+    rule picks below 64 MiB (up to 32 MiB the one that reports failure)."""
     from cswap_amd._lib import lib
 
     before = lib().cswap_zvc_set_single_pass_bytes(0 if request.param == "pipeline" else 64 << 20)
@@ -48,10 +48,10 @@ def test_size_rule_of_the_single_pass():
     mine = forced
     try:
         assert L.cswap_zvc_takes_single_pass(P * 512, P) == 2      # 32 MiB: the one-kernel form for small tensors
-        assert L.cswap_zvc_takes_single_pass(P * 512 + 32 * P, P) == 0   # 34 MiB: too large for it, three kernels
-        assert L.cswap_zvc_takes_single_pass(P * 64 + 5, P) == 0   # chunk length 65: three kernels
+        assert L.cswap_zvc_takes_single_pass(P * 512 + 32 * P, P) == 0   # 34 MiB: the small form's variant that cannot fail
+        assert L.cswap_zvc_takes_single_pass(P * 64 + 5, P) == 0   # chunk length 65: the same
         assert L.cswap_zvc_takes_single_pass(P * 1024, P) == 1     # 64 MiB: the pipeline kernel
-        assert L.cswap_zvc_takes_single_pass(P * 4096 + 5, P) == 0  # chunk length 4097: not whole half rows
+        assert L.cswap_zvc_takes_single_pass(P * 4096 + 5, P) == 0  # 256 MiB, chunk length 4097: three kernels
         assert L.cswap_zvc_takes_single_pass(1 << 30, 1024) == 0   # more tiles than the workspace has words for
     finally:
         L.cswap_zvc_set_single_pass_bytes(mine)
@@ -135,7 +135,8 @@ def test_expand_four_per_lane(torch_cuda, compact_form, n, process):
     LDS as for tensors beyond the cache size, which `compact_form` forces);
     the sizes end the last chunk inside a quad, inside a row and inside a refill
     group.  The same data is then expanded into a destination that is only
-    4-byte aligned, which takes the per-element kernel: both must agree."""
+    4-byte aligned, which takes the variants that store 16 bytes at any element: the checker's
+    result again, and nothing beside it."""
     import oracle
     from cswap_amd import api
 
@@ -154,6 +155,9 @@ def test_expand_four_per_lane(torch_cuda, compact_form, n, process):
     torch.cuda.synchronize()
     assert float(buf[0]) == -1.0
     assert np.array_equal(buf[1:].cpu().numpy().view(np.uint32), got[4].view(np.uint32))
+    want = x.copy()
+    want[x == 0] = 0.0
+    assert np.array_equal(buf[1:].cpu().numpy().view(np.uint32), want.view(np.uint32))
 
 
 @pytest.mark.parametrize("pct", [30, 50, 70, 90])

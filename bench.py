@@ -494,7 +494,8 @@ def zvc_extras(torch, api, dev, ex, config2_tensor, only_mib=0, cpu=False):
         full = ev_ms(torch, lambda: L.cswap_zvc_compress_fused(t.data_ptr(), n, api.PROCESS, ws.data_ptr(),
                                                                begin.data_ptr(), nnz.data_ptr(),
                                                                values.data_ptr(), mask.data_ptr(), st), reps)
-        single = bool(L.cswap_zvc_takes_single_pass(n, api.PROCESS))
+        # one kernel: the pipeline, or the form for tensors below 64 MiB of at most 262144 mask rows
+        single = L.cswap_zvc_takes_single_pass(n, api.PROCESS) == 1 or (4 * n < 64 << 20 and mask.numel() <= 2 * 262144)
         cnt = torch.zeros(api.PROCESS, dtype=torch.int32, device=dev)
         count = ev_ms(torch, lambda: L.cswap_zvc_count(t.data_ptr(), n, api.PROCESS, cnt.data_ptr(), st), reps)
         compact = ev_ms(torch, lambda: L.cswap_zvc_compact(t.data_ptr(), n, api.PROCESS, begin.data_ptr(),

@@ -343,22 +343,17 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_compact_rows_kernel(
 }
 
 // ------------------------------------------------------------------ expand
-// Same expansion with one lane = four consecutive elements and 16-byte stores
-// (with the nontemporal hint: 256 MiB expand in 63 instead of 88 us, 32 MiB in
+// One wavefront expands one chunk, one lane four consecutive elements with one 16-byte
+// store (with the nontemporal hint: 256 MiB expand in 63 instead of 88 us, 32 MiB in
 // 10.9 instead of 12.3 us, a reader of the result right after it no slower;
-// the same hint on the loads of the counting and compacting passes gains nothing):
-// the per-element form above issues one 4-byte store per lane and is bound by
-// that instruction stream, not by bytes.  A row is 256 elements = 8 mask words;
-// lane l keeps mask word 64*(row/8) + l of the chunk, together with the number
-// of set bits in the words before it inside its row, so a lane finds its nibble
-// and the rank of its first element with two cross-lane reads.
+// the same hint on the loads of the counting and compacting passes gains nothing).
+// With a 4-byte store per element the instruction stream bounds it, not the bytes.
+// A row is 256 elements = 8 mask words; lane l keeps mask word 64*(row/8) + l of the
+// chunk, together with the number of set bits in the words before it inside its row,
+// so a lane finds its nibble and the rank of its first element with two cross-lane reads.
 // ALIGNED: E % 4 == 0 and a 16-byte aligned destination, so every chunk starts on a
 // 16-byte boundary.  Otherwise the same 16-byte stores at any element, without the hint:
 // 60 MB in chunks of 1838 elements 16.3 us, against 18.6 us with a 4-byte store per element.
-// Chunks of at most so many mask words share a wavefront (zvc_expand_packed_kernel) where there are
-// more than so many of them: three or more to a wavefront.  Two to a wavefront measure the same as one
-// each, and few chunks are all in flight at once either way.
-constexpr int kPackedWords = 21, kPackedFrom = 2048;
 constexpr int kRowsInFlight = 8;  // divides the 8 rows one refill covers
 
 template <bool ALIGNED>
@@ -433,6 +428,10 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand4_kernel(
 // finds its chunk's end and offset by itself and the eight rows of a refill are full.
 // 16384 chunks, one wavefront per chunk -> this: 7 MB 11.3 -> 5.9 us, 25.7 MB 11.1 -> 8.4,
 // 33.6 MB (512 elements per chunk) 11.0 -> 8.7.
+// It takes chunks of at most kPackedWords mask words where there are more than kPackedFrom of
+// them: three or more to a wavefront.  Two to a wavefront measure the same as one each, and few
+// chunks are all in flight at once either way.
+constexpr int kPackedWords = 21, kPackedFrom = 2048;
 template <bool ALIGNED>
 __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand_packed_kernel(
     const float* __restrict__ values, const uint32_t* __restrict__ mask, const int* __restrict__ begin,
@@ -499,7 +498,7 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand_packed_kernel(
   }
 }
 
-// The same once more for tensors larger than the memory-side cache (the size from which
+// zvc_expand4_kernel once more, for tensors larger than the memory-side cache (the size from which
 // the compaction is staged, too): the packed values of four rows (1024 elements) are first
 // brought into an LDS region of the wavefront with aligned 16-byte loads -- whole lines per
 // instruction -- and picked from there, and the mask words of the next eight rows are asked
@@ -509,7 +508,7 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand_packed_kernel(
 // LDS per wavefront means more wavefronts per compute unit to hide the two loads each group
 // waits for, fewer rows per group means more groups) and the same where they come from the
 // cache; on small tensors the LDS costs more occupancy than the loads gain, so those keep
-// the kernel above.
+// the kernels above.
 constexpr int kRowsStaged = 4;  // divides kRowsInFlight
 
 template <bool ALIGNED>
@@ -1427,8 +1426,9 @@ extern "C" void cswap_zvc_debug_set_lookback(unsigned spin_limit, unsigned skip_
   g_skip_first.store(skip_first);
 }
 
-// Tensors of at least this many bytes take the single pass in cswap_zvc_compress_fused; smaller ones
-// finish sooner with the three kernels (a few rounds of the grid do not fill the pipeline).
+// Tensors of at least this many bytes take the pipeline kernel in cswap_zvc_compress_fused; smaller ones,
+// which do not fill the pipeline (a few rounds of the grid), finish sooner in the one-kernel form that
+// holds the whole tensor in registers: just below the limit 25 us, the pipeline 31 at it.
 static std::atomic<unsigned long long> g_single_pass_bytes{64ull << 20};  // cswap_zvc_set_single_pass_bytes
 
 extern "C" size_t cswap_zvc_set_single_pass_bytes(size_t bytes)
@@ -1476,8 +1476,8 @@ static bool single_pass_shape(const Geometry& g, int n, int process, StreamGeome
 }
 
 // Whether the one-kernel form for small tensors takes this shape (a tensor below the size from
-// which the pipeline kernel runs, whole half rows per chunk, the whole tensor in the registers
-// of one grid); fills the geometry, the grid and the rows per wavefront.
+// which the pipeline kernel runs, all of it in the registers of one grid, whole half rows per
+// chunk unless `any`); fills the geometry, the grid and the rows per wavefront.
 // `any`: also the shapes of the form's variants that cannot fail (zvc_small_kernel: kCountsItself),
 // chunks of any length and up to 64 rows per wavefront; a caller that has to know beforehand
 // whether the workspace decides about success (cswap_zvc_takes_single_pass) leaves those out.
@@ -1523,7 +1523,7 @@ extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, v
   uint32_t* ws = (uint32_t*)d_ws;
   const int cus = device_compute_units();
   StreamGeometry sg;
-  // anything the single pass does not take, or an output that is not 16-byte aligned, runs the three kernels
+  // what neither one-kernel form takes runs the three kernels (the pipeline needs a 16-byte aligned output, too)
   const bool single_pass = single_pass_shape(g, n, process, sg) && (reinterpret_cast<uintptr_t>(d_values) & 15u) == 0;
   int groups = 0, rows = 0;
   if (!single_pass && small_pass_shape(g, n, process, sg, &groups, &rows, true)) {

@@ -120,7 +120,7 @@ int cswap_zfp_decompress_i64_nd(const uint64_t* d_stream, int dims, size_t nx, s
  * 21 MB at 32), and by the decoder only from 16 bits per value on (at 8 it measured no
  * gain).  The smallest fields (below the same limits, up to 11 wavefronts of 16 blocks
  * per compute unit: about 11 MB; 22 for an encoder of a shape that the pair form does not
- * take) run a form with four lanes per block, at any shape and any maxbits that is a
+ * take, fewer at 16 to 30 bits per value, where LDS holds fewer at once) run a form with four lanes per block, at any shape and any maxbits that is a
  * multiple of 64.  0 = neither form, one lane per block; SIZE_MAX = the pair form
  * whenever the shape allows, whatever the size and rate, and never the one with four
  * lanes (tests and measurements).  Defaults: 40 MiB both.  `previous`, if not NULL, receives

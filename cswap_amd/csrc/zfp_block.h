@@ -112,6 +112,16 @@ inline Div31 make_div31(uint32_t d)
 }
 CSWAP_HD uint32_t div31(uint32_t b, Div31 d) { return (uint32_t)(((uint64_t)b * d.mul) >> d.shift); }
 
+// Which of a workgroup's 64 blocks the 16-byte piece p of its part of the stream belongs to, P =
+// maxbits / 128 pieces to a block.  by = ceil(65536 / P) is above 65536 / P by less than 1, so p * by is
+// above 65536 p / P by less than p < 64 P <= 65536 / P, which is how far p / P stays below the next
+// whole number (P <= 32).  0: blocks of an odd number of words.
+CSWAP_HD uint32_t piece_multiplier(unsigned maxbits)
+{
+  return (maxbits & 127u) ? 0u : (65536u + (maxbits >> 7) - 1u) / (maxbits >> 7);
+}
+CSWAP_HD uint32_t block_of_piece(uint32_t p, uint32_t by) { return (p * by) >> 16; }
+
 CSWAP_HD unsigned sub_sat(unsigned a, unsigned b)  // max(a - b, 0)
 {
 #if defined(__HIP_DEVICE_COMPILE__)

@@ -29,6 +29,7 @@ struct Field3 {
   int rows4;               // 1: as rows16, but the rows may start at any element, and nx >= 2
   int full;                // 1: rows4, and every block is a full one
   int stream16;            // 1: the stream pointer is 16-byte aligned
+  uint32_t by_piece;       // whole-word rates with an even number of words per block, else 0: the multiplier of block_of_piece
   int read_once;           // 1: the encoder should load the field with the nontemporal hint (see make_field)
   int once64;              // 1: the decoder of 64-bit elements should store its rows with the hint (see make_field)
   Div31 by_mx, by_my;      // block index -> block coordinates without a hardware divide
@@ -333,18 +334,93 @@ __device__ __forceinline__ void zero_region(uint4* lds_raw, unsigned lane, unsig
   for (unsigned i = lane; i < n16; i += 64) lds_raw[i] = make_uint4(0, 0, 0, 0);
 }
 
+// The blocks of a workgroup lie one behind the other in the stream, so its threads can move them as one
+// run of 16-byte pieces, thread t the pieces t, t + threads, ...: every instruction covers whole lines,
+// where lanes that move the words of their own block touch another line than their neighbour in each of
+// their instructions (64 lines at 16 bits per value, 32 at 8).  Four pieces at a time, all asked for
+// before the first is used: one by one, a stream that comes from memory costs its latency four times
+// (402.7 MB at 8 bits, from a cold stream, decoded in 104 us by own words, 109 one piece at a time, 92 four).
+// The decoder, own words -> pieces: 402.7 MB at 8 bits 88.9 -> 83.1 us (104 -> 92 cold), 201.3 MB 49.4 -> 45.0, at 16
+// bits 75.9 -> 62.7 (85 -> 71 cold), 50.3 MB 17.9 -> 17.3, at 16 bits 24.4 -> 20.3.  The encoder from 16 bits on:
+// 201.3 MB 72.2 -> 65.5 us; at 8 bits its lanes' 64 bytes of a line meet in the cache, and the pieces' addresses
+// cost more than they save (50.3 MB 21.3 / 21.8 us, 14x14 planes 16.4 / 17.1).
+// PAD: dwords between the blocks of the region.
+template <unsigned PAD>
+__device__ __forceinline__ uint32_t piece_dword(uint32_t p, uint32_t by)
+{
+  return 4 * p + PAD * (__umul24(p, by) >> 16);  // block_of_piece
+}
+
+// stream: the workgroup's first block.  B pieces of every thread; past the last piece all move that one.
+template <unsigned B, unsigned THREADS, unsigned PAD>
+__device__ __forceinline__ void store_batch(const uint32_t* lds, unsigned p0, unsigned last, uint32_t by, char* __restrict__ dst)
+{
+  ulonglong2 v[B];
+  unsigned p[B];
+#pragma unroll
+  for (unsigned k = 0; k < B; k++) {
+    p[k] = min(p0 + k * THREADS, last);
+    v[k] = *reinterpret_cast<const ulonglong2*>(lds + piece_dword<PAD>(p[k], by));
+  }
+#pragma unroll
+  for (unsigned k = 0; k < B; k++) *reinterpret_cast<ulonglong2*>(dst + (size_t)(16u * p[k])) = v[k];
+}
+
+template <unsigned B, unsigned THREADS, unsigned PAD>
+__device__ __forceinline__ void load_batch(uint32_t* lds, unsigned p0, unsigned last, uint32_t by, const char* __restrict__ src)
+{
+  ulonglong2 v[B];
+  unsigned p[B];
+#pragma unroll
+  for (unsigned k = 0; k < B; k++) {
+    p[k] = min(p0 + k * THREADS, last);
+    v[k] = *reinterpret_cast<const ulonglong2*>(src + (size_t)(16u * p[k]));
+  }
+#pragma unroll
+  for (unsigned k = 0; k < B; k++) {
+    uint64_t* dst = reinterpret_cast<uint64_t*>(lds + piece_dword<PAD>(p[k], by));
+    dst[0] = v[k].x;
+    dst[1] = v[k].y;
+  }
+}
+
+template <unsigned THREADS, unsigned PAD>
+__device__ __forceinline__ void store_pieces(const uint32_t* lds, unsigned t, uint32_t valid, unsigned maxbits, uint32_t by,
+                                             uint64_t* __restrict__ stream)
+{
+  const unsigned all = 64 * (maxbits >> 7), last = valid * (maxbits >> 7) - 1;
+  char* dst = reinterpret_cast<char*>(stream);
+  unsigned i = 0;
+  for (; i + 4 * THREADS <= all; i += 4 * THREADS) store_batch<4, THREADS, PAD>(lds, i + t, last, by, dst);
+  for (; i < all; i += THREADS) store_batch<1, THREADS, PAD>(lds, i + t, last, by, dst);
+}
+
+template <unsigned THREADS, unsigned PAD>
+__device__ __forceinline__ void load_pieces(uint32_t* lds, unsigned t, uint32_t valid, unsigned maxbits, uint32_t by,
+                                            const uint64_t* __restrict__ stream)
+{
+  const unsigned all = 64 * (maxbits >> 7), last = valid * (maxbits >> 7) - 1;
+  const char* src = reinterpret_cast<const char*>(stream);
+  unsigned i = 0;
+  for (; i + 4 * THREADS <= all; i += 4 * THREADS) load_batch<4, THREADS, PAD>(lds, i + t, last, by, src);
+  for (; i + 2 * THREADS <= all; i += 2 * THREADS) load_batch<2, THREADS, PAD>(lds, i + t, last, by, src);
+  for (; i < all; i += THREADS) load_batch<1, THREADS, PAD>(lds, i + t, last, by, src);
+}
+constexpr unsigned kSlackDwords = 4, kFenceDwords = 2;  // slot_bits and dec_slot_bits at whole-word rates of even word counts
+
 // the wave's coded blocks from LDS to the stream
-template <bool WHOLE>
+template <bool WHOLE, bool PIECES>
 __device__ __forceinline__ void store_region(const uint32_t* lds, unsigned lane, uint32_t first, uint32_t valid,
-                                             unsigned maxbits, int stream16, uint64_t* __restrict__ stream)
+                                             unsigned maxbits, const Field3& fd, uint64_t* __restrict__ stream)
 {
   if (WHOLE) {
-    // each lane stores the words of its own block (16-byte stores where aligned)
-    if (lane < valid) {
-      const unsigned W = maxbits >> 6;
+    const unsigned W = maxbits >> 6;
+    if (PIECES && fd.by_piece && fd.stream16) {
+      store_pieces<64, kSlackDwords>(lds, lane, valid, maxbits, fd.by_piece, stream + (size_t)first * W);
+    } else if (lane < valid) {  // each lane stores the words of its own block (16-byte stores where aligned)
       const uint64_t* src = reinterpret_cast<const uint64_t*>(lds + lane * (slot_bits(maxbits) / 32));
       uint64_t* dst = stream + (size_t)(first + lane) * W;
-      if ((W & 1u) == 0 && stream16) {
+      if ((W & 1u) == 0 && fd.stream16) {
         for (unsigned j = 0; j < W; j += 2)
           *reinterpret_cast<ulonglong2*>(dst + j) = *reinterpret_cast<const ulonglong2*>(src + j);
       } else {
@@ -361,31 +437,21 @@ __device__ __forceinline__ void store_region(const uint32_t* lds, unsigned lane,
 
 // the wave's coded blocks from the stream into LDS; whole-word rates get the
 // fence of ones behind every block that the fenced decoder relies on
-template <bool WHOLE, bool SLOT16 = true>
+template <bool WHOLE, unsigned PAD>
 __device__ __forceinline__ void load_region(uint32_t* lds, unsigned lane, uint32_t first, uint32_t valid,
-                                            unsigned maxbits, unsigned slot, int stream16,
+                                            unsigned maxbits, unsigned slot, const Field3& fd,
                                             const uint64_t* __restrict__ stream)
 {
   if (WHOLE) {
-    if (lane < valid) {
-      const unsigned W = maxbits >> 6;
-      uint64_t* dst = reinterpret_cast<uint64_t*>(lds + lane * (slot / 32));
+    const unsigned W = maxbits >> 6;
+    uint64_t* dst = reinterpret_cast<uint64_t*>(lds + lane * (slot / 32));
+    if (fd.by_piece && fd.stream16) {
+      load_pieces<64, PAD>(lds, lane, valid, maxbits, fd.by_piece, stream + (size_t)first * W);
+    } else if (lane < valid) {
       const uint64_t* src = stream + (size_t)(first + lane) * W;
-      if ((W & 1u) == 0 && stream16) {
-        for (unsigned j = 0; j < W; j += 2) {
-          const ulonglong2 v = *reinterpret_cast<const ulonglong2*>(src + j);
-          if (SLOT16) {
-            *reinterpret_cast<ulonglong2*>(dst + j) = v;
-          } else {
-            dst[j] = v.x;
-            dst[j + 1] = v.y;
-          }
-        }
-      } else {
-        for (unsigned j = 0; j < W; j++) dst[j] = src[j];
-      }
-      dst[W] = ~0ull;
+      for (unsigned j = 0; j < W; j++) dst[j] = src[j];
     }
+    if (lane < valid) dst[W] = ~0ull;
   } else {
     const unsigned nwords = (valid * maxbits + 63u) >> 6;
     const uint64_t* src = stream + (size_t)(first >> 6) * maxbits;
@@ -405,7 +471,8 @@ __device__ __forceinline__ void load_region(uint32_t* lds, unsigned lane, uint32
 // three per SIMD (402.7 MB at 16 bits per value: 130-133 us against 139-140 us with four
 // or five), the decoder with four (137-140 us against 143-156 us).
 // ROWS: a field for load_block_rows
-template <bool WHOLE, bool INT, bool ONCE, bool ROWS>
+// PIECES: for 16 bits per value and more, where the stream is stored as one run of pieces
+template <bool WHOLE, bool INT, bool ONCE, bool ROWS, bool PIECES>
 __device__ __forceinline__ void encode3_f32(const float* __restrict__ in, const Field3& fd, unsigned maxbits,
                                             uint64_t* __restrict__ stream)
 {
@@ -443,14 +510,14 @@ __device__ __forceinline__ void encode3_f32(const float* __restrict__ in, const 
   }
   __syncthreads();
   __builtin_amdgcn_s_setprio(3);
-  store_region<WHOLE>(lds, lane, first, valid, maxbits, fd.stream16, stream);
+  store_region<WHOLE, PIECES>(lds, lane, first, valid, maxbits, fd, stream);
 }
 
 template <bool WHOLE, bool INT = false, bool ONCE = false, int WPE = 5>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void zfp_encode3_f32_kernel(
     const float* __restrict__ in, Field3 fd, unsigned maxbits, uint64_t* __restrict__ stream)
 {
-  encode3_f32<WHOLE, INT, ONCE, false>(in, fd, maxbits, stream);
+  encode3_f32<WHOLE, INT, ONCE, false, WPE == 3>(in, fd, maxbits, stream);
 }
 // Kernels of their own for these fields: one kernel with both kinds of rows decoded full fields 2-6 %
 // slower (100 MB 29.2 instead of 27.5 us, 403 MB 89.7 instead of 87.4).
@@ -458,7 +525,7 @@ template <bool WHOLE, bool INT = false, int WPE = 5>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void zfp_encode3_rows_kernel(
     const float* __restrict__ in, Field3 fd, unsigned maxbits, uint64_t* __restrict__ stream)
 {
-  encode3_f32<WHOLE, INT, false, true>(in, fd, maxbits, stream);
+  encode3_f32<WHOLE, INT, false, true, WPE == 3>(in, fd, maxbits, stream);
 }
 
 // Five wavefronts per SIMD (at most 96 registers, which the row-wise finish
@@ -483,7 +550,7 @@ __device__ __forceinline__ void decode3_f32(const uint64_t* __restrict__ stream,
   // above the rest, 87.8 us with the last part below the planes as well (16 bits per value:
   // 137 -> 129 us); the last part below the lifting: 110 us.
   __builtin_amdgcn_s_setprio(3);
-  load_region<WHOLE, false>(lds, lane, first, valid, maxbits, slot, fd.stream16, stream);
+  load_region<WHOLE, kFenceDwords>(lds, lane, first, valid, maxbits, slot, fd, stream);
   __syncthreads();
 
   if (lane < valid) {
@@ -643,15 +710,9 @@ __global__ __launch_bounds__(128) void zfp_encode3_f32_pair_kernel(const float* 
   }
   if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) pair_encode_body<0>(in, fd, maxbits, lds, lane, first);
   else pair_encode_body<1>(in, fd, maxbits, lds, lane, first);
-  // Both halves are past the barrier of more() or done(): every block is coded.  Thread t
-  // moves half of block t / 2 (W / 2 words, W / 4 16-byte pieces).
-  const uint32_t blk = first + (tid >> 1);
-  if (blk < fd.nblocks) {
-    const unsigned W = maxbits >> 6;
-    const ulonglong2* src = reinterpret_cast<const ulonglong2*>(lds + (tid >> 1) * (slot_bits(maxbits) / 32) + (tid & 1u) * W);
-    ulonglong2* dst = reinterpret_cast<ulonglong2*>(stream + (size_t)blk * W + (tid & 1u) * (W / 2));
-    for (unsigned j = 0; j < W / 4; j++) dst[j] = src[j];
-  }
+  // Both halves are past the barrier of more() or done(): every block is coded.
+  store_pieces<128, kSlackDwords>(lds, tid, min(64u, fd.nblocks - first), maxbits, fd.by_piece,
+                                  stream + (size_t)first * (maxbits >> 6));
 }
 
 // The pair form of the decoder (zfp_block.h: pair_decode_half).  Dynamic LDS, in dwords:
@@ -746,22 +807,13 @@ __global__ __launch_bounds__(128) void zfp_decode3_f32_pair_kernel(const uint64_
   uint32_t* lds = reinterpret_cast<uint32_t*>(lds_raw);
   const unsigned tid = threadIdx.x, lane = tid & 63u;
   const uint32_t first = blockIdx.x * 64u;
-  {  // thread t brings in half of block t / 2; the fence of ones behind every block comes with the second half.
-     // The slots of blocks past the end of the field read as empty blocks.
-    const unsigned W = maxbits >> 6;
-    const uint32_t blk = first + (tid >> 1);
-    uint64_t* dst = reinterpret_cast<uint64_t*>(lds + (tid >> 1) * (dec_slot_bits(maxbits) / 32)) + (tid & 1u) * (W / 2);
-    if (blk < fd.nblocks) {
-      const ulonglong2* src = reinterpret_cast<const ulonglong2*>(stream + (size_t)blk * W + (tid & 1u) * (W / 2));
-      for (unsigned j = 0; j < W / 4; j++) {
-        const ulonglong2 v = src[j];
-        dst[2 * j] = v.x;
-        dst[2 * j + 1] = v.y;
-      }
-    } else {
-      for (unsigned j = 0; j < W / 2; j++) dst[j] = 0;
-    }
-    if (tid & 1u) dst[W / 2] = ~0ull;
+  {  // the fence of ones goes behind every block; the slots past the end of the field read as empty blocks
+    const unsigned W = maxbits >> 6, slot = dec_slot_bits(maxbits);
+    const uint32_t valid = min(64u, fd.nblocks - first);
+    load_pieces<128, kFenceDwords>(lds, tid, valid, maxbits, fd.by_piece, stream + (size_t)first * W);
+    uint64_t* own = reinterpret_cast<uint64_t*>(lds + lane * (slot / 32));
+    if (tid < 64) own[W] = ~0ull;
+    else if (lane >= valid) own[0] = 0;
   }
   __syncthreads();
   if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) pair_decode_body<0>(fd, maxbits, lds, lane, first, out);
@@ -1188,7 +1240,7 @@ __global__ __launch_bounds__(64) void zfp_encode3_w64_kernel(const uint64_t* __r
     encode_block_w64<!WHOLE, INT>(q, mem.bit0 + lane * slot_bits(maxbits), maxbits, mem);
   }
   __syncthreads();
-  store_region<WHOLE>(lds, lane, first, valid, maxbits, fd.stream16, stream);
+  store_region<WHOLE, true>(lds, lane, first, valid, maxbits, fd, stream);
 }
 
 // ONCE: rows stored with the nontemporal hint (Field3::once64)
@@ -1202,7 +1254,7 @@ __global__ __launch_bounds__(64) void zfp_decode3_w64_kernel(const uint64_t* __r
   const uint32_t first = blockIdx.x * 64u;
   const uint32_t valid = min(64u, fd.nblocks - first);
   __builtin_amdgcn_s_setprio(3);  // the 32-bit decoder's priorities (here, at two wavefronts per SIMD, worth 2.6 %)
-  load_region<WHOLE>(lds, lane, first, valid, maxbits, slot_bits(maxbits), fd.stream16, stream);
+  load_region<WHOLE, kSlackDwords>(lds, lane, first, valid, maxbits, slot_bits(maxbits), fd, stream);
   __syncthreads();
   if (lane < valid) {
     uint64_t q[64];
@@ -1432,6 +1484,7 @@ static int make_field(Field3& fd, const void* base, const void* stream, size_t n
              (unsigned long long)fd.sz * 4ull * elem * slabs < 0xfff00000ull;
   fd.full = fd.rows4 && ((nx | ny | nz) & 3u) == 0;
   fd.stream16 = ((uintptr_t)stream % 16) == 0;
+  fd.by_piece = piece_multiplier(maxbits);
   // Cache policy of the field's 16-byte rows (whole 128-byte lines per wave instruction).
   // The decoder always stores them with the nontemporal hint: 402.7 MB decode in 107 us
   // instead of 117 us, and the kernel that runs next no longer waits behind those lines

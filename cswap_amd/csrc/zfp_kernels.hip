@@ -79,6 +79,18 @@ struct LdsBits {
   __device__ __forceinline__ uint32_t ld32(unsigned d) const { return *at(d); }
 };
 
+// The same with the codec's table of expanded bytes (zfp_block.h: expand8) in front of the region: 512
+// bytes per workgroup, a 16-bit read per byte.  Most bytes are zero, so most lanes read one address.
+struct LdsBitsTable : LdsBits {
+  static constexpr bool kExpands = true;
+  const uint16_t* table;
+  __device__ __forceinline__ LdsBitsTable(uint32_t* region, const uint16_t* t) : LdsBits(region), table(t) {}
+  __device__ __forceinline__ uint32_t expanded(uint32_t word, int k) const { return table[(word >> (8 * k)) & 0xffu]; }
+};
+__constant__ const ExpandTable kExpandTable = make_expand_table();
+// A lane's 8 bytes of the table: asked for before anything else, written to LDS when the region is cleared.
+__device__ __forceinline__ uint2 table_piece(unsigned lane) { return reinterpret_cast<const uint2*>(kExpandTable.v)[lane]; }
+
 // Layout of the wave's LDS bit region.
 //  whole-word rates (maxbits % 64 == 0): every lane owns a private slot of
 //    maxbits + slack bits (slot a multiple of 128 bits), so the coder needs no
@@ -341,9 +353,8 @@ __device__ __forceinline__ void zero_region(uint4* lds_raw, unsigned lane, unsig
 // before the first is used: one by one, a stream that comes from memory costs its latency four times
 // (402.7 MB at 8 bits, from a cold stream, decoded in 104 us by own words, 109 one piece at a time, 92 four).
 // The decoder, own words -> pieces: 402.7 MB at 8 bits 88.9 -> 83.1 us (104 -> 92 cold), 201.3 MB 49.4 -> 45.0, at 16
-// bits 75.9 -> 62.7 (85 -> 71 cold), 50.3 MB 17.9 -> 17.3, at 16 bits 24.4 -> 20.3.  The encoder from 16 bits on:
-// 201.3 MB 72.2 -> 65.5 us; at 8 bits its lanes' 64 bytes of a line meet in the cache, and the pieces' addresses
-// cost more than they save (50.3 MB 21.3 / 21.8 us, 14x14 planes 16.4 / 17.1).
+// bits 75.9 -> 62.7 (85 -> 71 cold), 50.3 MB 17.9 -> 17.3, at 16 bits 24.4 -> 20.3.  The encoder: 201.3 MB at 8 bits
+// 49.3 -> 47.2, at 16 bits 72.2 -> 65.5, 402.7 MB 92.7 -> 89.3, 50.3 MB 17.8 -> 17.5.
 // PAD: dwords between the blocks of the region.
 template <unsigned PAD>
 __device__ __forceinline__ uint32_t piece_dword(uint32_t p, uint32_t by)
@@ -409,23 +420,18 @@ __device__ __forceinline__ void load_pieces(uint32_t* lds, unsigned t, uint32_t 
 constexpr unsigned kSlackDwords = 4, kFenceDwords = 2;  // slot_bits and dec_slot_bits at whole-word rates of even word counts
 
 // the wave's coded blocks from LDS to the stream
-template <bool WHOLE, bool PIECES>
+template <bool WHOLE>
 __device__ __forceinline__ void store_region(const uint32_t* lds, unsigned lane, uint32_t first, uint32_t valid,
                                              unsigned maxbits, const Field3& fd, uint64_t* __restrict__ stream)
 {
   if (WHOLE) {
     const unsigned W = maxbits >> 6;
-    if (PIECES && fd.by_piece && fd.stream16) {
+    if (fd.by_piece && fd.stream16) {
       store_pieces<64, kSlackDwords>(lds, lane, valid, maxbits, fd.by_piece, stream + (size_t)first * W);
-    } else if (lane < valid) {  // each lane stores the words of its own block (16-byte stores where aligned)
+    } else if (lane < valid) {  // an odd number of words, or a stream off 16 bytes: each lane stores its own block's
       const uint64_t* src = reinterpret_cast<const uint64_t*>(lds + lane * (slot_bits(maxbits) / 32));
       uint64_t* dst = stream + (size_t)(first + lane) * W;
-      if ((W & 1u) == 0 && fd.stream16) {
-        for (unsigned j = 0; j < W; j += 2)
-          *reinterpret_cast<ulonglong2*>(dst + j) = *reinterpret_cast<const ulonglong2*>(src + j);
-      } else {
-        for (unsigned j = 0; j < W; j++) dst[j] = src[j];
-      }
+      for (unsigned j = 0; j < W; j++) dst[j] = src[j];
     }
   } else {
     const unsigned nwords = (valid * maxbits + 63u) >> 6;
@@ -471,8 +477,7 @@ __device__ __forceinline__ void load_region(uint32_t* lds, unsigned lane, uint32
 // three per SIMD (402.7 MB at 16 bits per value: 130-133 us against 139-140 us with four
 // or five), the decoder with four (137-140 us against 143-156 us).
 // ROWS: a field for load_block_rows
-// PIECES: for 16 bits per value and more, where the stream is stored as one run of pieces
-template <bool WHOLE, bool INT, bool ONCE, bool ROWS, bool PIECES>
+template <bool WHOLE, bool INT, bool ONCE, bool ROWS>
 __device__ __forceinline__ void encode3_f32(const float* __restrict__ in, const Field3& fd, unsigned maxbits,
                                             uint64_t* __restrict__ stream)
 {
@@ -487,18 +492,22 @@ __device__ __forceinline__ void encode3_f32(const float* __restrict__ in, const 
   // the ones that are coding when both have an instruction to issue: its requests are what the
   // compute unit's other wavefronts will be computing behind (measured on 402.7 MB: encode 100 ->
   // 97 us at 8 bits per value, 129 -> 126 us at 16; the other way round 100 and 131 us).
+  __shared__ uint2 table[WHOLE ? 64 : 1];
   float f[64];
   __builtin_amdgcn_s_setprio(3);
+  uint2 piece;
+  if (WHOLE) piece = table_piece(lane);
   if (lane < valid) {  // in flight while the region is cleared
     if (ROWS) load_block_rows(in, fd, first, first + lane, f);
     else load_block<ONCE>(in, fd, first, first + lane, f);
   }
   zero_region(lds_raw, lane, maxbits);
+  if (WHOLE) table[lane] = piece;
   __syncthreads();
   __builtin_amdgcn_s_setprio(0);
 
   if (lane < valid) {
-    LdsBits mem(lds);
+    LdsBitsTable mem(lds, reinterpret_cast<const uint16_t*>(table));
     if (INT) {
       int32_t v[64];
 #pragma unroll
@@ -510,14 +519,14 @@ __device__ __forceinline__ void encode3_f32(const float* __restrict__ in, const 
   }
   __syncthreads();
   __builtin_amdgcn_s_setprio(3);
-  store_region<WHOLE, PIECES>(lds, lane, first, valid, maxbits, fd, stream);
+  store_region<WHOLE>(lds, lane, first, valid, maxbits, fd, stream);
 }
 
 template <bool WHOLE, bool INT = false, bool ONCE = false, int WPE = 5>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void zfp_encode3_f32_kernel(
     const float* __restrict__ in, Field3 fd, unsigned maxbits, uint64_t* __restrict__ stream)
 {
-  encode3_f32<WHOLE, INT, ONCE, false, WPE == 3>(in, fd, maxbits, stream);
+  encode3_f32<WHOLE, INT, ONCE, false>(in, fd, maxbits, stream);
 }
 // Kernels of their own for these fields: one kernel with both kinds of rows decoded full fields 2-6 %
 // slower (100 MB 29.2 instead of 27.5 us, 403 MB 89.7 instead of 87.4).
@@ -525,7 +534,7 @@ template <bool WHOLE, bool INT = false, int WPE = 5>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void zfp_encode3_rows_kernel(
     const float* __restrict__ in, Field3 fd, unsigned maxbits, uint64_t* __restrict__ stream)
 {
-  encode3_f32<WHOLE, INT, false, true, WPE == 3>(in, fd, maxbits, stream);
+  encode3_f32<WHOLE, INT, false, true>(in, fd, maxbits, stream);
 }
 
 // Five wavefronts per SIMD (at most 96 registers, which the row-wise finish
@@ -607,7 +616,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
 //                                                                               barrier  reads U_h
 //   planes       writes its 32 bits of 16 planes into U_h (k * 64 + lane)      barrier  reads both
 constexpr unsigned kPairMaxima = 128, kPairFlag = 4, kPairU = 1280;
-__host__ __device__ inline unsigned pair_lds_dwords(unsigned maxbits)
+__host__ __device__ inline unsigned pair_lds_dwords(unsigned maxbits)  // without the table of expanded bytes
 {
   return region_dwords(maxbits) + kPairMaxima + kPairFlag + 2 * kPairU;
 }
@@ -665,7 +674,7 @@ struct LdsExchange {
 
 template <int H>
 __device__ __forceinline__ void pair_encode_body(const float* __restrict__ in, const Field3& fd, unsigned maxbits,
-                                                 uint32_t* lds, unsigned lane, uint32_t first)
+                                                 uint32_t* lds, const uint16_t* table, unsigned lane, uint32_t first)
 {
   const bool live = first + lane < fd.nblocks;
   const uint32_t b = live ? first + lane : fd.nblocks - 1;
@@ -693,23 +702,27 @@ __device__ __forceinline__ void pair_encode_body(const float* __restrict__ in, c
   ex.mine = lds + region + kPairMaxima + kPairFlag + H * kPairU;
   ex.theirs = lds + region + kPairMaxima + kPairFlag + (1 - H) * kPairU;
   ex.lane = lane;
-  LdsBits mem(lds);
+  LdsBitsTable mem(lds, table);
   pair_encode_half<H>(p, q, live, mem.bit0 + lane * slot_bits(maxbits), maxbits, mem, ex);
 }
 
-__global__ __launch_bounds__(128) void zfp_encode3_f32_pair_kernel(const float* __restrict__ in, Field3 fd,
-                                                                   unsigned maxbits, uint64_t* __restrict__ stream)
+// Seven wavefronts per SIMD (72 registers; 75 without the limit) leave the LDS to bound how many are resident.
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(7, 8))) void zfp_encode3_f32_pair_kernel(
+    const float* __restrict__ in, Field3 fd, unsigned maxbits, uint64_t* __restrict__ stream)
 {
   extern __shared__ uint4 lds_raw[];
   uint32_t* lds = reinterpret_cast<uint32_t*>(lds_raw);
   const unsigned tid = threadIdx.x, lane = tid & 63u;
   const uint32_t first = blockIdx.x * 64u;
+  __shared__ uint2 pieces[64];
+  if (tid < 64) pieces[tid] = table_piece(tid);
+  const uint16_t* table = reinterpret_cast<const uint16_t*>(pieces);
   {  // the region starts out zero; the first exchange's barrier orders this before any coder's OR
     const unsigned n16 = region_dwords(maxbits) / 4;
     for (unsigned i = tid; i < n16; i += 128) lds_raw[i] = make_uint4(0, 0, 0, 0);
   }
-  if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) pair_encode_body<0>(in, fd, maxbits, lds, lane, first);
-  else pair_encode_body<1>(in, fd, maxbits, lds, lane, first);
+  if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) pair_encode_body<0>(in, fd, maxbits, lds, table, lane, first);
+  else pair_encode_body<1>(in, fd, maxbits, lds, table, lane, first);
   // Both halves are past the barrier of more() or done(): every block is coded.
   store_pieces<128, kSlackDwords>(lds, tid, min(64u, fd.nblocks - first), maxbits, fd.by_piece,
                                   stream + (size_t)first * (maxbits >> 6));
@@ -898,7 +911,7 @@ __device__ __forceinline__ void quad_load(const float* __restrict__ in, const Fi
 
 // One round of the coder: four planes, lane q's is x; acc and base (the OR of the planes so far
 // and the bit position behind them) are the same in the four lanes.
-__device__ __forceinline__ void quad_round(BlockEncoder<LdsBits, false>& enc, uint64_t x, uint32_t q, uint64_t& acc,
+__device__ __forceinline__ void quad_round(TableEncoder<LdsBitsTable>& enc, uint64_t x, uint32_t q, uint64_t& acc,
                                            unsigned& base)
 {
   const uint32_t from1 = q >= 1 ? ~0u : 0u, from2 = q >= 2 ? ~0u : 0u;
@@ -919,7 +932,7 @@ __device__ __forceinline__ void quad_round(BlockEncoder<LdsBits, false>& enc, ui
 
 // 16 planes: t as quad_planes leaves it, exchange: the block's exchange area
 __device__ __forceinline__ void quad_code16(const uint32_t (&t)[8], uint32_t* exchange, uint32_t q,
-                                            BlockEncoder<LdsBits, false>& enc, uint64_t& acc, unsigned& base)
+                                            TableEncoder<LdsBitsTable>& enc, uint64_t& acc, unsigned& base)
 {
 #pragma unroll
   for (int j = 0; j < 8; j++) exchange[4 * j + q] = t[j];
@@ -948,8 +961,11 @@ __global__ __launch_bounds__(64) void zfp_encode3_f32_quad_kernel(const float* _
   const unsigned slot = slot_bits(maxbits);
   uint32_t* ex = lds + quad_region_dwords(slot) + bl * kQuadStride;
 
+  __shared__ uint2 table[64];
+  const uint2 piece = table_piece(lane);
   float f[16];
   quad_load(in, fd, live ? b : fd.nblocks - 1, q, f);
+  table[lane] = piece;
   uint32_t to_seq[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) to_seq[i] = kQuadOrder.to_seq[q][i];
@@ -998,8 +1014,8 @@ __global__ __launch_bounds__(64) void zfp_encode3_f32_quad_kernel(const float* _
   }
   __syncthreads();
 
-  LdsBits mem(lds);
-  BlockEncoder<LdsBits, false> enc(mem, mem.bit0 + bl * slot, maxbits);
+  LdsBitsTable mem(lds, reinterpret_cast<const uint16_t*>(table));
+  TableEncoder<LdsBitsTable> enc(mem, mem.bit0 + bl * slot, maxbits);
   unsigned base = e ? enc.pos + 9 : enc.limit;  // an all-zero block or one past the end: nothing is written
   if (e && q == 0) enc.put(2 * e + 1, 9);
   uint64_t acc = 0;
@@ -1231,16 +1247,20 @@ __global__ __launch_bounds__(64) void zfp_encode3_w64_kernel(const uint64_t* __r
   const unsigned lane = threadIdx.x;
   const uint32_t first = blockIdx.x * 64u;
   const uint32_t valid = min(64u, fd.nblocks - first);
+  __shared__ uint2 table[WHOLE ? 64 : 1];
+  uint2 piece;
+  if (WHOLE) piece = table_piece(lane);
   uint64_t q[64];
   if (lane < valid) load_block_w64(in, fd, first + lane, q);  // in flight while the region is cleared
   zero_region(lds_raw, lane, maxbits);
+  if (WHOLE) table[lane] = piece;
   __syncthreads();
   if (lane < valid) {
-    LdsBits mem(lds);
+    LdsBitsTable mem(lds, reinterpret_cast<const uint16_t*>(table));
     encode_block_w64<!WHOLE, INT>(q, mem.bit0 + lane * slot_bits(maxbits), maxbits, mem);
   }
   __syncthreads();
-  store_region<WHOLE, true>(lds, lane, first, valid, maxbits, fd, stream);
+  store_region<WHOLE>(lds, lane, first, valid, maxbits, fd, stream);
 }
 
 // ONCE: rows stored with the nontemporal hint (Field3::once64)
@@ -1664,7 +1684,7 @@ static int compress3(const void* d_in, Elem elem, size_t nx, size_t ny, size_t n
     return check_launch();
   }
   if (elem == kF32 && pair_shape(fd, maxbits) && (unsigned long long)nx * ny * nz * 4ull < pair_below &&
-      pair_fits(grid, (size_t)pair_lds_dwords(maxbits) * 4, pair_below)) {
+      pair_fits(grid, (size_t)pair_lds_dwords(maxbits) * 4 + sizeof(ExpandTable), pair_below)) {
     hipLaunchKernelGGL(zfp_encode3_f32_pair_kernel, dim3(grid), dim3(128), (size_t)pair_lds_dwords(maxbits) * 4, st,
                        static_cast<const float*>(d_in), fd, maxbits, d_stream);
     return check_launch();

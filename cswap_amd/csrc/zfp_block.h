@@ -489,6 +489,40 @@ struct expands<Mem, decltype((void)Mem::kExpands)> {
   static constexpr bool value = Mem::kExpands;
 };
 
+// The way back: collapse8(b) is eight stream bits without the bit behind every one-bit that is not
+// itself such a bit, the first of them a coefficient's.
+constexpr uint8_t collapse8(unsigned b)
+{
+  uint8_t c = 0;
+  unsigned p = 0;
+  for (unsigned i = 0; i < 8; i++) {
+    if ((b >> i) & 1u) {
+      c = (uint8_t)(c | (1u << p));
+      i++;
+    }
+    p++;
+  }
+  return c;
+}
+struct CollapseTable {
+  uint8_t v[256];
+};
+constexpr CollapseTable make_collapse_table()
+{
+  CollapseTable t = {};
+  for (unsigned b = 0; b < 256; b++) t.v[b] = collapse8(b);
+  return t;
+}
+// As above: a member kCollapses, and mem.collapsed(word, k).
+template <class Mem, class = void>
+struct collapses {
+  static constexpr bool value = false;
+};
+template <class Mem>
+struct collapses<Mem, decltype((void)Mem::kCollapses)> {
+  static constexpr bool value = Mem::kCollapses;
+};
+
 CSWAP_HD unsigned popcount_add(uint32_t v, unsigned a) { return (unsigned)__builtin_popcount(v) + a; }
 
 // 32 coefficients with a 1 put in behind every one-bit: 32 + popcount(r) bits
@@ -499,6 +533,19 @@ CSWAP_HD uint64_t expand32(const Mem& mem, uint32_t r)
   const uint32_t w0 = e0 | (e1 << popcount_add(r & 0xffu, 8));
   const uint32_t w1 = e2 | (e3 << popcount_add(r & 0xff0000u, 8));
   return w0 | ((uint64_t)w1 << popcount_add(r & 0xffffu, 16));
+}
+
+// 32 stream bits of which v are coefficients' one-bits and u the group tests behind them, without the
+// tests.  A test at the start of a byte belongs to a one-bit of the byte before: the byte is looked up
+// without it, one place lower.
+template <class Mem>
+CSWAP_HD uint32_t collapse32(const Mem& mem, uint32_t v, uint32_t u)
+{
+  const uint32_t z = v | (u & 0xfefefefeu);
+  const uint32_t c0 = mem.collapsed(z, 0), c1 = mem.collapsed(z, 1), c2 = mem.collapsed(z, 2), c3 = mem.collapsed(z, 3);
+  const uint32_t w0 = c0 | (c1 << popcount_add(~u & 0x1feu, 0));
+  const uint32_t w1 = c2 | (c3 << popcount_add(~u & 0x1fe0000u, 0));
+  return w0 | (w1 << popcount_add(~u & 0x1fffeu, 0));
 }
 
 // ---------------------------------------------------------------- encoder
@@ -1256,6 +1303,8 @@ struct BlockDecoder {
     return x;
   }
 
+  CSWAP_HD uint64_t low_plane() { return plane(); }
+
   // One of the leading planes.  While no block of the wavefront has a significant
   // coefficient, a plane that is empty in all of them is one zero bit per block
   // (mirror of BlockEncoder::leading_plane).
@@ -1272,6 +1321,111 @@ struct BlockDecoder {
     return plane();
   }
 };
+
+// The fenced decoder for a Mem with the table of collapsed bytes; the fence has to be a one and 31 zeros
+// here, and reads go up to 192 bits past the block.  A plane's runs are read 32 stream bits at a time, without a step per coefficient found.
+// Between two zeros the one-bits are a coefficient's and a positive group test in turn, beginning with
+// a coefficient's, so the plane ends behind the first run of an odd number of ones: the zero there is
+// the negative group test.  Which ones are whose takes an addition: with a one added at the start of
+// every run that starts at an even place, those runs turn to zeros and the others stay, and a
+// coefficient's bits are the even places of the former and the odd ones of the latter.
+template <class Mem>
+struct TableDecoder : BlockDecoder<Mem, 64, true> {
+  using Base = BlockDecoder<Mem, 64, true>;
+  using Base::limit;
+  using Base::mem;
+  using Base::nrem;
+  using Base::pos;
+
+  CSWAP_HD TableDecoder(Mem& m, unsigned pos0, unsigned maxbits) : Base(m, pos0, maxbits) {}
+
+  CSWAP_HD uint64_t plane()
+  {
+    unsigned n = (unsigned)(63 - nrem);
+    const unsigned left = sub_sat(limit, pos);
+    const unsigned m = n < left ? n : left;
+    const unsigned runs = dword_of(pos + n + 1);  // where the runs begin, if there are any: read along with the verbatim bits
+    uint32_t r0 = mem.ld32(runs), r1 = mem.ld32(runs + 4);
+    const uint64_t w = this->window(pos);
+    uint64_t above = w >> (m & 63);               // what follows the m verbatim bits (m = 64: not used)
+    settle(above);
+    uint64_t x = w ^ (m < 64 ? above << m : 0);   // the low m bits of w
+    pos += m;
+    const bool go = nrem >= 0 && pos < limit;     // a group test follows (then m = n < 64)
+    const bool test = go && ((uint32_t)above & 1u);
+    pos += go ? 1u : 0u;
+    if (test) {
+      bool more;
+      do {  // at the start of each turn a coefficient's bit comes next, or the fence
+        const uint32_t s = funnel_shr(r1, r0, pos);
+        constexpr uint32_t even = 0x55555555u;
+        const uint32_t sum = s + (s & ~(s << 1) & even);
+        const uint32_t ones = s & (sum ^ even);     // coefficients' (up to the end of the plane)
+        const uint32_t end = ~s & (ones << 1);      // lowest bit: the negative group test
+        // the plane's bits among the 32, with that test; a last one whose test is not among them stays for the next turn
+        const uint32_t part = (end ^ (end - 1)) & ~(ones & 0x80000000u);
+        const uint32_t v = ones & part, u = (s ^ ones) & part;
+        const uint64_t y = (uint64_t)collapse32(mem, v, u) << n;
+        const unsigned taken = popcount_add(part, 0);
+        const unsigned behind = n + taken - popcount_add(u, 0) - (end ? 1u : 0u);  // coefficients read so far
+        unsigned next = pos + taken;
+        x |= y;
+        more = end == 0 && next <= limit;
+        // The last coefficient was reached: a one without a bit in the stream (unless the budget
+        // ended before).  Every one-bit before it has its group test.
+        if (behind > 63) {
+          next = pos + 63 - n + popcount_add((uint32_t)(y >> 32) & 0x7fffffffu, popcount_add((uint32_t)y, 0));
+          x |= (uint64_t)(next <= limit ? 0x80000000u : 0u) << 32;
+          next = next <= limit ? next : limit + 1;
+          more = false;
+        }
+        n = behind < 64 ? behind : 64;
+        pos = next;
+        if (more) {
+          const unsigned d = dword_of(pos);
+          r0 = mem.ld32(d);
+          r1 = mem.ld32(d + 4);
+        }
+      } while (more);
+      nrem = 63 - (int)n;
+    }
+    return x;
+  }
+
+  // One of the low planes, where most often every coefficient of every block is known.
+  CSWAP_HD uint64_t low_plane()
+  {
+    if (CSWAP_ANY(nrem >= 0)) return plane();
+    const unsigned left = sub_sat(limit, pos);
+    const uint64_t w = this->window(pos);
+    pos += left < 64 ? left : 64;
+    return left < 64 ? w & (((uint64_t)1 << (left & 63)) - 1) : w;
+  }
+
+  CSWAP_HD uint64_t leading_plane()
+  {
+    if (!CSWAP_ANY(nrem != 63)) {
+      const bool act = pos < limit;
+      const uint32_t bit = (mem.ld32(dword_of(pos)) >> (pos & 31)) & 1u;
+      if (!CSWAP_ANY(act && bit)) {
+        pos += act ? 1u : 0u;
+        return 0;
+      }
+    }
+    return plane();
+  }
+};
+
+template <class Mem, bool FENCED, bool TABLE>
+struct DecoderKind {
+  using type = BlockDecoder<Mem, 64, FENCED>;
+};
+template <class Mem>
+struct DecoderKind<Mem, true, true> {
+  using type = TableDecoder<Mem>;
+};
+template <class Mem, bool FENCED>
+using Decoder = typename DecoderKind<Mem, FENCED, collapses<Mem>::value>::type;
 
 // Block decode in two parts, so that a caller can finish, convert and store one
 // x-row at a time instead of holding 64 finished values:
@@ -1301,7 +1455,7 @@ CSWAP_HD uint32_t decode_planes32(Dec& dec, uint32_t (&lo)[32], uint32_t (&hi)[3
   if (CSWAP_ANY(dec.active())) {
 #pragma unroll
     for (int k = 15; k >= 0; k--) {
-      uint64_t x = dec.plane();
+      uint64_t x = dec.low_plane();
       lo[k] = (uint32_t)x;
       hi[k] = (uint32_t)(x >> 32);
     }
@@ -1400,7 +1554,7 @@ CSWAP_HD void decode_ints3(Dec& dec, int64_t (&ib)[64])
 template <bool INT, bool FENCED = false, class Mem>
 CSWAP_HD void decode_block_w64(Mem& mem, unsigned pos0, unsigned maxbits, uint64_t (&q)[64])
 {
-  BlockDecoder<Mem, 64, FENCED> dec(mem, pos0, maxbits);
+  Decoder<Mem, FENCED> dec(mem, pos0, maxbits);
   int emax = 0;
   if (!INT) {
     uint32_t h = (uint32_t)dec.window(pos0);
@@ -1427,7 +1581,7 @@ CSWAP_HD void decode_block_w64(Mem& mem, unsigned pos0, unsigned maxbits, uint64
 template <bool FENCED = false, class Mem>
 CSWAP_HD void decode_block_zy(Mem& mem, unsigned pos0, unsigned maxbits, int32_t (&ib)[64], float& w)
 {
-  BlockDecoder<Mem, 64, FENCED> dec(mem, pos0, maxbits);
+  Decoder<Mem, FENCED> dec(mem, pos0, maxbits);
   uint32_t h = (uint32_t)dec.window(pos0);
   // An empty block (flag bit 0) takes the same path with its bit budget already
   // spent: every plane then reads as zero, the coefficients come out as zero and
@@ -1442,7 +1596,7 @@ CSWAP_HD void decode_block_zy(Mem& mem, unsigned pos0, unsigned maxbits, int32_t
 template <bool FENCED = false, class Mem>
 CSWAP_HD void decode_block_i32_zy(Mem& mem, unsigned pos0, unsigned maxbits, int32_t (&ib)[64])
 {
-  BlockDecoder<Mem, 64, FENCED> dec(mem, pos0, maxbits);
+  Decoder<Mem, FENCED> dec(mem, pos0, maxbits);
   decode_ints3_zy(dec, ib);
 }
 
@@ -1510,7 +1664,7 @@ CSWAP_HD void pair_decode16(Dec& dec, uint64_t (&x)[16], bool top)
 #pragma unroll
   for (int k = 15; k >= 0; k--) {
     x[k] = 0;  // planes that no block of the wavefront can reach are zero without a read
-    if (CSWAP_ANY(dec.active())) x[k] = (top && k >= 12) ? dec.leading_plane() : dec.plane();
+    if (CSWAP_ANY(dec.active())) x[k] = !top ? dec.low_plane() : k >= 12 ? dec.leading_plane() : dec.plane();
   }
 }
 
@@ -1520,7 +1674,7 @@ CSWAP_HD void pair_decode16(Dec& dec, uint64_t (&x)[16], bool top)
 template <int H, class Ex, class Mem>
 CSWAP_HD void pair_decode_half(Mem& mem, unsigned pos0, unsigned maxbits, Ex& ex, float (&p)[16], float (&q)[16])
 {
-  BlockDecoder<Mem, 64, true> dec(mem, pos0, maxbits);
+  Decoder<Mem, true> dec(mem, pos0, maxbits);
   uint64_t x[16];
   bool any = false;
   if (H == 0) {

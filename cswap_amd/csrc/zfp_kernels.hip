@@ -46,7 +46,7 @@ constexpr unsigned long long kReadOnceBytes = CSWAP_READ_ONCE_BYTES;
 #define CSWAP_PAIR_ENCODE_BYTES (40ull << 20)
 #endif
 #ifndef CSWAP_PAIR_DECODE_BYTES
-#define CSWAP_PAIR_DECODE_BYTES (40ull << 20)   // and only from 16 bits per value on (kPairDecodeFromBits)
+#define CSWAP_PAIR_DECODE_BYTES (40ull << 20)   // and only where pair_decode_pays
 #endif
 
 // 16 bytes of the field as the compiler's own vector type (what the nontemporal builtins take)
@@ -90,6 +90,21 @@ struct LdsBitsTable : LdsBits {
 __constant__ const ExpandTable kExpandTable = make_expand_table();
 // A lane's 8 bytes of the table: asked for before anything else, written to LDS when the region is cleared.
 __device__ __forceinline__ uint2 table_piece(unsigned lane) { return reinterpret_cast<const uint2*>(kExpandTable.v)[lane]; }
+
+// For decoding, with the table of collapsed bytes: 256 bytes.
+struct LdsBitsCollapse : LdsBits {
+  static constexpr bool kCollapses = true;
+  const uint8_t* table;
+  __device__ __forceinline__ LdsBitsCollapse(uint32_t* region, const uint32_t* t)
+      : LdsBits(region), table(reinterpret_cast<const uint8_t*>(t))
+  {
+  }
+  __device__ __forceinline__ uint32_t collapsed(uint32_t word, int k) const { return table[(word >> (8 * k)) & 0xffu]; }
+};
+__constant__ const CollapseTable kCollapseTable = make_collapse_table();
+__device__ __forceinline__ uint32_t collapse_piece(unsigned lane) { return reinterpret_cast<const uint32_t*>(kCollapseTable.v)[lane]; }
+// What stands behind every block in the decoder's region.  A one, for the run that the budget cuts short, and zeros.
+constexpr uint64_t kFence = 1;
 
 // Layout of the wave's LDS bit region.
 //  whole-word rates (maxbits % 64 == 0): every lane owns a private slot of
@@ -457,7 +472,7 @@ __device__ __forceinline__ void load_region(uint32_t* lds, unsigned lane, uint32
       const uint64_t* src = stream + (size_t)(first + lane) * W;
       for (unsigned j = 0; j < W; j++) dst[j] = src[j];
     }
-    if (lane < valid) dst[W] = ~0ull;
+    if (lane < valid) dst[W] = kFence;
   } else {
     const unsigned nwords = (valid * maxbits + 63u) >> 6;
     const uint64_t* src = stream + (size_t)(first >> 6) * maxbits;
@@ -558,14 +573,16 @@ __device__ __forceinline__ void decode3_f32(const uint64_t* __restrict__ stream,
   // Measured on 402.7 MB: 97.5 us with one priority for everything, 94.3 us with the planes
   // above the rest, 87.8 us with the last part below the planes as well (16 bits per value:
   // 137 -> 129 us); the last part below the lifting: 110 us.
+  __shared__ uint32_t table[WHOLE ? 64 : 1];
   __builtin_amdgcn_s_setprio(3);
+  if (WHOLE) table[lane] = collapse_piece(lane);
   load_region<WHOLE, kFenceDwords>(lds, lane, first, valid, maxbits, slot, fd, stream);
   __syncthreads();
 
   if (lane < valid) {
     int32_t ib[64];
     float w;
-    LdsBits mem(lds);
+    LdsBitsCollapse mem(lds, table);
     if (INT) {
       w = 0.0f;
       decode_block_i32_zy<WHOLE>(mem, mem.bit0 + lane * slot, maxbits, ib);
@@ -782,8 +799,8 @@ struct LdsDecExchange {
 };
 
 template <int H>
-__device__ __forceinline__ void pair_decode_body(const Field3& fd, unsigned maxbits, uint32_t* lds, unsigned lane,
-                                                 uint32_t first, float* __restrict__ out)
+__device__ __forceinline__ void pair_decode_body(const Field3& fd, unsigned maxbits, uint32_t* lds, const uint32_t* table,
+                                                 unsigned lane, uint32_t first, float* __restrict__ out)
 {
   const unsigned region = dec_region_dwords(maxbits);
   LdsDecExchange<H> ex;
@@ -792,7 +809,7 @@ __device__ __forceinline__ void pair_decode_body(const Field3& fd, unsigned maxb
   ex.u0 = lds + region + kPairScales + kPairFlag;
   ex.u1 = ex.u0 + kPairDecU;
   ex.lane = lane;
-  LdsBits mem(lds);
+  LdsBitsCollapse mem(lds, table);
   float p[16], q[16];
   pair_decode_half<H>(mem, mem.bit0 + lane * dec_slot_bits(maxbits), maxbits, ex, p, q);
   if (first + lane < fd.nblocks) {
@@ -820,17 +837,19 @@ __global__ __launch_bounds__(128) void zfp_decode3_f32_pair_kernel(const uint64_
   uint32_t* lds = reinterpret_cast<uint32_t*>(lds_raw);
   const unsigned tid = threadIdx.x, lane = tid & 63u;
   const uint32_t first = blockIdx.x * 64u;
-  {  // the fence of ones goes behind every block; the slots past the end of the field read as empty blocks
+  __shared__ uint32_t table[64];
+  if (tid < 64) table[tid] = collapse_piece(tid);
+  {  // the fence goes behind every block; the slots past the end of the field read as empty blocks
     const unsigned W = maxbits >> 6, slot = dec_slot_bits(maxbits);
     const uint32_t valid = min(64u, fd.nblocks - first);
     load_pieces<128, kFenceDwords>(lds, tid, valid, maxbits, fd.by_piece, stream + (size_t)first * W);
     uint64_t* own = reinterpret_cast<uint64_t*>(lds + lane * (slot / 32));
-    if (tid < 64) own[W] = ~0ull;
+    if (tid < 64) own[W] = kFence;
     else if (lane >= valid) own[0] = 0;
   }
   __syncthreads();
-  if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) pair_decode_body<0>(fd, maxbits, lds, lane, first, out);
-  else pair_decode_body<1>(fd, maxbits, lds, lane, first, out);
+  if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) pair_decode_body<0>(fd, maxbits, lds, table, lane, first, out);
+  else pair_decode_body<1>(fd, maxbits, lds, table, lane, first, out);
 }
 
 // ------------------------------------------------------------- the quad form: four lanes per block
@@ -1052,6 +1071,8 @@ __global__ __launch_bounds__(64) void zfp_decode3_f32_quad_kernel(const uint64_t
   const bool live = b < fd.nblocks;
   const unsigned slot = dec_slot_bits(maxbits);
   uint32_t* ex = lds + quad_region_dwords(slot) + bl * kQuadStride;
+  __shared__ uint32_t table[64];
+  table[lane] = collapse_piece(lane);
   {  // the four lanes of a block bring its words; blocks past the end read as empty
     const unsigned W = maxbits >> 6;
     uint64_t* dst = reinterpret_cast<uint64_t*>(lds + bl * (slot / 32));
@@ -1067,15 +1088,15 @@ __global__ __launch_bounds__(64) void zfp_decode3_f32_quad_kernel(const uint64_t
     } else {
       for (unsigned j = q; j < W; j += 4) dst[j] = src[j];
     }
-    if (q == 0) dst[W] = ~0ull;
+    if (q == 0) dst[W] = kFence;
   }
   uint32_t to_xyz[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) to_xyz[i] = kQuadOrder.to_xyz[q][i];
   __syncthreads();
 
-  LdsBits mem(lds);
-  BlockDecoder<LdsBits, 64, true> dec(mem, mem.bit0 + bl * slot, maxbits);
+  LdsBitsCollapse mem(lds, table);
+  TableDecoder<LdsBitsCollapse> dec(mem, mem.bit0 + bl * slot, maxbits);
   const uint32_t h = (uint32_t)dec.window(dec.pos);
   const bool coded = (h & 1) != 0;
   dec.pos = coded ? dec.pos + 9 : dec.limit;
@@ -1094,7 +1115,7 @@ __global__ __launch_bounds__(64) void zfp_decode3_f32_quad_kernel(const uint64_t
   if (CSWAP_ANY(dec.active())) {
 #pragma unroll
     for (int k = 15; k >= 0; k--) {
-      const uint64_t x = dec.plane();
+      const uint64_t x = dec.low_plane();
       const uint32_t word = (q & 2u) ? (uint32_t)(x >> 32) : (uint32_t)x;
       if (k >= 8) l[k - 8] = word;
       else l[k] = byte_perm(l[k], word, mine);
@@ -1274,11 +1295,13 @@ __global__ __launch_bounds__(64) void zfp_decode3_w64_kernel(const uint64_t* __r
   const uint32_t first = blockIdx.x * 64u;
   const uint32_t valid = min(64u, fd.nblocks - first);
   __builtin_amdgcn_s_setprio(3);  // the 32-bit decoder's priorities (here, at two wavefronts per SIMD, worth 2.6 %)
+  __shared__ uint32_t table[WHOLE ? 64 : 1];
+  if (WHOLE) table[lane] = collapse_piece(lane);
   load_region<WHOLE, kSlackDwords>(lds, lane, first, valid, maxbits, slot_bits(maxbits), fd, stream);
   __syncthreads();
   if (lane < valid) {
     uint64_t q[64];
-    LdsBits mem(lds);
+    LdsBitsCollapse mem(lds, table);
     decode_block_w64<INT, WHOLE>(mem, mem.bit0 + lane * slot_bits(maxbits), maxbits, q);
     __builtin_amdgcn_s_setprio(1);
     store_block_w64<ONCE>(out, fd, first + lane, q);
@@ -1591,28 +1614,33 @@ static bool pair_fits(unsigned grid, size_t lds_bytes, unsigned long long limit)
   const double per_cu = 0.88 * 160.0 * 1024.0 / (double)lds_bytes;
   return (double)grid <= per_cu * (double)device_compute_units();
 }
-// The decoder's pair form gains nothing at 8 bits per value (the plane loop, which one half
-// runs alone, is 60 % of its time) and 3-7 % from 16 bits per value on, where the shared back
-// end weighs more.
-constexpr unsigned kPairDecodeFromBits = 1024;
+// The decoder's pair form, whose planes one half decodes alone, pays while every workgroup has a SIMD of
+// its own -- then what the halves share is worth its barriers -- and the planes are not all of the time:
+// lane / pair form at 16 bits per value 12.6 MB 13.35 / 12.7 us, 16.8 MB 13.0 / 12.4, 21 MB 14.6 / 14.6, 25.2 MB 14.3 / 15.2,
+// 41.9 MB 17.1 / 23.3; at 8 bits 12.6 MB 11.1 / 10.8, 16.8 MB 10.9 / 10.9; at 32 bits 12.6 MB 13.1 / 13.3, 16.8 MB 12.9 / 13.2.
+constexpr unsigned kPairDecodeFromBits = 1024, kPairDecodeBelowBits = 2048;
+static bool pair_decode_pays(unsigned grid, unsigned maxbits, unsigned long long limit)
+{
+  if (limit == ~0ull) return true;
+  return maxbits >= kPairDecodeFromBits && maxbits < kPairDecodeBelowBits && grid <= 4u * (unsigned)device_compute_units();
+}
 
 // The quad form pays while its wavefronts (16 blocks each) are few per compute unit: it trades
 // instructions (half as many again as the pair form's, for the same blocks) for short chains.
 // Microseconds, quad / pair / one lane per block at 8 bits per value by wavefronts per compute unit:
-//   encode  1 (1 MB) 6.1 / 7.9 / 10.7 · 4: 6.7 / 8.4 / 11.1 · 8: 8.1 / 9.6 / 11.7 · 12: 10.1 / 9.9 / 12.2 ·
-//           16: 11.1 / 10.2 / 12.6; where the pair form does not apply (odd planes): 8: 8.2 / - / 12.3 ·
-//           19: 14.9 / - / 17.7 · 30: 20.2 / - / 17.4
-//   decode  1: 9.2 / - / 11.8 · 4: 10.6 / - / 12.8 · 8: 11.2 / - / 12.4 · 12: 12.6 / - / 12.6 · 16: 13.9 / - / 13.4;
-//           odd planes 8: 11.6 / - / 14.2 · 10: 14.0 / - / 15.4 · 19: 21.0 / - / 18.3
-// Other rates, quad / the better of the other two.  Against the pair form and in the decoder the quad form
-// is ahead or level at its last size, 11, at all of them (encode 2 bits per value 8.6 / 10.3 · 16: 11.2 / 11.7 ·
-// 32: 12.5 / 14.4 · 64: 13.6 / 18.2; decode 10.4 / 10.3 · 14.6 / 14.7 · 14.8 / 16.0 · 15.5 / 17.8).  The encoder
-// of odd planes, 35x35: 2 bits 21: 12.0 / 13.3 · 16 bits 20: 16.2 / 17.8 · 22: 18.7 / 18.1 · 24 bits 18: 17.2 / 18.7 ·
-// 20: 20.5 / 19.3 · 28 bits 18: 17.8 / 19.5 · 20: 20.8 / 20.2 · 32 bits 20: 21.3 / 21.3 · 22: 22.3 / 22.3 ·
-// 40 bits 22: 23.7 / 24.6 · 64 bits 21: 25.8 / 40.7.  The steps are where the wavefronts' LDS no longer lets all of
-// them onto the chip at once; from 30 bits per value on one lane per block meets that limit, too.
-constexpr unsigned kQuadWaves = 11;        // per compute unit
-constexpr unsigned kQuadWavesNoPair = 22;  // the encoder's where the pair form does not apply
+//   encode  1 (1 MB) 4.5 / 6.1 / 7.6 · 4: 5.2 / 6.4 / 7.8 · 8: 6.6 / 7.6 / 8.5 · 12: 7.8 / 7.9 / 8.9 ·
+//           16: 9.2 / 8.2 / 9.3; where the pair form does not apply (odd planes): 8: 6.7 / - / 9.2 ·
+//           19: 10.7 / - / 11.9 · 23: 12.5 / - / 12.5 · 25: 14.1 / - / 13.1
+//   decode  1: 7.4 / 8.5 / 9.1 · 4: 8.1 / 8.9 / 9.5 · 8: 9.3 / 10.4 / 10.4 · 10: 10.8 / 10.6 / 10.8 · 14: 12.9 / 10.9 / 11.1;
+//           odd planes 8: 10.7 / - / 11.7 · 10: 12.8 / - / 12.2 · 15: 15.2 / - / 12.8
+// The decoder's lines cross at the same place at 4, 16 and 32 bits per value (9.6 / 9.5 / 9.6, 13.4 / 12.5 / 13.2 and
+// 13.6 / 13.2 / 13.1 at 10 wavefronts).  The encoder's against the pair form cross between 11 and 14 (12: 7.0 / 6.9 at 4
+// bits, 9.7 / 10.6 at 16, 11.8 / 13.4 at 32); of odd planes at 16 bits 19: 13.9 / 14.9 · 20: 15.3 / 15.2 · 21: 16.3 / 15.5, at 32 bits
+// 18: 18.1 / 18.4 · 25: 23.2 / 22.2.  The steps are where the wavefronts' LDS no longer lets all of them onto the chip at once;
+// from 30 bits per value on one lane per block meets that limit, too.
+constexpr unsigned kQuadWaves = 11;        // per compute unit, the encoder's where the pair form applies
+constexpr unsigned kQuadWavesNoPair = 22;  // where it does not
+constexpr unsigned kQuadWavesDecode = 9;
 constexpr unsigned kQuadOneRoundBelow = 1920;
 static double quad_waves_encode(const Field3& fd, unsigned maxbits)
 {
@@ -1743,7 +1771,7 @@ static int decompress3(const uint64_t* d_stream, Elem elem, size_t nx, size_t ny
   const bool whole = (maxbits & 63u) == 0;
   const bool is_int = elem == kI32 || elem == kI64;
   const unsigned long long pair_below = g_pair_decode_bytes.load(std::memory_order_relaxed);
-  if (quad && elem == kF32 && whole && quad_pays(fd.nblocks, kQuadWaves, (unsigned long long)nx * ny * nz * 4ull, pair_below,
+  if (quad && elem == kF32 && whole && quad_pays(fd.nblocks, kQuadWavesDecode, (unsigned long long)nx * ny * nz * 4ull, pair_below,
                                           device_compute_units())) {
     hipLaunchKernelGGL(zfp_decode3_f32_quad_kernel, dim3((fd.nblocks + kQuadBlocks - 1) / kQuadBlocks), dim3(64),
                        (size_t)quad_lds_dwords(dec_slot_bits(maxbits)) * 4, st, d_stream, fd, maxbits,
@@ -1751,8 +1779,7 @@ static int decompress3(const uint64_t* d_stream, Elem elem, size_t nx, size_t ny
     return check_launch();
   }
   if (elem == kF32 && pair_shape(fd, maxbits) && (unsigned long long)nx * ny * nz * 4ull < pair_below &&
-      (maxbits >= kPairDecodeFromBits || pair_below == ~0ull) &&
-      pair_fits(grid, (size_t)pair_dec_lds_dwords(maxbits) * 4, pair_below)) {
+      pair_decode_pays(grid, maxbits, pair_below)) {
     hipLaunchKernelGGL(zfp_decode3_f32_pair_kernel, dim3(grid), dim3(128), (size_t)pair_dec_lds_dwords(maxbits) * 4, st,
                        d_stream, fd, maxbits, static_cast<float*>(d_out));
     return check_launch();

@@ -51,6 +51,28 @@ extern "C" size_t cswap_policy_bytes(int policy, size_t n, size_t nnz, unsigned 
   }
 }
 
+// With d2h_hidden the outbound copy is taken to overlap with the layer's
+// compute (what the copy stream is for), so only the inbound copy is on the
+// critical path: the conservative view for a compressed option, whose kernels
+// and probe are not hidden.
+static double link_time_us(const cswap_costs& c, double bytes)
+{
+  double t = c.copy_latency_us + bytes / (c.bw_h2d_gbs * 1e3);
+  if (!c.d2h_hidden) t += c.copy_latency_us + bytes / (c.bw_d2h_gbs * 1e3);
+  return t;
+}
+static double min_gain_of(const cswap_costs& c) { return c.min_gain > 0 && c.min_gain <= 1.0 ? c.min_gain : 1.0; }
+
+bool cswap::made_payload_pays(size_t n, size_t bytes, const cswap_costs& c)
+{
+  const double in_bytes = 4.0 * (double)n;
+  if (c.bw_d2h_gbs <= 0 || c.bw_h2d_gbs <= 0 || c.zvc_expand_gbs <= 0 || in_bytes < (double)c.size_floor_bytes ||
+      (double)bytes >= c.sparse_max_ratio * in_bytes)
+    return false;
+  const double left = c.kernel_latency_us + in_bytes / (c.zvc_expand_gbs * 1e3) + link_time_us(c, (double)bytes);
+  return left < min_gain_of(c) * link_time_us(c, in_bytes);
+}
+
 static int select_core(size_t n, size_t nnz, size_t b_zfp, const cswap_costs* costs, cswap_choice* out)
 {
   if (!out || !n || nnz > n) return CSWAP_E_ARG;
@@ -58,15 +80,7 @@ static int select_core(size_t n, size_t nnz, size_t b_zfp, const cswap_costs* co
   if (costs) c = *costs; else cswap_costs_default(&c);
   if (c.bw_d2h_gbs <= 0 || c.bw_h2d_gbs <= 0) return CSWAP_E_ARG;
   const double in_bytes = 4.0 * (double)n;
-  // With d2h_hidden the outbound copy is taken to overlap with the layer's
-  // compute (what the copy stream is for), so only the inbound copy is on the
-  // critical path: the conservative view for a compressed option, whose kernels
-  // and probe are not hidden.
-  auto link_us = [&](double bytes) {
-    double t = c.copy_latency_us + bytes / (c.bw_h2d_gbs * 1e3);
-    if (!c.d2h_hidden) t += c.copy_latency_us + bytes / (c.bw_d2h_gbs * 1e3);
-    return t;
-  };
+  auto link_us = [&](double bytes) { return link_time_us(c, bytes); };
   const double inf = 1e300;
   // what deciding costs: the counting pass plus one host round trip for nnz; the
   // raw swap does not pay it, so every compressed option carries it
@@ -90,8 +104,7 @@ static int select_core(size_t n, size_t nnz, size_t b_zfp, const cswap_costs* co
   int pol = CSWAP_POLICY_NONE;
   double best = t_none;
   if ((size_t)in_bytes >= c.size_floor_bytes) {
-    const double gain = c.min_gain > 0 && c.min_gain <= 1.0 ? c.min_gain : 1.0;
-    double bar = gain * t_none;            // a compressed option must beat the raw swap by this margin
+    double bar = min_gain_of(c) * t_none;  // a compressed option must beat the raw swap by this margin
     if (t_sparse < bar) { best = t_sparse; pol = CSWAP_POLICY_SPARSE; }   // strict: ties stay raw
     const double need = pol == CSWAP_POLICY_SPARSE ? c.lossy_min_gain * best : bar;
     if (t_zfp < need) { best = t_zfp; pol = CSWAP_POLICY_ZFP; }

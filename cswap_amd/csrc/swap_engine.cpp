@@ -618,8 +618,11 @@ extern "C" int cswap_swap_out(cswap_engine* e, const float* d_in, size_t nx, siz
       cswap_choice ch;
       if ((rc = cswap_select_field(nx, ny, nz, t.nnz, t.maxbits, &costs, &ch))) { drop_device(e, t); return rc; }
       t.policy = ch.policy;
+      // The selector charges probe and compaction to the ZVC option.  Both have run by now: between sending
+      // this payload and dropping it for the raw tensor, only what is left to pay counts.
+      if (ch.policy == CSWAP_POLICY_NONE && cswap::made_payload_pays(n, t.bytes_out, costs)) t.policy = CSWAP_POLICY_SPARSE;
       want_probe = false;  // the count is known
-      if (ch.policy != CSWAP_POLICY_SPARSE) {
+      if (t.policy != CSWAP_POLICY_SPARSE) {
         drop_device(e, t);  // the pass has finished (its count is on the host): the block can go back at once
         rc = 1;             // on with the selector's choice below
       } else {

@@ -30,7 +30,8 @@ struct Field3 {
   int full;                // 1: rows4, and every block is a full one
   int stream16;            // 1: the stream pointer is 16-byte aligned
   uint32_t by_piece;       // whole-word rates with an even number of words per block, else 0: the multiplier of block_of_piece
-  int read_once;           // 1: the encoder should load the field with the nontemporal hint (see make_field)
+  int read_once;           // 1: a field of kReadOnceBytes and more (see make_field)
+  int store_hint;          // 1: the 32-bit decoder stores the field's rows with the nontemporal hint (see make_field)
   int once64;              // 1: the decoder of 64-bit elements should store its rows with the hint (see make_field)
   Div31 by_mx, by_my;      // block index -> block coordinates without a hardware divide
 };
@@ -598,7 +599,7 @@ __device__ __forceinline__ void decode3_f32(const uint64_t* __restrict__ stream,
     const uint32_t b = first + __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));  // lane id again
     __builtin_amdgcn_s_setprio(1);
     // (as one variant with the hint decided row by row, the compiler finishes all rows ahead and spills)
-    if (ROWS && fd.rows16) finish_and_store_rows<INT, true>(out, fd, first, b, ib, w);
+    if (ROWS && fd.store_hint) finish_and_store_rows<INT, true>(out, fd, first, b, ib, w);
     else if (ROWS) finish_and_store_rows<INT, false>(out, fd, first, b, ib, w);
     else finish_and_store_block<INT>(out, fd, first, b, ib, w);
   }
@@ -798,7 +799,7 @@ struct LdsDecExchange {
   }
 };
 
-template <int H>
+template <int H, bool HINT>
 __device__ __forceinline__ void pair_decode_body(const Field3& fd, unsigned maxbits, uint32_t* lds, const uint32_t* table,
                                                  unsigned lane, uint32_t first, float* __restrict__ out)
 {
@@ -824,14 +825,22 @@ __device__ __forceinline__ void pair_decode_body(const Field3& fd, unsigned maxb
     for (int y = 0; y < 4; y++) {
       const stream_f4 vp = {p[4 * y], p[4 * y + 1], p[4 * y + 2], p[4 * y + 3]};
       const stream_f4 vq = {q[4 * y], q[4 * y + 1], q[4 * y + 2], q[4 * y + 3]};
-      __builtin_nontemporal_store(vp, reinterpret_cast<stream_f4*>(base + (size_t)(me + (y * sy4 + ZP * sz4))));
-      __builtin_nontemporal_store(vq, reinterpret_cast<stream_f4*>(base + (size_t)(me + (y * sy4 + ZQ * sz4))));
+      stream_f4* dp = reinterpret_cast<stream_f4*>(base + (size_t)(me + (y * sy4 + ZP * sz4)));
+      stream_f4* dq = reinterpret_cast<stream_f4*>(base + (size_t)(me + (y * sy4 + ZQ * sz4)));
+      if (HINT) {
+        __builtin_nontemporal_store(vp, dp);
+        __builtin_nontemporal_store(vq, dq);
+      } else {
+        *dp = vp;
+        *dq = vq;
+      }
     }
   }
 }
 
-__global__ __launch_bounds__(128) void zfp_decode3_f32_pair_kernel(const uint64_t* __restrict__ stream, Field3 fd,
-                                                                   unsigned maxbits, float* __restrict__ out)
+template <bool HINT>
+__device__ __forceinline__ void pair_decode(const uint64_t* __restrict__ stream, const Field3& fd, unsigned maxbits,
+                                            float* __restrict__ out)
 {
   extern __shared__ uint4 lds_raw[];
   uint32_t* lds = reinterpret_cast<uint32_t*>(lds_raw);
@@ -848,8 +857,21 @@ __global__ __launch_bounds__(128) void zfp_decode3_f32_pair_kernel(const uint64_
     else if (lane >= valid) own[0] = 0;
   }
   __syncthreads();
-  if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) pair_decode_body<0>(fd, maxbits, lds, table, lane, first, out);
-  else pair_decode_body<1>(fd, maxbits, lds, table, lane, first, out);
+  if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) pair_decode_body<0, HINT>(fd, maxbits, lds, table, lane, first, out);
+  else pair_decode_body<1, HINT>(fd, maxbits, lds, table, lane, first, out);
+}
+
+__global__ __launch_bounds__(128) void zfp_decode3_f32_pair_kernel(const uint64_t* __restrict__ stream, Field3 fd,
+                                                                   unsigned maxbits, float* __restrict__ out)
+{
+  pair_decode<true>(stream, fd, maxbits, out);
+}
+// for rows that are not made of half lines (Field3::store_hint): 12.6 MB in 8x8 planes at 16 bits per value
+// 13.5 us, 17.4 with the hint, 12.8 MB in 28x28 planes 13.5 and 13.9
+__global__ __launch_bounds__(128) void zfp_decode3_f32_pair_plain_kernel(const uint64_t* __restrict__ stream, Field3 fd,
+                                                                         unsigned maxbits, float* __restrict__ out)
+{
+  pair_decode<false>(stream, fd, maxbits, out);
 }
 
 // ------------------------------------------------------------- the quad form: four lanes per block
@@ -1165,7 +1187,7 @@ __global__ __launch_bounds__(64) void zfp_decode3_f32_quad_kernel(const uint64_t
   const uint32_t bx = min(4u, fd.nx - x0), by = min(4u, fd.ny - y0), bz = min(4u, fd.nz - z0);
   if (!live || q >= bz) return;
   float* p = out + ((long long)x0 * fd.sx + (long long)y0 * fd.sy + (long long)(z0 + q) * fd.sz);
-  if (fd.full && fd.rows16) {
+  if (fd.full && fd.rows16) {  // few enough lines for the hint whatever the rows are (4.2 MB in 4x4 planes 7.5 us, 7.8 without)
 #pragma unroll
     for (int y = 0; y < 4; y++) {
       const stream_f4 v = {r[4 * y], r[4 * y + 1], r[4 * y + 2], r[4 * y + 3]};
@@ -1528,18 +1550,27 @@ static int make_field(Field3& fd, const void* base, const void* stream, size_t n
   fd.full = fd.rows4 && ((nx | ny | nz) & 3u) == 0;
   fd.stream16 = ((uintptr_t)stream % 16) == 0;
   fd.by_piece = piece_multiplier(maxbits);
-  // Cache policy of the field's 16-byte rows (whole 128-byte lines per wave instruction).
-  // The decoder always stores them with the nontemporal hint: 402.7 MB decode in 107 us
-  // instead of 117 us, and the kernel that runs next no longer waits behind those lines
-  // draining from the memory-side cache (33.6 MB: decode 14.5 instead of 17.6 us, and a
-  // reader of the result right after it is no slower).  The encoder loads with the hint
-  // only when the field is large against that cache (256 MB): a smaller tensor is still
-  // cached from the kernel that produced it, and hinted loads of cached lines are slower.
+  // Cache policy of the field's 16-byte rows.
+  // The decoder stores them with the nontemporal hint where a row is made of whole 128-byte lines, which
+  // one instruction then writes: 402.7 MB decode in 107 us instead of 117 us, and the kernel that runs next
+  // no longer waits behind those lines draining from the memory-side cache (33.6 MB: decode 14.5
+  // instead of 17.6 us, and a reader of the result right after it is no slower).  A line that several
+  // instructions write in parts leaves the cache in those parts, each a write of its own to memory; without
+  // the hint it is put together there.  Hint / none, decoded at 8 bits per value by bytes per row, warm: 16 (4x4
+  // planes) 33.6 MB 73.8 / 20.4 us, 134 MB 321 / 51 · 32: 33.6 MB 34.3 / 16.1, 134 MB 136 / 36 · 112: 51 MB 32.2 / 19.2, 411 MB
+  // 244 / 131 · 144: 64 MB 35.8 / 21.1 · 224: 206 MB 83 / 50; nothing cached: 272: 200 MB 84.6 / 68.7 · 784: 73.6 / 69.3 · 3088:
+  // 68.4 / 65.3, but 50 MB 21.3 / 21.8.  Rows of whole half lines, hint / none: 64 bytes 67 MB 26.8 / 22.9 cold, 134 MB 44.3 /
+  // 45.7, 268 MB warm 75.8 / 79.8 · 192: 75 MB 24.2 / 24.8, 227 MB 54.8 / 60.9.
+  // The encoder loads with the hint only when the field is large against that cache (256 MB): a smaller
+  // tensor is still cached from the kernel that produced it, and hinted loads of cached lines are slower.
   // Producer kernel + encoder, hinted / plain loads: 402.7 MB 205 / 220 us, 201.3 MB
-  // 95 / 109 us, 100.7 MB 43.6 / 43.2 us, 50.3 MB 26.1 / 24.5 us.  The stream keeps the
-  // default policy: a lane's piece of it is not a whole line, and the decoder or the copy
-  // engine reads it next.
+  // 95 / 109 us, 100.7 MB 43.6 / 43.2 us, 50.3 MB 26.1 / 24.5 us.  Rows shorter than a line and not made of half lines
+  // are fetched once per instruction that wants a part of it: hint / none, 32 bytes 268 MB 90 / 68 cold, 96: 151 MB 41.6 /
+  // 37.0 warm, 112: 411 MB 107 / 100; from a line on the hint is ahead again (224: 206 MB 51.8 / 54.8).
+  // The stream keeps the default policy: the decoder or the copy engine reads it next.
   fd.read_once = (unsigned long long)nx * ny * nz * elem >= kReadOnceBytes;
+  const unsigned long long pitch = (unsigned long long)fd.sy * elem;
+  fd.store_hint = fd.rows16 && (pitch % 128 == 0 || (fd.read_once ? pitch % 64 == 0 : pitch >= 1536));
   // 64-bit elements: a lane's row is two 16-byte pieces, half a line per store instruction.  The
   // hint on those stores gains 15 % at 537 MB and loses 20 % at 134 MB: only for fields of 256 MiB
   // and more (the memory-side cache's size).
@@ -1583,12 +1614,15 @@ static bool pair_shape(const Field3& fd, unsigned maxbits)
 
 // Whether the encoder loads with the nontemporal hint (make_field: read_once); the variants that do are
 // those of whole-word rates.
-static bool load_hint(const Field3& fd, bool whole) { return fd.read_once && fd.rows16 && whole; }
+static bool load_hint(const Field3& fd, bool whole)
+{
+  return fd.read_once && fd.rows16 && whole && (fd.sy % 16 == 0 || fd.sy >= 32);  // (elements; make_field has the reasons)
+}
 
 // Which fields the kernels for contiguous rows at any element take.  The encoder's: all that are not
 // whole blocks of aligned rows.  Both leave fields whose rows are aligned and whole along x to the other
 // kernel where that one has the hint: only the last block rows are cut off there, and the hint on the
-// others' whole lines is worth more.  The decoder's has it always (39 MB in 197 rows of 768: encode
+// others' whole lines is worth more.  The decoder's has it always, and takes no other fields (39 MB in 197 rows of 768: encode
 // 20.8 us either way, decode 16.2 with the other kernel, 17.1 with this; 57 MB in 197 rows of 196: encode
 // 28.1 and 26.3, decode 28.3 both), the encoder's on large fields (producer kernel + encoder, other kernel
 // / this, 197 rows of 768 or 3072: 201 MB at 8 bits per value 116 / 123 us, 290 MB 156 / 172, 402 MB
@@ -1599,7 +1633,7 @@ static bool encode_rows(const Field3& fd, bool whole)
 {
   return fd.rows4 && !(fd.full && fd.rows16) && !(load_hint(fd, whole) && (fd.nx & 3u) == 0);
 }
-static bool decode_rows(const Field3& fd) { return fd.rows4 && !(fd.rows16 && (fd.nx & 3u) == 0); }
+static bool decode_rows(const Field3& fd) { return fd.rows4 && !(fd.store_hint && (fd.nx & 3u) == 0); }
 
 static std::atomic<unsigned long long> g_pair_decode_bytes{CSWAP_PAIR_DECODE_BYTES};
 
@@ -1780,8 +1814,9 @@ static int decompress3(const uint64_t* d_stream, Elem elem, size_t nx, size_t ny
   }
   if (elem == kF32 && pair_shape(fd, maxbits) && (unsigned long long)nx * ny * nz * 4ull < pair_below &&
       pair_decode_pays(grid, maxbits, pair_below)) {
-    hipLaunchKernelGGL(zfp_decode3_f32_pair_kernel, dim3(grid), dim3(128), (size_t)pair_dec_lds_dwords(maxbits) * 4, st,
-                       d_stream, fd, maxbits, static_cast<float*>(d_out));
+    const auto kernel = fd.sy % 16 == 0 ? zfp_decode3_f32_pair_kernel : zfp_decode3_f32_pair_plain_kernel;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(128), (size_t)pair_dec_lds_dwords(maxbits) * 4, st, d_stream, fd, maxbits,
+                       static_cast<float*>(d_out));
     return check_launch();
   }
   if (elem_bytes(elem) == 4) {

@@ -427,7 +427,9 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand4_kernel(
 // keeps one word together with where its values start and where its elements go, so a word
 // finds its chunk's end and offset by itself and the eight rows of a refill are full.
 // 16384 chunks, one wavefront per chunk -> this: 7 MB 11.3 -> 5.9 us, 25.7 MB 11.1 -> 8.4,
-// 33.6 MB (512 elements per chunk) 11.0 -> 8.7.
+// 33.6 MB (512 elements per chunk) 11.0 -> 8.7.  Its stores have the hint at any element: several tensors in turn, 16384
+// chunks, without -> with: 19 MB (289 elements per chunk) 8.4 -> 7.8 us, 24 MB 11.4 -> 9.4, 32 MB 13.4 -> 11.3, compaction and
+// expansion 23.6 -> 21.2, 26.6 -> 24.0, 29.9 -> 29.1 (one tensor over and over 23.9 -> 23.4, 24.7 -> 24.4, 25.7 -> 26.5).
 // It takes chunks of at most kPackedWords mask words where there are more than kPackedFrom of
 // them: three or more to a wavefront.  Two to a wavefront measure the same as one each, and few
 // chunks are all in flight at once either way.
@@ -489,7 +491,7 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand_packed_kernel(
     if (j >= rows) break;
     float* q = out + to[j];
     if (left[j] >= 4) {
-      st_row4<ALIGNED>(q, x[j]);
+      st_row4<ALIGNED, true>(q, x[j]);
     } else {
       if (left[j] > 0) q[0] = x[j].x;
       if (left[j] > 1) q[1] = x[j].y;

@@ -18,7 +18,10 @@
 //    network instead of extracting each plane bit by bit.
 //  * The coder emits whole runs: "group test 1, t zeros, terminating 1" is two
 //    single-bit ORs into a zeroed bit region, placed with a count-trailing-zeros,
-//    not t+2 single-bit writes; nothing is accumulated or flushed.
+//    not t+2 single-bit writes; nothing is accumulated or flushed.  Where the caller
+//    has the tables (TableEncoder, TableDecoder: whole-word rates), all the runs of
+//    a plane are written from a byte table, 32 coefficients at a time, and read
+//    32 stream bits at a time.
 //  * The bit budget is applied as a cut of the unconstrained code at maxbits
 //    (the reference's per-bit budget counter stops the same sequence of writes
 //    at the same place, so the kept prefix is the same).
@@ -657,7 +660,11 @@ struct BlockEncoder {
 // The bits behind a plane's verbatim ones come from the table, 32 coefficients at a time, so that a
 // wavefront pays for a plane in which some of its blocks find any the same 60 to 95 instructions
 // however many they find, where the steps took 17 for each of the most that one block finds (45 a
-// wavefront in all on normally distributed values at 8 bits per value, in 8.5 planes).
+// wavefront in all on normally distributed values at 8 bits per value, in 8.5 planes).  Bound by instruction
+// issue and latency below 100 MB, by memory above; steps -> table at 8 bits per value: 1 MB 6.0 -> 4.6 us,
+// 16.8 MB 10.2 -> 8.2, 50.3 MB 21.2 -> 17.5, 100.7 MB 31.5 -> 26.8, 402.7 MB 96 -> 88; 2438 -> 2171 vector instructions
+// per 64 blocks at 55 instead of 45 active lanes.  Steps for planes with few runs and the table for the
+// others was no faster, wherever the line was drawn.
 template <class Mem>
 struct TableEncoder : BlockEncoder<Mem, false> {
   using Base = BlockEncoder<Mem, false>;
@@ -1329,6 +1336,11 @@ struct BlockDecoder {
 // the negative group test.  Which ones are whose takes an addition: with a one added at the start of
 // every run that starts at an even place, those runs turn to zeros and the others stay, and a
 // coefficient's bits are the even places of the former and the odd ones of the latter.
+// A turn is some 60 instructions, and 14 of them decode a wavefront's 64 blocks of normally distributed
+// values at 8 bits per value; a turn per coefficient took 45, each with an LDS read to wait for.  Turn per
+// coefficient -> this: 1 MB 9.2 -> 7.2 us, 16.8 MB 12.8 -> 10.0, 50.3 MB 17.1 -> 15.8, 201.3 MB at 16 bits 62.5 -> 57.8,
+// 402.7 MB 82.5 -> 82.0 (memory).  Asking for the first turn's bits along with the verbatim ones: 16.8 MB
+// 10.3 -> 10.0, 100 MB 25.3 -> 25.5.
 template <class Mem>
 struct TableDecoder : BlockDecoder<Mem, 64, true> {
   using Base = BlockDecoder<Mem, 64, true>;
@@ -1669,8 +1681,8 @@ CSWAP_HD void pair_decode16(Dec& dec, uint64_t (&x)[16], bool top)
 }
 
 // p, q receive the half's two z-slices ([x + 4y]; half 0: z = 0 and 3, half 1: z = 2 and 1).
-// The block owns [pos0, pos0 + maxbits) of the bit region behind mem, followed by a fence of
-// one-bits (only half 0 reads it).
+// The block owns [pos0, pos0 + maxbits) of the bit region behind mem, followed by its
+// fence (only half 0 reads it).
 template <int H, class Ex, class Mem>
 CSWAP_HD void pair_decode_half(Mem& mem, unsigned pos0, unsigned maxbits, Ex& ex, float (&p)[16], float (&q)[16])
 {

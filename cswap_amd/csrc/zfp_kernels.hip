@@ -121,9 +121,9 @@ __host__ __device__ inline unsigned region_dwords(unsigned maxbits)
 {
   return ((2u * slot_bits(maxbits) + 4u) + 3u) & ~3u;  // + padding for the 128-bit over-read / over-write
 }
-// The 32-bit decoder's slot is the block and its fence of 64 ones, nothing more: the
-// window it reads through reaches up to 64 bits further, into the next lane's block
-// (or the region's padding), and those bits are never looked at.  What this saves in
+// The 32-bit decoder's slot is the block and its fence (kFence), nothing more: its
+// reads reach up to 128 bits further, into the next lane's block (or the region's
+// padding), and those bits are never looked at.  What this saves in
 // LDS is two more wavefronts per compute unit at 16 bits per value (8720 bytes a
 // wavefront instead of 9232), and the stride of 2 (mod 4) dwords halves the bank
 // conflicts between lanes.  Slots are 8-byte aligned only.
@@ -225,9 +225,10 @@ __device__ __forceinline__ void padded_offsets(uint32_t n, uint32_t s, uint32_t 
 // selected in registers.  Only blocks whose reads would leave the field (the last block along
 // all three axes) go element by element.  nx = 1 stays out: four elements are up to four rows
 // there, and other blocks than the last could leave the field.  Against one predicated 4-byte
-// access per element with its own 64-bit address, at 8 bits per value: 60 MB in 35x35 planes
-// encoded in 26.2 instead of 28.1 us and decoded in 26.4 instead of 39.8, 321 MB of them in 90
-// instead of 108 and 119 instead of 166; 26 MB in 14x14 planes 16.9 / 19.6 and 18.7 / 26.5.
+// access per element with its own 64-bit address, at 8 bits per value and with the coders that step from
+// run to run: 60 MB in 35x35 planes encoded in 26.2 instead of 28.1 us and decoded in 26.4 instead of 39.8,
+// 321 MB of them in 90 instead of 108 and 119 instead of 166; 26 MB in 14x14 planes 16.9 / 19.6 and 18.7 / 26.5.
+// Now: 60 MB in 35x35 planes 21.9 and 22.9, 26 MB in 14x14 13.3 and 16.2.
 __device__ __forceinline__ void load_row(const char* src, float (&f)[64], int row)
 {
   const row_f4* p = reinterpret_cast<const row_f4*>(src);
@@ -458,7 +459,7 @@ __device__ __forceinline__ void store_region(const uint32_t* lds, unsigned lane,
 }
 
 // the wave's coded blocks from the stream into LDS; whole-word rates get the
-// fence of ones behind every block that the fenced decoder relies on
+// fence behind every block that the fenced decoder relies on
 template <bool WHOLE, unsigned PAD>
 __device__ __forceinline__ void load_region(uint32_t* lds, unsigned lane, uint32_t first, uint32_t valid,
                                             unsigned maxbits, unsigned slot, const Field3& fd,
@@ -490,8 +491,9 @@ __device__ __forceinline__ void load_region(uint32_t* lds, unsigned lane, uint32
 // WPE: wavefronts per SIMD the kernel is built for and held to.  Five, except from 16 bits
 // per value on: there a wavefront's LDS region (9 KB and more) lets 16 or 17 wavefronts
 // into a compute unit, unevenly over its SIMDs, and the encoder measured fastest with
-// three per SIMD (402.7 MB at 16 bits per value: 130-133 us against 139-140 us with four
-// or five), the decoder with four (137-140 us against 143-156 us).
+// three per SIMD (201.3 MB at 16 bits per value: 72.7 us, 73.1 with four and 74.3 with five, 72.1 with two
+// but 50 MB 26.4 instead of 21.9), the decoder with four (402.7 MB, stepping from run to run, 137-140 us
+// against 143-156 us).  Now 58 us each for 201.3 MB, 111 and 110 for 402.7 MB.
 // ROWS: a field for load_block_rows
 template <bool WHOLE, bool INT, bool ONCE, bool ROWS>
 __device__ __forceinline__ void encode3_f32(const float* __restrict__ in, const Field3& fd, unsigned maxbits,
@@ -506,8 +508,8 @@ __device__ __forceinline__ void encode3_f32(const float* __restrict__ in, const 
 
   // A wavefront in one of its memory phases (the loads here, the stores at the end) goes before
   // the ones that are coding when both have an instruction to issue: its requests are what the
-  // compute unit's other wavefronts will be computing behind (measured on 402.7 MB: encode 100 ->
-  // 97 us at 8 bits per value, 129 -> 126 us at 16; the other way round 100 and 131 us).
+  // compute unit's other wavefronts will be computing behind (201.3 MB, nothing cached: 51.7 -> 49.9 us at
+  // 8 bits per value, 61.8 -> 59.1 at 16; 402.7 MB 94.0 and 93.9).
   __shared__ uint2 table[WHOLE ? 64 : 1];
   float f[64];
   __builtin_amdgcn_s_setprio(3);
@@ -545,7 +547,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
   encode3_f32<WHOLE, INT, ONCE, false>(in, fd, maxbits, stream);
 }
 // Kernels of their own for these fields: one kernel with both kinds of rows decoded full fields 2-6 %
-// slower (100 MB 29.2 instead of 27.5 us, 403 MB 89.7 instead of 87.4).
+// slower (100 MB 29.2 instead of 27.5 us, 403 MB 89.7 instead of 87.4; measured with a step per run).
 template <bool WHOLE, bool INT = false, int WPE = 5>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void zfp_encode3_rows_kernel(
     const float* __restrict__ in, Field3 fd, unsigned maxbits, uint64_t* __restrict__ stream)
@@ -571,7 +573,7 @@ __device__ __forceinline__ void decode3_f32(const uint64_t* __restrict__ stream,
   // Issue priorities: the load of the stream and the bit planes (a dependent chain through LDS
   // reads) go first, the lifting along z and y inside decode_block_zy fills the slots that are
   // left, and the last part -- lifting along x, cast, the row stores -- sits between the two.
-  // Measured on 402.7 MB: 97.5 us with one priority for everything, 94.3 us with the planes
+  // Measured on 402.7 MB, with a step per run: 97.5 us with one priority for everything, 94.3 us with the planes
   // above the rest, 87.8 us with the last part below the planes as well (16 bits per value:
   // 137 -> 129 us); the last part below the lifting: 110 us.
   __shared__ uint32_t table[WHOLE ? 64 : 1];
@@ -887,8 +889,8 @@ __global__ __launch_bounds__(128) void zfp_decode3_f32_pair_plain_kernel(const u
 //            decode every plane, each keeps its quarter, and the exchange that the encoder needs falls away
 // A lane's rows are loaded by the padding rule's addresses, so the form takes every field of
 // floats at a whole-word rate.  What bounds it is the chain left in a wavefront: the encoder's
-// four rounds of planes, the decoder's 13 to 16 planes one after the other.  4.2 MB at 8 bits
-// per value: encode 8.4 (pair form) -> 6.7 us, decode 12.8 -> 10.6; the rule is at quad_pays.
+// four rounds of planes, the decoder's 13 to 16 planes one after the other.  4.2 MB at 8 bits per value,
+// quad / one lane per block: encode 5.2 / 7.8 us (pair form 6.4), decode 8.1 / 9.5; the rule is at quad_pays.
 constexpr unsigned kQuadBlocks = 16;   // blocks of a wavefront
 constexpr unsigned kQuadStride = 68;   // dwords of a block's exchange area: 64 and four to spread the banks
 __host__ __device__ inline unsigned quad_region_dwords(unsigned slot) { return (kQuadBlocks * slot / 32 + 4u + 3u) & ~3u; }

@@ -276,7 +276,10 @@ typedef enum { CSWAP_POLICY_AUTO = -1, CSWAP_POLICY_NONE = 2, CSWAP_POLICY_SPARS
                 * (Execution.h:89-95) -- and asks the selector with that count.  If the answer is
                 * still ZVC the payload is there already; if not, the selector's choice runs as
                 * it would have after a probe.  Never a wrong result, one wasted pass when the
-                * expectation was wrong. */
+                * expectation was wrong.  Where the compaction was the probe (here, and for
+                * CSWAP_POLICY_AUTO on tensors that the one-kernel form takes) and the selector says
+                * raw, the payload that is there is sent all the same if what is left to pay for it,
+                * link and expansion, is less than min_gain times the raw swap. */
                CSWAP_POLICY_AUTO_SPARSE = -3 } cswap_policy;
 
 typedef struct {

@@ -471,7 +471,7 @@ constexpr uint16_t expand8(unsigned b)
   }
   return e;
 }
-struct ExpandTable {
+struct alignas(16) ExpandTable {
   uint16_t v[256];
 };
 constexpr ExpandTable make_expand_table()
@@ -507,7 +507,7 @@ constexpr uint8_t collapse8(unsigned b)
   }
   return c;
 }
-struct CollapseTable {
+struct alignas(16) CollapseTable {
   uint8_t v[256];
 };
 constexpr CollapseTable make_collapse_table()

@@ -45,14 +45,14 @@ def bench_schedule(dev, batch: int = 128, seed: int = 0) -> dict:
     for e in sched:
         x = torch.from_numpy(config4_tensor(e, seed)).to(dev)
         out = torch.empty_like(x)
-        lat, chosen, phases = {}, None, None
+        lat, chosen, remembered, phases = {}, None, swap.NONE, None
         for label in ("none", "auto", "remembered"):
             if label == "none":
                 pol = swap.NONE
             elif label == "auto":
                 pol = swap.AUTO
             else:
-                pol = swap.AUTO_SPARSE if chosen.policy == swap.SPARSE else chosen.policy
+                pol = swap.AUTO_SPARSE if remembered == swap.SPARSE else remembered
             best = None
             for _ in range(5):
                 torch.cuda.synchronize()
@@ -64,7 +64,7 @@ def bench_schedule(dev, batch: int = 128, seed: int = 0) -> dict:
                 torch.cuda.synchronize()
                 t1 = time.perf_counter()
                 info = eng.info(tk)
-                tm = eng.timing(tk)
+                tm, decision = eng.timing(tk), eng.decision(tk)
                 eng.release(tk)
                 if best is None or t1 - t0 < best:
                     best = t1 - t0
@@ -72,7 +72,7 @@ def bench_schedule(dev, batch: int = 128, seed: int = 0) -> dict:
                         phases = tm
             lat[label] = best * 1e3
             if label == "auto":
-                chosen = info
+                chosen, remembered = info, decision
         # dummy compute alone, to report how much of it the swap hides
         torch.cuda.synchronize()
         t0 = time.perf_counter(); dummy_layer_compute(a, b, 2); torch.cuda.synchronize()
@@ -85,8 +85,8 @@ def bench_schedule(dev, batch: int = 128, seed: int = 0) -> dict:
                                    "copy_in": round(phases.copy_in_us, 1), "decompress": round(phases.decompress_us, 1)}})
         for k in tot:
             tot[k] += lat[k]
-        if chosen.policy != swap.NONE:
-            for k in worst:
+        for k, pol in (("auto", chosen.policy), ("remembered", remembered)):
+            if pol != swap.NONE:
                 worst[k] = max(worst[k], lat[k] / lat["none"])
         del x, out
     eng.close()

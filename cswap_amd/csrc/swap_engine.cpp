@@ -101,6 +101,7 @@ enum TicketState { kFree = 0, kOutInFlight = 1, kOnHost = 2, kInInFlight = 3, kP
 struct Ticket {
   int state = kFree;
   int policy = CSWAP_POLICY_NONE;
+  int decision = CSWAP_POLICY_NONE;  // what to remember for the next time (cswap_swap_decision)
   int process = 0;  // ZVC chunk count this tensor was compacted with
   unsigned maxbits = 0;  // ZFP bits per block this tensor was (or would be) coded with: the engine's rate at its swap-out
   size_t n = 0, nnz = 0, nx = 0, ny = 0, nz = 0;
@@ -580,7 +581,7 @@ extern "C" int cswap_swap_out(cswap_engine* e, const float* d_in, size_t nx, siz
   }
   Ticket& t = e->tickets[(size_t)id];
   const int requested = policy;
-  t.policy = policy; t.n = n; t.nnz = n; t.nx = nx; t.ny = ny; t.nz = nz;
+  t.policy = t.decision = policy; t.n = n; t.nnz = n; t.nx = nx; t.ny = ny; t.nz = nz;
   t.dev_held = false;
   t.probe_held = false;
   t.out_pending = t.done_pending = t.keep_staged = false;
@@ -620,7 +621,9 @@ extern "C" int cswap_swap_out(cswap_engine* e, const float* d_in, size_t nx, siz
       t.policy = ch.policy;
       // The selector charges probe and compaction to the ZVC option.  Both have run by now: between sending
       // this payload and dropping it for the raw tensor, only what is left to pay counts.
+      // The answer itself stays: a caller that remembers "raw" pays for neither of them the next time.
       if (ch.policy == CSWAP_POLICY_NONE && cswap::made_payload_pays(n, t.bytes_out, costs)) t.policy = CSWAP_POLICY_SPARSE;
+      t.decision = ch.policy;
       want_probe = false;  // the count is known
       if (t.policy != CSWAP_POLICY_SPARSE) {
         drop_device(e, t);  // the pass has finished (its count is on the host): the block can go back at once
@@ -660,6 +663,7 @@ extern "C" int cswap_swap_out(cswap_engine* e, const float* d_in, size_t nx, siz
   }
 
   if ((rc = reserve_blocks(e, t, requested))) return rc;
+  t.decision = t.policy;
   const void* src = nullptr;
   rc = compress_tensor(e, t, d_in, compute, &src);
   if (!rc) rc = start_outbound_copy(e, t, src, compute);
@@ -855,6 +859,16 @@ extern "C" int cswap_swap_info(cswap_engine* e, int ticket, cswap_ticket_info* i
   info->bytes_out = t->bytes_out;
   // to the caller a released ticket is free, and a payload that a prefetch found still staged is prefetched
   info->state = t->state == kReleasing ? (int)kFree : (t->state == kOutInFlight && t->keep_staged ? (int)kPrefetched : t->state);
+  return CSWAP_OK;
+}
+
+extern "C" int cswap_swap_decision(cswap_engine* e, int ticket, int* policy)
+{
+  if (!e || !policy) return CSWAP_E_ARG;
+  std::lock_guard<std::mutex> lock(e->mu);
+  Ticket* t = get_ticket(e, ticket);
+  if (!t) return CSWAP_E_ARG;
+  *policy = t->decision;
   return CSWAP_OK;
 }
 

@@ -17,6 +17,8 @@ from __future__ import annotations
 import torch
 
 from . import swap
+from ._lib import CswapError
+from .hooks import E_NOMEM
 
 CONV, POOL, ACT, BN, FC, MASKFILL = range(6)   # Layer_type, CSWAP+/Execution.h:28-35
 
@@ -85,7 +87,7 @@ class Execution:
             if act == 1:
                 self._dropped.add(tid)
                 continue
-            remember = False
+            remember, asked = False, act
             if act == swap.AUTO and self.recheck > 0:
                 m = self._memo.get(tid)
                 if m and m[0] == t.numel() and m[2] < self.recheck and m[1] in (swap.ZFP, swap.NONE):
@@ -96,9 +98,15 @@ class Execution:
                     remember = True
                     if m and m[0] == t.numel() and m[1] == swap.SPARSE:
                         act = swap.AUTO_SPARSE   # the selector, with the compaction itself as its probe
-            ticket = self.engine.pre(t, act)
+            try:
+                ticket = self.engine.pre(t, act)
+            except CswapError as err:
+                if err.code != E_NOMEM or act == asked:
+                    raise
+                remember = True              # no room for what is remembered: the selector may find some
+                ticket = self.engine.pre(t, asked)
             if remember:
-                self._memo[tid] = [t.numel(), self.engine.info(ticket).policy, 0]
+                self._memo[tid] = [t.numel(), self.engine.decision(ticket), 0]
             self._tickets[tid] = (ticket, tuple(t.shape))
             self._pending.append(tid)
 

@@ -86,7 +86,8 @@ class swap_saved_tensors(torch.autograd.graph.saved_tensors_hooks):
     under (k, element count).  A remembered "ZFP" or "raw" is passed to the engine
     as an explicit policy and costs no probe; a remembered "ZVC" goes in as
     ``AUTO_SPARSE``: the one-kernel compaction runs first and its count is the
-    selector's probe, so the choice is confirmed every time.  After ``recheck`` uses
+    selector's probe, so the choice is confirmed every time.  (A payload that went out only
+    because the probe had made it is remembered as raw, the selector's answer.)  After ``recheck`` uses
     a ZFP or raw entry is probed again, so a layer whose sparsity drifts is noticed.
 
     ``only``: when set to a tensor, nothing but that tensor (the same contiguous
@@ -200,7 +201,7 @@ class swap_saved_tensors(torch.autograd.graph.saved_tensors_hooks):
             return False                 # pinned pool, staging pool or tickets exhausted: the tensor stays on the device
         info = self.engine.info(ticket)
         if self.memo is not None and policy in (swap.AUTO, swap.AUTO_SPARSE):
-            self.memo[slot] = (info.policy, 0)
+            self.memo[slot] = (self.engine.decision(ticket), 0)
         self.stats["swapped"] += 1
         self.stats["bytes_in"] += info.bytes_in
         self.stats["bytes_out"] += info.bytes_out

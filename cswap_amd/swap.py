@@ -125,6 +125,13 @@ class SwapEngine:
         check(lib().cswap_swap_timing(self._h, ticket, C.byref(t)), "cswap_swap_timing")
         return t
 
+    def decision(self, ticket: int) -> int:
+        """What to remember of this ticket for the next time: its policy, or NONE where a payload was
+        sent only because the probe had made it."""
+        p = C.c_int(0)
+        check(lib().cswap_swap_decision(self._h, ticket, C.byref(p)), "cswap_swap_decision")
+        return p.value
+
     def info(self, ticket: int) -> TicketInfo:
         i = TicketInfo()
         check(lib().cswap_swap_info(self._h, ticket, C.byref(i)), "cswap_swap_info")

@@ -94,6 +94,7 @@ class Execution {
         continue;
       }
       const size_t n = in.nx * in.ny * in.nz;
+      const int asked = act;
       Memo* memo = nullptr;
       if (act == CSWAP_POLICY_AUTO && recheck > 0) {
         memo = &memo_[in.tensor_id];
@@ -112,14 +113,16 @@ class Execution {
       }
       int ticket = -1;
       int rc = cswap_swap_out(engine_, in.d_tensor, in.nx, in.ny, in.nz, act, compute, &ticket);
+      if (rc == CSWAP_E_NOMEM && act != asked) {  // no room for what is remembered: the selector may find some
+        memo = &memo_[in.tensor_id];
+        rc = cswap_swap_out(engine_, in.d_tensor, in.nx, in.ny, in.nz, asked, compute, &ticket);
+      }
       if (rc) return rc;
-      if (memo) {  // the selector decided: remember what
-        cswap_ticket_info info;
-        if (cswap_swap_info(engine_, ticket, &info) == CSWAP_OK) {
-          memo->n = n;
-          memo->policy = info.policy;
-          memo->uses = 0;
-        }
+      int decision;
+      if (memo && cswap_swap_decision(engine_, ticket, &decision) == CSWAP_OK) {  // the selector decided: remember what
+        memo->n = n;
+        memo->policy = decision;
+        memo->uses = 0;
       }
       tickets_[in.tensor_id] = ticket;
       pending_.push_back(in.tensor_id);

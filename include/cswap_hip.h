@@ -279,7 +279,8 @@ typedef enum { CSWAP_POLICY_AUTO = -1, CSWAP_POLICY_NONE = 2, CSWAP_POLICY_SPARS
                 * expectation was wrong.  Where the compaction was the probe (here, and for
                 * CSWAP_POLICY_AUTO on tensors that the one-kernel form takes) and the selector says
                 * raw, the payload that is there is sent all the same if what is left to pay for it,
-                * link and expansion, is less than min_gain times the raw swap. */
+                * link and expansion, is less than min_gain times the raw swap.  That holds for the
+                * one call: the selector's answer stays raw (cswap_swap_decision). */
                CSWAP_POLICY_AUTO_SPARSE = -3 } cswap_policy;
 
 typedef struct {
@@ -421,6 +422,11 @@ int cswap_swap_prefetch(cswap_engine* e, int ticket);
  * and the ticket number is not handed out again before that. */
 int cswap_swap_release(cswap_engine* e, int ticket);
 int cswap_swap_info(cswap_engine* e, int ticket, cswap_ticket_info* info);
+/* What a caller that remembers the selector's decisions should remember of this ticket: NONE,
+ * SPARSE or ZFP.  The same as `policy` in cswap_swap_info but where a payload was sent only
+ * because the probe had made it: the selector's answer is NONE there, and asked for outright
+ * it costs neither the probe nor the wait for its count. */
+int cswap_swap_decision(cswap_engine* e, int ticket, int* policy);
 /* Phase times of a ticket so far (see cswap_ticket_timing); does not wait for anything.
  * CSWAP_E_UNSUPPORTED on an engine created without config.timing. */
 int cswap_swap_timing(cswap_engine* e, int ticket, cswap_ticket_timing* out);

@@ -65,8 +65,9 @@ __device__ __forceinline__ void st_stream4(float4* p, float4 v)
 }
 
 // The same where the address may be any element's.  The wavefront then writes partial lines at both
-// ends, and the hint pays for large tensors only: expansion of 314 MB 84 us with it, 108 without,
-// 257 MB 61 and 61, 60 MB 19.2 and 16.2.
+// ends, and the hint does not always pay.  Long chunks, from the size of zvc_expand4_staged_kernel on only:
+// expansion of 314 MB 84 us with it, 108 without, 257 MB 61 and 61, 60 MB 19.2 and 16.2.  Short chunks:
+// packed_hint.
 template <bool ALIGNED, bool HINT = false>
 __device__ __forceinline__ void st_row4(float* p, float4 v)
 {
@@ -427,14 +428,20 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand4_kernel(
 // keeps one word together with where its values start and where its elements go, so a word
 // finds its chunk's end and offset by itself and the eight rows of a refill are full.
 // 16384 chunks, one wavefront per chunk -> this: 7 MB 11.3 -> 5.9 us, 25.7 MB 11.1 -> 8.4,
-// 33.6 MB (512 elements per chunk) 11.0 -> 8.7.  Its stores have the hint at any element: several tensors in turn, 16384
-// chunks, without -> with: 19 MB (289 elements per chunk) 8.4 -> 7.8 us, 24 MB 11.4 -> 9.4, 32 MB 13.4 -> 11.3, compaction and
-// expansion 23.6 -> 21.2, 26.6 -> 24.0, 29.9 -> 29.1 (one tensor over and over 23.9 -> 23.4, 24.7 -> 24.4, 25.7 -> 26.5).
+// 33.6 MB (512 elements per chunk) 11.0 -> 8.7.
 // It takes chunks of at most kPackedWords mask words where there are more than kPackedFrom of
 // them: three or more to a wavefront.  Two to a wavefront measure the same as one each, and few
 // chunks are all in flight at once either way.
 constexpr int kPackedWords = 21, kPackedFrom = 2048;
-template <bool ALIGNED>
+// Whether its stores at any element carry the nontemporal hint.  Compaction and expansion of one tensor over and over
+// / of several in turn, us, hint against none.  16384 chunks: 19 MB 23.4 : 24.0 / 22.4 : 24.2 · 24 MB 24.4 : 24.2 / 25.1 : 26.6 ·
+// 29 MB 26.4 : 25.0 / 28.9 : 29.2 · 32 MB 26.4 : 25.4 / 29.6 : 30.0 · 42 MB 36.8 : 34.4 / 39.8 : 40.3; 32768 chunks: 24 MB 24.4 : 24.6 /
+// 25.4 : 27.1 · 30.5 MB 24.5 : 25.1 / 27.8 : 30.0 · 38 MB 35.9 : 34.1 / 38.7 : 38.5; 65536 chunks: 34 MB 35.2 : 33.5 / 37.9 : 36.5 · 87 MB
+// 83.9 : 79.5 / 91.9 : 91.8 · 168 MB 134 : 154 / 150 : 158.  Expansion with a reader right behind it gains from the
+// lines that plain stores leave in the cache: 17 MB 25.7 : 26.3 / 25.1 : 24.0, 42 MB 34.0 : 30.1 / 39.1 : 35.8.
+constexpr size_t kPackedHintBelow = 28u << 20, kPackedHintFrom = 128u << 20;
+static bool packed_hint(size_t bytes) { return bytes < kPackedHintBelow || bytes >= kPackedHintFrom; }
+template <bool ALIGNED, bool HINT>
 __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand_packed_kernel(
     const float* __restrict__ values, const uint32_t* __restrict__ mask, const int* __restrict__ begin,
     Geometry g, int per, float* __restrict__ out)
@@ -491,7 +498,7 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand_packed_kernel(
     if (j >= rows) break;
     float* q = out + to[j];
     if (left[j] >= 4) {
-      st_row4<ALIGNED, true>(q, x[j]);
+      st_row4<ALIGNED, HINT>(q, x[j]);
     } else {
       if (left[j] > 0) q[0] = x[j].x;
       if (left[j] > 1) q[1] = x[j].y;
@@ -1356,6 +1363,8 @@ extern "C" int cswap_zvc_compact(const float* d_in, int n, int process, const in
   return check_launch();
 }
 
+extern "C" int cswap_test_zvc_packed_hint(size_t bytes) { return packed_hint(bytes); }
+
 extern "C" int cswap_zvc_expand(const float* d_values, const uint32_t* d_mask, const int* d_begin, int n,
                                 int process, float* d_out, cswap_stream_t stream)
 {
@@ -1374,12 +1383,11 @@ extern "C" int cswap_zvc_expand(const float* d_values, const uint32_t* d_mask, c
     const int per = 64 / g.W;
     const unsigned waves = (unsigned)((g.active + per - 1) / per);
     const dim3 packed_grid((waves + kWavesPerGroup - 1) / kWavesPerGroup);
-    if (aligned)
-      hipLaunchKernelGGL(zvc_expand_packed_kernel<true>, packed_grid, dim3(64 * kWavesPerGroup), 0, (hipStream_t)stream,
-                         d_values, d_mask, d_begin, g, per, d_out);
-    else
-      hipLaunchKernelGGL(zvc_expand_packed_kernel<false>, packed_grid, dim3(64 * kWavesPerGroup), 0, (hipStream_t)stream,
-                         d_values, d_mask, d_begin, g, per, d_out);
+    const auto kernel = aligned                   ? zvc_expand_packed_kernel<true, true>
+                        : packed_hint(4 * (size_t)n) ? zvc_expand_packed_kernel<false, true>
+                                                     : zvc_expand_packed_kernel<false, false>;
+    hipLaunchKernelGGL(kernel, packed_grid, dim3(64 * kWavesPerGroup), 0, (hipStream_t)stream, d_values, d_mask, d_begin, g,
+                       per, d_out);
   } else if (staged && aligned) CSWAP_EXPAND(zvc_expand4_staged_kernel<true>);
   else if (staged) CSWAP_EXPAND(zvc_expand4_staged_kernel<false>);
   else if (aligned) CSWAP_EXPAND(zvc_expand4_kernel<true>);

@@ -27,6 +27,10 @@ void cswap_zvc_debug_set_lookback(unsigned spin_limit, unsigned skip_first);
  * workgroup comes on top).  Host only. */
 int cswap_test_zvc_stream_groups(int tiles, int compute_units);
 
+/* 1 if the expansion of many short chunks that start on no 16-byte boundary stores a tensor of this many
+ * bytes with the nontemporal hint.  Host only. */
+int cswap_test_zvc_packed_hint(size_t bytes);
+
 /* Which of the encoder's one-lane-per-block kernels a 3-D field of 32-bit elements with contiguous
  * x-rows runs where no other form takes it: 0 the general one, 1 the one for rows at any element,
  * 2 the general one with the nontemporal load hint; or an error code.  sy, sz: strides in elements

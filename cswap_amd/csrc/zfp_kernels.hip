@@ -31,7 +31,7 @@ struct Field3 {
   int stream16;            // 1: the stream pointer is 16-byte aligned
   uint32_t by_piece;       // whole-word rates with an even number of words per block, else 0: the multiplier of block_of_piece
   int read_once;           // 1: a field of kReadOnceBytes and more (see make_field)
-  int store_hint;          // 1: the 32-bit decoder stores the field's rows with the nontemporal hint (see make_field)
+  int store_hint;          // 1: the 32-bit decoder stores the field's rows with the nontemporal hint (row_store_hint)
   int once64;              // 1: the decoder of 64-bit elements should store its rows with the hint (see make_field)
   Div31 by_mx, by_my;      // block index -> block coordinates without a hardware divide
 };
@@ -868,8 +868,8 @@ __global__ __launch_bounds__(128) void zfp_decode3_f32_pair_kernel(const uint64_
 {
   pair_decode<true>(stream, fd, maxbits, out);
 }
-// for rows that are not made of half lines (Field3::store_hint): 12.6 MB in 8x8 planes at 16 bits per value
-// 13.5 us, 17.4 with the hint, 12.8 MB in 28x28 planes 13.5 and 13.9
+// without the hint (Field3::store_hint): 11 MB in 8x8 planes at 16 bits per value, several in turn, 13.7 us, 15.6 with it,
+// in 4x4 planes 14.6 and 31
 __global__ __launch_bounds__(128) void zfp_decode3_f32_pair_plain_kernel(const uint64_t* __restrict__ stream, Field3 fd,
                                                                          unsigned maxbits, float* __restrict__ out)
 {
@@ -1520,6 +1520,39 @@ static int make_field_low(FieldLow& fd, int dims, const void* base, const void* 
 }
 
 // ------------------------------------------------------------- host side
+// Whether the decoder stores a field's aligned rows with the nontemporal hint: base, pitch (row to row) and plane
+// (plane to plane) in bytes.  Where every row starts on a 128-byte line one instruction writes whole lines, and the hint
+// pays at any size: 402.7 MB decode in 107 us instead of 117, and the kernel that runs next no longer waits behind those
+// lines draining from the memory-side cache (33.6 MB: 14.5 instead of 17.6 us, a reader of the result right after it
+// no slower).  A line that several instructions write in parts leaves the cache in those parts, each a write of its own to
+// memory; without the hint it is put together there.  That hurts where the parts are small or many; a field of some 20 MB
+// is through before it does.  Microseconds at 8 bits per value, one tensor over and over / several in turn, hint : none --
+//   half lines: 64 bytes a row 18 MB 12.2 : 13.0 / 11.6 : 14.1 · 36: 15.3 : 16.2 / 16.5 : 17.3 · 43: 17.7 : 16.6 / 18.4 : 17.9 ·
+//     110: 38.4 : 29.7 / 38.3 : 35.8 · 140: 45.5 : 36.0 / 45.0 : 45.7 (268 MB 75.8 : 79.8); 192 bytes 36: 13.7 : 15.9 / 14.5 : 17.1 ·
+//     58: 18.9 : 19.1 / 19.1 : 20.5 · 110: 31.9 : 29.1 / 32.3 : 35.3; 320 bytes 58: 18.3 : 19.0 / 18.4 : 20.5 · 110: 29.9 : 29.1 / 30.2 : 35.2 ·
+//     140: 35.8 : 35.4 / 35.8 : 43.5
+//   smaller parts: 16 bytes 11 MB 12.7 : 12.4 / 23.9 : 12.6; 32 bytes 15: 11.3 : 12.0 / 16.2 : 12.5; 112 bytes 15: 11.9 : 12.0 / 13.2 : 12.7 · 43: 25.6 :
+//     17.0 / 27.0 : 19.8; 160 bytes 25: 13.5 : 13.8 / 14.8 : 15.9 · 30: 15.5 : 14.2 / 16.8 : 16.6; 784 bytes 21: 13.2 : 13.3 / 13.1 : 15.3 · 30: 15.3 : 14.3 /
+//     15.5 : 17.1 · 50: 22.2 : 17.7 / 22.5 : 22.9; 1552 to 6160 bytes 50: 19.7-22.4 : 17.4-18.0 / 20.1-22.5 : 21.3-22.2 · 100: 36-40 : 28-30 /
+//     36-40 : 37-39 · 200, in turn: 68.4 : 65.3.  They take more at 4 bits (24 MB of 160 bytes 12.3 : 12.2 / 13.1 : 14.1) and less at 16 (36: 21.3 :
+//     20.4 / 22.3 : 23.5; 18 MB of 96 bytes 14.9 : 15.7 / 16.3 : 18.5)
+//   rows of whole lines that start 16 bytes into one: 128 bytes 21 MB 12.9 : 13.3 / 14.4 : 15.1 · 50: 26.8 : 17.6 / 27.8 : 19.4 · 140: 73.1 : 36.0 / 73.4 :
+//     46.7; 512 bytes 36: 15.1 : 16.2 / 15.9 : 17.9 · 50: 19.9 : 17.5 / 20.1 : 19.4; 3072 bytes 50: 20.2 : 17.3 / 20.5 : 21.0 · 200: 66 : 47 / 66 : 62
+static bool row_store_hint(unsigned long long base, unsigned long long pitch, unsigned long long plane, unsigned long long bytes,
+                           unsigned maxbits)
+{
+  const unsigned long long starts = base | pitch | plane;
+  const unsigned long long mib = bytes >> 20;
+  if (starts % 128 == 0) return true;
+  if (starts % 64 == 0) return bytes >= kReadOnceBytes || pitch >= 320 || mib < (pitch >= 192 ? 56u : 38u);
+  if (bytes >= kReadOnceBytes) return false;
+  if (pitch >= 1536) return true;
+  if (pitch >= 256 && pitch % 64 == 0) return mib < 36;
+  const unsigned rate = maxbits / 64;  // bits per value
+  if (pitch >= 160) return mib < (rate < 20 ? 16 + rate : 36);
+  return pitch >= 96 && pitch * maxbits >= 128 * 512 && mib < 20;
+}
+
 static int make_field(Field3& fd, const void* base, const void* stream, size_t nx, size_t ny, size_t nz,
                       ptrdiff_t sx, ptrdiff_t sy, ptrdiff_t sz, unsigned maxbits, unsigned elem)
 {
@@ -1553,16 +1586,7 @@ static int make_field(Field3& fd, const void* base, const void* stream, size_t n
   fd.stream16 = ((uintptr_t)stream % 16) == 0;
   fd.by_piece = piece_multiplier(maxbits);
   // Cache policy of the field's 16-byte rows.
-  // The decoder stores them with the nontemporal hint where a row is made of whole 128-byte lines, which
-  // one instruction then writes: 402.7 MB decode in 107 us instead of 117 us, and the kernel that runs next
-  // no longer waits behind those lines draining from the memory-side cache (33.6 MB: decode 14.5
-  // instead of 17.6 us, and a reader of the result right after it is no slower).  A line that several
-  // instructions write in parts leaves the cache in those parts, each a write of its own to memory; without
-  // the hint it is put together there.  Hint / none, decoded at 8 bits per value by bytes per row, warm: 16 (4x4
-  // planes) 33.6 MB 73.8 / 20.4 us, 134 MB 321 / 51 · 32: 33.6 MB 34.3 / 16.1, 134 MB 136 / 36 · 112: 51 MB 32.2 / 19.2, 411 MB
-  // 244 / 131 · 144: 64 MB 35.8 / 21.1 · 224: 206 MB 83 / 50; nothing cached: 272: 200 MB 84.6 / 68.7 · 784: 73.6 / 69.3 · 3088:
-  // 68.4 / 65.3, but 50 MB 21.3 / 21.8.  Rows of whole half lines, hint / none: 64 bytes 67 MB 26.8 / 22.9 cold, 134 MB 44.3 /
-  // 45.7, 268 MB warm 75.8 / 79.8 · 192: 75 MB 24.2 / 24.8, 227 MB 54.8 / 60.9.
+  // The decoder's stores: row_store_hint.
   // The encoder loads with the hint only when the field is large against that cache (256 MB): a smaller
   // tensor is still cached from the kernel that produced it, and hinted loads of cached lines are slower.
   // Producer kernel + encoder, hinted / plain loads: 402.7 MB 205 / 220 us, 201.3 MB
@@ -1571,8 +1595,8 @@ static int make_field(Field3& fd, const void* base, const void* stream, size_t n
   // 37.0 warm, 112: 411 MB 107 / 100; from a line on the hint is ahead again (224: 206 MB 51.8 / 54.8).
   // The stream keeps the default policy: the decoder or the copy engine reads it next.
   fd.read_once = (unsigned long long)nx * ny * nz * elem >= kReadOnceBytes;
-  const unsigned long long pitch = (unsigned long long)fd.sy * elem;
-  fd.store_hint = fd.rows16 && (pitch % 128 == 0 || (fd.read_once ? pitch % 64 == 0 : pitch >= 1536));
+  fd.store_hint = fd.rows16 && row_store_hint((uintptr_t)base, (unsigned long long)fd.sy * elem, (unsigned long long)fd.sz * elem,
+                                             (unsigned long long)nx * ny * nz * elem, maxbits);
   // 64-bit elements: a lane's row is two 16-byte pieces, half a line per store instruction.  The
   // hint on those stores gains 15 % at 537 MB and loses 20 % at 134 MB: only for fields of 256 MiB
   // and more (the memory-side cache's size).
@@ -1714,6 +1738,12 @@ extern "C" int cswap_test_zfp_encode_route(size_t nx, size_t ny, size_t nz, ptrd
   return encode_rows(fd, whole) ? 1 : load_hint(fd, whole) ? 2 : 0;
 }
 
+extern "C" int cswap_test_zfp_store_hint(unsigned long long base, unsigned long long pitch, unsigned long long plane,
+                                         unsigned long long bytes, unsigned maxbits)
+{
+  return row_store_hint(base, pitch, plane, bytes, maxbits);
+}
+
 #define CSWAP_LAUNCH3(KERNEL_, T_, ARG0_, ARG3_)                                                                   \
   do {                                                                                                              \
     if (whole && !is_int)                                                                                           \
@@ -1816,7 +1846,7 @@ static int decompress3(const uint64_t* d_stream, Elem elem, size_t nx, size_t ny
   }
   if (elem == kF32 && pair_shape(fd, maxbits) && (unsigned long long)nx * ny * nz * 4ull < pair_below &&
       pair_decode_pays(grid, maxbits, pair_below)) {
-    const auto kernel = fd.sy % 16 == 0 ? zfp_decode3_f32_pair_kernel : zfp_decode3_f32_pair_plain_kernel;
+    const auto kernel = fd.store_hint ? zfp_decode3_f32_pair_kernel : zfp_decode3_f32_pair_plain_kernel;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(128), (size_t)pair_dec_lds_dwords(maxbits) * 4, st, d_stream, fd, maxbits,
                        static_cast<float*>(d_out));
     return check_launch();

@@ -82,15 +82,24 @@ struct LdsBits {
 
 // The same with the codec's table of expanded bytes (zfp_block.h: expand8) in front of the region: 512
 // bytes per workgroup, a 16-bit read per byte.  Most bytes are zero, so most lanes read one address.
+typedef uint16_t table_u16 __attribute__((may_alias));  // the table's pieces are written 8 bytes at a time
 struct LdsBitsTable : LdsBits {
   static constexpr bool kExpands = true;
-  const uint16_t* table;
-  __device__ __forceinline__ LdsBitsTable(uint32_t* region, const uint16_t* t) : LdsBits(region), table(t) {}
+  const table_u16* table;
+  __device__ __forceinline__ LdsBitsTable(uint32_t* region, const uint2* pieces)
+      : LdsBits(region), table(reinterpret_cast<const table_u16*>(pieces))
+  {
+  }
   __device__ __forceinline__ uint32_t expanded(uint32_t word, int k) const { return table[(word >> (8 * k)) & 0xffu]; }
 };
 __constant__ const ExpandTable kExpandTable = make_expand_table();
 // A lane's 8 bytes of the table: asked for before anything else, written to LDS when the region is cleared.
-__device__ __forceinline__ uint2 table_piece(unsigned lane) { return reinterpret_cast<const uint2*>(kExpandTable.v)[lane]; }
+__device__ __forceinline__ uint2 table_piece(unsigned lane)
+{
+  uint2 piece;
+  __builtin_memcpy(&piece, kExpandTable.v + 4 * lane, sizeof piece);
+  return piece;
+}
 
 // For decoding, with the table of collapsed bytes: 256 bytes.
 struct LdsBitsCollapse : LdsBits {
@@ -103,7 +112,12 @@ struct LdsBitsCollapse : LdsBits {
   __device__ __forceinline__ uint32_t collapsed(uint32_t word, int k) const { return table[(word >> (8 * k)) & 0xffu]; }
 };
 __constant__ const CollapseTable kCollapseTable = make_collapse_table();
-__device__ __forceinline__ uint32_t collapse_piece(unsigned lane) { return reinterpret_cast<const uint32_t*>(kCollapseTable.v)[lane]; }
+__device__ __forceinline__ uint32_t collapse_piece(unsigned lane)
+{
+  uint32_t piece;
+  __builtin_memcpy(&piece, kCollapseTable.v + 4 * lane, sizeof piece);
+  return piece;
+}
 // What stands behind every block in the decoder's region.  A one, for the run that the budget cuts short, and zeros.
 constexpr uint64_t kFence = 1;
 
@@ -525,7 +539,7 @@ __device__ __forceinline__ void encode3_f32(const float* __restrict__ in, const 
   __builtin_amdgcn_s_setprio(0);
 
   if (lane < valid) {
-    LdsBitsTable mem(lds, reinterpret_cast<const uint16_t*>(table));
+    LdsBitsTable mem(lds, table);
     if (INT) {
       int32_t v[64];
 #pragma unroll
@@ -694,7 +708,7 @@ struct LdsExchange {
 
 template <int H>
 __device__ __forceinline__ void pair_encode_body(const float* __restrict__ in, const Field3& fd, unsigned maxbits,
-                                                 uint32_t* lds, const uint16_t* table, unsigned lane, uint32_t first)
+                                                 uint32_t* lds, const uint2* table, unsigned lane, uint32_t first)
 {
   const bool live = first + lane < fd.nblocks;
   const uint32_t b = live ? first + lane : fd.nblocks - 1;
@@ -734,9 +748,8 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(7, 8))) voi
   uint32_t* lds = reinterpret_cast<uint32_t*>(lds_raw);
   const unsigned tid = threadIdx.x, lane = tid & 63u;
   const uint32_t first = blockIdx.x * 64u;
-  __shared__ uint2 pieces[64];
-  if (tid < 64) pieces[tid] = table_piece(tid);
-  const uint16_t* table = reinterpret_cast<const uint16_t*>(pieces);
+  __shared__ uint2 table[64];
+  if (tid < 64) table[tid] = table_piece(tid);
   {  // the region starts out zero; the first exchange's barrier orders this before any coder's OR
     const unsigned n16 = region_dwords(maxbits) / 4;
     for (unsigned i = tid; i < n16; i += 128) lds_raw[i] = make_uint4(0, 0, 0, 0);
@@ -1057,7 +1070,7 @@ __global__ __launch_bounds__(64) void zfp_encode3_f32_quad_kernel(const float* _
   }
   __syncthreads();
 
-  LdsBitsTable mem(lds, reinterpret_cast<const uint16_t*>(table));
+  LdsBitsTable mem(lds, table);
   TableEncoder<LdsBitsTable> enc(mem, mem.bit0 + bl * slot, maxbits);
   unsigned base = e ? enc.pos + 9 : enc.limit;  // an all-zero block or one past the end: nothing is written
   if (e && q == 0) enc.put(2 * e + 1, 9);
@@ -1301,7 +1314,7 @@ __global__ __launch_bounds__(64) void zfp_encode3_w64_kernel(const uint64_t* __r
   if (WHOLE) table[lane] = piece;
   __syncthreads();
   if (lane < valid) {
-    LdsBitsTable mem(lds, reinterpret_cast<const uint16_t*>(table));
+    LdsBitsTable mem(lds, table);
     encode_block_w64<!WHOLE, INT>(q, mem.bit0 + lane * slot_bits(maxbits), maxbits, mem);
   }
   __syncthreads();

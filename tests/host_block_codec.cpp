@@ -22,6 +22,23 @@ struct WatchedBits {          // the same for reading, remembering the highest d
     return dw[d / 4];
   }
 };
+// The same regions with the coder's tables, as the kernels for whole-word rates have them.  Without them the codec
+// steps from run to run: the second opinion.
+constexpr cswap::ExpandTable kExpand = cswap::make_expand_table();
+constexpr cswap::CollapseTable kCollapse = cswap::make_collapse_table();
+template <class Bits>
+struct WithTables : Bits {
+  static constexpr bool kExpands = true, kCollapses = true;
+  uint32_t expanded(uint32_t word, int k) const { return kExpand.v[(word >> (8 * k)) & 0xffu]; }
+  uint32_t collapsed(uint32_t word, int k) const { return kCollapse.v[(word >> (8 * k)) & 0xffu]; }
+};
+template <class Bits>
+struct Plain : Bits {};
+template <class Mem>
+constexpr uint64_t fence_of()  // what stands behind a block for the fenced decoder
+{
+  return cswap::collapses<Mem>::value ? 1u : ~(uint64_t)0;
+}
 }
 
 extern "C" {
@@ -47,7 +64,9 @@ void host_zfp_encode3(const float* in, size_t nx, size_t ny, size_t nz, unsigned
 // zeroed slot of maxbits + 128 bits, as the device does for whole-word rates, and
 // only its first maxbits bits are kept.  Returns the highest dword index (relative
 // to the slot) that any block wrote a non-zero value to.
-unsigned host_zfp_encode3_slots(const float* in, size_t nx, size_t ny, size_t nz, unsigned maxbits, uint64_t* stream)
+}  // extern "C"
+template <class Mem>
+static unsigned encode3_slots(const float* in, size_t nx, size_t ny, size_t nz, unsigned maxbits, uint64_t* stream)
 {
   size_t mx = (nx + 3) / 4, my = (ny + 3) / 4, mz = (nz + 3) / 4;
   const unsigned W = maxbits / 64;  // maxbits % 64 == 0
@@ -63,13 +82,20 @@ unsigned host_zfp_encode3_slots(const float* in, size_t nx, size_t ny, size_t nz
       f[x + 4 * y + 16 * z] = in[(x0 + x) + nx * ((y0 + y) + ny * (z0 + z))];
     if (bx < 4 || by < 4 || bz < 4) cswap::pad_block3(f, bx, by, bz);
     memset(slot, 0, 4 * (size_t)slot_dwords);
-    ArrayBits mem{slot};
+    Mem mem{{slot}};
     cswap::encode_block<false>(f, 0u, maxbits, mem);
     memcpy(stream + b * W, slot, 8 * (size_t)W);
     for (unsigned d = 0; d < slot_dwords; d++) if (slot[d] && d > top) top = d;
   }
   delete[] slot;
   return top;
+}
+
+extern "C" {
+unsigned host_zfp_encode3_slots(const float* in, size_t nx, size_t ny, size_t nz, unsigned maxbits, uint64_t* stream, int table)
+{
+  return table ? encode3_slots<WithTables<ArrayBits>>(in, nx, ny, nz, maxbits, stream)
+               : encode3_slots<Plain<ArrayBits>>(in, nx, ny, nz, maxbits, stream);
 }
 
 void host_zfp_decode3(const uint64_t* stream, size_t nx, size_t ny, size_t nz, unsigned maxbits, float* out)
@@ -87,11 +113,13 @@ void host_zfp_decode3(const uint64_t* stream, size_t nx, size_t ny, size_t nz, u
 }
 
 // Same decode through the fenced variant: every block is copied into a private
-// slot that is followed by 64 one bits, as the device does for whole-word rates,
-// and then by whatever the next lane's slot happens to hold (here: `junk`,
+// slot that is followed by its fence (64 one bits for the steps from run to run, a one and
+// zeros with the tables), as the device does for whole-word rates, and then by whatever the next lane's slot happens to hold (here: `junk`,
 // different for every block).  Returns the highest dword index, relative to the
 // slot, that any block read.
-unsigned host_zfp_decode3_fenced(const uint64_t* stream, size_t nx, size_t ny, size_t nz, unsigned maxbits, float* out,
+}  // extern "C"
+template <class Mem>
+static unsigned decode3_fenced(const uint64_t* stream, size_t nx, size_t ny, size_t nz, unsigned maxbits, float* out,
                                  uint32_t junk)
 {
   size_t mx = (nx + 3) / 4, my = (ny + 3) / 4, mz = (nz + 3) / 4;
@@ -102,16 +130,25 @@ unsigned host_zfp_decode3_fenced(const uint64_t* stream, size_t nx, size_t ny, s
     size_t x0 = (b % mx) * 4, y0 = ((b / mx) % my) * 4, z0 = (b / (mx * my)) * 4;
     unsigned bx = nx - x0 < 4 ? nx - x0 : 4, by = ny - y0 < 4 ? ny - y0 : 4, bz = nz - z0 < 4 ? nz - z0 : 4;
     memcpy(slot, stream + b * W, 8 * (size_t)W);
-    slot[2 * W] = slot[2 * W + 1] = 0xffffffffu;
+    const uint64_t fence = fence_of<Mem>();
+    memcpy(slot + 2 * W, &fence, 8);
     for (unsigned d = 2 * W + 2; d < 2 * W + 16; d++) slot[d] = junk = junk * 1664525u + 1013904223u + (uint32_t)b;
     float f[64];
-    WatchedBits mem{slot, &top};
+    Mem mem{{slot, &top}};
     cswap::decode_block<true>(mem, 0u, maxbits, f);
     for (unsigned z = 0; z < bz; z++) for (unsigned y = 0; y < by; y++) for (unsigned x = 0; x < bx; x++)
       out[(x0 + x) + nx * ((y0 + y) + ny * (z0 + z))] = f[x + 4 * y + 16 * z];
   }
   delete[] slot;
   return top;
+}
+
+extern "C" {
+unsigned host_zfp_decode3_fenced(const uint64_t* stream, size_t nx, size_t ny, size_t nz, unsigned maxbits, float* out,
+                                 uint32_t junk, int table)
+{
+  return table ? decode3_fenced<WithTables<WatchedBits>>(stream, nx, ny, nz, maxbits, out, junk)
+               : decode3_fenced<Plain<WatchedBits>>(stream, nx, ny, nz, maxbits, out, junk);
 }
 
 // 2-D field a[ny][nx] (ny = 0: 1-D field a[nx])
@@ -335,7 +372,7 @@ struct HostExchange {
 struct PairJob {
   const float* in; size_t nx, ny, nz; unsigned maxbits; uint32_t* slots; unsigned slot_dwords; PairShared* sh;
 };
-template <int H>
+template <int H, class Mem>
 void* pair_thread(void* arg)
 {
   PairJob& j = *static_cast<PairJob*>(arg);
@@ -349,7 +386,7 @@ void* pair_thread(void* arg)
       p[x + 4 * y] = j.in[(x0 + x) + j.nx * ((y0 + y) + j.ny * (z0 + zp))];
       q[x + 4 * y] = j.in[(x0 + x) + j.nx * ((y0 + y) + j.ny * (z0 + zq))];
     }
-    AtomicBits mem{j.slots + b * j.slot_dwords};
+    Mem mem{{j.slots + b * j.slot_dwords}};
     cswap::pair_encode_half<H>(p, q, true, 0u, j.maxbits, mem, ex);
   }
   return nullptr;
@@ -359,7 +396,7 @@ void* pair_thread(void* arg)
 extern "C" {
 // nx, ny, nz multiples of 4; maxbits a multiple of 64.  Returns the highest dword index
 // (relative to its slot) that any block wrote a non-zero value to, or ~0u on a setup error.
-unsigned host_zfp_encode3_pair(const float* in, size_t nx, size_t ny, size_t nz, unsigned maxbits, uint64_t* stream)
+unsigned host_zfp_encode3_pair(const float* in, size_t nx, size_t ny, size_t nz, unsigned maxbits, uint64_t* stream, int table)
 {
   if (nx % 4 || ny % 4 || nz % 4 || maxbits % 64) return ~0u;
   const size_t nb = (nx / 4) * (ny / 4) * (nz / 4);
@@ -370,8 +407,8 @@ unsigned host_zfp_encode3_pair(const float* in, size_t nx, size_t ny, size_t nz,
   if (pthread_barrier_init(&sh.bar, nullptr, 2)) return ~0u;
   PairJob job{in, nx, ny, nz, maxbits, slots.data(), slot_dwords, &sh};
   pthread_t t0, t1;
-  pthread_create(&t0, nullptr, pair_thread<0>, &job);
-  pthread_create(&t1, nullptr, pair_thread<1>, &job);
+  pthread_create(&t0, nullptr, table ? pair_thread<0, WithTables<AtomicBits>> : pair_thread<0, Plain<AtomicBits>>, &job);
+  pthread_create(&t1, nullptr, table ? pair_thread<1, WithTables<AtomicBits>> : pair_thread<1, Plain<AtomicBits>>, &job);
   pthread_join(t0, nullptr);
   pthread_join(t1, nullptr);
   pthread_barrier_destroy(&sh.bar);
@@ -383,15 +420,17 @@ unsigned host_zfp_encode3_pair(const float* in, size_t nx, size_t ny, size_t nz,
   return top;
 }
 
-// BlockEncoder::skip_plane against BlockEncoder::plane on one plane: starting from n known
+// BlockEncoder::skip_plane against BlockEncoder::plane or, with the table, TableEncoder::plane on one plane: starting from n known
 // coefficients (acc = their mask) at bit position pos of a zeroed region, returns 1 if both
 // leave the same n and pos.
-int host_skip_plane_agrees(uint64_t x, unsigned n, unsigned pos, unsigned maxbits)
+}
+template <class Mem>
+static int skip_plane_agrees(uint64_t x, unsigned n, unsigned pos, unsigned maxbits)
 {
   uint32_t region[64];
   memset(region, 0, sizeof region);
-  ArrayBits mem{region};
-  cswap::BlockEncoder<ArrayBits, false> a(mem, 0u, maxbits), b(mem, 0u, maxbits);
+  Mem mem{{region}};
+  cswap::Encoder<Mem, false> a(mem, 0u, maxbits), b(mem, 0u, maxbits);
   a.pos = b.pos = pos;
   a.n = b.n = n;
   uint64_t acc = n >= 64 ? ~0ull : (n ? ((~0ull) >> (64 - n)) : 0ull);  // any mask whose highest one-bit is n - 1 does
@@ -400,6 +439,9 @@ int host_skip_plane_agrees(uint64_t x, unsigned n, unsigned pos, unsigned maxbit
   b.skip_plane(x, acc);
   return a.n == b.n && a.pos == b.pos;
 }
+extern "C" int host_skip_plane_agrees(uint64_t x, unsigned n, unsigned pos, unsigned maxbits, int table)
+{
+  return table ? skip_plane_agrees<WithTables<ArrayBits>>(x, n, pos, maxbits) : skip_plane_agrees<Plain<ArrayBits>>(x, n, pos, maxbits);
 }
 
 // ---- the decoder's pair form, the same way: two threads, the kernel's reuse of its shared words
@@ -434,7 +476,7 @@ struct HostDecExchange {
 struct PairDecJob {
   const uint32_t* slots; unsigned slot_dwords; size_t nx, ny, nz; unsigned maxbits; float* out; PairDecShared* sh;
 };
-template <int H>
+template <int H, class Mem>
 void* pair_dec_thread(void* arg)
 {
   PairDecJob& j = *static_cast<PairDecJob*>(arg);
@@ -443,7 +485,7 @@ void* pair_dec_thread(void* arg)
   for (size_t b = 0; b < mx * my * mz; b++) {
     const size_t x0 = (b % mx) * 4, y0 = ((b / mx) % my) * 4, z0 = (b / (mx * my)) * 4;
     const int zp = H == 0 ? 0 : 2, zq = H == 0 ? 3 : 1;
-    ArrayBits mem{const_cast<uint32_t*>(j.slots + b * j.slot_dwords)};
+    Mem mem{{const_cast<uint32_t*>(j.slots + b * j.slot_dwords)}};
     float p[16], q[16];
     cswap::pair_decode_half<H>(mem, 0u, j.maxbits, ex, p, q);
     for (int y = 0; y < 4; y++) for (int x = 0; x < 4; x++) {
@@ -456,17 +498,18 @@ void* pair_dec_thread(void* arg)
 }
 }
 
-extern "C" int host_zfp_decode3_pair(const uint64_t* stream, size_t nx, size_t ny, size_t nz, unsigned maxbits, float* out)
+extern "C" int host_zfp_decode3_pair(const uint64_t* stream, size_t nx, size_t ny, size_t nz, unsigned maxbits, float* out, int table)
 {
   if (nx % 4 || ny % 4 || nz % 4 || maxbits % 64) return -1;
   const size_t nb = (nx / 4) * (ny / 4) * (nz / 4);
   const unsigned W = maxbits / 64, slot_dwords = 2 * W + 16;
   std::vector<uint32_t> slots(nb * slot_dwords);
   uint32_t junk = 12345u;
-  for (size_t b = 0; b < nb; b++) {  // the block, its fence of 64 ones, then whatever
+  const uint64_t fence = table ? fence_of<WithTables<ArrayBits>>() : fence_of<Plain<ArrayBits>>();
+  for (size_t b = 0; b < nb; b++) {  // the block, its fence, then whatever
     uint32_t* s = slots.data() + b * slot_dwords;
     memcpy(s, stream + b * W, 8 * (size_t)W);
-    s[2 * W] = s[2 * W + 1] = 0xffffffffu;
+    memcpy(s + 2 * W, &fence, 8);
     for (unsigned d = 2 * W + 2; d < slot_dwords; d++) s[d] = junk = junk * 1664525u + 1013904223u;
   }
   PairDecShared sh;
@@ -474,10 +517,52 @@ extern "C" int host_zfp_decode3_pair(const uint64_t* stream, size_t nx, size_t n
   if (pthread_barrier_init(&sh.bar, nullptr, 2)) return -1;
   PairDecJob job{slots.data(), slot_dwords, nx, ny, nz, maxbits, out, &sh};
   pthread_t t0, t1;
-  pthread_create(&t0, nullptr, pair_dec_thread<0>, &job);
-  pthread_create(&t1, nullptr, pair_dec_thread<1>, &job);
+  pthread_create(&t0, nullptr, table ? pair_dec_thread<0, WithTables<ArrayBits>> : pair_dec_thread<0, Plain<ArrayBits>>, &job);
+  pthread_create(&t1, nullptr, table ? pair_dec_thread<1, WithTables<ArrayBits>> : pair_dec_thread<1, Plain<ArrayBits>>, &job);
   pthread_join(t0, nullptr);
   pthread_join(t1, nullptr);
   pthread_barrier_destroy(&sh.bar);
   return 0;
+}
+
+// Blocks of 64 values of 32-bit integers (kind 0), doubles (1) or 64-bit integers (2) one after the other, with the
+// tables: each coded without the guard into a zeroed slot and decoded from a fenced one, its neighbours' bits behind it.
+// Returns the highest dword, relative to its slot, that a block wrote a one-bit to or read.
+template <class Mem>
+static void code_one(const uint64_t* in, int kind, unsigned maxbits, Mem& mem)
+{
+  uint64_t q[64];
+  int32_t v[64];
+  memcpy(q, in, sizeof q);
+  for (int i = 0; i < 64; i++) v[i] = (int32_t)q[i];
+  if (kind == 0) cswap::encode_block_i32<false>(v, 0u, maxbits, mem);
+  else if (kind == 1) cswap::encode_block_w64<false, false>(q, 0u, maxbits, mem);
+  else cswap::encode_block_w64<false, true>(q, 0u, maxbits, mem);
+}
+extern "C" unsigned host_zfp_blocks_table(const uint64_t* in, int kind, size_t nb, unsigned maxbits, uint64_t* stream, uint64_t* out)
+{
+  const unsigned W = maxbits / 64;
+  unsigned top = 0;
+  for (size_t b = 0; b < nb; b++) {
+    std::vector<uint32_t> slot(2 * W + 16, 0u);
+    WithTables<ArrayBits> w{{slot.data()}};
+    code_one(in + 64 * b, kind, maxbits, w);
+    for (unsigned d = 0; d < slot.size(); d++) if (slot[d] && d > top) top = d;
+    memcpy(stream + b * W, slot.data(), 8 * (size_t)W);
+  }
+  for (size_t b = 0; b < nb; b++) {
+    std::vector<uint32_t> slot(2 * W + 16, 0xa5a5a5a5u);
+    memcpy(slot.data(), stream + b * W, 8 * (size_t)W);
+    const uint64_t fence = fence_of<WithTables<ArrayBits>>();
+    memcpy(slot.data() + 2 * W, &fence, 8);
+    WithTables<WatchedBits> m{{slot.data(), &top}};
+    int32_t v[64];
+    uint64_t* o = out + 64 * b;
+    if (kind == 0) cswap::decode_block_i32<true>(m, 0u, maxbits, v);
+    else if (kind == 1) cswap::decode_block_w64<false, true>(m, 0u, maxbits, *reinterpret_cast<uint64_t(*)[64]>(o));
+    else cswap::decode_block_w64<true, true>(m, 0u, maxbits, *reinterpret_cast<uint64_t(*)[64]>(o));
+    if (kind == 0)
+      for (int i = 0; i < 64; i++) o[i] = (uint64_t)(uint32_t)v[i];
+  }
+  return top;
 }

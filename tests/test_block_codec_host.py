@@ -23,9 +23,9 @@ def host():
     L.host_zfp_encode3.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t, C.c_size_t, C.c_uint, C.c_void_p]
     L.host_zfp_decode3.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t, C.c_size_t, C.c_uint, C.c_void_p]
     L.host_zfp_decode3_fenced.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t, C.c_size_t, C.c_uint, C.c_void_p,
-                                          C.c_uint32]
+                                          C.c_uint32, C.c_int]
     L.host_zfp_decode3_fenced.restype = C.c_uint
-    L.host_zfp_encode3_slots.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t, C.c_size_t, C.c_uint, C.c_void_p]
+    L.host_zfp_encode3_slots.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t, C.c_size_t, C.c_uint, C.c_void_p, C.c_int]
     L.host_zfp_encode3_slots.restype = C.c_uint
     L.host_transpose32.argtypes = [C.c_void_p]
     L.host_zfp_encode_low.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t, C.c_uint, C.c_void_p]
@@ -85,21 +85,21 @@ def test_block_codec_matches_golden_vectors(host, golden):
         k = min(sb.size, stream.size)
         assert np.array_equal(sb[:k], stream[:k]), (name, rate)
         assert not sb[k:].any() and not stream[k:].any()
-        if maxbits % 64 == 0:  # the encoder variant the device uses for whole-word rates
+        for table in (0, 1) if maxbits % 64 == 0 else ():  # the encoder variant for whole-word rates; the device has the table
             s2 = np.zeros(words, dtype=np.uint64)
-            top = host.host_zfp_encode3_slots(f.ctypes.data, nx, ny, nz, maxbits, s2.ctypes.data)
-            assert np.array_equal(s2.view(np.uint8)[:k], stream[:k]), (name, rate, "slots")
+            top = host.host_zfp_encode3_slots(f.ctypes.data, nx, ny, nz, maxbits, s2.ctypes.data, table)
+            assert np.array_equal(s2.view(np.uint8)[:k], stream[:k]), (name, rate, "slots", table)
             assert top < maxbits // 32 + 4, (name, rate, "wrote past the 128 bits of slack")
         g = np.zeros((words + 2) * 8, dtype=np.uint8)
         g[:k] = stream[:k]
         o = np.zeros_like(f)
         host.host_zfp_decode3(g.ctypes.data, nx, ny, nz, maxbits, o.ctypes.data)
         assert np.array_equal(o.view(np.uint32), dec.view(np.uint32)), (name, rate)
-        if maxbits % 64 == 0:  # the variant the device uses for whole-word rates
+        for table in (0, 1) if maxbits % 64 == 0 else ():  # the decoder variant for whole-word rates
             o2 = np.zeros_like(f)
-            top = host.host_zfp_decode3_fenced(g.ctypes.data, nx, ny, nz, maxbits, o2.ctypes.data, n)
-            assert np.array_equal(o2.view(np.uint32), dec.view(np.uint32)), (name, rate, "fenced")
-            assert top < maxbits // 32 + 4, (name, rate, top)
+            top = host.host_zfp_decode3_fenced(g.ctypes.data, nx, ny, nz, maxbits, o2.ctypes.data, n, table)
+            assert np.array_equal(o2.view(np.uint32), dec.view(np.uint32)), (name, rate, "fenced", table)
+            assert top < maxbits // 32 + (6 if table else 4), (name, rate, top)
         n += 1
     assert n >= 100
 
@@ -210,12 +210,13 @@ def test_64_bit_block_codec_agrees_with_checker_on_tiny_and_huge_doubles(host):
             assert np.array_equal(o.view(np.uint64), d.view(np.uint64)), (scale, maxbits)
 
 
-def test_unguarded_encoder_stays_inside_its_slack(host):
+@pytest.mark.parametrize("table", [0, 1], ids=["steps", "table"])
+def test_unguarded_encoder_stays_inside_its_slack(host, table):
     """The encoder variant without end-of-block guards lets a block that runs out
     of budget finish its bit plane.  On noise, where a plane that starts with few
     significant coefficients finds many at once, what it writes past the block's
     end must stay within the 128 bits of slack, and the kept bits must equal the
-    guarded encoder's."""
+    guarded encoder's.  Steps from run to run, and the table that the kernels use."""
     rng = np.random.default_rng(11)
     for maxbits in (64, 128, 192, 256, 512):
         for scale in (1.0, 1e-3, 1e4):
@@ -226,17 +227,20 @@ def test_unguarded_encoder_stays_inside_its_slack(host):
             a = np.zeros(words + 2, dtype=np.uint64)
             host.host_zfp_encode3(f.ctypes.data, nx, ny, nz, maxbits, a.ctypes.data)
             b = np.zeros(words, dtype=np.uint64)
-            top = host.host_zfp_encode3_slots(f.ctypes.data, nx, ny, nz, maxbits, b.ctypes.data)
+            top = host.host_zfp_encode3_slots(f.ctypes.data, nx, ny, nz, maxbits, b.ctypes.data, table)
             assert np.array_equal(a[:words], b), (maxbits, scale)
             assert top < maxbits // 32 + 4, (maxbits, scale, top)
 
 
-def test_fenced_decoder_ignores_what_lies_behind_its_fence(host):
-    """The device gives every lane a slot of the block's bits and 64 one bits; what
-    the decoder reads beyond those (the window it looks through is wider than what
-    it uses) belongs to the next lane.  On noise and on fields with outliers, at
-    every whole-word rate: the result does not depend on those bits, and no read
-    goes further than 128 bits past the block."""
+@pytest.mark.parametrize("table", [0, 1], ids=["steps", "table"])
+def test_fenced_decoder_ignores_what_lies_behind_its_fence(host, table):
+    """The device gives every lane a slot of the block's bits and a fence of 64 bits (a one
+    and zeros; the decoder that steps from run to run, its second opinion here, takes 64
+    ones); what the decoder reads beyond those (the window it looks through is wider than
+    what it uses) belongs to the next lane.  On noise and on fields with outliers, at
+    every whole-word rate: the result does not depend on those bits, and no read goes
+    further than the region has room for behind its last block: the 64 bits of fence and
+    128 of padding (dec_region_dwords), of which the steps use 64."""
     rng = np.random.default_rng(12)
     for maxbits in (64, 128, 192, 256, 512, 1024, 2048):
         for scale in (1.0, 1e-3, 1e4):
@@ -251,25 +255,26 @@ def test_fenced_decoder_ignores_what_lies_behind_its_fence(host):
             host.host_zfp_decode3(a.ctypes.data, nx, ny, nz, maxbits, plain.ctypes.data)
             for junk in (0, 1, 0xffffffff, 12345):
                 o = np.zeros_like(f)
-                top = host.host_zfp_decode3_fenced(a.ctypes.data, nx, ny, nz, maxbits, o.ctypes.data, junk)
+                top = host.host_zfp_decode3_fenced(a.ctypes.data, nx, ny, nz, maxbits, o.ctypes.data, junk, table)
                 assert np.array_equal(o.view(np.uint32), plain.view(np.uint32)), (maxbits, scale, junk)
-                assert top < maxbits // 32 + 4, (maxbits, scale, top)
+                assert top < maxbits // 32 + (6 if table else 4), (maxbits, scale, top)
 
 
 # ---- the encoder's pair form: a block shared by two wavefronts (here: two host threads)
 def _pair(host):
-    host.host_zfp_encode3_pair.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t, C.c_size_t, C.c_uint, C.c_void_p]
+    host.host_zfp_encode3_pair.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t, C.c_size_t, C.c_uint, C.c_void_p, C.c_int]
     host.host_zfp_encode3_pair.restype = C.c_uint
-    host.host_skip_plane_agrees.argtypes = [C.c_uint64, C.c_uint, C.c_uint, C.c_uint]
+    host.host_skip_plane_agrees.argtypes = [C.c_uint64, C.c_uint, C.c_uint, C.c_uint, C.c_int]
     host.host_skip_plane_agrees.restype = C.c_int
-    host.host_zfp_decode3_pair.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t, C.c_size_t, C.c_uint, C.c_void_p]
+    host.host_zfp_decode3_pair.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t, C.c_size_t, C.c_uint, C.c_void_p, C.c_int]
     host.host_zfp_decode3_pair.restype = C.c_int
     return host
 
 
 @pytest.mark.timeout(300)
-def test_skipping_a_plane_in_closed_form_leaves_the_coder_where_coding_it_does(host):
-    """BlockEncoder::skip_plane against BlockEncoder::plane (the coder of
+@pytest.mark.parametrize("table", [0, 1], ids=["steps", "table"])
+def test_skipping_a_plane_in_closed_form_leaves_the_coder_where_coding_it_does(host, table):
+    """BlockEncoder::skip_plane against BlockEncoder::plane and TableEncoder::plane (the coder of
     encode.cuh:331-344) on single planes: every count of known coefficients, planes
     that are empty, full, sparse, dense, that end in the last coefficient."""
     L = _pair(host)
@@ -285,13 +290,14 @@ def test_skipping_a_plane_in_closed_form_leaves_the_coder_where_coding_it_does(h
     for x in planes:
         for n in list(range(0, 65, 3)) + [1, 2, 62, 63, 64]:
             for pos in (9, 200, 511):
-                if not L.host_skip_plane_agrees(x, n, pos, 2048):
+                if not L.host_skip_plane_agrees(x, n, pos, 2048, table):
                     bad.append((hex(x), n, pos))
     assert not bad, bad[:10]
 
 
 @pytest.mark.timeout(600)
-def test_pair_form_of_the_encoder_matches_golden_vectors_and_the_block_encoder(host, golden):
+@pytest.mark.parametrize("table", [0, 1], ids=["steps", "table"])
+def test_pair_form_of_the_encoder_matches_golden_vectors_and_the_block_encoder(host, golden, table):
     """The pair form (two halves of a workgroup per block; here two threads with the
     kernel's reuse of its shared words) gives the streams of the golden vectors and of
     encode_block on random fields, at every whole-word rate incl. the ones that code the
@@ -304,7 +310,7 @@ def test_pair_form_of_the_encoder_matches_golden_vectors_and_the_block_encoder(h
             continue
         words = (nx // 4) * (ny // 4) * (nz // 4) * maxbits // 64
         s = np.zeros(words, dtype=np.uint64)
-        top = L.host_zfp_encode3_pair(f.ctypes.data, nx, ny, nz, maxbits, s.ctypes.data)
+        top = L.host_zfp_encode3_pair(f.ctypes.data, nx, ny, nz, maxbits, s.ctypes.data, table)
         assert top != 0xFFFFFFFF
         assert np.array_equal(s.view(np.uint8), stream[:words * 8]), (name, rate)
         assert top < maxbits // 32 + 4, (name, rate, "wrote past the 128 bits of slack")
@@ -329,13 +335,14 @@ def test_pair_form_of_the_encoder_matches_golden_vectors_and_the_block_encoder(h
                 want = np.zeros(words + 2, dtype=np.uint64)
                 host.host_zfp_encode3(f.ctypes.data, nx, ny, nz, maxbits, want.ctypes.data)
                 s = np.zeros(words, dtype=np.uint64)
-                top = L.host_zfp_encode3_pair(f.ctypes.data, nx, ny, nz, maxbits, s.ctypes.data)
+                top = L.host_zfp_encode3_pair(f.ctypes.data, nx, ny, nz, maxbits, s.ctypes.data, table)
                 assert np.array_equal(s, want[:words]), (kind, shape, maxbits)
                 assert top < maxbits // 32 + 4, (kind, shape, maxbits, top)
 
 
 @pytest.mark.timeout(600)
-def test_pair_form_of_the_decoder_matches_golden_vectors_and_the_block_decoder(host, golden):
+@pytest.mark.parametrize("table", [0, 1], ids=["steps", "table"])
+def test_pair_form_of_the_decoder_matches_golden_vectors_and_the_block_decoder(host, golden, table):
     """The decoder's pair form (half 0 decodes the bit planes, both halves share what follows; here
     two threads with the kernel's reuse of its shared words) gives the decoded values of the golden
     vectors and of decode_block on the streams of random fields, at every whole-word rate."""
@@ -349,7 +356,7 @@ def test_pair_form_of_the_decoder_matches_golden_vectors_and_the_block_decoder(h
         g = np.zeros(words * 8, dtype=np.uint8)
         g[:] = stream[:words * 8]
         o = np.full(f.shape, -7.0, dtype=np.float32)
-        assert L.host_zfp_decode3_pair(g.ctypes.data, nx, ny, nz, maxbits, o.ctypes.data) == 0
+        assert L.host_zfp_decode3_pair(g.ctypes.data, nx, ny, nz, maxbits, o.ctypes.data, table) == 0
         assert np.array_equal(o.view(np.uint32), dec.view(np.uint32)), (name, rate)
         n += 1
     assert n >= 20, n
@@ -373,5 +380,32 @@ def test_pair_form_of_the_decoder_matches_golden_vectors_and_the_block_decoder(h
                 want = np.zeros_like(f)
                 host.host_zfp_decode3(s.ctypes.data, nx, ny, nz, maxbits, want.ctypes.data)
                 o = np.full(f.shape, -7.0, dtype=np.float32)
-                assert L.host_zfp_decode3_pair(s.ctypes.data, nx, ny, nz, maxbits, o.ctypes.data) == 0
+                assert L.host_zfp_decode3_pair(s.ctypes.data, nx, ny, nz, maxbits, o.ctypes.data, table) == 0
                 assert np.array_equal(o.view(np.uint32), want.view(np.uint32)), (kind, shape, maxbits)
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2], ids=["int32", "double", "int64"])
+def test_other_scalar_types_through_the_tables(host, kind):
+    """The blocks of the kernels for int32, double and int64 at whole-word rates, coded and decoded with the tables,
+    against the checker; no one-bit is written further than 128 bits past a block and none read further than 192."""
+    import oracle
+
+    host.host_zfp_blocks_table.argtypes = [C.c_void_p, C.c_int, C.c_size_t, C.c_uint, C.c_void_p, C.c_void_p]
+    host.host_zfp_blocks_table.restype = C.c_uint
+    rng = np.random.default_rng(kind)
+    nb = 48
+    blocks = rng.standard_normal((nb, 4, 4, 4)) * np.exp2(rng.integers(-12, 24, (nb, 1, 1, 1)))
+    blocks[rng.random(blocks.shape) < 0.1] *= 50.0
+    blocks[-1] = 0.0
+    f = blocks.astype((np.int32, np.float64, np.int64)[kind])
+    q = np.ascontiguousarray(f.astype(np.int64) if kind == 0 else f).view(np.uint64)
+    field = np.ascontiguousarray(f.reshape(nb * 4, 4, 4))
+    for maxbits in (64, 128, 192, 512, 1024, 2048, 4096):
+        s, out = np.zeros(nb * maxbits // 64, dtype=np.uint64), np.zeros((nb, 64), dtype=np.uint64)
+        top = host.host_zfp_blocks_table(q.ctypes.data, kind, nb, maxbits, s.ctypes.data, out.ctypes.data)
+        want = oracle.zfp_encode_i32(field, maxbits) if kind == 0 else oracle.zfp_encode_64(field, maxbits)
+        assert np.array_equal(s, want[: s.size]), maxbits
+        back = oracle.zfp_decode_i32(want, field.shape, maxbits) if kind == 0 else oracle.zfp_decode_64(want, field.shape, maxbits, field.dtype)
+        got = out.astype(np.uint32) if kind == 0 else out
+        assert np.array_equal(got.ravel(), back.view(got.dtype).ravel()), maxbits
+        assert top < maxbits // 32 + 6, (maxbits, top)

@@ -557,7 +557,9 @@ CSWAP_HD uint32_t collapse32(const Mem& mem, uint32_t v, uint32_t u)
 // The block owns [pos0, pos0 + maxbits).  GUARD = true cuts every write at the
 // end of the block (needed when the next block's bits follow immediately);
 // GUARD = false lets the last plane spill up to 128 bits past the end, which the
-// caller must provide as slack and ignore.
+// caller must provide as slack and ignore.  The kernels run it guarded (rates that are no whole
+// words, one and two dimensions); without the guard they run TableEncoder, and this form's steps
+// from run to run are what the host checks hold against it.
 template <class Mem, bool GUARD, int SIZE = 64>
 struct BlockEncoder {
   Mem& mem;
@@ -1220,7 +1222,8 @@ constexpr QuadOrder make_quad_order()
 // the end of the block (the values are never used).
 // FENCED: the caller guarantees that the bit right after the block reads as one.
 // A run of zeros that the bit budget cuts short then ends at that bit by itself,
-// and the step loop does not have to clamp the run to the bits that are left.
+// and the step loop does not have to clamp the run to the bits that are left.  The kernels run it
+// without the fence; with one they run TableDecoder, and this form is its second opinion on the host.
 template <class Mem, int SIZE = 64, bool FENCED = false>
 struct BlockDecoder {
   Mem& mem;

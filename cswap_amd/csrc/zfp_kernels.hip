@@ -133,14 +133,13 @@ __host__ __device__ inline unsigned slot_bits(unsigned maxbits)
 }
 __host__ __device__ inline unsigned region_dwords(unsigned maxbits)
 {
-  return ((2u * slot_bits(maxbits) + 4u) + 3u) & ~3u;  // + padding for the 128-bit over-read / over-write
+  return ((2u * slot_bits(maxbits) + 4u) + 3u) & ~3u;  // + padding of 128 bits for what reads and OR-ed zeros reach past the last slot
 }
 // The 32-bit decoder's slot is the block and its fence (kFence), nothing more: its
 // reads reach up to 128 bits further, into the next lane's block (or the region's
-// padding), and those bits are never looked at.  What this saves in
-// LDS is two more wavefronts per compute unit at 16 bits per value (8720 bytes a
-// wavefront instead of 9232), and the stride of 2 (mod 4) dwords halves the bank
-// conflicts between lanes.  Slots are 8-byte aligned only.
+// padding of as many bits), and those bits are never looked at.  The stride is then 2 (mod 4)
+// dwords at even word counts.  Against slots as the encoder's: 10 bits per value 50 MB 16.0 / 16.7 us,
+// 100 MB 26.9 / 27.5; at 4, 8, 16, 24 and 32 level or up to 1 % ahead.  Slots are 8-byte aligned only.
 __host__ __device__ inline unsigned dec_slot_bits(unsigned maxbits)
 {
   return (maxbits & 63u) ? maxbits : maxbits + 64u;
@@ -504,10 +503,11 @@ __device__ __forceinline__ void load_region(uint32_t* lds, unsigned lane, uint32
 // ONCE: the field is loaded with the nontemporal hint (Field3::read_once)
 // WPE: wavefronts per SIMD the kernel is built for and held to.  Five, except from 16 bits
 // per value on: there a wavefront's LDS region (9 KB and more) lets 16 or 17 wavefronts
-// into a compute unit, unevenly over its SIMDs, and the encoder measured fastest with
-// three per SIMD (201.3 MB at 16 bits per value: 72.7 us, 73.1 with four and 74.3 with five, 72.1 with two
-// but 50 MB 26.4 instead of 21.9), the decoder with four (402.7 MB, stepping from run to run, 137-140 us
-// against 143-156 us).  Now 58 us each for 201.3 MB, 111 and 110 for 402.7 MB.
+// into a compute unit, unevenly over its SIMDs.  The encoder, three / four / five per SIMD, us, one tensor over
+// and over (several in turn): 16 bits 100 MB 32.0 / 30.9 / 33.2 (35.2 / 34.8 / 35.7), 201 MB 57.2 / 55.4 / 57.8 (59.1 / 58.5 / 60.1); 24 bits 37.7 / 39.4 /
+// 41.0 (42.2 / 43.4 / 44.4), 66.2 / 67.6 / 68.6; 32 bits 45.7 / 47.0 / 47.3, 79.4 / 80.8 / 81.0; in 35x35 planes the same.  Three for all of
+// these rates (84 registers, so it is the attribute that holds it there).  The decoder, three / four / five: 16 bits 100 MB 34.9 /
+// 34.1 / 35.6, 201 MB 62.8 / 57.2 / 60.1 (70.2 / 65.9 / 67.0); 24 and 32 bits within 1.5 %.  Four.  Below 36 MB all are level.
 // ROWS: a field for load_block_rows
 template <bool WHOLE, bool INT, bool ONCE, bool ROWS>
 __device__ __forceinline__ void encode3_f32(const float* __restrict__ in, const Field3& fd, unsigned maxbits,
@@ -1688,10 +1688,13 @@ static bool pair_fits(unsigned grid, size_t lds_bytes, unsigned long long limit)
   return (double)grid <= per_cu * (double)device_compute_units();
 }
 // The decoder's pair form, whose planes one half decodes alone, pays while every workgroup has a SIMD of
-// its own -- then what the halves share is worth its barriers -- and the planes are not all of the time:
-// lane / pair form at 16 bits per value 12.6 MB 13.35 / 12.7 us, 16.8 MB 13.0 / 12.4, 21 MB 14.6 / 14.6, 25.2 MB 14.3 / 15.2,
-// 41.9 MB 17.1 / 23.3; at 8 bits 12.6 MB 11.1 / 10.8, 16.8 MB 10.9 / 10.9; at 32 bits 12.6 MB 13.1 / 13.3, 16.8 MB 12.9 / 13.2.
-constexpr unsigned kPairDecodeFromBits = 1024, kPairDecodeBelowBits = 2048;
+// its own -- then what the halves share is worth its barriers -- and the planes are not all of the time.  One lane
+// per block / pair form, us, one tensor over and over (several in turn), 16.5 MB: 16 bits per value in 64x64 planes 12.3 / 11.9 (13.0 /
+// 12.7), 28x28 16.1 / 15.0 (16.5 / 15.3), 8x8 14.7 / 14.1 (16.7 / 16.0); 20 bits 12.5 / 12.4 (13.3 / 13.4), 16.2 / 15.4 (16.9 / 16.4), 14.9 / 14.6;
+// 24 bits 12.5 / 12.6 (13.6 / 14.0), 16.2 / 15.8 (17.0 / 16.8), 14.9 / 14.9; 28 bits 12.6 / 13.0 (14.0 / 14.5), 16.4 / 16.2 (17.4 / 17.5), 15.2 / 15.3; 10 MB
+// alike.  Beyond one workgroup per SIMD, at 16 bits: 21 MB 14.6 / 14.6, 25.2 MB 14.3 / 15.2, 41.9 MB 17.1 / 23.3.  At 8 bits 12.6 MB 11.1 /
+// 10.8, 16.8 MB 10.9 / 10.9.
+constexpr unsigned kPairDecodeFromBits = 1024, kPairDecodeBelowBits = 1792;
 static bool pair_decode_pays(unsigned grid, unsigned maxbits, unsigned long long limit)
 {
   if (limit == ~0ull) return true;

@@ -1716,13 +1716,22 @@ static bool pair_decode_pays(unsigned grid, unsigned maxbits, unsigned long long
 // from 30 bits per value on one lane per block meets that limit, too.
 constexpr unsigned kQuadWaves = 11;        // per compute unit, the encoder's where the pair form applies
 constexpr unsigned kQuadWavesNoPair = 22;  // where it does not
-constexpr unsigned kQuadWavesDecode = 9;
+constexpr unsigned kQuadWavesDecode = 9;  // the decoder's; kQuadWaves in rows of at most 32 bytes, where no other form stores with the hint
 constexpr unsigned kQuadOneRoundBelow = 1920;
 static double quad_waves_encode(const Field3& fd, unsigned maxbits)
 {
   if (pair_shape(fd, maxbits)) return kQuadWaves;
   const double fit = 0.92 * 160.0 * 1024.0 / (4.0 * (double)quad_lds_dwords(slot_bits(maxbits)));
   return maxbits < kQuadOneRoundBelow && fit < kQuadWavesNoPair ? fit : kQuadWavesNoPair;
+}
+// Rows of 16 and 32 bytes: the quad form, whose stores have the hint at any length of row, against what else takes the
+// field, one tensor over and over (several in turn), us, 10.4 MB: 16 bytes 8 bits per value 11.2 / 12.0 (11.1 / 12.5), 4 bits 10.0 /
+// 10.8 (11.7 / 11.1), 32 bits 13.7 / 14.9 (14.5 / 16.8); 32 bytes 11.0 / 11.2 (10.7 / 11.6), 10.0 / 9.9 (9.5 / 10.2), 13.5 / 14.2 (14.5 / 16.4); 80 bytes
+// 12.5 / 11.3 (11.1 / 11.7).  Where the pair form applies 16 bytes at 16 bits 13.7 / 13.9 (13.8 / 14.6), 32 bytes 13.7 / 12.7 (13.8 / 13.6).
+static double quad_waves_decode(const Field3& fd, unsigned maxbits)
+{
+  const bool pair = pair_shape(fd, maxbits) && maxbits >= kPairDecodeFromBits && maxbits < kPairDecodeBelowBits;
+  return fd.full && fd.rows16 && fd.sy <= 8 && !pair ? kQuadWaves : kQuadWavesDecode;
 }
 static bool quad_pays(uint32_t nblocks, double waves, unsigned long long bytes, unsigned long long pair_below, int compute_units)
 {
@@ -1752,6 +1761,17 @@ extern "C" int cswap_test_zfp_encode_route(size_t nx, size_t ny, size_t nz, ptrd
                                               CSWAP_PAIR_ENCODE_BYTES, compute_units))
     return 3;
   return encode_rows(fd, whole) ? 1 : load_hint(fd, whole) ? 2 : 0;
+}
+
+extern "C" int cswap_test_zfp_decode_quad(size_t nx, size_t ny, size_t nz, ptrdiff_t sy, ptrdiff_t sz, unsigned maxbits,
+                                          int compute_units)
+{
+  Field3 fd;
+  const void* aligned = reinterpret_cast<const void*>((uintptr_t)4096);
+  int rc = make_field(fd, aligned, aligned, nx, ny, nz, 1, sy, sz, maxbits, 4);
+  if (rc) return rc;
+  return (maxbits & 63u) == 0 && quad_pays(fd.nblocks, quad_waves_decode(fd, maxbits), (unsigned long long)nx * ny * nz * 4ull,
+                                           CSWAP_PAIR_DECODE_BYTES, compute_units);
 }
 
 extern "C" int cswap_test_zfp_store_hint(unsigned long long base, unsigned long long pitch, unsigned long long plane,
@@ -1853,8 +1873,8 @@ static int decompress3(const uint64_t* d_stream, Elem elem, size_t nx, size_t ny
   const bool whole = (maxbits & 63u) == 0;
   const bool is_int = elem == kI32 || elem == kI64;
   const unsigned long long pair_below = g_pair_decode_bytes.load(std::memory_order_relaxed);
-  if (quad && elem == kF32 && whole && quad_pays(fd.nblocks, kQuadWavesDecode, (unsigned long long)nx * ny * nz * 4ull, pair_below,
-                                          device_compute_units())) {
+  if (quad && elem == kF32 && whole && quad_pays(fd.nblocks, quad_waves_decode(fd, maxbits), (unsigned long long)nx * ny * nz * 4ull,
+                                                 pair_below, device_compute_units())) {
     hipLaunchKernelGGL(zfp_decode3_f32_quad_kernel, dim3((fd.nblocks + kQuadBlocks - 1) / kQuadBlocks), dim3(64),
                        (size_t)quad_lds_dwords(dec_slot_bits(maxbits)) * 4, st, d_stream, fd, maxbits,
                        static_cast<float*>(d_out));

@@ -40,6 +40,11 @@ int cswap_test_zvc_packed_hint(size_t bytes);
 int cswap_test_zfp_encode_route(size_t nx, size_t ny, size_t nz, ptrdiff_t sy, ptrdiff_t sz, unsigned misaligned,
                                 unsigned maxbits, int compute_units);
 
+/* 1 if a 3-D field of floats with contiguous, 16-byte aligned x-rows is decoded by the form with four lanes per block on a
+ * part with `compute_units` of them.  sy, sz: strides in elements (0 = packed).  Host only. */
+int cswap_test_zfp_decode_quad(size_t nx, size_t ny, size_t nz, ptrdiff_t sy, ptrdiff_t sz, unsigned maxbits,
+                               int compute_units);
+
 /* 1 if the decoder stores a field of 16-byte aligned rows with the nontemporal hint.  base: the field's address
  * (its alignment counts), pitch, plane: bytes from row to row and from plane to plane, bytes: of the field.  Host only. */
 int cswap_test_zfp_store_hint(unsigned long long base, unsigned long long pitch, unsigned long long plane,

@@ -387,7 +387,7 @@ def test_pair_form_of_the_decoder_matches_golden_vectors_and_the_block_decoder(h
 @pytest.mark.parametrize("kind", [0, 1, 2], ids=["int32", "double", "int64"])
 def test_other_scalar_types_through_the_tables(host, kind):
     """The blocks of the kernels for int32, double and int64 at whole-word rates, coded and decoded with the tables,
-    against the checker; no one-bit is written further than 128 bits past a block and none read further than 192."""
+    against the oracle; no one-bit is written further than 128 bits past a block and none read further than 192."""
     import oracle
 
     host.host_zfp_blocks_table.argtypes = [C.c_void_p, C.c_int, C.c_size_t, C.c_uint, C.c_void_p, C.c_void_p]

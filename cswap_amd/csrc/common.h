@@ -28,6 +28,13 @@ int zfp_decompress_f32_no_quad(const uint64_t* d_stream, size_t nx, size_t ny, s
 // tensor of n elements has left to pay for it (link and expansion) against the raw swap.
 bool made_payload_pays(size_t n, size_t bytes, const cswap_costs& costs);
 
+// A copy between device memory and pinned host memory as a kernel on the stream (link_kernels.hip).  Addresses and
+// bytes are multiples of 4.
+hipError_t link_copy(void* dst, const void* src, size_t bytes, hipStream_t stream);
+
+// *host (pinned memory) becomes *count
+hipError_t publish_count(int* host, const int* count, hipStream_t stream);
+
 // to be called right after a kernel launch: picks up launch-configuration errors
 inline int check_launch()
 {

@@ -5,11 +5,12 @@
 //   swap_out  = pre  : (probe, select,) compress on the compute stream, then an
 //                      async device-to-host copy on a dedicated copy stream
 //   swap_wait = post : wait for that copy; the device tensor may then be freed
-//   swap_in          : async host-to-device copy on a second copy stream (the link
-//                      carries both directions at once), then decompress on the
-//                      compute stream; a compressed tensor whose outbound copy has
-//                      not finished yet is decompressed straight from its staging
-//                      block, without touching the link
+//   prefetch         : async host-to-device copy on a second copy stream (the link
+//                      carries both directions at once)
+//   swap_in          : decompress on the compute stream, behind a prefetch or behind
+//                      a host-to-device copy on the compute stream itself; a compressed
+//                      tensor whose outbound copy has not finished yet is decompressed
+//                      straight from its staging block, without touching the link
 // Nothing here makes the host wait unless it has to: a staging block whose copy
 // has finished is taken back the next time somebody needs room (an event query),
 // a released ticket whose work is still in flight gives its memory back when that
@@ -115,7 +116,8 @@ struct Ticket {
   bool done_pending = false;      // a decompression that reads the staging block (ev_done) is not known to have finished
   bool keep_staged = false;       // a prefetch found the payload still in its staging block: it stays there
   unsigned long long seq = 0;     // order of the swap-outs: the oldest work in flight is waited for first
-  hipEvent_t ev_ready = nullptr;  // compute stream: compressed data / destination ready
+  bool made = false;              // the host has seen the payload finished: ev_ready is not recorded
+  hipEvent_t ev_ready = nullptr;  // compute stream: compressed data ready
   hipEvent_t ev_copy = nullptr;   // copy stream: transfer finished
   hipEvent_t ev_done = nullptr;   // compute stream: decompression finished
   // engines with timing only: where each phase starts on its stream (its end is one of the three above)
@@ -250,9 +252,9 @@ extern "C" int cswap_engine_create(cswap_engine** out, const cswap_engine_config
     // default priority on purpose; non-blocking so it never serialises with the null stream
     if ((err = hipStreamCreateWithFlags(&e->copy, hipStreamNonBlocking)) != hipSuccess) { fail(err); break; }
     if ((err = hipStreamCreateWithFlags(&e->copy_in, hipStreamNonBlocking)) != hipSuccess) { fail(err); break; }
-    if ((err = hipHostMalloc((void**)&e->h_base, cfg.pinned_pool_bytes, hipHostMallocDefault)) != hipSuccess) { fail(err); break; }
+    if ((err = hipHostMalloc((void**)&e->h_base, cfg.pinned_pool_bytes, hipHostMallocCoherent)) != hipSuccess) { fail(err); break; }
     if ((err = hipMalloc((void**)&e->d_base, cfg.device_pool_bytes)) != hipSuccess) { fail(err); break; }
-    if ((err = hipHostMalloc((void**)&e->h_nnz, 256, hipHostMallocDefault)) != hipSuccess) { fail(err); break; }
+    if ((err = hipHostMalloc((void**)&e->h_nnz, 256, hipHostMallocCoherent)) != hipSuccess) { fail(err); break; }
     if ((err = hipMalloc((void**)&e->d_nnz, 256)) != hipSuccess) { fail(err); break; }
     if ((err = hipMalloc(&e->d_ws, cswap_zvc_workspace_bytes(kWsProcess))) != hipSuccess) { fail(err); break; }
     if ((rc = cswap_zvc_workspace_clear(e->d_ws, kWsProcess, nullptr)) != CSWAP_OK) break;
@@ -405,6 +407,16 @@ static void abandon_device(cswap_engine* e, Ticket& t, hipStream_t compute)
 // ---- the four steps of a swap-out.  Each leaves the ticket consistent on failure:
 // whatever it holds is given back by abandon_device / the caller.
 
+// The count that a kernel queued on the compute stream leaves in d_nnz.  Everything queued there so far has run by then.
+static int count_to_host(cswap_engine* e, hipStream_t compute, int* count)
+{
+  CSWAP_HIP_TRY(cswap::publish_count(e->h_nnz, e->d_nnz, compute));
+  CSWAP_HIP_TRY(hipEventRecord(e->ev_probe, compute));
+  CSWAP_HIP_TRY(hipEventSynchronize(e->ev_probe));
+  *count = *e->h_nnz;
+  return CSWAP_OK;
+}
+
 // Counts the non-zeros of the tensor (one host round trip, Execution.h:92) and
 // leaves the per-chunk counts, scanned into offsets, in the ticket's probe block.
 // Without room for that block: CSWAP_E_NOMEM if the probe is required, else the
@@ -422,12 +434,10 @@ static int probe_tensor(cswap_engine* e, Ticket& t, const float* d_in, hipStream
   int* d_counts = (int*)(e->d_base + off);
   int rc = cswap_zvc_count(d_in, (int)t.n, t.process, d_counts, compute);
   if (!rc) rc = cswap_zvc_scan(d_counts, cswap_zvc_active_chunks((int)t.n, t.process), e->d_nnz, compute);
+  int count = 0;
+  if (!rc) rc = count_to_host(e, compute, &count);
   if (rc) { abandon_device(e, t, compute); return rc; }
-  hipError_t err = hipMemcpyAsync(e->h_nnz, e->d_nnz, sizeof(int), hipMemcpyDeviceToHost, compute);
-  if (err == hipSuccess) err = hipEventRecord(e->ev_probe, compute);
-  if (err == hipSuccess) err = hipEventSynchronize(e->ev_probe);
-  if (err != hipSuccess) { abandon_device(e, t, compute); return hip_fail(err); }
-  t.nnz = (size_t)*e->h_nnz;
+  t.nnz = (size_t)count;
   e->probes++;
   return CSWAP_OK;
 }
@@ -455,21 +465,19 @@ static int single_pass_sparse(cswap_engine* e, Ticket& t, const float* d_in, hip
   char* base = e->d_base + off;
   int rc = cswap_zvc_compress_fused(d_in, (int)t.n, t.process, e->d_ws, (int*)base, e->d_nnz, (float*)(base + hdr),
                                     (uint32_t*)(base + 4 * (size_t)t.process), compute);
-  hipError_t err = hipSuccess;
-  if (!rc) err = hipMemcpyAsync(e->h_nnz, e->d_nnz, sizeof(int), hipMemcpyDeviceToHost, compute);
-  if (!rc && err == hipSuccess) err = hipEventRecord(e->ev_probe, compute);
-  if (!rc && err == hipSuccess) err = hipEventSynchronize(e->ev_probe);
-  if (rc || err != hipSuccess) {
+  int count = 0;
+  if (!rc) rc = count_to_host(e, compute, &count);
+  if (rc) {
     (void)hipStreamSynchronize(compute);
     e->dpool.free(off, worst);
-    return rc ? rc : hip_fail(err);
+    return rc;
   }
-  if (*e->h_nnz < 0) {  // kernels have finished (the event): the block can go back at once
+  if (count < 0) {  // the kernel has finished (its count is here): the block can go back at once
     e->dpool.free(off, worst);
     (void)cswap_zvc_workspace_clear(e->d_ws, kWsProcess, compute);  // a failed run leaves the workspace unusable
     return 1;
   }
-  t.nnz = (size_t)*e->h_nnz;
+  t.nnz = (size_t)count;
   t.bytes_out = hdr + 4 * t.nnz;
   e->dpool.shrink(off, worst, t.bytes_out);
   t.dev_off = off; t.dev_bytes = t.bytes_out; t.dev_held = true;
@@ -540,11 +548,28 @@ static int compress_tensor(cswap_engine* e, Ticket& t, const float* d_in, hipStr
   return rc;
 }
 
-// Device-to-host copy on the copy stream, ordered after the compression by an event.
-static int start_outbound_copy(cswap_engine* e, Ticket& t, const void* src, hipStream_t compute)
+// A payload in, on the compute stream.  Beside copies out the runtime's copy it is: the copy kernel's reads of host
+// memory and their writes are in each other's way (8 MB each way at once: 222 us and more, with the runtime's copy both ways
+// 182).  The kernel's launch needs the engine's GPU to be the thread's current one, and addresses at whole words.
+static hipError_t copy_in_here(const cswap_engine* e, void* dst, const void* src, size_t bytes, hipStream_t compute)
 {
-  hipError_t err = hipEventRecord(t.ev_ready, compute);
-  if (err == hipSuccess) err = hipStreamWaitEvent(e->copy, t.ev_ready, 0);
+  bool outbound = false;
+  for (auto& t : e->tickets)
+    if (!outbound && t.state != kFree && t.out_pending) outbound = !event_done(t.ev_copy);
+  int device = -1;
+  if (!outbound && (((uintptr_t)dst | (uintptr_t)src | bytes) & 3u) == 0 && hipGetDevice(&device) == hipSuccess && device == e->device)
+    return cswap::link_copy(dst, src, bytes, compute);
+  return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, compute);
+}
+
+// Device-to-host copy on the copy stream, ordered after the compression by an event -- unless the host has seen the
+// compression end (`made`).  To have a stream wait for an event that has not fired costs 15 us of the host's time.
+static int start_outbound_copy(cswap_engine* e, Ticket& t, const void* src, hipStream_t compute, bool made = false)
+{
+  t.made = made;
+  hipError_t err = hipSuccess;
+  if (!made || e->timing) err = hipEventRecord(t.ev_ready, compute);
+  if (err == hipSuccess && !made) err = hipStreamWaitEvent(e->copy, t.ev_ready, 0);
   if (err == hipSuccess) err = phase_start(e, t, kPhaseCopyOut, e->copy);
   if (err == hipSuccess)
     err = hipMemcpyAsync(e->h_base + t.host_off, src, t.bytes_out, hipMemcpyDeviceToHost, e->copy);
@@ -640,7 +665,7 @@ extern "C" int cswap_swap_out(cswap_engine* e, const float* d_in, size_t nx, siz
         return CSWAP_E_NOMEM;
       }
       t.host_off = hoff; t.host_bytes = t.bytes_out;
-      rc = start_outbound_copy(e, t, payload, compute);
+      rc = start_outbound_copy(e, t, payload, compute, true);  // its count is here: the kernel has run
       if (rc) {
         (void)hipStreamSynchronize(compute);
         (void)hipStreamSynchronize(e->copy);
@@ -781,7 +806,7 @@ extern "C" int cswap_swap_in(cswap_engine* e, int ticket, float* d_out, cswap_st
     // the payload is complete when the compression has run (ev_ready); the outbound copy goes on
     // reading the same block, which stays with the ticket until both are done
     src = e->d_base + t->dev_off;
-    err = hipStreamWaitEvent(compute, t->ev_ready, 0);
+    if (!t->made) err = hipStreamWaitEvent(compute, t->ev_ready, 0);
   } else if (t->state == kPrefetched) {
     src = e->d_base + t->dev_off;
     err = hipStreamWaitEvent(compute, t->ev_copy, 0);
@@ -795,13 +820,9 @@ extern "C" int cswap_swap_in(cswap_engine* e, int ticket, float* d_out, cswap_st
       t->dev_off = off; t->dev_bytes = t->bytes_out; t->dev_held = true;
       src = e->d_base + off;
     }
-    // the copy may not overtake earlier work of the compute stream on d_out
-    err = hipEventRecord(t->ev_ready, compute);
-    if (err == hipSuccess) err = hipStreamWaitEvent(e->copy_in, t->ev_ready, 0);
-    if (err == hipSuccess) err = phase_start(e, *t, kPhaseCopyIn, e->copy_in);
-    if (err == hipSuccess) err = hipMemcpyAsync(src, e->h_base + t->host_off, t->bytes_out, hipMemcpyHostToDevice, e->copy_in);
-    if (err == hipSuccess) err = hipEventRecord(t->ev_copy, e->copy_in);
-    if (err == hipSuccess) err = hipStreamWaitEvent(compute, t->ev_copy, 0);
+    err = phase_start(e, *t, kPhaseCopyIn, compute);
+    if (err == hipSuccess) err = copy_in_here(e, src, e->h_base + t->host_off, t->bytes_out, compute);
+    if (err == hipSuccess && e->timing) err = hipEventRecord(t->ev_copy, compute);
     t->in_copied = true;
   }
   if (err == hipSuccess) err = phase_start(e, *t, kPhaseDecompress, compute);
@@ -1016,9 +1037,8 @@ extern "C" int cswap_engine_calibrate(cswap_engine* e, cswap_costs* out_costs)
       for (int i = 0; i < reps && er2 == hipSuccess && !rc; i++) {
         rc = cswap_zvc_count(d_x, small_n, small_proc, d_begin, s);
         if (!rc) rc = cswap_zvc_scan(d_begin, cswap_zvc_active_chunks(small_n, small_proc), e->d_nnz, s);
-        if (!rc) er2 = hipMemcpyAsync(e->h_nnz, e->d_nnz, sizeof(int), hipMemcpyDeviceToHost, s);
-        if (!rc && er2 == hipSuccess) er2 = hipEventRecord(e->ev_probe, s);
-        if (!rc && er2 == hipSuccess) er2 = hipEventSynchronize(e->ev_probe);
+        int count;
+        if (!rc) rc = count_to_host(e, s, &count);
       }
       auto t1 = std::chrono::steady_clock::now();
       if (rc) break;

@@ -370,7 +370,7 @@ typedef struct {
  *   copy_out_us    the device-to-host copy on the copy stream (what the reference splits into
  *                  the part under the consumer's kernel, slot 0, and the wait after it,
  *                  slot 1: Execution.h:285-295)
- *   copy_in_us     the host-to-device copy on the inbound copy stream
+ *   copy_in_us     the host-to-device copy, on `compute` or (prefetched) on the inbound copy stream
  *   decompress_us  the decompression kernel on the compute stream */
 typedef struct {
   double compress_us, copy_out_us, copy_in_us, decompress_us;
@@ -400,9 +400,9 @@ int cswap_swap_out(cswap_engine* e, const float* d_in, size_t nx, size_t ny, siz
  * returns, so it may go back to a stream-ordered allocator at once and nobody
  * has to wait.  Also answered after a cswap_swap_in that came first. */
 int cswap_swap_wait(cswap_engine* e, int ticket);
-/* Backward side: copy back on the engine's inbound copy stream (its own: both
- * directions of the link can be busy at once), then decompress into d_out on
- * `compute` (ordered by an event).  Returns at once; the data is ready when
+/* Backward side: copy back and decompress into d_out, both on `compute`.  A
+ * prefetched payload came over the link on the engine's inbound copy stream (its
+ * own: both directions can be busy at once) and is ordered by an event.  Returns at once; the data is ready when
  * `compute` reaches this point.  A compressed tensor whose outbound copy has not
  * finished yet is still in its staging block and is decompressed from there: no
  * wait for the copy, nothing on the link. */

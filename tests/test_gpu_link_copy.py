@@ -1,0 +1,60 @@
+"""Payloads that come in on the compute stream: the copy kernel at the edges of its pieces and of its grid, and the
+runtime's copy in its place beside a copy out."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def engine():
+    from cswap_amd import swap
+
+    e = swap.SwapEngine(pinned_bytes=256 << 20, device_bytes=256 << 20)
+    yield e
+    e.close()
+
+
+# pieces of 16 bytes, 256 to a workgroup, 64 workgroups a turn: below and above each, and remainders of 1 to 3 words
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 1023, 1024, 1027, 65535, 65536, 65539, 200001])
+@pytest.mark.parametrize("shift", [0, 1, 2, 3])
+def test_raw_payload_comes_back_at_any_element(engine, n, shift):
+    import torch
+
+    from cswap_amd import swap
+
+    for _ in range(2):  # the second time through the same pinned block, with other values
+        x = torch.randn(1, 1, 1, n, device="cuda")
+        room = torch.full((n + 8,), -7.0, device="cuda")
+        ticket = engine.pre(x, swap.NONE)
+        engine.post(ticket)
+        engine.swap_in(ticket, room[shift:shift + n])
+        engine.release(ticket)
+        torch.cuda.synchronize()
+        assert torch.equal(room[shift:shift + n], x.view(-1))
+        assert bool((room[:shift] == -7.0).all()) and bool((room[shift + n:] == -7.0).all())
+
+
+@pytest.mark.parametrize("policy", ["none", "sparse", "zfp"])
+def test_payload_comes_in_beside_a_copy_out(engine, policy):
+    import torch
+
+    from cswap_amd import swap
+
+    pol = {"none": swap.NONE, "sparse": swap.SPARSE, "zfp": swap.ZFP}[policy]
+    x = torch.randn(64, 64, 16, 16, device="cuda").clamp_(min=0.0)
+    big = torch.randn(1, 32, 1024, 1024, device="cuda")
+    alone, beside, back = torch.empty_like(x), torch.empty_like(x), torch.empty_like(big)
+    for out, other in ((alone, False), (beside, True)):
+        ticket = engine.pre(x, pol)
+        engine.post(ticket)
+        outbound = engine.pre(big, swap.NONE) if other else None
+        engine.swap_in(ticket, out)
+        engine.release(ticket)
+        if other:
+            engine.post(outbound)
+            engine.swap_in(outbound, back)
+            engine.release(outbound)
+    torch.cuda.synchronize()
+    assert torch.equal(alone, beside) and torch.equal(back, big)
+    if policy != "zfp":
+        assert torch.equal(alone, x)

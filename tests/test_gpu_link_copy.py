@@ -58,3 +58,50 @@ def test_payload_comes_in_beside_a_copy_out(engine, policy):
     assert torch.equal(alone, beside) and torch.equal(back, big)
     if policy != "zfp":
         assert torch.equal(alone, x)
+
+
+@pytest.mark.parametrize("n", [1001, 1 << 20])
+@pytest.mark.parametrize("order", ["in", "in_post", "prefetch_in", "prefetch_post_in", "prefetch_release"])
+def test_raw_tensor_asked_back_behind_its_copy_out(engine, order, n):
+    """A long copy out goes ahead, so that the tensor's own is still to come when it is asked back."""
+    import torch
+
+    from cswap_amd import swap
+
+    big = torch.randn(1, 16, 1024, 1024, device="cuda")
+    for _ in range(2):
+        x = torch.randn(1, 1, 1, n, device="cuda")
+        want, out = x.clone(), torch.empty_like(x)
+        torch.cuda.synchronize()
+        ahead = engine.pre(big, swap.NONE)
+        ticket = engine.pre(x, swap.NONE)
+        if order.startswith("prefetch"):
+            engine.prefetch(ticket)
+        if order == "prefetch_post_in":
+            engine.post(ticket)
+            x.fill_(3.0)
+        if order != "prefetch_release":
+            engine.swap_in(ticket, out)
+        if order == "in_post":
+            engine.post(ticket)
+            x.fill_(3.0)
+        engine.release(ticket)
+        engine.post(ahead)
+        engine.release(ahead)
+        torch.cuda.synchronize()
+        assert order == "prefetch_release" or torch.equal(out, want)
+
+
+def test_raw_tensor_comes_back_into_itself(engine):
+    import torch
+
+    from cswap_amd import swap
+
+    x = torch.randn(1, 4, 1024, 1024, device="cuda")
+    want = x.clone()
+    for _ in range(3):
+        ticket = engine.pre(x, swap.NONE)
+        engine.swap_in(ticket, x)
+        engine.release(ticket)
+    torch.cuda.synchronize()
+    assert torch.equal(x, want)

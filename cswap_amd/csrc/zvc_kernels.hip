@@ -20,6 +20,7 @@
 #include "../../include/cswap_hip.h"
 #include "../../include/cswap_test_hooks.h"
 #include "common.h"
+#include "zfp_block.h"  // Div31
 
 namespace cswap {
 
@@ -1005,241 +1006,287 @@ __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
 }
 
 // ------------------------------------------------------------------ one kernel for small tensors
-// Up to 64 MiB the whole tensor fits in the registers of one grid: every workgroup (one per
-// compute unit, sixteen wavefronts) loads its share once -- wavefront v of workgroup w owns R
-// consecutive rows of 64 elements of the mask layout --, counts it, writes its mask words, and
-// publishes its count.  There is no scanner: every workgroup reads the counts of the workgroups
-// before it itself, one trip through memory instead of two, takes their sum as its offset, and
-// stores its non-zeros straight from the registers (at these sizes the values array stays in the
-// memory-side cache, where whole-line stores through an LDS stage gain nothing).  The last
-// workgroup, which has read every count but its own, writes the total.  Nobody waits for a
-// workgroup with a higher number than its own, so the grid makes progress however few of its
-// workgroups the hardware runs at a time (they are started in order).
+// Below 64 MiB the whole tensor fits in the registers of one grid.  It is cut into at most 512 tiles of consecutive
+// elements, a workgroup each: W wavefronts of R rows of 64 elements.  A workgroup loads its tile, counts it,
+// publishes the count, reads the counts of the workgroups before it (one trip through memory), takes their sum as
+// its offset and stores its non-zeros straight from the registers (at these sizes the values array stays in the
+// memory-side cache, where whole-line stores through an LDS stage gain nothing).  The last workgroup, which has read
+// every count but its own, writes the total.  Nobody waits for a workgroup with a higher number than its own, so the
+// grid makes progress however few of its workgroups the hardware runs at a time (they are started in order).
 //
-// RAGGED: chunks of any length.  A half row of the mask layout is then up to 32 elements of one
-// chunk, at any element of the tensor, and a lane works out place and existence of its element
-// row by row (about 12 instructions a row, behind the loads that are already on their way).
-// Measured, three kernels -> this one: 60 MB in 8192 chunks of 1838 elements 35 -> 25.3 us (30.5
-// with the counting pass's 16-byte loads at any element), 30 MB 17.3 -> 14.6, 7 MB 12.3 -> 8.4,
-// 1.6 MB in 16384 chunks 14.4 -> 8.2.  64 rows per wavefront instead of the three kernels
-// (33.6 to 67 MB): 63.7 MB 31 -> 25.
+// Rows are rows of the tensor, whatever the chunks are: a row's ballot is 64 bits of the flat bit mask.  Where
+// chunks are whole half rows that is the mask layout.  Elsewhere (RAGGED) the tile's bits go to LDS, and a lane makes a
+// mask word from the 32 bits at its first element; a word belongs to the tile that has its first element, and the last
+// wavefront looks one row further than the tile for the bits of the tile's last words.
 //
-// The counts live in two arrays of 256 words, used in turns: run k publishes into array k & 1 and
-// every workgroup clears its word of the other one, which nobody reads any more;
-// ws[kWsSmallRuns] counts the runs.  The grid is the same for every size and the arrays have one
-// place in every workspace (status words 65024 to 65535, which the pipeline kernel leaves out),
-// whatever chunk count a call comes with, so every word is cleared every time.  Failure works as
-// in the pipeline kernel: a wait that runs out raises the sticky flag, the offsets are kept inside
-// the tensor, and the wavefront that gave up writes -1 after the last workgroup has stepped the
-// run counter.
-// The variants that took over shapes of the three kernels (RAGGED, 64 rows) must not fail where
-// those did not: a workgroup that finds the workspace unusable or whose wait runs out counts the
-// elements before its own by itself, which costs time and nothing else.  The last workgroup alone
-// steps the run counter, and only when it has seen everybody's count, so that everybody has taken
-// the same array: had it stepped past a workgroup that is still to start, that one would publish
-// into the next run's array.  If its wait runs out it leaves the counter and raises the flag
-// instead, which keeps later runs away from the words until they are cleared.
-constexpr int kQWaves = 16;
-constexpr int kQGroupsMax = 256;
+// Groups of 64 tiles.  A tile's count is read by every later tile of its group; the last tile of a group, when it has
+// read them all, publishes the group's total, which every tile of later groups reads.  So an offset takes two trips
+// through memory, 1 us each.  Every count has 32 bytes to itself: what workgroups on different dies store into one
+// line is stored one after the other, 5 ns and more a store, and with the counts side by side those were the time (33.6 MB in
+// 512 tiles 13.6 -> 11.7 us, 60 MB in 919 tiles 22.1 -> 18.8; how often they are read, and that 64 tiles read one, does
+// not show).  A tile that has its offset marks its own count, and the counts of a group in which all are marked are
+// cleared: by the last tile of the group after next, those of the last three groups by the last tile.  (A counter per group on
+// which the tiles add, and whose last adder clears: 33.6 MB 2.4 us more, 60 MB 3.3.)
+//
+// The totals live in two arrays of 256 words, used in turns: run k publishes into array k & 1 and clears the other one, which
+// nobody reads any more; ws[kWsSmallRuns] counts the runs.  The entries that a run has no group for are its
+// last workgroup's, so every entry is written and cleared every time.  The arrays have one
+// place in every workspace (status words 65024 to 65535, which the pipeline kernel leaves out; the counts are in front of
+// them), whatever chunk count a call comes with.  The last workgroup alone steps the run counter, and only when it has
+// its offset, so that everybody has taken the same array: had it stepped past a workgroup that is still to
+// start, that one would publish into the next run's array.
+//
+// Failure works as in the pipeline kernel for the shapes that take_single_pass says 2 for (may_fail): a wait that runs
+// out raises the sticky flag, the offsets are kept inside the tensor, and the wavefront that gave up writes -1 after the
+// last workgroup has stepped the run counter.  The other shapes must not fail: a workgroup that finds the workspace
+// unusable or whose wait runs out counts the elements before its own by itself, which costs time and nothing else; the
+// flag goes up all the same, since counts that nobody clears would be the next run's.
+//
+// Bound by the two trips (some 2 us), by the loads before and the stores behind them, which overlap only as far as tiles
+// differ in when they get their offset, and by instruction issue (14 a row).  Against one workgroup of sixteen wavefronts on
+// every compute unit, whatever the size, with one trip for 256 counts side by side, us alone / with the expansion behind it: 1 MB 7.5 -> 4.8 /
+// 11.9 -> 9.4, 4.2 MB 8.0 -> 5.8 / 13.0 -> 11.1, 16.8 MB 10.2 -> 8.1 / 18.2 -> 16.7, 33.6 MB 13.2 -> 12.4 / 24.4 -> 23.6, 50 MB 21.5 -> 17.3 / 34.8 -> 31.0;
+// chunks of any length: 22 MB 13.5 -> 9.7 / 24.1 -> 21.3, 60 MB 24.4 -> 20.5 / 40.4 -> 36.3.
+constexpr unsigned kGroupTiles = 64, kGroupsMax = 64;  // a lane for each
+constexpr unsigned kCountWords = 8;                    // from one count to the next
+constexpr uint32_t kTileThrough = 1u << 30;            // the tile has its offset
 constexpr int kWsSmallRuns = 4;
 constexpr int kStatusWordsMin = 65536;  // status words of the smallest workspace
-constexpr int kSmallWords = 2 * kQGroupsMax;
+constexpr int kSmallTotals = 256;
+constexpr int kSmallWords = 2 * kSmallTotals;
 constexpr int kSmallCounts = kStatusWordsMin - kSmallWords;  // status word at which the two arrays start
+static_assert(kGroupsMax * kGroupTiles * kCountWords <= (unsigned)kSmallCounts, "the counts are in front of the totals");
 
-template <int R, bool RAGGED>
-__global__ __launch_bounds__(64 * kQWaves) void zvc_small_kernel(
-    const float* __restrict__ in, StreamGeometry g, uint32_t* __restrict__ ws, uint32_t* __restrict__ counts,
-    int* __restrict__ begin, int* __restrict__ nnz, float* __restrict__ values, uint32_t* __restrict__ mask,
-    unsigned spin_limit, unsigned skip_first)
+struct SmallGeometry {
+  unsigned n, E, W, process;
+  unsigned tiles;
+  unsigned spread;            // log2 of the words from one group's total to the next
+  unsigned mask_words, tail;  // words of the mask, and the first of those that hold no element
+  Div31 by_E, by_W;
+};
+
+// old with lane `lane` replaced by the uniform v
+__device__ uint32_t write_lane(uint32_t v, uint32_t lane, uint32_t old) __asm("llvm.amdgcn.writelane.i32");
+
+template <int W, int R, bool RAGGED>
+__global__ __launch_bounds__(64 * W, 8) void zvc_small_kernel(
+    const float* __restrict__ in, SmallGeometry g, uint32_t* __restrict__ ws, int* __restrict__ begin, int* __restrict__ nnz,
+    float* __restrict__ values, uint32_t* __restrict__ mask, int may_fail, unsigned spin_limit, unsigned skip_first)
 {
-  constexpr int kHeld = (R + 31) / 32;  // registers of mask words: lane l of register h holds half row 64h + l
-  __shared__ unsigned s_cnt[kQWaves];
-  __shared__ unsigned s_head[5];        // refused, parity, my offset, total, count for myself
-  const int G = (int)gridDim.x, w = (int)blockIdx.x;
-  const unsigned lane = lane_id();
+  constexpr unsigned kElems = 64u * W * R, kHalves = 2u * W * R;
+  static_assert(R <= 32, "64 half rows to a wavefront");
+  __shared__ uint32_t bits[kHalves + 2];  // the tile's bits, and those of the row behind it
+  __shared__ uint16_t pre[kHalves];       // set bits of the wavefront's half rows before this one
+  __shared__ unsigned s_cnt[W], s_before[W];  // set bits of each wavefront's rows, and of the rows before them
+  __shared__ unsigned s_head[4];              // refused, offset, gave up, failure flag
+  const unsigned t = blockIdx.x, lane = lane_id();
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int r0 = (w * kQWaves + wv) * R;  // my first row
+  const unsigned first = t * kElems, mine = first + 64u * R * wv;  // my tile's first element, my wavefront's
+  const unsigned end = min(first + kElems, g.n);
 
-  constexpr bool kCountsItself = RAGGED || R > 32;
-  const unsigned long long w_magic = ((1ull << 40) + (unsigned)g.W - 1) / (unsigned)g.W;
+  // is the workspace usable, and which count array is this run's: asked for together with the data
+  uint32_t magic = kWsMagic, flag = 0, runs = 0;
+  if (wv == 0) {
+    magic = ld_status(&ws[0]);
+    flag = ld_status(&ws[kWsFlag]);
+    runs = ld_status(&ws[kWsSmallRuns]);
+  }
 
-  // ---- my rows; what does not exist is read from an element that does and ignored
+  // ---- my rows
   float x[R];
-  int left = 0;             // !RAGGED: elements that exist from my first row on
-  uint32_t exists[kHeld];   // RAGGED: bit j % 32 of register j / 32: my element of row j exists
-  if (RAGGED) {
-    const unsigned half = 2u * (unsigned)r0 + (lane >> 5);
-    const unsigned c = (unsigned)(((unsigned long long)half * w_magic) >> 40);
-    const unsigned row_elems = 32u * (unsigned)g.W, E = (unsigned)g.E;  // a chunk's elements in the mask layout, and in the tensor
-    unsigned e = 32u * (half - c * (unsigned)g.W) + (lane & 31u);       // place in the chunk
-    unsigned idx = E * c + e;
-    const unsigned chunks = 64u / row_elems, rest = 64u - chunks * row_elems;  // one row further
-    const unsigned step = chunks * E + rest, wrapped = step + E - row_elems, last = (unsigned)g.n - 1u;
+  const int left = mine < g.n ? (int)min(g.n - mine, 64u * R) : 0;  // elements that exist
+  if (left == 64 * R) {
 #pragma unroll
-    for (int h = 0; h < kHeld; h++) exists[h] = 0;
-#pragma unroll
-    for (int j = 0; j < R; j++) {
-      x[j] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(in) + (size_t)(4u * min(idx, last)));
-      exists[j / 32] |= (e < E && idx <= last ? 1u : 0u) << (j % 32);
-      e += rest;
-      const bool wraps = e >= row_elems;
-      e -= wraps ? row_elems : 0u;
-      idx += wraps ? wrapped : step;
-      // row after row, and the bits in a register: not a pair of scalars per row
-      asm volatile("" : "+v"(exists[j / 32]), "+v"(e), "+v"(idx));
-    }
-  } else {
-    const long long first = (long long)r0 * 64;
-    long long left_ll = (long long)g.n - first;
-    left_ll = left_ll < 0 ? 0 : (left_ll > R * 64 ? R * 64 : left_ll);
-    left = (int)left_ll;
-    const float* base = in + (left > 0 ? first : 0);
+    for (int j = 0; j < R; j++) x[j] = in[mine + lane + 64u * j];
+  } else {  // what does not exist is read from an element that does, and is a zero from here on
+    const float* base = in + (left > 0 ? mine : 0u);
     const unsigned last = (unsigned)max(left - 1, 0);
 #pragma unroll
-    for (int j = 0; j < R; j++)
-      x[j] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + (size_t)(4u * min(lane + 64u * j, last)));
-  }
-  if (threadIdx.x == 0) {  // together with the data: is the workspace usable, and which count array is this run's
-    const uint32_t magic = ld_status(&ws[0]), flag = ld_status(&ws[kWsFlag]), runs = ld_status(&ws[kWsSmallRuns]);
-    s_head[0] = (magic != kWsMagic || flag != 0u) ? 1u : 0u;
-    s_head[1] = runs;
-  }
-
-  // ---- count, and the mask words (two per row, straight from the ballots)
-  unsigned cnt = 0;
-  uint32_t held[kHeld];
+    for (int j = 0; j < R; j++) x[j] = base[min(lane + 64u * j, last)];
 #pragma unroll
-  for (int h = 0; h < kHeld; h++) held[h] = 0;
+    for (int j = 0; j < R; j++) x[j] = (int)lane < left - 64 * j ? x[j] : 0.0f;
+  }
+  float behind = 0.0f;
+  if (RAGGED && wv == W - 1 && first + kElems + lane < g.n) behind = in[first + kElems + lane];
+
+  // ---- count: lane l < 2R keeps half row l of my rows
+  uint32_t held = 0;
 #pragma unroll
   for (int j = 0; j < R; j++) {
-    // an element that does not exist is a zero from here on
-    if (RAGGED) x[j] = __uint_as_float(__float_as_uint(x[j]) & (0u - ((exists[j / 32] >> (j % 32)) & 1u)));
-    else x[j] = (int)lane < left - 64 * j ? x[j] : 0.0f;
-    asm volatile("" : "+v"(x[j]));
+    asm volatile("" : "+v"(x[j]));  // row after row: the ballots are made again below, 32 scalar pairs would not last
     const unsigned long long m = __ballot(x[j] != 0.0f);
-    cnt += popc64(m);
-    unsigned me = lane;
-    asm volatile("" : "+v"(me));  // compared afresh for every row: kept, the conditions would not last in scalars either
-    if (me == 2u * (j % 32)) held[j / 32] = (uint32_t)m;
-    if (me == 2u * (j % 32) + 1u) held[j / 32] = (uint32_t)(m >> 32);
+    held = write_lane((uint32_t)m, 2 * j, held);
+    held = write_lane((uint32_t)(m >> 32), 2 * j + 1, held);
   }
-#pragma unroll
-  for (int h = 0; h < kHeld; h++) {
-    const long long word = ((long long)r0 + 32 * h) * 2 + lane;
-    if ((int)lane < 2 * (R - 32 * h) && word < (long long)g.mask_words) mask[word] = held[h];
+  const unsigned in_half = (unsigned)__popc(held), upto = wave_inclusive_scan(in_half);
+  if (lane < 2u * R) {
+    if (RAGGED) bits[2 * R * wv + lane] = held;
+    pre[2 * R * wv + lane] = (uint16_t)(upto - in_half);
+    if (!RAGGED && mine / 32 + lane < g.tail) mask[mine / 32 + lane] = held;
   }
-  if (lane == 0) s_cnt[wv] = cnt;
+  if (RAGGED && wv == W - 1) {
+    const unsigned long long m = __ballot(behind != 0.0f);
+    if (lane == 0) {
+      bits[kHalves] = (uint32_t)m;
+      bits[kHalves + 1] = (uint32_t)(m >> 32);
+    }
+  }
+  if (lane == 63) s_cnt[wv] = upto;
+  if (wv == 0 && lane == 0) s_head[0] = (magic != kWsMagic || flag != 0u) ? 1u : 0u;
   __syncthreads();
   const bool refused = s_head[0] != 0u;
-  if (!kCountsItself && refused) {  // nothing is published, nothing written but the result
-    if (w == 0 && threadIdx.x == 0) *nnz = -1;
+  if (may_fail && refused) {  // nothing is published, no value written
+    if (t == 0 && threadIdx.x == 0) *nnz = -1;
     return;
   }
-  const uint32_t runs0 = s_head[1];
-  uint32_t* mine_arr = counts + (runs0 & 1u) * kQGroupsMax;
-  const unsigned wave_cnt = lane < (unsigned)kQWaves ? s_cnt[lane] : 0u;
-  const unsigned wave_incl = wave_inclusive_scan(wave_cnt);
-  const unsigned group_total = (unsigned)__builtin_amdgcn_readlane((int)wave_incl, kQWaves - 1);
-  const unsigned woff = (unsigned)__builtin_amdgcn_readlane((int)(wave_incl - wave_cnt), wv);
-  if (!refused && threadIdx.x == 0) {
-    st_status(&counts[((runs0 & 1u) ^ 1u) * kQGroupsMax + w], 0u);
-    if (!(skip_first && w == 0)) st_status(&mine_arr[w], kTileReady | group_total);
-  }
+  const unsigned wave_cnt = lane < (unsigned)W ? s_cnt[lane] : 0u, wave_upto = wave_inclusive_scan(wave_cnt);
+  const unsigned total = (unsigned)__builtin_amdgcn_readlane((int)wave_upto, W - 1);
+  const unsigned before_wave = (unsigned)__builtin_amdgcn_readlane((int)(wave_upto - wave_cnt), wv);
+  if (wv == 1 && lane < (unsigned)W) s_before[lane] = wave_upto - wave_cnt;
+  const bool last_tile = t == g.tiles - 1;
 
-  // ---- wavefront 0 collects the counts of the workgroups before this one: lane l looks at workgroups 4l .. 4l+3
   bool gave_up = false;
   if (wv == 0) {
-    uint32_t v[4];
-    unsigned spins = 0;
-    for (;;) {
-      bool missing = false;
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int k = 4 * (int)lane + r;
-        v[r] = k < w ? ld_status(&mine_arr[k]) : kTileReady;
-        missing |= (v[r] & kTileReady) == 0u;
+    // ---- publish, and collect what is before me
+    const unsigned group = t / kGroupTiles, place = t % kGroupTiles;
+    uint32_t* const counts = ws + 16 + (size_t)group * (kGroupTiles * kCountWords);  // my group's
+    uint32_t* const totals = ws + 16 + kSmallCounts + (runs & 1u) * kSmallTotals;
+    uint32_t* const others = ws + 16 + kSmallCounts + ((runs & 1u) ^ 1u) * kSmallTotals;
+    const bool ends_group = place == kGroupTiles - 1, silent = skip_first && t == 0;
+    unsigned in_group = 0, groups_before = 0, spins = 0;
+    bool need_count = lane < place, need_total = lane < group;
+    bool counts_open = !refused;
+    if (!refused) {
+      if (lane == 0 && !silent) st_status(&counts[place * kCountWords], kTileReady | total);
+      if (last_tile)  // the other array, and the entries of this one that are no whole group's total
+        for (unsigned k = lane; k < (unsigned)kSmallTotals; k += 64) {
+          if (k % (1u << g.spread) != 0u || k >> g.spread >= (t + 1) / kGroupTiles) st_status(&totals[k], kTileReady);
+          st_status(&others[k], 0u);
+        }
+    }
+    while (!refused) {
+      uint32_t count = 0, group_total = 0;
+      if (need_count) count = ld_status(&counts[lane * kCountWords]);
+      if (need_total) group_total = ld_status(&totals[lane << g.spread]);
+      if (count & kTileReady) {
+        in_group = count & (kTileThrough - 1u);
+        need_count = false;
       }
-      if (__ballot(missing) == 0ull && !refused) break;
-      if (refused || ++spins > spin_limit) {
-        if (!refused && (!kCountsItself || w == G - 1) && lane == 0) atomicOr(&ws[kWsFlag], 1u);
+      if (group_total & kTileReady) {
+        groups_before = group_total & ~kTileReady;
+        need_total = false;
+      }
+      if (counts_open && __ballot(need_count) == 0ull) {
+        counts_open = false;
+        if (ends_group) {
+          const unsigned sum = (unsigned)__builtin_amdgcn_readlane((int)wave_inclusive_scan(in_group), 63);
+          if (lane == 0) st_status(&totals[group << g.spread], kTileReady | (sum + total));
+        }
+      }
+      if (!counts_open && __ballot(need_total) == 0ull) break;
+      spins++;
+      if (spins > spin_limit || (spins % kFlagEvery == 0 && ld_status(&ws[kWsFlag]) != 0u)) {
+        if (lane == 0) atomicOr(&ws[kWsFlag], 1u);
         gave_up = true;
         break;
       }
-      __builtin_amdgcn_s_sleep(2);
+      __builtin_amdgcn_s_sleep(1);
     }
-    unsigned c[4], lane_sum = 0;
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      c[r] = v[r] & ~kTileReady;
-      lane_sum += c[r];
-    }
-    const unsigned incl = wave_inclusive_scan(lane_sum);
-    // counts of the workgroups before mine: whole lanes below lane w/4, and the first w%4 of that lane
-    unsigned part = incl - lane_sum;
-#pragma unroll
-    for (int r = 0; r < 3; r++) part += r < (w & 3) ? c[r] : 0u;
-    const unsigned before_me = (unsigned)__builtin_amdgcn_readlane((int)part, w >> 2);
-    const unsigned total = (unsigned)__builtin_amdgcn_readlane((int)incl, 63) + group_total;  // the last workgroup's is the tensor's
+    if (refused) gave_up = true;
+    if (!gave_up && lane == 0 && !silent) st_status(&counts[place * kCountWords], kTileReady | kTileThrough | total);
+    const unsigned before = (unsigned)__builtin_amdgcn_readlane((int)wave_inclusive_scan(in_group + groups_before), 63);
     if (lane == 0) {
-      // whatever the words held: what this workgroup writes stays inside the tensor
-      s_head[2] = min(before_me, (unsigned)g.n - group_total);
-      s_head[3] = total;
-      s_head[4] = gave_up ? 1u : 0u;
+      s_head[1] = min(before, g.n - total);  // whatever the words held: what this workgroup writes stays inside the tensor
+      s_head[2] = gave_up ? 1u : 0u;
+      if (may_fail && last_tile) s_head[3] = ld_status(&ws[kWsFlag]);
     }
+  } else {
+    // ---- meanwhile the mask words that start in my tile, and my share of those that hold no element
+    if (RAGGED) {
+      const unsigned c0 = div31(first, g.by_E), c1 = div31(end, g.by_E);
+      const unsigned from = c0 * g.W + (first - c0 * g.E + 31u) / 32u;
+      const unsigned stop = end == g.n ? g.tail : c1 * g.W + (end - c1 * g.E + 31u) / 32u;
+      for (unsigned f = from + threadIdx.x - 64u; f < stop; f += 64u * (W - 1)) {
+        const unsigned c = div31(f, g.by_W), e = c * g.E + 32u * (f - c * g.W), at = e - first;
+        const unsigned len = min(c * g.E + g.E, g.n) - e;  // elements of the chunk from here on
+        uint32_t w = __builtin_amdgcn_alignbit(bits[at / 32u + 1], bits[at / 32u], at & 31u);
+        if (len < 32u) w &= (1u << len) - 1u;
+        mask[f] = w;
+      }
+    }
+    for (unsigned f = g.tail + t * 64u * (W - 1) + threadIdx.x - 64u; f < g.mask_words; f += g.tiles * 64u * (W - 1)) mask[f] = 0;
   }
   __syncthreads();
-  if (kCountsItself && s_head[4] != 0u) {
-    const unsigned half = 2u * (unsigned)(w * kQWaves * R);  // my workgroup's first half row
-    const unsigned c = (unsigned)(((unsigned long long)half * w_magic) >> 40);
-    const unsigned long long from = (unsigned long long)(unsigned)g.E * c + min(32u * (half - c * (unsigned)g.W), (unsigned)g.E);
-    const unsigned end = (unsigned)(from < (unsigned long long)g.n ? from : (unsigned long long)g.n);
-    int before = 0;
-    for (unsigned i = threadIdx.x; i < end; i += 64 * kQWaves) before += in[i] != 0.0f;
-    before = wave_sum(before);
-    if (lane == 0) s_cnt[wv] = (unsigned)before;  // woff and group_total have been taken out of it
+  unsigned offset = s_head[1];
+  const bool counts_itself = !may_fail && s_head[2] != 0u;
+  if (counts_itself) {
+    unsigned before = 0;
+    for (unsigned i = threadIdx.x; i < first; i += 64u * W) before += in[i] != 0.0f;
+    before = (unsigned)wave_sum((int)before);
+    if (lane == 0) s_cnt[wv] = before;  // what was in it has been taken out
     __syncthreads();
-    if (threadIdx.x == 0) {
-      unsigned sum = 0;
-      for (int v = 0; v < kQWaves; v++) sum += s_cnt[v];
-      s_head[2] = sum;
-      s_head[3] = sum + group_total;
-    }
-    __syncthreads();
-    gave_up = false;
+    offset = 0;
+    for (int k = 0; k < W; k++) offset += s_cnt[k];
   }
-  uint32_t flag_late = 0;
-  if (!kCountsItself && w == G - 1 && threadIdx.x == 0) flag_late = ld_status(&ws[kWsFlag]);  // asked for now, looked at when the rows are out
 
-  // ---- my non-zeros, row by row, straight from the lanes that hold them; chunk starts on the way
-  unsigned at = s_head[2] + woff;
-#pragma unroll
-  for (int j = 0; j < R; j++) asm volatile("" : "+v"(x[j]));  // the ballots below are made again: two scalars per row would not last
-#pragma unroll
-  for (int h = 0; h < kHeld; h++) {
-    const unsigned in_word = (unsigned)__popc(held[h]);
-    const unsigned before = wave_inclusive_scan(in_word) - in_word;
-    const unsigned half = 2u * ((unsigned)r0 + 32u * h) + lane;
-    const unsigned c = (unsigned)(((unsigned long long)half * w_magic) >> 40);
-    if ((int)lane < 2 * (R - 32 * h) && c * (unsigned)g.W == half && (int)c < g.active)
-      begin[c] = (int)(at + before);
-#pragma unroll
-    for (int j = 32 * h; j < R && j < 32 * h + 32; j++) {
-      const float v = x[j];
-      const bool nz = v != 0.0f;
-      const unsigned long long m = __ballot(nz);
-      if (nz) values[at + rank_below(m)] = v;
-      at += popc64(m);
+  // ---- where the chunks that start in my tile start among the values
+  {
+    const unsigned c0 = div31(first + g.E - 1u, g.by_E), c1 = div31(end + g.E - 1u, g.by_E);
+    for (unsigned c = c0 + threadIdx.x; c < c1; c += 64u * W) {
+      const unsigned at = c * g.E - first, h = at / 32u, w = h / (2u * R);
+      unsigned o = offset + s_before[w] + pre[h];
+      if (RAGGED) o += (unsigned)__popc(bits[h] & ((1u << (at & 31u)) - 1u));
+      begin[c] = (int)o;
     }
+  }
+  // ---- the counts that I clear, if I clear any: asked for now, looked at when my rows are out
+  const unsigned group = t / kGroupTiles, groups = (g.tiles + kGroupTiles - 1) / kGroupTiles;
+  const bool clears = wv == 0 && !gave_up && (last_tile || ((t + 1) % kGroupTiles == 0 && group >= 2 && group + 1 < groups));
+  const unsigned clear_at = (group < 2 ? 0u : group - 2u) * kGroupTiles + lane;
+  const unsigned clear_end = last_tile ? g.tiles : (group < 2 ? 0u : group - 1u) * kGroupTiles;
+  uint32_t* const clear = ws + 16 + (size_t)clear_at * kCountWords;
+  uint32_t through[3] = {kTileThrough, kTileThrough, kTileThrough};
+  auto ask = [&] {
+#pragma unroll
+    for (unsigned k = 0; k < 3; k++)
+      if (clear_at + k * kGroupTiles < clear_end) through[k] = ld_status(clear + (size_t)k * kGroupTiles * kCountWords);
+  };
+  if (clears) ask();
+  // ---- my non-zeros, row by row, straight from the lanes that hold them
+  float* const out = values + (offset + before_wave);
+  unsigned at = 0;
+#pragma unroll
+  for (int j = 0; j < R; j++) {
+    asm volatile("" : "+v"(x[j]));
+    const bool nz = x[j] != 0.0f;
+    const unsigned long long m = __ballot(nz);
+    const unsigned slot = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, at));
+    if (nz) *reinterpret_cast<float*>(reinterpret_cast<char*>(out) + (size_t)(4u * slot)) = x[j];
+    at += popc64(m);
+  }
+
+  if (clears) {
+    for (unsigned spins = 0; __ballot((through[0] & through[1] & through[2] & kTileThrough) == 0u) != 0ull; spins++) {
+      if (spins > spin_limit || (spins % kFlagEvery == kFlagEvery - 1 && ld_status(&ws[kWsFlag]) != 0u)) {
+        if (lane == 0) atomicOr(&ws[kWsFlag], 1u);
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+      ask();
+    }
+#pragma unroll
+    for (unsigned k = 0; k < 3; k++)
+      if (clear_at + k * kGroupTiles < clear_end) st_status(clear + (size_t)k * kGroupTiles * kCountWords, 0u);
   }
 
   // ---- the result
-  if (w == G - 1 && threadIdx.x == 0) {
-    *nnz = (gave_up || flag_late != 0u) ? -1 : (int)s_head[3];
+  if (last_tile && threadIdx.x == 0) {
+    const bool failed = may_fail && (gave_up || s_head[3] != 0u);
+    *nnz = failed ? -1 : (int)(offset + total);
     __threadfence();
-    if (!refused && !(kCountsItself && s_head[4] != 0u)) __hip_atomic_fetch_add(&ws[kWsSmallRuns], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  } else if (gave_up && w != G - 1) {  // (wavefront 0 of another workgroup) after the last workgroup has spoken
-    for (unsigned spins = 0; ld_status(&ws[kWsSmallRuns]) == runs0 && spins < spin_limit; spins++)
-      __builtin_amdgcn_s_sleep(2);
+    if (!refused && !counts_itself) __hip_atomic_fetch_add(&ws[kWsSmallRuns], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  } else if (may_fail && gave_up && !last_tile) {  // (wavefront 0 of another workgroup) after the last workgroup has spoken
+    for (unsigned spins = 0; ld_status(&ws[kWsSmallRuns]) == runs && spins < spin_limit; spins++) __builtin_amdgcn_s_sleep(2);
     if (lane == 0) *nnz = -1;
   }
 }
@@ -1485,42 +1532,38 @@ static bool single_pass_shape(const Geometry& g, int n, int process, StreamGeome
          device_compute_units() > 1 && 4ull * (unsigned long long)n >= g_single_pass_bytes;
 }
 
-// Whether the one-kernel form for small tensors takes this shape (a tensor below the size from
-// which the pipeline kernel runs, all of it in the registers of one grid, whole half rows per
-// chunk unless `any`); fills the geometry, the grid and the rows per wavefront.
-// `any`: also the shapes of the form's variants that cannot fail (zvc_small_kernel: kCountsItself),
-// chunks of any length and up to 64 rows per wavefront; a caller that has to know beforehand
-// whether the workspace decides about success (cswap_zvc_takes_single_pass) leaves those out.
-static bool small_pass_shape(const Geometry& g, int n, int process, StreamGeometry& sg, int* groups, int* rows_per_wave,
-                             bool any)
+// Whether the one-kernel form for small tensors takes this shape: a tensor below the size from which the pipeline
+// kernel runs, in at most kGroupsMax groups of its largest tiles.  Fills the geometry but for its tiles.
+static bool small_pass_shape(const Geometry& g, int n, SmallGeometry& sg)
 {
-  sg.n = n; sg.E = g.E; sg.W = g.W; sg.process = process; sg.active = g.active;
-  const long long mask_words = (long long)g.W * process;
-  sg.mask_words = (int)mask_words;
-  sg.rows = (int)((mask_words + 1) / 2);
-  sg.tiles = sg.status_at = sg.offset_at = 0;
-  const int cus = device_compute_units();
-  const int G = cus < kQGroupsMax ? cus : kQGroupsMax;
   const unsigned long long single_from = g_single_pass_bytes.load();
-  if (G < 1 || (!any && g.E % 32 != 0) || mask_words >= (1ll << 31) - 64 || single_from == ~0ull || 4ull * (unsigned long long)n >= single_from) return false;
-  // every row of the mask layout has an owner, also the rows of chunks that hold no data (their words are zero)
-  const int most = any ? 64 : 32;
-  int R = 8;
-  while (R <= most && (long long)G * kQWaves * R < (long long)sg.rows) R *= 2;
-  if (R > most) return false;
-  *groups = G;
-  *rows_per_wave = R;
+  const long long mask_words = (long long)g.W * g.process;
+  if (single_from == ~0ull || 4ull * (unsigned long long)n >= single_from || n > (int)(kGroupsMax * kGroupTiles * 64 * 8 * 32) || mask_words >= (1ll << 31) - 64) return false;
+  sg.n = (unsigned)n; sg.E = (unsigned)g.E; sg.W = (unsigned)g.W; sg.process = (unsigned)g.process;
+  sg.mask_words = (unsigned)mask_words;
+  const unsigned in_last = (unsigned)(n - (long long)(g.active - 1) * g.E);  // elements of the last chunk that has any
+  sg.tail = (unsigned)(g.active - 1) * sg.W + (in_last + 31u) / 32u;
+  sg.by_E = make_div31(sg.E);
+  sg.by_W = make_div31(sg.W);
   return true;
+}
+// Whether a run of it reports failure where the workspace fails it (zvc_small_kernel: may_fail): whole half rows per
+// chunk, at most 131072 rows of the mask layout on a part of 256 compute units.
+static bool small_pass_may_fail(const Geometry& g)
+{
+  const int cus = device_compute_units();
+  const long long rows = ((long long)g.W * g.process + 1) / 2;
+  return g.E % 32 == 0 && cus > 0 && rows <= (long long)(cus < 256 ? cus : 256) * 512;
 }
 
 extern "C" int cswap_zvc_takes_single_pass(int n, int process)
 {
   Geometry g;
   StreamGeometry sg;
-  int groups, rows;
+  SmallGeometry small;
   if (make_geometry(g, n, process) != CSWAP_OK) return 0;
   if (single_pass_shape(g, n, process, sg)) return 1;
-  return small_pass_shape(g, n, process, sg, &groups, &rows, false) ? 2 : 0;
+  return small_pass_shape(g, n, small) && small_pass_may_fail(g) ? 2 : 0;
 }
 
 extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, void* d_ws, int* d_begin,
@@ -1535,18 +1578,31 @@ extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, v
   StreamGeometry sg;
   // what neither one-kernel form takes runs the three kernels (the pipeline needs a 16-byte aligned output, too)
   const bool single_pass = single_pass_shape(g, n, process, sg) && (reinterpret_cast<uintptr_t>(d_values) & 15u) == 0;
-  int groups = 0, rows = 0;
-  if (!single_pass && small_pass_shape(g, n, process, sg, &groups, &rows, true)) {
-    uint32_t* counts = ws + 16 + kSmallCounts;
-#define CSWAP_SMALL(R, RAGGED)                                                                                     \
-  hipLaunchKernelGGL((zvc_small_kernel<R, RAGGED>), dim3(groups), dim3(64 * kQWaves), 0, (hipStream_t)stream, d_in, \
-                     sg, ws, counts, d_begin, d_nnz, d_values, d_mask, g_spin_limit.load(), g_skip_first.load())
-    const bool ragged = g.E % 32 != 0;
-    if (rows == 8) { if (ragged) CSWAP_SMALL(8, true); else CSWAP_SMALL(8, false); }
-    else if (rows == 16) { if (ragged) CSWAP_SMALL(16, true); else CSWAP_SMALL(16, false); }
-    else if (rows == 32) { if (ragged) CSWAP_SMALL(32, true); else CSWAP_SMALL(32, false); }
-    else { if (ragged) CSWAP_SMALL(64, true); else CSWAP_SMALL(64, false); }
+  SmallGeometry small;
+  if (!single_pass && small_pass_shape(g, n, small)) {
+    const int may_fail = small_pass_may_fail(g) ? 1 : 0;
+#define CSWAP_SMALL_AS(W, R, RAGGED)                                                                                \
+  hipLaunchKernelGGL((zvc_small_kernel<W, R, RAGGED>), dim3(small.tiles), dim3(64 * W), 0, (hipStream_t)stream, d_in, small, ws, \
+                     d_begin, d_nnz, d_values, d_mask, may_fail, g_spin_limit.load(), g_skip_first.load())
+#define CSWAP_SMALL(W, R)                                       \
+  do {                                                          \
+    small.tiles = ((unsigned)n + 64 * W * R - 1) / (64 * W * R); \
+    if (small.tiles > kGroupsMax * kGroupTiles) return CSWAP_E_ARG; \
+    small.spread = 2; \
+    while (small.spread < 7 && (small.tiles + kGroupTiles - 1) / kGroupTiles <= (unsigned)kSmallTotals >> (small.spread + 1)) small.spread++; \
+    if (g.E % 32 != 0) CSWAP_SMALL_AS(W, R, true);              \
+    else CSWAP_SMALL_AS(W, R, false);                           \
+  } while (0)
+    // The tile by size, us for the compaction alone / with the expansion behind it, tiles of 16 x 8 rows : 16 x 16 : 8 x 32: 1 MB 4.8 : 5.5 :
+    // 6.2 / 9.4 : 10.1 : 10.5 · 4.2 MB 5.8 : 6.2 : 6.9 / 11.1 : 11.2 : 11.6 · 8.4 MB 6.3 : 6.6 : 7.2 / 12.9 : 13.4 : 13.8 · 16.8 MB 8.2 : 8.1 : 8.8 /
+    // 17.7 : 16.7 : 17.5 · 33.6 MB 16.8 : 12.4 : 12.7 / 26.4 : 23.6 : 24.2 · 50 MB 22.3 : 19.3 : 17.3 / 35.8 : 33.0 : 31.0.  Small tiles while each has a compute
+    // unit to itself; then those of sixteen wavefronts while two on every compute unit hold the tensor, then
+    // those of eight with twice the rows, four to a compute unit.
+    if (n <= 256 * 64 * 16 * 8) CSWAP_SMALL(16, 8);
+    else if (n <= 512 * 64 * 16 * 16) CSWAP_SMALL(16, 16);
+    else CSWAP_SMALL(8, 32);
 #undef CSWAP_SMALL
+#undef CSWAP_SMALL_AS
     return check_launch();
   }
   if (!single_pass) return cswap_zvc_compress(d_in, n, process, d_begin, d_nnz, d_values, d_mask, stream);

@@ -184,9 +184,8 @@ int cswap_zvc_compress(const float* d_in, int n, int process, int* d_begin, int*
  * write mask, offsets and packed values, so HBM traffic is the algorithmic
  * 4 + 1/8 + 4*density bytes per element.  Smaller tensors than
  * cswap_zvc_set_single_pass_bytes says (64 MiB) do not fill that pipeline; they run
- * another one-kernel form -- the whole tensor in the registers of one grid, every
- * workgroup reads the counts of the workgroups before it -- while their mask layout
- * has at most 262144 rows of 64 elements (64 MiB).  d_ws is a
+ * another one-kernel form: the whole tensor in the registers of one grid, and every
+ * workgroup reads the counts of the workgroups before it.  d_ws is a
  * workspace of cswap_zvc_workspace_bytes(process) bytes (at least 256 KiB) that
  * cswap_zvc_workspace_clear has prepared once, after it was allocated; every call
  * that succeeds leaves it ready for the next one (the kernel clears each status
@@ -223,7 +222,7 @@ int cswap_zvc_workspace_clear(void* d_ws, int process, cswap_stream_t stream);
  * d_values): 1 the pipeline kernel, 2 the one-kernel form for small tensors (chunk
  * lengths that are multiples of 32, at most 131072 rows of 64 elements, 32 MiB), 0 a
  * form that does not need the workspace to succeed: the three kernels, or the small
- * form of tensors of other chunk lengths and of up to 262144 rows, whose workgroups
+ * form of tensors of other chunk lengths or more rows, whose workgroups
  * count for themselves where the workspace fails them.  Host only. */
 int cswap_zvc_takes_single_pass(int n, int process);
 /* No counterpart in the reference: the tensor size in bytes from which

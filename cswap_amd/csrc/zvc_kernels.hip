@@ -1006,7 +1006,7 @@ __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
 }
 
 // ------------------------------------------------------------------ one kernel for small tensors
-// Below 64 MiB the whole tensor fits in the registers of one grid.  It is cut into at most 512 tiles of consecutive
+// Below 64 MiB the whole tensor fits in the registers of one grid.  It is cut into tiles of consecutive
 // elements, a workgroup each: W wavefronts of R rows of 64 elements.  A workgroup loads its tile, counts it,
 // publishes the count, reads the counts of the workgroups before it (one trip through memory), takes their sum as
 // its offset and stores its non-zeros straight from the registers (at these sizes the values array stays in the
@@ -1532,13 +1532,15 @@ static bool single_pass_shape(const Geometry& g, int n, int process, StreamGeome
          device_compute_units() > 1 && 4ull * (unsigned long long)n >= g_single_pass_bytes;
 }
 
-// Whether the one-kernel form for small tensors takes this shape: a tensor below the size from which the pipeline
-// kernel runs, in at most kGroupsMax groups of its largest tiles.  Fills the geometry but for its tiles.
+// Whether the one-kernel form for small tensors takes a shape that the pipeline kernel does not: up to kGroupsMax groups of its
+// largest tiles, 256 MiB.  Chunks of any length from 64 MiB on, three kernels -> this form, us alone / on tensors in turn / with the
+// expansion behind it: 68 MB 35.9 -> 22.5 / 42.2 -> 30.3 / 53.8 -> 40.4, 120 MB 54.2 -> 34.9 / 64.3 -> 44.3 / 87.2 -> 71.6, 241 MB 102.9 -> 85.9 /
+// 113 -> 85 / 183 -> 146.  Whole half rows stay with the pipeline there, 241 MB of which take 73.  Fills the geometry but for its tiles.
 static bool small_pass_shape(const Geometry& g, int n, SmallGeometry& sg)
 {
   const unsigned long long single_from = g_single_pass_bytes.load();
   const long long mask_words = (long long)g.W * g.process;
-  if (single_from == ~0ull || 4ull * (unsigned long long)n >= single_from || n > (int)(kGroupsMax * kGroupTiles * 64 * 8 * 32) || mask_words >= (1ll << 31) - 64) return false;
+  if (single_from == 0 || single_from == ~0ull || n > (int)(kGroupsMax * kGroupTiles * 64 * 8 * 32) || mask_words >= (1ll << 31) - 64) return false;
   sg.n = (unsigned)n; sg.E = (unsigned)g.E; sg.W = (unsigned)g.W; sg.process = (unsigned)g.process;
   sg.mask_words = (unsigned)mask_words;
   const unsigned in_last = (unsigned)(n - (long long)(g.active - 1) * g.E);  // elements of the last chunk that has any
@@ -1580,7 +1582,7 @@ extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, v
   const bool single_pass = single_pass_shape(g, n, process, sg) && (reinterpret_cast<uintptr_t>(d_values) & 15u) == 0;
   SmallGeometry small;
   if (!single_pass && small_pass_shape(g, n, small)) {
-    const int may_fail = small_pass_may_fail(g) ? 1 : 0;
+    const int may_fail = small_pass_may_fail(g) && 4ull * (unsigned long long)n < g_single_pass_bytes.load() ? 1 : 0;
 #define CSWAP_SMALL_AS(W, R, RAGGED)                                                                                \
   hipLaunchKernelGGL((zvc_small_kernel<W, R, RAGGED>), dim3(small.tiles), dim3(64 * W), 0, (hipStream_t)stream, d_in, small, ws, \
                      d_begin, d_nnz, d_values, d_mask, may_fail, g_spin_limit.load(), g_skip_first.load())
@@ -1597,7 +1599,7 @@ extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, v
     // 6.2 / 9.4 : 10.1 : 10.5 · 4.2 MB 5.8 : 6.2 : 6.9 / 11.1 : 11.2 : 11.6 · 8.4 MB 6.3 : 6.6 : 7.2 / 12.9 : 13.4 : 13.8 · 16.8 MB 8.2 : 8.1 : 8.8 /
     // 17.7 : 16.7 : 17.5 · 33.6 MB 16.8 : 12.4 : 12.7 / 26.4 : 23.6 : 24.2 · 50 MB 22.3 : 19.3 : 17.3 / 35.8 : 33.0 : 31.0.  Small tiles while each has a compute
     // unit to itself; then those of sixteen wavefronts while two on every compute unit hold the tensor, then
-    // those of eight with twice the rows, four to a compute unit.
+    // those of eight with twice the rows, four to a compute unit: all of them at once up to 64 MiB.
     if (n <= 256 * 64 * 16 * 8) CSWAP_SMALL(16, 8);
     else if (n <= 512 * 64 * 16 * 16) CSWAP_SMALL(16, 16);
     else CSWAP_SMALL(8, 32);

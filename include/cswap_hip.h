@@ -184,8 +184,9 @@ int cswap_zvc_compress(const float* d_in, int n, int process, int* d_begin, int*
  * write mask, offsets and packed values, so HBM traffic is the algorithmic
  * 4 + 1/8 + 4*density bytes per element.  Smaller tensors than
  * cswap_zvc_set_single_pass_bytes says (64 MiB) do not fill that pipeline; they run
- * another one-kernel form: the whole tensor in the registers of one grid, and every
- * workgroup reads the counts of the workgroups before it.  d_ws is a
+ * another one-kernel form: the tensor in the registers of one grid, and every
+ * workgroup reads the counts of the workgroups before it.  So do, up to 256 MiB, larger
+ * ones that the pipeline does not take (unless that size is set to 0).  d_ws is a
  * workspace of cswap_zvc_workspace_bytes(process) bytes (at least 256 KiB) that
  * cswap_zvc_workspace_clear has prepared once, after it was allocated; every call
  * that succeeds leaves it ready for the next one (the kernel clears each status
@@ -194,7 +195,7 @@ int cswap_zvc_compress(const float* d_in, int n, int process, int* d_begin, int*
  * workspace must not overlap.  Shapes the one-kernel forms do not take -- for the
  * pipeline a chunk length that is not a multiple of 32, d_values not 16-byte
  * aligned or more tiles of 12288 elements than the workspace has room for (32512, more with
- * `process` above 65536) -- run the three kernels instead.  The workgroups
+ * `process` above 65536) and more than 256 MiB -- run the three kernels instead.  The workgroups
  * wait for each other's counts; that wait is bounded, and if it ever runs out (for
  * example because the pipeline kernel, whose 256 workgroups all have to run at the
  * same time, does not get the whole GPU) the kernel still finishes

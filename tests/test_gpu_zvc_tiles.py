@@ -1,15 +1,16 @@
-"""The one-kernel compaction of small tensors where its tiles and its groups of 64 tiles begin and end, against the
-three kernels: values, mask, offsets and count, three runs on one workspace with other data in each."""
+"""The one-kernel compaction of small tensors, and of larger ones in chunks that are no whole half rows, where its tiles
+and its groups of 64 tiles begin and end, against the three kernels: values, mask, offsets and count, three runs on one
+workspace with other data in each."""
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 KB = 1024
-# tiles of 8192 elements up to 2 M elements, of 16384 above; whole half rows per chunk, and any length
+# tiles of 8192 elements up to 2 M elements, of 16384 above, 4096 of them at most; whole half rows per chunk, and any length
 SHAPES = [(1, 1), (8191, 16), (8192, 256), (8193, 7), (64 * 8192, 1024), (64 * 8192 + 1, 1024), (65 * 8192 - 5, 333),
           (128 * 8192, 4096), (129 * 8192 + 31, 16384), (192 * 8192 + 1, 50), (2048 * KB, 2048), (2048 * KB + 1, 2048),
           (2048 * KB + 64, 2049), (64 * 16384 * 3 - 1, 16384), (8192 * KB, 16384), (8192 * KB + 1, 8192), (8192 * KB + 16384, 16383),
-          (16384 * KB - 1, 16384), (3_000_000, 1), (3_000_001, 65536), (700_000, 700_000)]
+          (16384 * KB - 1, 16384), (16384 * KB + 1, 16384), (30_105_600, 16384), (65536 * KB - 49157, 16384), (3_000_000, 1), (3_000_001, 65536), (700_000, 700_000)]
 
 
 @pytest.mark.parametrize("n,process", SHAPES)
@@ -42,3 +43,23 @@ def test_tiles_against_three_kernels(n, process):
         assert int(words[16:].count_nonzero().item()) == 256  # the totals of the last run, nothing else
     finally:
         L.cswap_zvc_set_single_pass_bytes(before)
+
+
+def test_more_than_the_groups_hold_runs_the_three_kernels():
+    import torch
+
+    from cswap_amd import api
+    from cswap_amd._lib import check, lib
+
+    n, process = 65536 * KB + 1, 16384
+    L = lib()
+    x = torch.randn(n, device="cuda").clamp_(min=0.0)
+    want = api.zvc_compress(x, process)
+    got = [torch.zeros_like(o) for o in want]
+    ws = api.zvc_workspace(process)
+    check(L.cswap_zvc_compress_fused(x.data_ptr(), n, process, ws.data_ptr(), got[2].data_ptr(), got[3].data_ptr(),
+                                     got[0].data_ptr(), got[1].data_ptr(), None), "fused")
+    torch.cuda.synchronize()
+    k = int(want[3].item())
+    assert int(got[3].item()) == k and torch.equal(got[0][:k], want[0][:k]) and torch.equal(got[1], want[1])
+    assert int(ws.view(torch.int32)[4].item()) == 0

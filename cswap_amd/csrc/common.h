@@ -24,6 +24,9 @@ int zfp_compress_f32_no_quad(const float* d_in, size_t nx, size_t ny, size_t nz,
 int zfp_decompress_f32_no_quad(const uint64_t* d_stream, size_t nx, size_t ny, size_t nz, unsigned maxbits, float* d_out,
                                hipStream_t stream);
 
+// Whether cswap_zvc_compress_fused runs one kernel for a shape that cswap_zvc_takes_single_pass says 0 for: one that cannot fail.
+bool zvc_small_any_chunk(int n, int process);
+
 // Whether a ZVC payload of `bytes` that is already made is worth sending: by the selector's model, what a
 // tensor of n elements has left to pay for it (link and expansion) against the raw swap.
 bool made_payload_pays(size_t n, size_t bytes, const cswap_costs& costs);

@@ -442,6 +442,10 @@ static int probe_tensor(cswap_engine* e, Ticket& t, const float* d_in, hipStream
   return CSWAP_OK;
 }
 
+// The selector's probe is the compaction itself where that costs no more than counting and scanning: the small form up to
+// this size, in whole half rows (cswap_zvc_takes_single_pass: 2) or in chunks of any length.
+constexpr size_t kProbeBySmallFormUpTo = (size_t)32 << 20;
+
 // An explicit ZVC request for a tensor that one of the single-kernel forms takes: count, scan and
 // compaction in one pass over the tensor, straight into a staging block of the worst-case size that is cut back to what was
 // needed once the non-zero count is on the host (the same small round trip a probe makes).
@@ -454,7 +458,9 @@ static int single_pass_sparse(cswap_engine* e, Ticket& t, const float* d_in, hip
 {
   if (t.process > kWsProcess) return 1;
   const int form = cswap_zvc_takes_single_pass((int)t.n, t.process);
-  if (form == 0 || (small_form_only && form != 2)) return 1;
+  const bool any_chunk = form == 0 && cswap::zvc_small_any_chunk((int)t.n, t.process);
+  if (form == 0 && !any_chunk) return 1;
+  if (small_form_only && form != 2 && !(any_chunk && 4 * t.n <= kProbeBySmallFormUpTo)) return 1;
   const size_t hdr = zvc_header_bytes((int)t.n, t.process);
   const size_t worst = hdr + 4 * t.n;
   size_t off;

@@ -1568,6 +1568,13 @@ extern "C" int cswap_zvc_takes_single_pass(int n, int process)
   return small_pass_shape(g, n, small) && small_pass_may_fail(g) ? 2 : 0;
 }
 
+bool cswap::zvc_small_any_chunk(int n, int process)
+{
+  Geometry g;
+  SmallGeometry small;
+  return make_geometry(g, n, process) == CSWAP_OK && cswap_zvc_takes_single_pass(n, process) == 0 && small_pass_shape(g, n, small);
+}
+
 extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, void* d_ws, int* d_begin,
                                         int* d_nnz, float* d_values, uint32_t* d_mask, cswap_stream_t stream)
 {

@@ -386,7 +386,7 @@ void cswap_engine_destroy(cswap_engine* e);
  * compression by an event.  The tensor is the field a[nz][ny][nx].
  * The probe of an AUTO request is the counting pass of the compactor, whose per-chunk
  * counts the compaction then reuses (Execution.h:89-95); for tensors small enough for the
- * one-kernel form of the compactor (cswap_zvc_takes_single_pass == 2, up to 32 MiB) it is
+ * one-kernel form of the compactor (up to 32 MiB, chunks of any length) it is
  * that kernel itself, into a staging block of the worst-case size when the pool has one
  * to spare: a tensor that turns out sparse is compacted by the time its count is known.
  * Calls that probe hold the engine's lock over the host round trip (about 20 us): two

@@ -81,6 +81,19 @@ __device__ __forceinline__ void st_row4(float* p, float4 v)
   }
 }
 
+// A tensor's elements as the single-pass kernels read them, each of them once.  ONCE: with the nontemporal hint, which leaves the
+// memory-side cache (256 MB) to the values that go out and to what other kernels have there.  Tensors of kReadOnceFrom bytes and more: below
+// that the next reader of the tensor itself, the layer that it is the input of, finds it evicted.  Plain loads -> hint, us, tensors in turn:
+// compaction and expansion (half zeros) 67 MB 49.4 -> 50.6, 100 MB 70.1 -> 67.0, 201 MB 133.8 -> 119.0, 268 MB 169.5 -> 163.3, odd chunks 89 MB 61.4 -> 57.2,
+// 180 MB 125.3 -> 117.4; producer, compaction and a reader behind it 60 MB 60.6 -> 64.6, 89 MB 90.2 -> 90.3, 134 MB 137.6 -> 132.9, 241 MB 247 -> 233.
+// The same tensor over and over, which the cache holds up to its size, loses: 120 MB 36.3 -> 40.7 by itself (45.4 -> 43.2 in turn).
+constexpr unsigned long long kReadOnceFrom = 80ull << 20;
+template <bool ONCE>
+__device__ __forceinline__ float ld_once(const float* p)
+{
+  return ONCE ? __builtin_nontemporal_load(p) : *p;
+}
+
 struct Geometry {
   int n;        // elements
   int E;        // elements per chunk
@@ -777,7 +790,10 @@ __device__ void zvc_stream_scanner(uint32_t* ws, const StreamGeometry& g, int st
   }
 }
 
-template <bool HINT>
+// HINT: the values leave with the nontemporal hint, from 5/3 of the size from which the three kernels' compaction is staged on (320 MiB).  Below,
+// whoever reads them next finds them in the memory-side cache: compaction and expansion of 201 MB 133.8 -> 119.0 us and of 268 MB 169.5 -> 147.5 over
+// one tensor and -> 163.3 in turn, the compaction alone 87.8 and 88.2; 537 MB with the hint 317, without 327.
+template <bool ONCE, bool HINT>
 __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
     const float* __restrict__ in, StreamGeometry g, uint32_t* __restrict__ ws, int* __restrict__ begin,
     int* __restrict__ nnz, float* __restrict__ values, uint32_t* __restrict__ mask, unsigned spin_limit,
@@ -896,7 +912,7 @@ __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
       rows_of(w + k * G, base, exist);
       have[k] = exist;
 #pragma unroll
-      for (int j = 0; j < kSRows; j++) x[k][j] = base[min(lane + 64u * j, (unsigned)max(exist - 1, 0))];
+      for (int j = 0; j < kSRows; j++) x[k][j] = ld_once<ONCE>(base + min(lane + 64u * j, (unsigned)max(exist - 1, 0)));
     }
   }
 #pragma unroll
@@ -957,7 +973,7 @@ __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
             at += popc64(m);
             if (lane == 2u * j) held = (uint32_t)m;
             if (lane == 2u * j + 1u) held = (uint32_t)(m >> 32);
-            x[(s + kSAhead) % kSSlots][j] = base[lane + 64u * j];
+            x[(s + kSAhead) % kSSlots][j] = ld_once<ONCE>(base + lane + 64u * j);
           }
         } else {
 #pragma unroll
@@ -971,7 +987,7 @@ __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
             at += popc64(m);
             if (lane == 2u * j) held = (uint32_t)m;
             if (lane == 2u * j + 1u) held = (uint32_t)(m >> 32);
-            x[(s + kSAhead) % kSSlots][j] = base[min(lane + 64u * j, last)];
+            x[(s + kSAhead) % kSSlots][j] = ld_once<ONCE>(base + min(lane + 64u * j, last));
           }
         }
         // lane k < 32 holds mask word k of my rows = half row 2*r0 + k; a chunk starts there
@@ -1068,7 +1084,7 @@ struct SmallGeometry {
 // old with lane `lane` replaced by the uniform v
 __device__ uint32_t write_lane(uint32_t v, uint32_t lane, uint32_t old) __asm("llvm.amdgcn.writelane.i32");
 
-template <int W, int R, bool RAGGED>
+template <int W, int R, bool RAGGED, bool ONCE>
 __global__ __launch_bounds__(64 * W, 8) void zvc_small_kernel(
     const float* __restrict__ in, SmallGeometry g, uint32_t* __restrict__ ws, int* __restrict__ begin, int* __restrict__ nnz,
     float* __restrict__ values, uint32_t* __restrict__ mask, int may_fail, unsigned spin_limit, unsigned skip_first)
@@ -1097,7 +1113,7 @@ __global__ __launch_bounds__(64 * W, 8) void zvc_small_kernel(
   const int left = mine < g.n ? (int)min(g.n - mine, 64u * R) : 0;  // elements that exist
   if (left == 64 * R) {
 #pragma unroll
-    for (int j = 0; j < R; j++) x[j] = in[mine + lane + 64u * j];
+    for (int j = 0; j < R; j++) x[j] = ld_once<ONCE>(in + (mine + lane + 64u * j));
   } else {  // what does not exist is read from an element that does, and is a zero from here on
     const float* base = in + (left > 0 ? mine : 0u);
     const unsigned last = (unsigned)max(left - 1, 0);
@@ -1590,26 +1606,27 @@ extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, v
   SmallGeometry small;
   if (!single_pass && small_pass_shape(g, n, small)) {
     const int may_fail = small_pass_may_fail(g) && 4ull * (unsigned long long)n < g_single_pass_bytes.load() ? 1 : 0;
-#define CSWAP_SMALL_AS(W, R, RAGGED)                                                                                \
-  hipLaunchKernelGGL((zvc_small_kernel<W, R, RAGGED>), dim3(small.tiles), dim3(64 * W), 0, (hipStream_t)stream, d_in, small, ws, \
+#define CSWAP_SMALL_AS(W, R, RAGGED, ONCE)                                                                          \
+  hipLaunchKernelGGL((zvc_small_kernel<W, R, RAGGED, ONCE>), dim3(small.tiles), dim3(64 * W), 0, (hipStream_t)stream, d_in, small, ws, \
                      d_begin, d_nnz, d_values, d_mask, may_fail, g_spin_limit.load(), g_skip_first.load())
-#define CSWAP_SMALL(W, R)                                       \
+#define CSWAP_SMALL(W, R, ONCE)                                 \
   do {                                                          \
     small.tiles = ((unsigned)n + 64 * W * R - 1) / (64 * W * R); \
     if (small.tiles > kGroupsMax * kGroupTiles) return CSWAP_E_ARG; \
     small.spread = 2; \
     while (small.spread < 7 && (small.tiles + kGroupTiles - 1) / kGroupTiles <= (unsigned)kSmallTotals >> (small.spread + 1)) small.spread++; \
-    if (g.E % 32 != 0) CSWAP_SMALL_AS(W, R, true);              \
-    else CSWAP_SMALL_AS(W, R, false);                           \
+    if (g.E % 32 != 0) CSWAP_SMALL_AS(W, R, true, ONCE);        \
+    else CSWAP_SMALL_AS(W, R, false, ONCE);                     \
   } while (0)
     // The tile by size, us for the compaction alone / with the expansion behind it, tiles of 16 x 8 rows : 16 x 16 : 8 x 32: 1 MB 4.8 : 5.5 :
     // 6.2 / 9.4 : 10.1 : 10.5 · 4.2 MB 5.8 : 6.2 : 6.9 / 11.1 : 11.2 : 11.6 · 8.4 MB 6.3 : 6.6 : 7.2 / 12.9 : 13.4 : 13.8 · 16.8 MB 8.2 : 8.1 : 8.8 /
     // 17.7 : 16.7 : 17.5 · 33.6 MB 16.8 : 12.4 : 12.7 / 26.4 : 23.6 : 24.2 · 50 MB 22.3 : 19.3 : 17.3 / 35.8 : 33.0 : 31.0.  Small tiles while each has a compute
     // unit to itself; then those of sixteen wavefronts while two on every compute unit hold the tensor, then
     // those of eight with twice the rows, four to a compute unit: all of them at once up to 64 MiB.
-    if (n <= 256 * 64 * 16 * 8) CSWAP_SMALL(16, 8);
-    else if (n <= 512 * 64 * 16 * 16) CSWAP_SMALL(16, 16);
-    else CSWAP_SMALL(8, 32);
+    if (n <= 256 * 64 * 16 * 8) CSWAP_SMALL(16, 8, false);
+    else if (n <= 512 * 64 * 16 * 16) CSWAP_SMALL(16, 16, false);
+    else if (4ull * (unsigned long long)n < kReadOnceFrom) CSWAP_SMALL(8, 32, false);
+    else CSWAP_SMALL(8, 32, true);
 #undef CSWAP_SMALL
 #undef CSWAP_SMALL_AS
     return check_launch();
@@ -1617,12 +1634,12 @@ extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, v
   if (!single_pass) return cswap_zvc_compress(d_in, n, process, d_begin, d_nnz, d_values, d_mask, stream);
   // one workgroup per compute unit, the last of them the scanner
   const int data_groups = stream_data_groups(sg.tiles, cus);
-  if (4ull * (unsigned long long)n >= g_staged_compact_bytes)
-    hipLaunchKernelGGL(zvc_stream_kernel<true>, dim3(data_groups + 1), dim3(64 * kSWaves), 0, (hipStream_t)stream,
-                       d_in, sg, ws, d_begin, d_nnz, d_values, d_mask, g_spin_limit.load(), g_skip_first.load());
-  else
-    hipLaunchKernelGGL(zvc_stream_kernel<false>, dim3(data_groups + 1), dim3(64 * kSWaves), 0, (hipStream_t)stream,
-                       d_in, sg, ws, d_begin, d_nnz, d_values, d_mask, g_spin_limit.load(), g_skip_first.load());
+  const unsigned long long bytes = 4ull * (unsigned long long)n;
+  const auto kernel = bytes * 3 >= g_staged_compact_bytes.load() * 5 ? zvc_stream_kernel<true, true>
+                      : bytes >= kReadOnceFrom                       ? zvc_stream_kernel<true, false>
+                                                                     : zvc_stream_kernel<false, false>;
+  hipLaunchKernelGGL(kernel, dim3(data_groups + 1), dim3(64 * kSWaves), 0, (hipStream_t)stream, d_in, sg, ws, d_begin, d_nnz,
+                     d_values, d_mask, g_spin_limit.load(), g_skip_first.load());
   return check_launch();
 }
 

@@ -63,3 +63,28 @@ def test_more_than_the_groups_hold_runs_the_three_kernels():
     k = int(want[3].item())
     assert int(got[3].item()) == k and torch.equal(got[0][:k], want[0][:k]) and torch.equal(got[1], want[1])
     assert int(ws.view(torch.int32)[4].item()) == 0
+
+
+# either side of the sizes from which the pipeline kernel reads its input, and stores its values, with the nontemporal hint
+@pytest.mark.parametrize("mib,off", [(80, -16384), (80, 0), (80, 16384), (320, -16384), (320, 0), (328, 0)])
+def test_pipeline_hints_against_three_kernels(mib, off):
+    import torch
+
+    from cswap_amd import api
+    from cswap_amd._lib import check, lib
+
+    process = 16384
+    n = (mib << 18) + 32 * off
+    L = lib()
+    assert L.cswap_zvc_takes_single_pass(n, process) == 1
+    x = torch.empty(n, device="cuda").normal_(generator=torch.Generator(device="cuda").manual_seed(mib)).clamp_(min=0.0)
+    want = api.zvc_compress(x, process)
+    got = [torch.zeros_like(o) for o in want]
+    ws = api.zvc_workspace(process)
+    for _ in range(2):
+        check(L.cswap_zvc_compress_fused(x.data_ptr(), n, process, ws.data_ptr(), got[2].data_ptr(), got[3].data_ptr(),
+                                         got[0].data_ptr(), got[1].data_ptr(), None), "fused")
+    torch.cuda.synchronize()
+    k = int(want[3].item())
+    assert int(got[3].item()) == k and torch.equal(got[0][:k], want[0][:k])
+    assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])

@@ -115,6 +115,7 @@ _SIGNATURES = {
     "cswap_zvc_debug_set_lookback": (None, [u, u]),        # include/cswap_test_hooks.h
     "cswap_test_zvc_stream_groups": (i32, [i32, i32]),      # include/cswap_test_hooks.h
     "cswap_test_zfp_decode_quad": (i32, [sz, sz, sz, pd, pd, u, i32]),
+    "cswap_test_zfp_decode_runs": (i32, [sz, sz, sz, pd, pd, u]),
     "cswap_test_zfp_store_hint": (i32, [C.c_ulonglong] * 4 + [u]),
     "cswap_test_zvc_packed_hint": (i32, [sz]),
     "cswap_test_zfp_encode_route": (i32, [sz, sz, sz, pd, pd, u, u, i32]),

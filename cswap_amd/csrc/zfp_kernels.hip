@@ -11,10 +11,12 @@
 // the stream is needed (the reference pre-zeroes the stream and adds every bit
 // with a global atomic, CSWAP+/zfp/encode.cuh:252-299, encode3.cuh:152).
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <atomic>
 #include "../../include/cswap_hip.h"
 #include "../../include/cswap_test_hooks.h"
 #include "zfp_block.h"
+#include "zfp_runs.h"
 #include "common.h"
 
 namespace cswap {
@@ -632,6 +634,136 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) 
     const uint64_t* __restrict__ stream, Field3 fd, unsigned maxbits, float* __restrict__ out)
 {
   decode3_f32<WHOLE, INT, true>(stream, fd, maxbits, out);
+}
+
+// ------------------------------------------------------------- rows that are not made of whole lines
+// The decoder for packed fields whose rows are no multiple of 128 bytes (zfp_runs.h).  One lane per block and a row store
+// per lane, as above, leaves rows of 28 bytes in parts of a line that are 16 bytes long, and one instruction touches
+// as many lines as it has rows: 160 MB in 7x7 planes took three times as long as in 32x32.  Here a wavefront takes whole
+// block rows, and one plane of them at a time goes through LDS (4 KB in the place of the decoded stream, so as many
+// wavefronts are resident as before): written as whole blocks, 16 bytes a lane without conflicts, read and stored
+// in the order of memory.  Where a unit stands and goes is worked out once and holds for all four planes.  What it
+// costs: two trips through LDS a plane, and lanes that are left over (64 / mx block rows fit).  Lanes without a block decode the
+// last one once more, units past the end store the last one again.  Bound by memory where rows are whole
+// 16 bytes (28x28: 4.6 MB a us at 150 MB, as 32x32), by the 4-byte stores and the vector unit at odd lengths.  8 bits per
+// value, one tensor over and over (several in turn), row stores -> this, us:
+//   units of 16 bytes  4x4 20 MB 16.1 -> 13.0 (16.6 -> 12.2), 60 MB 28.6 -> 21.8 (29.5 -> 21.9), 160 MB 57 -> 48 (68 -> 49) · 28x28 20 MB 13.3 -> 12.6
+//     (14.8 -> 11.8), 60 MB 20.1 -> 18.8 (23.9 -> 19.0), 160 MB 40.4 -> 38.5 (54.3 -> 38.9) · 56x56 60 MB 19.7 -> 18.9 (23.5 -> 19.1)
+//   of 8  14x14 20 MB 15.2 -> 13.1 (16.2 -> 12.8), 60 MB 27.2 -> 22.8 (28.1 -> 24.6), 160 MB 51 -> 46 (65 -> 51)
+//   of 4  7x7 20 MB 21.4 -> 14.9 (21.7 -> 15.9), 60 MB 44 -> 24.5 (45 -> 26.2), 160 MB 97 -> 51 (106 -> 58) · 35x35 20 MB 14.2 -> 14.4 (15.6 ->
+//     13.2), 60 MB 22.8 -> 21.3 (26.5 -> 23.9), 160 MB 44 -> 43 (60 -> 51)
+//   4 bits per value, 100 MB  28x28 26.4 -> 25.6 (35.4 -> 25.9); 16 bits 38.4 -> 36.3 (48.9 -> 40.6), 35x35 41.8 -> 41.2 (52.9 -> 49.3)
+template <int V>
+struct RunUnit;
+template <>
+struct RunUnit<4> {
+  typedef stream_f4 type;
+};
+template <>
+struct RunUnit<2> {
+  typedef float type __attribute__((ext_vector_type(2)));
+};
+template <>
+struct RunUnit<1> {
+  typedef float type;
+};
+
+// Computes these sixteen values where this stands
+__device__ __forceinline__ void pin16(int32_t (&ib)[64], int i)
+{
+  asm volatile(""
+               : "+v"(ib[i]), "+v"(ib[i + 1]), "+v"(ib[i + 2]), "+v"(ib[i + 3]), "+v"(ib[i + 4]), "+v"(ib[i + 5]), "+v"(ib[i + 6]),
+                 "+v"(ib[i + 7]), "+v"(ib[i + 8]), "+v"(ib[i + 9]), "+v"(ib[i + 10]), "+v"(ib[i + 11]), "+v"(ib[i + 12]),
+                 "+v"(ib[i + 13]), "+v"(ib[i + 14]), "+v"(ib[i + 15]));
+}
+
+// The last lifting pass, the cast and the stores, a plane at a time.  V: elements of a unit.  The pins keep the compiler
+// from working ahead on later planes, whose values it would hold twice over: without them it spills at 96 registers.
+template <int V, bool HINT>
+__device__ __forceinline__ void finish_and_store_runs(float* __restrict__ out, const Runs& p, const RunsWave& wave, char* image,
+                                                      int32_t (&ib)[64], float w)
+{
+  typedef typename RunUnit<V>::type unit_t;
+  constexpr int kUnits = 16 / V;
+  uint32_t src[kUnits], dst[kUnits];
+  uint32_t zero = 0;
+  asm volatile("" : "+v"(zero) : "v"(ib[0]));
+  const uint32_t lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+  char* mine = image + 16 * runs_block(p, min(lane, wave.blocks - 1));
+  const uint32_t row = 16 * p.mx;
+  char* plane = reinterpret_cast<char*>(out) + (size_t)wave.slab * 16u * V * p.plane;
+#pragma unroll
+  for (int z = 0; z < 4; z++) {
+    if (z) pin16(ib, 16 * z);
+#pragma unroll
+    for (int y = 0; y < 4; y++) {
+      float r[4];
+      decode_row(ib, y + 4 * z, w, r);
+      const stream_f4 v = {r[0], r[1], r[2], r[3]};
+      *reinterpret_cast<stream_f4*>(mine + y * row) = v;
+    }
+    if (z == 0) {
+      uint32_t l = lane;
+      asm volatile("" : "+v"(l) : "v"(ib[0]));
+#pragma unroll
+      for (int j = 0; j < kUnits; j++) {
+        runs_unit(p, wave, min(l + 64u * j, wave.total - 1), src[j], dst[j]);
+        src[j] *= 4 * V;
+        dst[j] *= 4 * V;
+      }
+    } else if (z == p.planes_last && wave.cut != ~0u) {  // from here on without the last slab: its units store the first one again
+      if (wave.cut == 0) return;
+#pragma unroll
+      for (int j = 0; j < kUnits; j++) {
+        const bool gone = dst[j] >= wave.cut * (4 * V);
+        src[j] = gone ? 0 : src[j];
+        dst[j] = gone ? wave.skip * (4 * V) : dst[j];
+      }
+    }
+    __syncthreads();
+    constexpr int kBatch = kUnits < 8 ? kUnits : 4;
+#pragma unroll
+    for (int b = 0; b < kUnits; b += kBatch) {
+      if (b) __builtin_amdgcn_sched_barrier(0);
+      unit_t v[kBatch];
+#pragma unroll
+      for (int j = 0; j < kBatch; j++) v[j] = *reinterpret_cast<const unit_t*>(image + src[b + j]);
+#pragma unroll
+      for (int j = 0; j < kBatch; j++) {
+        asm volatile("" : "+v"(dst[b + j]));  // a 32-bit offset to the plane's address, not a 64-bit one per unit
+        unit_t* to = reinterpret_cast<unit_t*>(plane + (size_t)dst[b + j]);
+        if (HINT) __builtin_nontemporal_store(v[j], to);
+        else *to = v[j];
+      }
+    }
+    __syncthreads();
+    plane += (size_t)4u * V * p.plane;
+  }
+}
+
+template <int V, bool HINT, int WPE>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void zfp_decode3_runs_kernel(
+    const uint64_t* __restrict__ stream, Field3 fd, Runs runs, unsigned maxbits, float* __restrict__ out)
+{
+  extern __shared__ uint4 lds_raw[];
+  uint32_t* lds = reinterpret_cast<uint32_t*>(lds_raw);
+  const unsigned lane = threadIdx.x;
+  const RunsWave wave = runs_wave(runs, blockIdx.x);
+  const unsigned slot = dec_slot_bits(maxbits);
+  __shared__ uint32_t table[64];
+  __builtin_amdgcn_s_setprio(3);
+  table[lane] = collapse_piece(lane);
+  load_region<true, kFenceDwords>(lds, lane, wave.first, wave.blocks, maxbits, slot, fd, stream);
+  __syncthreads();
+  int32_t ib[64];
+  float w;
+  LdsBitsCollapse mem(lds, table);
+  decode_block_zy<true>(mem, mem.bit0 + min(lane, wave.blocks - 1) * slot, maxbits, ib, w);
+#pragma unroll
+  for (int i = 0; i < 64; i += 16) pin16(ib, i);
+  __builtin_amdgcn_s_setprio(1);
+  __syncthreads();  // the image takes the stream's place
+  finish_and_store_runs<V, HINT>(out, runs, wave, reinterpret_cast<char*>(lds), ib, w);
 }
 
 // ------------------------------------------------------------- the pair form: two wavefronts per 64 blocks
@@ -1674,6 +1806,37 @@ static bool encode_rows(const Field3& fd, bool whole)
 }
 static bool decode_rows(const Field3& fd) { return fd.rows4 && !(fd.store_hint && (fd.nx & 3u) == 0); }
 
+// Which packed fields of floats the decoder stores as runs through LDS, and whether with the hint; us at 8 bits per value,
+// one tensor over and over (several in turn).
+//  - Rows of whole 16 bytes: with the hint, at all sizes and down to 48 lanes of 64 with a block (52x52 52 lanes, 60 MB
+//    20.0 -> 19.5 (24.7 -> 19.4); 100x100 50 lanes, 150 MB 37.8 -> 38.1 (52.8 -> 39.4)).  Not where rows are whole lines, nor where row stores
+//    do as well: half lines from 320 bytes a row on (80x80 60 MB 18.4 and 18.4 (18.7 and 18.6); 112x112 19 MB 11.2 and 12.6 (11.6 and
+//    11.8)), 192 bytes below 38 MiB (20 MB 11.3 and 12.7 (11.7 and 12.0); 60 MB 19.6 -> 18.6 (21.1 -> 18.7)).
+//  - Other rows: their runs end inside lines.  Below 40 MiB the hint pays all the same (plain / hint: 35x35 20 MB 14.3 / 14.4 (15.6 /
+//    13.2), 31x31 36 MB 17.6 / 15.9 (19.2 / 16.3), 33x33 36 MB 21.2 / 19.6 (23.1 / 20.0; row stores 21.0 and 23.5)) unless a plane is
+//    shorter than two lines (6x6 36 MB 20.3 / 24.3 (21.6 / 25.6)).  From there on it costs (35x35 60 MB 21.3 / 25.7 (23.9 / 26.2)),
+//    and without it lanes left over and padding tell.  A last block of one column never pays: 5x5 150 MB 101 -> 105 (108 -> 107), 13x13
+//    64 -> 67 (73 -> 70), 17x17 60 MB 30.6 -> 33.4 (33.1 -> 35.9), 33x33 27.7 -> 28.7 (30.5 -> 31.2).  Other rows of 16 elements and more are asked
+//    to fill 7/8 of what a wavefront can hold (30x30 0.88: 22.8 -> 22.2 (24.1 -> 23.8); 50x50 0.75: 21.4 -> 22.1 (25.9 -> 24.5)), shorter
+//    ones gain whatever they fill (15x15 30 -> 24 (31 -> 25), 6x6 38 -> 30 (41 -> 33), 3x3 58 -> 33 (60 -> 42)), and rows from
+//    252 bytes on gain nothing (63x63 60 MB 20.8 -> 20.9 (22.8 -> 23.3), 127x127 20.0 -> 20.5 (22.3 -> 22.6)).
+enum RunsRoute { kNoRuns, kRunsPlain, kRunsHint };
+static RunsRoute decode_runs(const Field3& fd, uintptr_t base)
+{
+  const bool packed = fd.rows4 && fd.sy == (long long)fd.nx && fd.sz == fd.sy * (long long)fd.ny;
+  if (!packed || fd.mx > 64 || fd.sz >= (long long)kRunsPlaneElements || fd.nx % 32 == 0) return kNoRuns;
+  const unsigned lanes = 64 / fd.mx * fd.mx;
+  if (lanes < 48) return kNoRuns;
+  const unsigned long long bytes = 4ull * fd.nx * fd.ny * fd.nz;
+  if (fd.nx % 4 == 0 && base % 16 == 0) {
+    if (fd.nx % 16 == 0 && base % 64 == 0 && (fd.nx >= 80 || (fd.nx == 48 && bytes < (38ull << 20)))) return kNoRuns;
+    return kRunsHint;
+  }
+  if (bytes < (40ull << 20)) return 4 * fd.sz >= 256 ? kRunsHint : kRunsPlain;
+  const unsigned long long held = (unsigned long long)lanes * fd.nx * fd.ny, room = 64ull * 16 * fd.mx * fd.my;
+  return fd.nx % 4 != 1 && (fd.nx < 16 || (fd.nx < 63 && 8 * held >= 7 * room)) ? kRunsPlain : kNoRuns;
+}
+
 static std::atomic<unsigned long long> g_pair_decode_bytes{CSWAP_PAIR_DECODE_BYTES};
 
 // The pair form pays while all of a field's workgroups are on the chip at once (twice the
@@ -1772,6 +1935,14 @@ extern "C" int cswap_test_zfp_decode_quad(size_t nx, size_t ny, size_t nz, ptrdi
   if (rc) return rc;
   return (maxbits & 63u) == 0 && quad_pays(fd.nblocks, quad_waves_decode(fd, maxbits), (unsigned long long)nx * ny * nz * 4ull,
                                            CSWAP_PAIR_DECODE_BYTES, compute_units);
+}
+
+extern "C" int cswap_test_zfp_decode_runs(size_t nx, size_t ny, size_t nz, ptrdiff_t sy, ptrdiff_t sz, unsigned base)
+{
+  Field3 fd;
+  const void* at = reinterpret_cast<const void*>((uintptr_t)4096 + base);
+  int rc = make_field(fd, at, reinterpret_cast<const void*>((uintptr_t)4096), nx, ny, nz, 1, sy, sz, 512, 4);
+  return rc ? rc : (int)decode_runs(fd, (uintptr_t)at);
 }
 
 extern "C" int cswap_test_zfp_store_hint(unsigned long long base, unsigned long long pitch, unsigned long long plane,
@@ -1890,6 +2061,22 @@ static int decompress3(const uint64_t* d_stream, Elem elem, size_t nx, size_t ny
   if (elem_bytes(elem) == 4) {
     float* out = static_cast<float*>(d_out);
     lds_bytes = (size_t)dec_region_dwords(maxbits) * 4;
+    const RunsRoute route = elem == kF32 && whole ? decode_runs(fd, (uintptr_t)d_out) : kNoRuns;
+    if (route != kNoRuns) {
+      const Runs runs = make_runs(fd.nx, fd.ny, fd.nz, (uintptr_t)d_out);
+      const bool fewer = maxbits >= kFewerWavesFrom;
+      const auto kernel =
+          runs.unit == 4 ? (fewer ? zfp_decode3_runs_kernel<4, true, 4> : zfp_decode3_runs_kernel<4, true, 5>)
+          : runs.unit == 2
+              ? (route == kRunsHint ? (fewer ? zfp_decode3_runs_kernel<2, true, 4> : zfp_decode3_runs_kernel<2, true, 5>)
+                                    : (fewer ? zfp_decode3_runs_kernel<2, false, 4> : zfp_decode3_runs_kernel<2, false, 5>))
+              : (route == kRunsHint ? (fewer ? zfp_decode3_runs_kernel<1, true, 4> : zfp_decode3_runs_kernel<1, true, 5>)
+                                    : (fewer ? zfp_decode3_runs_kernel<1, false, 4> : zfp_decode3_runs_kernel<1, false, 5>));
+      lds_bytes = std::max(lds_bytes, (size_t)kRunsImageDwords * 4);
+      hipLaunchKernelGGL(kernel, dim3((runs.block_rows + runs.rows - 1) / runs.rows), dim3(64), lds_bytes, st, d_stream, fd,
+                         runs, maxbits, out);
+      return check_launch();
+    }
     if (decode_rows(fd)) {
       if (whole && maxbits >= kFewerWavesFrom && !is_int)
         hipLaunchKernelGGL((zfp_decode3_rows_kernel<true, false, 4>), dim3(grid), dim3(64), lds_bytes, st, d_stream, fd,

@@ -50,6 +50,11 @@ int cswap_test_zfp_decode_quad(size_t nx, size_t ny, size_t nz, ptrdiff_t sy, pt
 int cswap_test_zfp_store_hint(unsigned long long base, unsigned long long pitch, unsigned long long plane,
                               unsigned long long bytes, unsigned maxbits);
 
+/* How the decoder's kernel for whole-word rates with one lane per block stores a 3-D field of floats with contiguous x-rows:
+ * 0 row by row, 1 as runs through LDS, 2 as runs with the nontemporal hint; or an error code.  sy, sz: strides in
+ * elements (0 = packed), base: the field's distance from a 128-byte line.  Host only. */
+int cswap_test_zfp_decode_runs(size_t nx, size_t ny, size_t nz, ptrdiff_t sy, ptrdiff_t sz, unsigned base);
+
 #ifdef __cplusplus
 }
 #endif

@@ -405,8 +405,8 @@ int cswap_swap_wait(cswap_engine* e, int ticket);
  * own: both directions can be busy at once) and is ordered by an event.  Returns at once; the data is ready when
  * `compute` reaches this point.  A compressed tensor whose outbound copy has not
  * finished yet is still in its staging block and is decompressed from there: no
- * wait for the copy, nothing on the link.  A raw one comes in behind that copy (in
- * engines with config.timing the host waits for it). */
+ * wait for the copy, nothing on the link.  A raw one comes in behind that copy
+ * where other payloads are staged; else, and in engines with config.timing, the host waits for it. */
 int cswap_swap_in(cswap_engine* e, int ticket, float* d_out, cswap_stream_t compute);
 /* Backward side, ahead of time: start the host-to-device copy of the payload
  * into the engine's device staging pool on the copy stream, before a

@@ -105,3 +105,34 @@ def test_raw_tensor_comes_back_into_itself(engine):
         engine.release(ticket)
     torch.cuda.synchronize()
     assert torch.equal(x, want)
+
+
+@pytest.mark.parametrize("order", ["in", "prefetch_in", "prefetch_release"])
+def test_raw_tensor_asked_back_while_another_payload_is_staged(engine, order):
+    """A long copy out goes ahead of both, so the raw tensor's own copy is still to come and the other's payload
+    still staged: the stream waits, and the other comes back from its staging block."""
+    import torch
+
+    from cswap_amd import swap
+
+    big = torch.randn(1, 16, 1024, 1024, device="cuda")
+    for _ in range(2):
+        x = torch.randn(1, 1, 1, 200001, device="cuda")
+        y = torch.randn(1, 8, 256, 256, device="cuda").clamp_(min=0.0)
+        want, out, back = x.clone(), torch.empty_like(x), torch.empty_like(y)
+        torch.cuda.synchronize()
+        ahead = engine.pre(big, swap.NONE)
+        other = engine.pre(y, swap.SPARSE)
+        ticket = engine.pre(x, swap.NONE)
+        if order.startswith("prefetch"):
+            engine.prefetch(ticket)
+        if order != "prefetch_release":
+            engine.swap_in(ticket, out)
+        engine.release(ticket)
+        engine.swap_in(other, back)
+        engine.release(other)
+        engine.post(ahead)
+        engine.release(ahead)
+        torch.cuda.synchronize()
+        assert torch.equal(back, y)
+        assert order == "prefetch_release" or torch.equal(out, want)

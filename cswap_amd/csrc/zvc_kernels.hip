@@ -66,9 +66,7 @@ __device__ __forceinline__ void st_stream4(float4* p, float4 v)
 }
 
 // The same where the address may be any element's.  The wavefront then writes partial lines at both
-// ends, and the hint does not always pay.  Long chunks, from the size of zvc_expand4_staged_kernel on only:
-// expansion of 314 MB 84 us with it, 108 without, 257 MB 61 and 61, 60 MB 19.2 and 16.2.  Short chunks:
-// packed_hint.
+// ends, and the hint does not always pay.  Long chunks: never (60 MB 19.2 us with it, 16.2 without).  Short chunks: packed_hint.
 template <bool ALIGNED, bool HINT = false>
 __device__ __forceinline__ void st_row4(float* p, float4 v)
 {
@@ -521,6 +519,39 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand_packed_kernel(
   }
 }
 
+// How many elements of its line lie in front of a chunk that goes to q
+__device__ __forceinline__ unsigned line_phase(const float* q) { return (unsigned)(reinterpret_cast<uintptr_t>(q) >> 2) & 31u; }
+
+// The mask words of a chunk moved up by `phase` bits: lane l's word behind the one of the lane before, whose
+// last lane's word of the refill before is `carry`.  Returns the shifted word and steps carry.
+__device__ __forceinline__ uint32_t shifted_words(uint32_t word, unsigned phase, unsigned lane, uint32_t& carry)
+{
+  uint32_t before = (uint32_t)__shfl_up((int)word, 1, 64);
+  if (lane == 0) before = carry;
+  carry = (uint32_t)__builtin_amdgcn_readlane((int)word, 63);
+  return (uint32_t)((((uint64_t)word << 32) | before) >> (32u - phase));
+}
+
+// Mask word w of a chunk of len elements: bits past its end carry no data
+__device__ __forceinline__ uint32_t chunk_word(uint32_t word, int w, unsigned len)
+{
+  const unsigned first = (unsigned)w * 32u;
+  return first + 32 <= len ? word : first >= len ? 0u : word & ((1u << (len - first)) - 1u);
+}
+
+// Four elements at place k of rows that start `phase` elements before the chunk and end with it at `end`; q: the start of the rows
+__device__ __forceinline__ void store_lane(float* q, unsigned k, unsigned phase, unsigned end, float4 v)
+{
+  if (k >= phase && k + 4 <= end) {
+    st_stream4(reinterpret_cast<float4*>(q + k), v);
+  } else {
+    if (k >= phase && k < end) q[k] = v.x;
+    if (k + 1 >= phase && k + 1 < end) q[k + 1] = v.y;
+    if (k + 2 >= phase && k + 2 < end) q[k + 2] = v.z;
+    if (k + 3 >= phase && k + 3 < end) q[k + 3] = v.w;
+  }
+}
+
 // zvc_expand4_kernel once more, for tensors larger than the memory-side cache (the size from which
 // the compaction is staged, too): the packed values of four rows (1024 elements) are first
 // brought into an LDS region of the wavefront with aligned 16-byte loads -- whole lines per
@@ -532,9 +563,15 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand_packed_kernel(
 // waits for, fewer rows per group means more groups) and the same where they come from the
 // cache; on small tensors the LDS costs more occupancy than the loads gain, so those keep
 // the kernels above.
+// The rows start where the line starts that the chunk begins in, whatever the chunk's length: its mask is moved up by as many
+// bits (shifted_words), and every store but a chunk's first and last is one of whole lines.  Rows that started with
+// the chunk put every line together from two instructions, each part a write of its own to memory.  One tensor over and
+// over (several in turn), us: chunks of 3308 elements 217 MB 57.9 -> 52.1 (73.2 -> 70.5), 3675 241 MB 64.6 -> 57.1 (67.0 -> 61.2), 4738 311 MB
+// 82.8 -> 74.6 (105.4 -> 99.2), 5025 329 MB 87.0 -> 78.5 (110.2 -> 102.9); 4096 (always a line's start) 268 MB 62.5 and 62.4 (77.0 and 76.8).
+// The same in zvc_expand4_kernel gains nothing reliable below that size (60 MB 16.4 -> 16.7 (24.7 -> 25.7), 188 MB 52.7 -> 45.3 (64 -> 65)
+// but whole lines 34 MB 8.2 -> 8.7 (9.7 -> 10.4)).
 constexpr int kRowsStaged = 4;  // divides kRowsInFlight
 
-template <bool ALIGNED>
 __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand4_staged_kernel(
     const float* __restrict__ values, const uint32_t* __restrict__ mask, const int* __restrict__ begin,
     Geometry g, float* __restrict__ out)
@@ -547,19 +584,19 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand4_staged_kernel
   const long long b = (long long)g.E * c;
   const int len = (int)min((long long)g.E, (long long)g.n - b);
   const uint32_t* mrow = mask + (size_t)c * g.W;
-  float* q = out + b;
+  const unsigned phase = line_phase(out + b), end = phase + (unsigned)len;  // below 2^31 + 32
+  float* q = out + b - phase;
   unsigned off = (unsigned)begin[c];
-  const int rows = (len + 255) >> 8;
+  const int rows = (int)((end + 255u) >> 8);
   const unsigned sub = lane & 7u;  // my nibble inside the word I read
   const uint32_t below = (1u << (4u * sub)) - 1u;
-  uint32_t held_next = (int)lane < g.W ? mrow[lane] : 0u;
+  uint32_t held_next = (int)lane < g.W ? mrow[lane] : 0u, carry = 0;
   for (int r0 = 0; r0 < rows; r0 += kRowsInFlight) {
-    uint32_t held = held_next, pre;  // pre: low half = set bits before my word in its row, high half = through it
+    uint32_t held, pre;  // pre: low half = set bits before my word in its row, high half = through it
     {  // 64 words = 8 rows; the next 64 are asked for now
       const int w = (r0 >> 3) * 64 + (int)lane;
+      held = shifted_words(chunk_word(held_next, w, (unsigned)len), phase, lane, carry);
       held_next = w + 64 < g.W ? mrow[w + 64] : 0u;
-      const int first = w * 32;  // bits past the end of the chunk carry no data
-      if (first + 32 > len) held = first >= len ? 0u : (held & ((1u << (len - first)) - 1u));
       const uint32_t cnt = (uint32_t)__popc(held);
       uint32_t s = cnt;
 #pragma unroll
@@ -582,13 +619,13 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand4_staged_kernel
       // the last group of four is fetched element by element so that nothing past the values is read
       const unsigned shift = off & 3u;
       const float* src = values + (off - shift);
-      const unsigned end = shift + total;
+      const unsigned until = shift + total;
       lds_order();  // the picks of the previous group are done
-      for (unsigned k = 4u * lane; k < end; k += 256u) {
-        if (k + 4u <= end) {
+      for (unsigned k = 4u * lane; k < until; k += 256u) {
+        if (k + 4u <= until) {
           *reinterpret_cast<float4*>(lds + k) = *reinterpret_cast<const float4*>(src + k);
         } else {
-          for (unsigned e = k; e < end; e++) lds[e] = src[e];
+          for (unsigned e = k; e < until; e++) lds[e] = src[e];
         }
       }
       lds_order();
@@ -613,14 +650,7 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand4_staged_kernel
       off += total;
 #pragma unroll
       for (int j = 0; j < kRowsStaged; j++) {
-        const int k = (r0 + h + j) * 256 + 4 * (int)lane;
-        if (k + 4 <= len) {
-          st_row4<ALIGNED, true>(q + k, x[j]);
-        } else {  // ragged end of the last chunk
-          if (k < len) q[k] = x[j].x;
-          if (k + 1 < len) q[k + 1] = x[j].y;
-          if (k + 2 < len) q[k + 2] = x[j].z;
-        }
+        store_lane(q, 256u * (unsigned)(r0 + h + j) + 4u * lane, phase, end, x[j]);
       }
     }
   }
@@ -1451,8 +1481,7 @@ extern "C" int cswap_zvc_expand(const float* d_values, const uint32_t* d_mask, c
                                                      : zvc_expand_packed_kernel<false, false>;
     hipLaunchKernelGGL(kernel, packed_grid, dim3(64 * kWavesPerGroup), 0, (hipStream_t)stream, d_values, d_mask, d_begin, g,
                        per, d_out);
-  } else if (staged && aligned) CSWAP_EXPAND(zvc_expand4_staged_kernel<true>);
-  else if (staged) CSWAP_EXPAND(zvc_expand4_staged_kernel<false>);
+  } else if (staged) CSWAP_EXPAND(zvc_expand4_staged_kernel);
   else if (aligned) CSWAP_EXPAND(zvc_expand4_kernel<true>);
   else CSWAP_EXPAND(zvc_expand4_kernel<false>);
 #undef CSWAP_EXPAND

@@ -88,3 +88,32 @@ def test_pipeline_hints_against_three_kernels(mib, off):
     k = int(want[3].item())
     assert int(got[3].item()) == k and torch.equal(got[0][:k], want[0][:k])
     assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
+
+
+# the staged expansion lays its rows out from the line that a chunk begins in: chunks below and above one word, one row and
+# the eight rows of a turn, destinations at every kind of place in a line, nothing stored outside
+@pytest.mark.parametrize("length", [1, 31, 32, 33, 255, 257, 2016, 2017, 2048, 2049, 4133])
+@pytest.mark.parametrize("off", [0, 1, 4, 15, 31])
+@pytest.mark.parametrize("short", [0, 1])
+def test_staged_expansion_at_any_place_of_a_line(length, off, short):
+    import torch
+
+    from cswap_amd import api
+    from cswap_amd._lib import check, lib
+
+    process = 37
+    n = length * process - min(short, length - 1)
+    x = torch.randn(n, device="cuda").clamp_(min=0.0)
+    values, mask, begin, _ = api.zvc_compress(x, process)
+    L = lib()
+    before = L.cswap_zvc_set_staged_compact_bytes(0)
+    try:
+        room = torch.full((n + 96,), -7.0, device="cuda")
+        at = 32 + off
+        check(L.cswap_zvc_expand(values.data_ptr(), mask.data_ptr(), begin.data_ptr(), n, process,
+                                 room.data_ptr() + 4 * at, torch.cuda.current_stream().cuda_stream), "expand")
+        torch.cuda.synchronize()
+    finally:
+        L.cswap_zvc_set_staged_compact_bytes(before)
+    assert torch.equal(room[at:at + n], x)
+    assert bool((room[:at] == -7.0).all()) and bool((room[at + n:] == -7.0).all())

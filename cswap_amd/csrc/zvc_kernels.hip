@@ -66,7 +66,9 @@ __device__ __forceinline__ void st_stream4(float4* p, float4 v)
 }
 
 // The same where the address may be any element's.  The wavefront then writes partial lines at both
-// ends, and the hint does not always pay.  Long chunks: never (60 MB 19.2 us with it, 16.2 without).  Short chunks: packed_hint.
+// ends, and the hint does not always pay.  Long chunks: below kPackedHintBelow, one tensor over and over (several in turn), us, without ->
+// with it 16 MB 7.0 -> 6.7 (7.9 -> 7.2), 20 MB 8.1 -> 7.6 (9.6 -> 8.1), 24 MB 8.2 -> 8.2 (9.1 -> 9.0); from there on it takes from one tensor what it gives
+// to several (30 MB 10.0 -> 10.6 (13.9 -> 11.4), 45 MB 12.9 -> 14.3 (19.7 -> 16.5), 60 MB 15.8 -> 18.9 (24.3 -> 22.9)).  Short chunks: packed_hint.
 template <bool ALIGNED, bool HINT = false>
 __device__ __forceinline__ void st_row4(float* p, float4 v)
 {
@@ -365,11 +367,11 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_compact_rows_kernel(
 // chunk, together with the number of set bits in the words before it inside its row,
 // so a lane finds its nibble and the rank of its first element with two cross-lane reads.
 // ALIGNED: E % 4 == 0 and a 16-byte aligned destination, so every chunk starts on a
-// 16-byte boundary.  Otherwise the same 16-byte stores at any element, without the hint:
+// 16-byte boundary.  Otherwise the same 16-byte stores at any element, without the hint from 28 MiB on:
 // 60 MB in chunks of 1838 elements 16.3 us, against 18.6 us with a 4-byte store per element.
 constexpr int kRowsInFlight = 8;  // divides the 8 rows one refill covers
 
-template <bool ALIGNED>
+template <bool ALIGNED, bool HINT>
 __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand4_kernel(
     const float* __restrict__ values, const uint32_t* __restrict__ mask, const int* __restrict__ begin,
     Geometry g, float* __restrict__ out)
@@ -425,7 +427,7 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand4_kernel(
     for (int j = 0; j < kRowsInFlight; j++) {
       const int k = (r0 + j) * 256 + 4 * (int)lane;
       if (k + 4 <= len) {
-        st_row4<ALIGNED>(q + k, x[j]);
+        st_row4<ALIGNED, HINT>(q + k, x[j]);
       } else {  // ragged end of the last chunk
         if (k < len) q[k] = x[j].x;
         if (k + 1 < len) q[k + 1] = x[j].y;
@@ -1482,8 +1484,9 @@ extern "C" int cswap_zvc_expand(const float* d_values, const uint32_t* d_mask, c
     hipLaunchKernelGGL(kernel, packed_grid, dim3(64 * kWavesPerGroup), 0, (hipStream_t)stream, d_values, d_mask, d_begin, g,
                        per, d_out);
   } else if (staged) CSWAP_EXPAND(zvc_expand4_staged_kernel);
-  else if (aligned) CSWAP_EXPAND(zvc_expand4_kernel<true>);
-  else CSWAP_EXPAND(zvc_expand4_kernel<false>);
+  else if (aligned) CSWAP_EXPAND((zvc_expand4_kernel<true, true>));
+  else if (4 * (size_t)n < kPackedHintBelow) CSWAP_EXPAND((zvc_expand4_kernel<false, true>));
+  else CSWAP_EXPAND((zvc_expand4_kernel<false, false>));
 #undef CSWAP_EXPAND
   return check_launch();
 }

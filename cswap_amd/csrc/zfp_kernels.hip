@@ -1814,7 +1814,8 @@ static bool decode_rows(const Field3& fd) { return fd.rows4 && !(fd.store_hint &
 //    11.8)), 192 bytes below 38 MiB (20 MB 11.3 and 12.7 (11.7 and 12.0); 60 MB 19.6 -> 18.6 (21.1 -> 18.7)).
 //  - Other rows: their runs end inside lines.  Below 40 MiB the hint pays all the same (plain / hint: 35x35 20 MB 14.3 / 14.4 (15.6 /
 //    13.2), 31x31 36 MB 17.6 / 15.9 (19.2 / 16.3), 33x33 36 MB 21.2 / 19.6 (23.1 / 20.0; row stores 21.0 and 23.5)) unless a plane is
-//    shorter than two lines (6x6 36 MB 20.3 / 24.3 (21.6 / 25.6)).  From there on it costs (35x35 60 MB 21.3 / 25.7 (23.9 / 26.2)),
+//    shorter than two lines (6x6 36 MB 20.3 / 24.3 (21.6 / 25.6)); fewer than 56 lanes only below 24 MiB (softmax values: 49x49 22 MB row
+//    stores 17.4, runs 17.0 (17.6, 16.2), 39 MB at 4 bits 17.8 and 18.9).  From there on it costs (35x35 60 MB 21.3 / 25.7 (23.9 / 26.2)),
 //    and without it lanes left over and padding tell.  A last block of one column never pays: 5x5 150 MB 101 -> 105 (108 -> 107), 13x13
 //    64 -> 67 (73 -> 70), 17x17 60 MB 30.6 -> 33.4 (33.1 -> 35.9), 33x33 27.7 -> 28.7 (30.5 -> 31.2).  Other rows of 16 elements and more are asked
 //    to fill 7/8 of what a wavefront can hold (30x30 0.88: 22.8 -> 22.2 (24.1 -> 23.8); 50x50 0.75: 21.4 -> 22.1 (25.9 -> 24.5)), shorter
@@ -1832,7 +1833,7 @@ static RunsRoute decode_runs(const Field3& fd, uintptr_t base)
     if (fd.nx % 16 == 0 && base % 64 == 0 && (fd.nx >= 80 || (fd.nx == 48 && bytes < (38ull << 20)))) return kNoRuns;
     return kRunsHint;
   }
-  if (bytes < (40ull << 20)) return 4 * fd.sz >= 256 ? kRunsHint : kRunsPlain;
+  if (bytes < ((lanes < 56 ? 24ull : 40ull) << 20)) return 4 * fd.sz >= 256 ? kRunsHint : kRunsPlain;
   const unsigned long long held = (unsigned long long)lanes * fd.nx * fd.ny, room = 64ull * 16 * fd.mx * fd.my;
   return fd.nx % 4 != 1 && (fd.nx < 16 || (fd.nx < 63 && 8 * held >= 7 * room)) ? kRunsPlain : kNoRuns;
 }

@@ -30,6 +30,7 @@ def test_route():
     assert [route(35, 35, mb) for mb in (20, 60)] == [2, 1] and [route(7, 7, mb) for mb in (20, 60)] == [1, 1]
     assert [route(n, n, 20) for n in (17, 33, 49, 63)] == [2] * 4 and [route(n, n, 60) for n in (17, 33, 49, 63)] == [0] * 4
     assert [route(n, n, 60) for n in (2, 6, 10, 15, 13, 30, 50)] == [1, 1, 1, 1, 0, 1, 0]
+    assert [route(n, n, 30) for n in (17, 33, 49, 197)] == [2, 2, 0, 0]              # lanes left over
     assert route(28, 28, 60, base=4) == 1 and route(28, 28, 60, base=8) == 1      # off 16 bytes
     assert route(28, 28, 60, sy=29) == 0 and route(28, 28, 60, sz=28 * 28 + 4) == 0 and route(28, 28, 60, sy=28, sz=28 * 28) == 2
     assert route(132, 64, 20) == 0 and route(260, 64, 20) == 0                    # lanes left over; longer than a wavefront

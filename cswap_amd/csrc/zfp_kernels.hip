@@ -243,7 +243,8 @@ __device__ __forceinline__ void padded_offsets(uint32_t n, uint32_t s, uint32_t 
 // access per element with its own 64-bit address, at 8 bits per value and with the coders that step from
 // run to run: 60 MB in 35x35 planes encoded in 26.2 instead of 28.1 us and decoded in 26.4 instead of 39.8,
 // 321 MB of them in 90 instead of 108 and 119 instead of 166; 26 MB in 14x14 planes 16.9 / 19.6 and 18.7 / 26.5.
-// Now: 60 MB in 35x35 planes 21.9 and 22.9, 26 MB in 14x14 13.3 and 16.2.
+// Now: 60 MB in 35x35 planes 21.9 and 22.9, 26 MB in 14x14 13.3 and 16.2.  (Packed fields are decoded by zfp_decode3_runs_kernel where
+// that is faster.)
 __device__ __forceinline__ void load_row(const char* src, float (&f)[64], int row)
 {
   const row_f4* p = reinterpret_cast<const row_f4*>(src);

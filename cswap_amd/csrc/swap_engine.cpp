@@ -23,6 +23,7 @@
 // the pinned allocator per tensor, Execution.h:76,97-99,114); several tensors
 // can be in flight at once (the reference has one dataptr_/buffer per Execution,
 // Execution.h:432-441).
+#include <algorithm>
 #include <chrono>
 #include <map>
 #include <mutex>
@@ -1047,27 +1048,30 @@ extern "C" int cswap_engine_calibrate(cswap_engine* e, cswap_costs* out_costs)
       if ((rc = ms(sd, 20, &td))) break;
       c.zfp_latency_us = 0.5 * (tc + td) * 1e3;
     }
-    // the probe: counting pass throughput, and the fixed cost of count + scan +
-    // 4-byte copy + host wait measured on a tensor too small to matter
+    // the probe: counting pass throughput, and the fixed cost of count + scan + the
+    // count's way to the host + host wait measured on a tensor too small to matter
     auto cnt = [&]() { return cswap_zvc_count(d_x, (int)n, proc, d_begin, s); };
     if ((rc = ms(cnt, 2, &t))) break;
     if ((rc = ms(cnt, 10, &t))) break;
     c.probe_gbs = gb / (t * 1e-3);
     {
-      const int small_n = 1 << 16, reps = 10;
+      // The median of turns that are timed one by one, after one that is not: the first launch of a kernel in a process
+      // loads its code, 400 us and more (as a tenth of ten turns it was 40 of 61 us, 20 to 24 afterwards).
+      const int small_n = 1 << 16, turns = 11;
       const int small_proc = process_for(e, (size_t)small_n);
-      hipError_t er2 = hipStreamSynchronize(s);
-      auto t0 = std::chrono::steady_clock::now();
-      for (int i = 0; i < reps && er2 == hipSuccess && !rc; i++) {
+      double took[turns];
+      if ((er = hipStreamSynchronize(s)) != hipSuccess) { rc = hip_fail(er); break; }
+      for (int i = -1; i < turns && !rc; i++) {
+        const auto t0 = std::chrono::steady_clock::now();
         rc = cswap_zvc_count(d_x, small_n, small_proc, d_begin, s);
         if (!rc) rc = cswap_zvc_scan(d_begin, cswap_zvc_active_chunks(small_n, small_proc), e->d_nnz, s);
         int count;
         if (!rc) rc = count_to_host(e, s, &count);
+        if (i >= 0) took[i] = std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count();
       }
-      auto t1 = std::chrono::steady_clock::now();
       if (rc) break;
-      if (er2 != hipSuccess) { rc = hip_fail(er2); break; }
-      c.probe_latency_us = std::chrono::duration<double, std::micro>(t1 - t0).count() / reps;
+      std::sort(took, took + turns);
+      c.probe_latency_us = took[turns / 2];
     }
     e->costs = c;
   } while (0);

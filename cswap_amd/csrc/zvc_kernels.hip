@@ -670,8 +670,9 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void zvc_expand4_staged_kernel
 // is some tens of milliseconds, two orders of magnitude above what the kernel takes for 1 GiB.
 constexpr unsigned kSpinLimit = 1u << 15;
 constexpr unsigned kFlagEvery = 32;  // a waiting wavefront looks at the failure flag every so many turns
-// cswap_zvc_debug_set_lookback: the bound of the waits, and whether tile 0 is never published
-static std::atomic<unsigned> g_spin_limit{kSpinLimit}, g_skip_first{0};
+// cswap_zvc_debug_set_lookback: the bound of the waits, and what is left out
+static std::atomic<unsigned> g_spin_limit{kSpinLimit}, g_skip{0};
+constexpr unsigned kSkipFirstCount = 1, kSkipFirstMark = 2, kRefuseLastTile = 4;
 
 // Head of a workspace.  ws[0]: kWsMagic once cswap_zvc_workspace_clear has prepared it;
 // ws[1]: not 0 after a run whose bounded waits ran out (stays until the next clear, and
@@ -829,7 +830,7 @@ template <bool ONCE, bool HINT>
 __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
     const float* __restrict__ in, StreamGeometry g, uint32_t* __restrict__ ws, int* __restrict__ begin,
     int* __restrict__ nnz, float* __restrict__ values, uint32_t* __restrict__ mask, unsigned spin_limit,
-    unsigned skip_first)
+    unsigned skip)
 {
   __shared__ __attribute__((aligned(16))) float stage[kSTileElems + 8];
   __shared__ unsigned s_cnt[kSSlots][kSWaves];
@@ -886,7 +887,7 @@ __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
     const unsigned incl = wave_inclusive_scan(mine);
     total[slot] = (unsigned)__builtin_amdgcn_readlane((int)incl, kSWaves - 1);
     woff[slot] = (unsigned)__builtin_amdgcn_readlane((int)(incl - mine), wv);
-    if (wv == 0 && exists && lane == 0 && !(skip_first && t == 0)) st_status(&status[t], kTileReady | total[slot]);
+    if (wv == 0 && exists && lane == 0 && !((skip & kSkipFirstCount) && t == 0)) st_status(&status[t], kTileReady | total[slot]);
   };
   // waits (bounded) until the scanner has published the offset of tile t
   bool gave_up = false;
@@ -1085,8 +1086,9 @@ __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
 // start, that one would publish into the next run's array.
 //
 // Failure works as in the pipeline kernel for the shapes that take_single_pass says 2 for (may_fail): a wait that runs
-// out raises the sticky flag, the offsets are kept inside the tensor, and the wavefront that gave up writes -1 after the
-// last workgroup has stepped the run counter.  The other shapes must not fail: a workgroup that finds the workspace
+// out, for a count or before a clearing, raises the sticky flag, the offsets are kept inside the tensor, and the wavefront
+// that gave up writes -1 after the last workgroup has stepped the run counter; a workgroup that starts when the flag is up leaves,
+// and if it is the last one it writes -1.  The other shapes must not fail: a workgroup that finds the workspace
 // unusable or whose wait runs out counts the elements before its own by itself, which costs time and nothing else; the
 // flag goes up all the same, since counts that nobody clears would be the next run's.
 //
@@ -1119,7 +1121,7 @@ __device__ uint32_t write_lane(uint32_t v, uint32_t lane, uint32_t old) __asm("l
 template <int W, int R, bool RAGGED, bool ONCE>
 __global__ __launch_bounds__(64 * W, 8) void zvc_small_kernel(
     const float* __restrict__ in, SmallGeometry g, uint32_t* __restrict__ ws, int* __restrict__ begin, int* __restrict__ nnz,
-    float* __restrict__ values, uint32_t* __restrict__ mask, int may_fail, unsigned spin_limit, unsigned skip_first)
+    float* __restrict__ values, uint32_t* __restrict__ mask, int may_fail, unsigned spin_limit, unsigned skip)
 {
   constexpr unsigned kElems = 64u * W * R, kHalves = 2u * W * R;
   static_assert(R <= 32, "64 half rows to a wavefront");
@@ -1180,18 +1182,19 @@ __global__ __launch_bounds__(64 * W, 8) void zvc_small_kernel(
     }
   }
   if (lane == 63) s_cnt[wv] = upto;
-  if (wv == 0 && lane == 0) s_head[0] = (magic != kWsMagic || flag != 0u) ? 1u : 0u;
+  const bool last_tile = t == g.tiles - 1;
+  if (wv == 0 && lane == 0) s_head[0] = (magic != kWsMagic || flag != 0u || ((skip & kRefuseLastTile) && last_tile)) ? 1u : 0u;
   __syncthreads();
   const bool refused = s_head[0] != 0u;
   if (may_fail && refused) {  // nothing is published, no value written
-    if (t == 0 && threadIdx.x == 0) *nnz = -1;
+    // The last tile says so whatever the first one found: the flag may have gone up since.
+    if ((t == 0 || last_tile) && threadIdx.x == 0) *nnz = -1;
     return;
   }
   const unsigned wave_cnt = lane < (unsigned)W ? s_cnt[lane] : 0u, wave_upto = wave_inclusive_scan(wave_cnt);
   const unsigned total = (unsigned)__builtin_amdgcn_readlane((int)wave_upto, W - 1);
   const unsigned before_wave = (unsigned)__builtin_amdgcn_readlane((int)(wave_upto - wave_cnt), wv);
   if (wv == 1 && lane < (unsigned)W) s_before[lane] = wave_upto - wave_cnt;
-  const bool last_tile = t == g.tiles - 1;
 
   bool gave_up = false;
   if (wv == 0) {
@@ -1200,7 +1203,7 @@ __global__ __launch_bounds__(64 * W, 8) void zvc_small_kernel(
     uint32_t* const counts = ws + 16 + (size_t)group * (kGroupTiles * kCountWords);  // my group's
     uint32_t* const totals = ws + 16 + kSmallCounts + (runs & 1u) * kSmallTotals;
     uint32_t* const others = ws + 16 + kSmallCounts + ((runs & 1u) ^ 1u) * kSmallTotals;
-    const bool ends_group = place == kGroupTiles - 1, silent = skip_first && t == 0;
+    const bool ends_group = place == kGroupTiles - 1, silent = (skip & kSkipFirstCount) && t == 0;
     unsigned in_group = 0, groups_before = 0, spins = 0;
     bool need_count = lane < place, need_total = lane < group;
     bool counts_open = !refused;
@@ -1241,7 +1244,7 @@ __global__ __launch_bounds__(64 * W, 8) void zvc_small_kernel(
       __builtin_amdgcn_s_sleep(1);
     }
     if (refused) gave_up = true;
-    if (!gave_up && lane == 0 && !silent) st_status(&counts[place * kCountWords], kTileReady | kTileThrough | total);
+    if (!gave_up && lane == 0 && !silent && !((skip & kSkipFirstMark) && t == 0)) st_status(&counts[place * kCountWords], kTileReady | kTileThrough | total);
     const unsigned before = (unsigned)__builtin_amdgcn_readlane((int)wave_inclusive_scan(in_group + groups_before), 63);
     if (lane == 0) {
       s_head[1] = min(before, g.n - total);  // whatever the words held: what this workgroup writes stays inside the tensor
@@ -1317,6 +1320,7 @@ __global__ __launch_bounds__(64 * W, 8) void zvc_small_kernel(
     for (unsigned spins = 0; __ballot((through[0] & through[1] & through[2] & kTileThrough) == 0u) != 0ull; spins++) {
       if (spins > spin_limit || (spins % kFlagEvery == kFlagEvery - 1 && ld_status(&ws[kWsFlag]) != 0u)) {
         if (lane == 0) atomicOr(&ws[kWsFlag], 1u);
+        gave_up = true;  // my rows are out, but what is left in the workspace makes this a failed run like any other
         break;
       }
       __builtin_amdgcn_s_sleep(1);
@@ -1525,10 +1529,10 @@ extern "C" size_t cswap_zvc_workspace_bytes(int process)
   return process > 0 ? ((size_t)status_words(process) + 16) * sizeof(uint32_t) : 0;
 }
 
-extern "C" void cswap_zvc_debug_set_lookback(unsigned spin_limit, unsigned skip_first)
+extern "C" void cswap_zvc_debug_set_lookback(unsigned spin_limit, unsigned skip)
 {
   g_spin_limit.store(spin_limit ? spin_limit : kSpinLimit);
-  g_skip_first.store(skip_first);
+  g_skip.store(skip);
 }
 
 // Tensors of at least this many bytes take the pipeline kernel in cswap_zvc_compress_fused; smaller ones,
@@ -1640,7 +1644,7 @@ extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, v
     const int may_fail = small_pass_may_fail(g) && 4ull * (unsigned long long)n < g_single_pass_bytes.load() ? 1 : 0;
 #define CSWAP_SMALL_AS(W, R, RAGGED, ONCE)                                                                          \
   hipLaunchKernelGGL((zvc_small_kernel<W, R, RAGGED, ONCE>), dim3(small.tiles), dim3(64 * W), 0, (hipStream_t)stream, d_in, small, ws, \
-                     d_begin, d_nnz, d_values, d_mask, may_fail, g_spin_limit.load(), g_skip_first.load())
+                     d_begin, d_nnz, d_values, d_mask, may_fail, g_spin_limit.load(), g_skip.load())
 #define CSWAP_SMALL(W, R, ONCE)                                 \
   do {                                                          \
     small.tiles = ((unsigned)n + 64 * W * R - 1) / (64 * W * R); \
@@ -1671,7 +1675,7 @@ extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, v
                       : bytes >= kReadOnceFrom                       ? zvc_stream_kernel<true, false>
                                                                      : zvc_stream_kernel<false, false>;
   hipLaunchKernelGGL(kernel, dim3(data_groups + 1), dim3(64 * kSWaves), 0, (hipStream_t)stream, d_in, sg, ws, d_begin, d_nnz,
-                     d_values, d_mask, g_spin_limit.load(), g_skip_first.load());
+                     d_values, d_mask, g_spin_limit.load(), g_skip.load());
   return check_launch();
 }
 

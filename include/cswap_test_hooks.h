@@ -17,10 +17,12 @@ extern "C" {
 
 /* The single-pass ZVC kernels wait, bounded, for status words of other workgroups.
  * spin_limit: how many times in all a wavefront asks again before it gives up
- * (0 = the default, some tens of milliseconds' worth); skip_first: if not 0 the
- * count of the first tile is never published, so that everything after it waits in
- * vain.  (0, 0) restores normal operation. */
-void cswap_zvc_debug_set_lookback(unsigned spin_limit, unsigned skip_first);
+ * (0 = the default, some tens of milliseconds' worth).  skip, bits: 1 the count of the first
+ * tile is never published, so that everything after it waits in vain; 2 (small form)
+ * the first tile never says that it has its offset, so that whoever clears its count
+ * waits in vain; 4 (small form) the last tile takes the workspace for unusable, as one does
+ * that starts after another's wait has run out.  (0, 0) restores normal operation. */
+void cswap_zvc_debug_set_lookback(unsigned spin_limit, unsigned skip);
 
 /* Data workgroups the pipeline kernel of cswap_zvc_compress_fused is launched with for a
  * tensor of `tiles` tiles on a part with `compute_units` compute units (the scanner's

@@ -24,8 +24,13 @@ int zfp_compress_f32_no_quad(const float* d_in, size_t nx, size_t ny, size_t nz,
 int zfp_decompress_f32_no_quad(const uint64_t* d_stream, size_t nx, size_t ny, size_t nz, unsigned maxbits, float* d_out,
                                hipStream_t stream);
 
-// Whether cswap_zvc_compress_fused runs one kernel for a shape that cswap_zvc_takes_single_pass says 0 for: one that cannot fail.
+// Whether cswap_zvc_compress_fused runs one kernel for a shape that cswap_zvc_takes_single_pass says 0 for.
 bool zvc_small_any_chunk(int n, int process);
+
+// cswap_zvc_compress_fused for a caller that looks at the count: shapes whose workgroups would count for themselves where
+// the workspace fails them, which takes the square of the tensor's size, write -1 instead.
+int zvc_compress_fused_reporting(const float* d_in, int n, int process, void* d_ws, int* d_begin, int* d_nnz, float* d_values,
+                                 uint32_t* d_mask, hipStream_t stream);
 
 // Whether a ZVC payload of `bytes` that is already made is worth sending: by the selector's model, what a
 // tensor of n elements has left to pay for it (link and expansion) against the raw swap.

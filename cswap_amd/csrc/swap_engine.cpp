@@ -470,8 +470,8 @@ static int single_pass_sparse(cswap_engine* e, Ticket& t, const float* d_in, hip
     if (!e->dpool.alloc(worst, &off)) return 1;
   }
   char* base = e->d_base + off;
-  int rc = cswap_zvc_compress_fused(d_in, (int)t.n, t.process, e->d_ws, (int*)base, e->d_nnz, (float*)(base + hdr),
-                                    (uint32_t*)(base + 4 * (size_t)t.process), compute);
+  int rc = cswap::zvc_compress_fused_reporting(d_in, (int)t.n, t.process, e->d_ws, (int*)base, e->d_nnz, (float*)(base + hdr),
+                                               (uint32_t*)(base + 4 * (size_t)t.process), compute);
   int count = 0;
   if (!rc) rc = count_to_host(e, compute, &count);
   if (rc) {

@@ -1627,8 +1627,9 @@ bool cswap::zvc_small_any_chunk(int n, int process)
   return make_geometry(g, n, process) == CSWAP_OK && cswap_zvc_takes_single_pass(n, process) == 0 && small_pass_shape(g, n, small);
 }
 
-extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, void* d_ws, int* d_begin,
-                                        int* d_nnz, float* d_values, uint32_t* d_mask, cswap_stream_t stream)
+// report: the small form reports failure whatever the shape
+static int compress_fused(const float* d_in, int n, int process, void* d_ws, int* d_begin, int* d_nnz, float* d_values,
+                          uint32_t* d_mask, bool report, cswap_stream_t stream)
 {
   if (!d_in || !d_ws || !d_begin || !d_nnz || !d_values || !d_mask) return CSWAP_E_ARG;
   Geometry g;
@@ -1641,7 +1642,7 @@ extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, v
   const bool single_pass = single_pass_shape(g, n, process, sg) && (reinterpret_cast<uintptr_t>(d_values) & 15u) == 0;
   SmallGeometry small;
   if (!single_pass && small_pass_shape(g, n, small)) {
-    const int may_fail = small_pass_may_fail(g) && 4ull * (unsigned long long)n < g_single_pass_bytes.load() ? 1 : 0;
+    const int may_fail = report || (small_pass_may_fail(g) && 4ull * (unsigned long long)n < g_single_pass_bytes.load()) ? 1 : 0;
 #define CSWAP_SMALL_AS(W, R, RAGGED, ONCE)                                                                          \
   hipLaunchKernelGGL((zvc_small_kernel<W, R, RAGGED, ONCE>), dim3(small.tiles), dim3(64 * W), 0, (hipStream_t)stream, d_in, small, ws, \
                      d_begin, d_nnz, d_values, d_mask, may_fail, g_spin_limit.load(), g_skip.load())
@@ -1677,6 +1678,18 @@ extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, v
   hipLaunchKernelGGL(kernel, dim3(data_groups + 1), dim3(64 * kSWaves), 0, (hipStream_t)stream, d_in, sg, ws, d_begin, d_nnz,
                      d_values, d_mask, g_spin_limit.load(), g_skip.load());
   return check_launch();
+}
+
+extern "C" int cswap_zvc_compress_fused(const float* d_in, int n, int process, void* d_ws, int* d_begin,
+                                        int* d_nnz, float* d_values, uint32_t* d_mask, cswap_stream_t stream)
+{
+  return compress_fused(d_in, n, process, d_ws, d_begin, d_nnz, d_values, d_mask, false, stream);
+}
+
+int cswap::zvc_compress_fused_reporting(const float* d_in, int n, int process, void* d_ws, int* d_begin, int* d_nnz,
+                                        float* d_values, uint32_t* d_mask, hipStream_t stream)
+{
+  return compress_fused(d_in, n, process, d_ws, d_begin, d_nnz, d_values, d_mask, true, stream);
 }
 
 // ------------------------------------------------------------------ no allocation

@@ -1112,8 +1112,20 @@ struct SmallGeometry {
   unsigned tiles;
   unsigned spread;            // log2 of the words from one group's total to the next
   unsigned mask_words, tail;  // words of the mask, and the first of those that hold no element
+  unsigned clearers;          // workgroups behind the tiles that clear those; 0: the tiles do
   Div31 by_E, by_W;
 };
+
+// How many workgroups of `threads` clear the mask words that hold no element, where the tiles would take more than
+// eight turns each.  Few elements in many chunks: the one tile of 8192 elements took 8.0 us with 65536 chunks, 15.0 with 262144
+// and 43 with 2^20; with these workgroups 5.7, 5.6 and 6.0 (16384 chunks, cleared by the tile, 6.0).
+static unsigned small_clearers(const SmallGeometry& g, unsigned threads)
+{
+  const unsigned words = g.mask_words - g.tail;
+  if (words <= 8ull * threads * g.tiles) return 0;
+  const unsigned groups = (words + 4 * threads - 1) / (4 * threads);
+  return groups < 1024 ? groups : 1024;
+}
 
 // old with lane `lane` replaced by the uniform v
 __device__ uint32_t write_lane(uint32_t v, uint32_t lane, uint32_t old) __asm("llvm.amdgcn.writelane.i32");
@@ -1131,6 +1143,10 @@ __global__ __launch_bounds__(64 * W, 8) void zvc_small_kernel(
   __shared__ unsigned s_head[4];              // refused, offset, gave up, failure flag
   const unsigned t = blockIdx.x, lane = lane_id();
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (t >= g.tiles) {  // no tile: a share of the mask words that hold no element
+    for (unsigned f = g.tail + (t - g.tiles) * 64u * W + threadIdx.x; f < g.mask_words; f += g.clearers * 64u * W) mask[f] = 0;
+    return;
+  }
   const unsigned first = t * kElems, mine = first + 64u * R * wv;  // my tile's first element, my wavefront's
   const unsigned end = min(first + kElems, g.n);
 
@@ -1265,7 +1281,8 @@ __global__ __launch_bounds__(64 * W, 8) void zvc_small_kernel(
         mask[f] = w;
       }
     }
-    for (unsigned f = g.tail + t * 64u * (W - 1) + threadIdx.x - 64u; f < g.mask_words; f += g.tiles * 64u * (W - 1)) mask[f] = 0;
+    if (g.clearers == 0)
+      for (unsigned f = g.tail + t * 64u * (W - 1) + threadIdx.x - 64u; f < g.mask_words; f += g.tiles * 64u * (W - 1)) mask[f] = 0;
   }
   __syncthreads();
   unsigned offset = s_head[1];
@@ -1644,7 +1661,7 @@ static int compress_fused(const float* d_in, int n, int process, void* d_ws, int
   if (!single_pass && small_pass_shape(g, n, small)) {
     const int may_fail = report || (small_pass_may_fail(g) && 4ull * (unsigned long long)n < g_single_pass_bytes.load()) ? 1 : 0;
 #define CSWAP_SMALL_AS(W, R, RAGGED, ONCE)                                                                          \
-  hipLaunchKernelGGL((zvc_small_kernel<W, R, RAGGED, ONCE>), dim3(small.tiles), dim3(64 * W), 0, (hipStream_t)stream, d_in, small, ws, \
+  hipLaunchKernelGGL((zvc_small_kernel<W, R, RAGGED, ONCE>), dim3(small.tiles + small.clearers), dim3(64 * W), 0, (hipStream_t)stream, d_in, small, ws, \
                      d_begin, d_nnz, d_values, d_mask, may_fail, g_spin_limit.load(), g_skip.load())
 #define CSWAP_SMALL(W, R, ONCE)                                 \
   do {                                                          \
@@ -1652,6 +1669,7 @@ static int compress_fused(const float* d_in, int n, int process, void* d_ws, int
     if (small.tiles > kGroupsMax * kGroupTiles) return CSWAP_E_ARG; \
     small.spread = 2; \
     while (small.spread < 7 && (small.tiles + kGroupTiles - 1) / kGroupTiles <= (unsigned)kSmallTotals >> (small.spread + 1)) small.spread++; \
+    small.clearers = small_clearers(small, 64 * W);             \
     if (g.E % 32 != 0) CSWAP_SMALL_AS(W, R, true, ONCE);        \
     else CSWAP_SMALL_AS(W, R, false, ONCE);                     \
   } while (0)

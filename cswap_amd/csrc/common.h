@@ -28,7 +28,7 @@ int zfp_decompress_f32_no_quad(const uint64_t* d_stream, size_t nx, size_t ny, s
 bool zvc_small_any_chunk(int n, int process);
 
 // cswap_zvc_compress_fused for a caller that looks at the count: shapes whose workgroups would count for themselves where
-// the workspace fails them, which takes the square of the tensor's size, write -1 instead.
+// the workspace fails them, at milliseconds a call, write -1 instead.
 int zvc_compress_fused_reporting(const float* d_in, int n, int process, void* d_ws, int* d_begin, int* d_nnz, float* d_values,
                                  uint32_t* d_mask, hipStream_t stream);
 

@@ -1085,12 +1085,15 @@ __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
 // its offset, so that everybody has taken the same array: had it stepped past a workgroup that is still to
 // start, that one would publish into the next run's array.
 //
-// Failure works as in the pipeline kernel for the shapes that take_single_pass says 2 for (may_fail): a wait that runs
+// Failure works as in the pipeline kernel for the shapes that take_single_pass says 2 for (MAY_FAIL): a wait that runs
 // out, for a count or before a clearing, raises the sticky flag, the offsets are kept inside the tensor, and the wavefront
 // that gave up writes -1 after the last workgroup has stepped the run counter; a workgroup that starts when the flag is up leaves,
-// and if it is the last one it writes -1.  The other shapes must not fail: a workgroup that finds the workspace
-// unusable or whose wait runs out counts the elements before its own by itself, which costs time and nothing else; the
-// flag goes up all the same, since counts that nobody clears would be the next run's.
+// and if it is the last one it writes -1.  The other shapes must not fail.  A workgroup whose wait runs out counts the elements
+// before its own by itself; the flag goes up all the same, since counts that nobody clears would be the next run's.  Where the
+// workspace is found unusable the last tile of every group compacts the whole group, and the others write their mask words and leave:
+// they have published nothing, so that tile is refused as well or its wait for them runs out.  What it costs, until the workspace is
+// cleared, is to read what is in front of a group at one workgroup's rate: 60 MB 1.6 ms, 92 MB 2.3, 235 MB 9.6 (20, 34 and 79 us with
+// the workspace; with every tile on its own, the square of the size: 7.3, 19 and 86 ms).
 //
 // Bound by the two trips (some 2 us), by the loads before and the stores behind them, which overlap only as far as tiles
 // differ in when they get their offset, and by instruction issue (14 a row).  Against one workgroup of sixteen wavefronts on
@@ -1130,10 +1133,64 @@ static unsigned small_clearers(const SmallGeometry& g, unsigned threads)
 // old with lane `lane` replaced by the uniform v
 __device__ uint32_t write_lane(uint32_t v, uint32_t lane, uint32_t old) __asm("llvm.amdgcn.writelane.i32");
 
-template <int W, int R, bool RAGGED, bool ONCE>
+// What a workgroup does without the others' counts: counts the elements before `from` by itself, and compacts from there to
+// `end`, all but the mask.  Returns the count of non-zeros before `end`.  `from` is a multiple of 64 * W * 8.
+template <int W>
+__device__ __forceinline__ unsigned compact_alone(const float* __restrict__ in, unsigned from, unsigned end, Div31 by_E, unsigned E,
+                                                  unsigned* s_cnt, int* __restrict__ begin, float* __restrict__ values)
+{
+  const unsigned lane = lane_id(), wv = threadIdx.x >> 6;
+  constexpr unsigned kStep = 4 * 64 * W;
+  auto nonzero = [](any_f4 v) { return (unsigned)(v.x != 0.0f) + (v.y != 0.0f) + (v.z != 0.0f) + (v.w != 0.0f); };
+  unsigned mine = 0, i = 4 * threadIdx.x;
+  for (; i + 7 * kStep < from; i += 8 * kStep) {  // 8 loads on their way: one workgroup's rate is what this takes
+    any_f4 v[8];
+#pragma unroll
+    for (unsigned j = 0; j < 8; j++) v[j] = *reinterpret_cast<const any_f4*>(in + i + j * kStep);
+#pragma unroll
+    for (unsigned j = 0; j < 8; j++) mine += nonzero(v[j]);
+  }
+  for (; i < from; i += kStep) mine += nonzero(*reinterpret_cast<const any_f4*>(in + i));
+  mine = (unsigned)wave_sum((int)mine);
+  if (lane == 0) s_cnt[wv] = mine;
+  __syncthreads();
+  unsigned offset = 0;
+  for (int k = 0; k < W; k++) offset += s_cnt[k];
+  for (unsigned base = from; base < end; base += 64 * W * 8) {
+    const unsigned e = base + 512 * wv + lane;
+    float v[8];
+#pragma unroll
+    for (unsigned j = 0; j < 8; j++) {
+      v[j] = in[min(e + 64 * j, end - 1)];
+      if (e + 64 * j >= end) v[j] = 0.0f;
+    }
+    unsigned cnt = 0;
+#pragma unroll
+    for (unsigned j = 0; j < 8; j++) cnt += popc64(__ballot(v[j] != 0.0f));
+    __syncthreads();  // s_cnt has been read
+    if (lane == 0) s_cnt[wv] = cnt;
+    __syncthreads();
+    unsigned at = offset;
+    for (unsigned k = 0; k < (unsigned)W; k++) {
+      at += k < wv ? s_cnt[k] : 0u;
+      offset += s_cnt[k];
+    }
+#pragma unroll
+    for (unsigned j = 0; j < 8; j++) {
+      const unsigned long long m = __ballot(v[j] != 0.0f);
+      const unsigned slot = at + rank_below(m), me = e + 64 * j, c = div31(me, by_E);
+      if (v[j] != 0.0f) values[slot] = v[j];
+      if (me < end && c * E == me) begin[c] = (int)slot;
+      at += popc64(m);
+    }
+  }
+  return offset;
+}
+
+template <int W, int R, bool RAGGED, bool ONCE, bool MAY_FAIL>
 __global__ __launch_bounds__(64 * W, 8) void zvc_small_kernel(
     const float* __restrict__ in, SmallGeometry g, uint32_t* __restrict__ ws, int* __restrict__ begin, int* __restrict__ nnz,
-    float* __restrict__ values, uint32_t* __restrict__ mask, int may_fail, unsigned spin_limit, unsigned skip)
+    float* __restrict__ values, uint32_t* __restrict__ mask, unsigned spin_limit, unsigned skip)
 {
   constexpr unsigned kElems = 64u * W * R, kHalves = 2u * W * R;
   static_assert(R <= 32, "64 half rows to a wavefront");
@@ -1143,10 +1200,6 @@ __global__ __launch_bounds__(64 * W, 8) void zvc_small_kernel(
   __shared__ unsigned s_head[4];              // refused, offset, gave up, failure flag
   const unsigned t = blockIdx.x, lane = lane_id();
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  if (t >= g.tiles) {  // no tile: a share of the mask words that hold no element
-    for (unsigned f = g.tail + (t - g.tiles) * 64u * W + threadIdx.x; f < g.mask_words; f += g.clearers * 64u * W) mask[f] = 0;
-    return;
-  }
   const unsigned first = t * kElems, mine = first + 64u * R * wv;  // my tile's first element, my wavefront's
   const unsigned end = min(first + kElems, g.n);
 
@@ -1175,6 +1228,11 @@ __global__ __launch_bounds__(64 * W, 8) void zvc_small_kernel(
   float behind = 0.0f;
   if (RAGGED && wv == W - 1 && first + kElems + lane < g.n) behind = in[first + kElems + lane];
 
+  if (__builtin_expect(t >= g.tiles, 0)) {  // no tile (and element 0 loaded for it): a share of the mask words that hold no element
+    for (unsigned f = g.tail + (t - g.tiles) * 64u * W + threadIdx.x; f < g.mask_words; f += g.clearers * 64u * W) mask[f] = 0;
+    return;
+  }
+
   // ---- count: lane l < 2R keeps half row l of my rows
   uint32_t held = 0;
 #pragma unroll
@@ -1201,8 +1259,9 @@ __global__ __launch_bounds__(64 * W, 8) void zvc_small_kernel(
   const bool last_tile = t == g.tiles - 1;
   if (wv == 0 && lane == 0) s_head[0] = (magic != kWsMagic || flag != 0u || ((skip & kRefuseLastTile) && last_tile)) ? 1u : 0u;
   __syncthreads();
-  const bool refused = s_head[0] != 0u;
-  if (may_fail && refused) {  // nothing is published, no value written
+  const bool refused = __builtin_amdgcn_readfirstlane((int)s_head[0]) != 0;
+  static_assert(kElems % (64 * W * 8) == 0, "compact_alone");
+  if (MAY_FAIL && refused) {  // nothing is published, no value written
     // The last tile says so whatever the first one found: the flag may have gone up since.
     if ((t == 0 || last_tile) && threadIdx.x == 0) *nnz = -1;
     return;
@@ -1265,7 +1324,7 @@ __global__ __launch_bounds__(64 * W, 8) void zvc_small_kernel(
     if (lane == 0) {
       s_head[1] = min(before, g.n - total);  // whatever the words held: what this workgroup writes stays inside the tensor
       s_head[2] = gave_up ? 1u : 0u;
-      if (may_fail && last_tile) s_head[3] = ld_status(&ws[kWsFlag]);
+      if (MAY_FAIL && last_tile) s_head[3] = ld_status(&ws[kWsFlag]);
     }
   } else {
     // ---- meanwhile the mask words that start in my tile, and my share of those that hold no element
@@ -1285,78 +1344,82 @@ __global__ __launch_bounds__(64 * W, 8) void zvc_small_kernel(
       for (unsigned f = g.tail + t * 64u * (W - 1) + threadIdx.x - 64u; f < g.mask_words; f += g.tiles * 64u * (W - 1)) mask[f] = 0;
   }
   __syncthreads();
-  unsigned offset = s_head[1];
-  const bool counts_itself = !may_fail && s_head[2] != 0u;
-  if (counts_itself) {
-    unsigned before = 0;
-    for (unsigned i = threadIdx.x; i < first; i += 64u * W) before += in[i] != 0.0f;
-    before = (unsigned)wave_sum((int)before);
-    if (lane == 0) s_cnt[wv] = before;  // what was in it has been taken out
-    __syncthreads();
-    offset = 0;
-    for (int k = 0; k < W; k++) offset += s_cnt[k];
-  }
+  // Two ifs, and not one with an else: the compiler lays both sides out one behind the other and would keep the rows in registers
+  // through compact_alone, 36 bytes a lane of them in scratch memory (92 MB in chunks of any length 34.2 -> 36.5 us).
+  int alone = !MAY_FAIL && __builtin_amdgcn_readfirstlane((int)s_head[2]) != 0;
+  if (!alone) {
+    const unsigned offset = s_head[1];
 
-  // ---- where the chunks that start in my tile start among the values
-  {
-    const unsigned c0 = div31(first + g.E - 1u, g.by_E), c1 = div31(end + g.E - 1u, g.by_E);
-    for (unsigned c = c0 + threadIdx.x; c < c1; c += 64u * W) {
-      const unsigned at = c * g.E - first, h = at / 32u, w = h / (2u * R);
-      unsigned o = offset + s_before[w] + pre[h];
-      if (RAGGED) o += (unsigned)__popc(bits[h] & ((1u << (at & 31u)) - 1u));
-      begin[c] = (int)o;
-    }
-  }
-  // ---- the counts that I clear, if I clear any: asked for now, looked at when my rows are out
-  const unsigned group = t / kGroupTiles, groups = (g.tiles + kGroupTiles - 1) / kGroupTiles;
-  const bool clears = wv == 0 && !gave_up && (last_tile || ((t + 1) % kGroupTiles == 0 && group >= 2 && group + 1 < groups));
-  const unsigned clear_at = (group < 2 ? 0u : group - 2u) * kGroupTiles + lane;
-  const unsigned clear_end = last_tile ? g.tiles : (group < 2 ? 0u : group - 1u) * kGroupTiles;
-  uint32_t* const clear = ws + 16 + (size_t)clear_at * kCountWords;
-  uint32_t through[3] = {kTileThrough, kTileThrough, kTileThrough};
-  auto ask = [&] {
-#pragma unroll
-    for (unsigned k = 0; k < 3; k++)
-      if (clear_at + k * kGroupTiles < clear_end) through[k] = ld_status(clear + (size_t)k * kGroupTiles * kCountWords);
-  };
-  if (clears) ask();
-  // ---- my non-zeros, row by row, straight from the lanes that hold them
-  float* const out = values + (offset + before_wave);
-  unsigned at = 0;
-#pragma unroll
-  for (int j = 0; j < R; j++) {
-    asm volatile("" : "+v"(x[j]));
-    const bool nz = x[j] != 0.0f;
-    const unsigned long long m = __ballot(nz);
-    const unsigned slot = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, at));
-    if (nz) *reinterpret_cast<float*>(reinterpret_cast<char*>(out) + (size_t)(4u * slot)) = x[j];
-    at += popc64(m);
-  }
-
-  if (clears) {
-    for (unsigned spins = 0; __ballot((through[0] & through[1] & through[2] & kTileThrough) == 0u) != 0ull; spins++) {
-      if (spins > spin_limit || (spins % kFlagEvery == kFlagEvery - 1 && ld_status(&ws[kWsFlag]) != 0u)) {
-        if (lane == 0) atomicOr(&ws[kWsFlag], 1u);
-        gave_up = true;  // my rows are out, but what is left in the workspace makes this a failed run like any other
-        break;
+    // ---- where the chunks that start in my tile start among the values
+    {
+      const unsigned c0 = div31(first + g.E - 1u, g.by_E), c1 = div31(end + g.E - 1u, g.by_E);
+      for (unsigned c = c0 + threadIdx.x; c < c1; c += 64u * W) {
+        const unsigned at = c * g.E - first, h = at / 32u, w = h / (2u * R);
+        unsigned o = offset + s_before[w] + pre[h];
+        if (RAGGED) o += (unsigned)__popc(bits[h] & ((1u << (at & 31u)) - 1u));
+        begin[c] = (int)o;
       }
-      __builtin_amdgcn_s_sleep(1);
-      ask();
     }
+    // ---- the counts that I clear, if I clear any: asked for now, looked at when my rows are out
+    const unsigned group = t / kGroupTiles, groups = (g.tiles + kGroupTiles - 1) / kGroupTiles;
+    const bool clears = wv == 0 && !gave_up && (last_tile || ((t + 1) % kGroupTiles == 0 && group >= 2 && group + 1 < groups));
+    const unsigned clear_at = (group < 2 ? 0u : group - 2u) * kGroupTiles + lane;
+    const unsigned clear_end = last_tile ? g.tiles : (group < 2 ? 0u : group - 1u) * kGroupTiles;
+    uint32_t* const clear = ws + 16 + (size_t)clear_at * kCountWords;
+    uint32_t through[3] = {kTileThrough, kTileThrough, kTileThrough};
+    auto ask = [&] {
 #pragma unroll
-    for (unsigned k = 0; k < 3; k++)
-      if (clear_at + k * kGroupTiles < clear_end) st_status(clear + (size_t)k * kGroupTiles * kCountWords, 0u);
-  }
+      for (unsigned k = 0; k < 3; k++)
+        if (clear_at + k * kGroupTiles < clear_end) through[k] = ld_status(clear + (size_t)k * kGroupTiles * kCountWords);
+    };
+    if (clears) ask();
+    // ---- my non-zeros, row by row, straight from the lanes that hold them
+    float* const out = values + (offset + before_wave);
+    unsigned at = 0;
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      asm volatile("" : "+v"(x[j]));
+      const bool nz = x[j] != 0.0f;
+      const unsigned long long m = __ballot(nz);
+      const unsigned slot = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, at));
+      if (nz) *reinterpret_cast<float*>(reinterpret_cast<char*>(out) + (size_t)(4u * slot)) = x[j];
+      at += popc64(m);
+    }
 
-  // ---- the result
-  if (last_tile && threadIdx.x == 0) {
-    const bool failed = may_fail && (gave_up || s_head[3] != 0u);
-    *nnz = failed ? -1 : (int)(offset + total);
-    __threadfence();
-    if (!refused && !counts_itself) __hip_atomic_fetch_add(&ws[kWsSmallRuns], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  } else if (may_fail && gave_up && !last_tile) {  // (wavefront 0 of another workgroup) after the last workgroup has spoken
-    for (unsigned spins = 0; ld_status(&ws[kWsSmallRuns]) == runs && spins < spin_limit; spins++) __builtin_amdgcn_s_sleep(2);
-    if (lane == 0) *nnz = -1;
+    if (clears) {
+      for (unsigned spins = 0; __ballot((through[0] & through[1] & through[2] & kTileThrough) == 0u) != 0ull; spins++) {
+        if (spins > spin_limit || (spins % kFlagEvery == kFlagEvery - 1 && ld_status(&ws[kWsFlag]) != 0u)) {
+          if (lane == 0) atomicOr(&ws[kWsFlag], 1u);
+          gave_up = true;  // my rows are out, but what is left in the workspace makes this a failed run like any other
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+        ask();
+      }
+#pragma unroll
+      for (unsigned k = 0; k < 3; k++)
+        if (clear_at + k * kGroupTiles < clear_end) st_status(clear + (size_t)k * kGroupTiles * kCountWords, 0u);
+    }
+
+    // ---- the result
+    if (last_tile && threadIdx.x == 0) {
+      const bool failed = MAY_FAIL && (gave_up || s_head[3] != 0u);
+      *nnz = failed ? -1 : (int)(offset + total);
+      __threadfence();
+      __hip_atomic_fetch_add(&ws[kWsSmallRuns], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else if (MAY_FAIL && gave_up && !last_tile) {  // (wavefront 0 of another workgroup) after the last workgroup has spoken
+      for (unsigned spins = 0; ld_status(&ws[kWsSmallRuns]) == runs && spins < spin_limit; spins++) __builtin_amdgcn_s_sleep(2);
+      if (lane == 0) *nnz = -1;
+    }
+  }
+  asm volatile("" : "+v"(alone));
+  if (!MAY_FAIL && __builtin_amdgcn_readfirstlane(alone) != 0) {
+    const bool ends_group = (t + 1) % kGroupTiles == 0 || last_tile;
+    // (a refused tile that does not end its group leaves: the one that does is refused or gives up, too)
+    if (refused && !ends_group) return;
+    const unsigned from = ends_group ? t / kGroupTiles * kGroupTiles * kElems : first;
+    const unsigned count = compact_alone<W>(in, from, end, g.by_E, g.E, s_cnt, begin, values);
+    if (last_tile && threadIdx.x == 0) *nnz = (int)count;
   }
 }
 
@@ -1618,7 +1681,7 @@ static bool small_pass_shape(const Geometry& g, int n, SmallGeometry& sg)
   sg.by_W = make_div31(sg.W);
   return true;
 }
-// Whether a run of it reports failure where the workspace fails it (zvc_small_kernel: may_fail): whole half rows per
+// Whether a run of it reports failure where the workspace fails it (zvc_small_kernel: MAY_FAIL): whole half rows per
 // chunk, at most 131072 rows of the mask layout on a part of 256 compute units.
 static bool small_pass_may_fail(const Geometry& g)
 {
@@ -1659,10 +1722,11 @@ static int compress_fused(const float* d_in, int n, int process, void* d_ws, int
   const bool single_pass = single_pass_shape(g, n, process, sg) && (reinterpret_cast<uintptr_t>(d_values) & 15u) == 0;
   SmallGeometry small;
   if (!single_pass && small_pass_shape(g, n, small)) {
-    const int may_fail = report || (small_pass_may_fail(g) && 4ull * (unsigned long long)n < g_single_pass_bytes.load()) ? 1 : 0;
+    const bool may_fail = report || (small_pass_may_fail(g) && 4ull * (unsigned long long)n < g_single_pass_bytes.load());
 #define CSWAP_SMALL_AS(W, R, RAGGED, ONCE)                                                                          \
-  hipLaunchKernelGGL((zvc_small_kernel<W, R, RAGGED, ONCE>), dim3(small.tiles + small.clearers), dim3(64 * W), 0, (hipStream_t)stream, d_in, small, ws, \
-                     d_begin, d_nnz, d_values, d_mask, may_fail, g_spin_limit.load(), g_skip.load())
+  hipLaunchKernelGGL((may_fail ? zvc_small_kernel<W, R, RAGGED, ONCE, true> : zvc_small_kernel<W, R, RAGGED, ONCE, false>), \
+                     dim3(small.tiles + small.clearers), dim3(64 * W), 0, (hipStream_t)stream, d_in, small, ws, d_begin, d_nnz, \
+                     d_values, d_mask, g_spin_limit.load(), g_skip.load())
 #define CSWAP_SMALL(W, R, ONCE)                                 \
   do {                                                          \
     small.tiles = ((unsigned)n + 64 * W * R - 1) / (64 * W * R); \

@@ -207,8 +207,10 @@ int cswap_zvc_compress(const float* d_in, int n, int process, int* d_begin, int*
  * cswap_zvc_takes_single_pass is 0 never report failure: where the workspace was not
  * prepared, or a failure has been left in it, or their own wait runs out (which leaves
  * one for the calls of other shapes), they count again what they cannot read there, so
- * their result is right and takes longer.  They use the workspace all the same while
- * it is good: calls that overlap on one are wrong for them, too. */
+ * their result is right and takes longer: 60 MB 1.6 ms instead of 20 us, 235 MB 9.6 ms
+ * instead of 79 us, every time until cswap_zvc_workspace_clear has been called.  They use
+ * the workspace all the same while it is good: calls that overlap on one are wrong for
+ * them, too. */
 size_t cswap_zvc_workspace_bytes(int process);
 int cswap_zvc_compress_fused(const float* d_in, int n, int process, void* d_ws, int* d_begin,
                              int* d_nnz, float* d_values, uint32_t* d_mask, cswap_stream_t stream);
@@ -224,7 +226,8 @@ int cswap_zvc_workspace_clear(void* d_ws, int process, cswap_stream_t stream);
  * lengths that are multiples of 32, at most 131072 rows of 64 elements, 32 MiB), 0 a
  * form that does not need the workspace to succeed: the three kernels, or the small
  * form of tensors of other chunk lengths or more rows, whose workgroups
- * count for themselves where the workspace fails them.  Host only. */
+ * count for themselves where the workspace fails them (for what that costs see
+ * cswap_zvc_compress_fused).  Host only. */
 int cswap_zvc_takes_single_pass(int n, int process);
 /* No counterpart in the reference: the tensor size in bytes from which
  * cswap_zvc_compress_fused runs the pipeline kernel (default 64 MiB; 0 = whenever

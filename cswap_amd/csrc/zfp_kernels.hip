@@ -1822,15 +1822,21 @@ static bool decode_rows(const Field3& fd) { return fd.rows4 && !(fd.store_hint &
 //    to fill 7/8 of what a wavefront can hold (30x30 0.88: 22.8 -> 22.2 (24.1 -> 23.8); 50x50 0.75: 21.4 -> 22.1 (25.9 -> 24.5)), shorter
 //    ones gain whatever they fill (15x15 30 -> 24 (31 -> 25), 6x6 38 -> 30 (41 -> 33), 3x3 58 -> 33 (60 -> 42)), and rows from
 //    252 bytes on gain nothing (63x63 60 MB 20.8 -> 20.9 (22.8 -> 23.3), 127x127 20.0 -> 20.5 (22.3 -> 22.6)).
+//  - Either only where blocks are full enough: most of the image is padding with one row to a plane (28x1 150 MB 97 -> 106 (97 -> 109),
+//    15x1 30 MB 1.19 times), and with two in rows of more than 8 (100x2 150 MB 1.23 times (1.10), 35x2 30 MB 1.04 (1.07)).
+//    With the hint a plane that is not whole 64-byte sectors ends inside one, which is then written twice, and a short plane is little
+//    else: 150 MB in 4x2 3.0 times (2.3), 8x7 1.59 (1.14), 12x3 2.2 (1.6), 28x7 1.32 (1.01), 24x7 1.22 (0.96); from 1 KB on 28x10 1.01 (0.75),
+//    100x3 1.18 (0.87), 252x9 0.99 (0.75); whole sectors 8x6 1.01 (0.76), 16x3 0.58 (0.49).
 enum RunsRoute { kNoRuns, kRunsPlain, kRunsHint };
 static RunsRoute decode_runs(const Field3& fd, uintptr_t base)
 {
   const bool packed = fd.rows4 && fd.sy == (long long)fd.nx && fd.sz == fd.sy * (long long)fd.ny;
   if (!packed || fd.mx > 64 || fd.sz >= (long long)kRunsPlaneElements || fd.nx % 32 == 0) return kNoRuns;
   const unsigned lanes = 64 / fd.mx * fd.mx;
-  if (lanes < 48) return kNoRuns;
+  if (lanes < 48 || fd.ny == 1 || (fd.ny == 2 && fd.nx > 8 && fd.nx % 16 != 0)) return kNoRuns;
   const unsigned long long bytes = 4ull * fd.nx * fd.ny * fd.nz;
   if (fd.nx % 4 == 0 && base % 16 == 0) {
+    if (fd.sz % 16 != 0 && 4 * fd.sz < 1024) return kNoRuns;
     if (fd.nx % 16 == 0 && base % 64 == 0 && (fd.nx >= 80 || (fd.nx == 48 && bytes < (38ull << 20)))) return kNoRuns;
     return kRunsHint;
   }

@@ -1730,7 +1730,6 @@ static int compress_fused(const float* d_in, int n, int process, void* d_ws, int
 #define CSWAP_SMALL(W, R, ONCE)                                 \
   do {                                                          \
     small.tiles = ((unsigned)n + 64 * W * R - 1) / (64 * W * R); \
-    if (small.tiles > kGroupsMax * kGroupTiles) return CSWAP_E_ARG; \
     small.spread = 2; \
     while (small.spread < 7 && (small.tiles + kGroupTiles - 1) / kGroupTiles <= (unsigned)kSmallTotals >> (small.spread + 1)) small.spread++; \
     small.clearers = small_clearers(small, 64 * W);             \

@@ -86,7 +86,8 @@ __device__ __forceinline__ void st_row4(float* p, float4 v)
 // that the next reader of the tensor itself, the layer that it is the input of, finds it evicted.  Plain loads -> hint, us, tensors in turn:
 // compaction and expansion (half zeros) 67 MB 49.4 -> 50.6, 100 MB 70.1 -> 67.0, 201 MB 133.8 -> 119.0, 268 MB 169.5 -> 163.3, odd chunks 89 MB 61.4 -> 57.2,
 // 180 MB 125.3 -> 117.4; producer, compaction and a reader behind it 60 MB 60.6 -> 64.6, 89 MB 90.2 -> 90.3, 134 MB 137.6 -> 132.9, 241 MB 247 -> 233.
-// The same tensor over and over, which the cache holds up to its size, loses: 120 MB 36.3 -> 40.7 by itself (45.4 -> 43.2 in turn).
+// One tensor over and over, which the cache holds, loses up to 160 MB, and that is the price: the compaction by itself (in turn) 94 MB
+// 37.5 -> 41.0 (43.0 -> 41.1), 120 MB 43.7 -> 47.8 (50.3 -> 47.8), 159 MB 52.9 -> 57.0 (60.6 -> 58.4), 199 MB 68.9 -> 66.5 (70.4 -> 68.8).
 constexpr unsigned long long kReadOnceFrom = 80ull << 20;
 template <bool ONCE>
 __device__ __forceinline__ float ld_once(const float* p)
@@ -735,8 +736,8 @@ __device__ __forceinline__ void st_status(uint32_t* p, uint32_t v)
 // clearing.
 //
 // Measured on one MI355X, half of the elements zero (this kernel / count + scan + compact):
-// 512 MiB 0.161 / 0.240 ms, 256 MiB 0.082 / 0.115 ms, 128 MiB 0.046 / 0.056, 64 MiB 0.031 /
-// 0.033, 32 MiB 0.021 / 0.020 ms (a tensor of a few rounds of the grid does not fill the
+// 512 MiB 0.157 / 0.241 ms, 256 MiB 0.085 / 0.115 ms, 128 MiB 0.051 / 0.057, 64 MiB 0.032 /
+// 0.033, 32 MiB 0.022 / 0.020 ms (a tensor of a few rounds of the grid does not fill the
 // pipeline).
 constexpr int kSWaves = 16, kSRows = 12;
 constexpr int kSTileRows = kSWaves * kSRows, kSTileElems = kSTileRows * 64;
@@ -824,8 +825,9 @@ __device__ void zvc_stream_scanner(uint32_t* ws, const StreamGeometry& g, int st
 }
 
 // HINT: the values leave with the nontemporal hint, from 5/3 of the size from which the three kernels' compaction is staged on (320 MiB).  Below,
-// whoever reads them next finds them in the memory-side cache: compaction and expansion of 201 MB 133.8 -> 119.0 us and of 268 MB 169.5 -> 147.5 over
-// one tensor and -> 163.3 in turn, the compaction alone 87.8 and 88.2; 537 MB with the hint 317, without 327.
+// whoever reads them next finds them in the memory-side cache.  The compaction by itself is within 3 % either way.  With the expansion behind
+// it, with the hint / without, us over one tensor (in turn): 268 MB 170 / 148 (170 / 163), 302 194 / 167 (194 / 195), 346 216 / 186 (217 / 208), 417 262 /
+// 222 (262 / 243), 470 286 / 245 (288 / 261), 537 317 / 328 (319 / 323): the line could lie at 480 MiB.
 template <bool ONCE, bool HINT>
 __global__ __launch_bounds__(64 * kSWaves) void zvc_stream_kernel(
     const float* __restrict__ in, StreamGeometry g, uint32_t* __restrict__ ws, int* __restrict__ begin,
@@ -1617,7 +1619,7 @@ extern "C" void cswap_zvc_debug_set_lookback(unsigned spin_limit, unsigned skip)
 
 // Tensors of at least this many bytes take the pipeline kernel in cswap_zvc_compress_fused; smaller ones,
 // which do not fill the pipeline (a few rounds of the grid), finish sooner in the one-kernel form that
-// holds the whole tensor in registers: just below the limit 25 us, the pipeline 31 at it.
+// holds the whole tensor in registers: 60 MiB 21 us, the pipeline 32.
 static std::atomic<unsigned long long> g_single_pass_bytes{64ull << 20};  // cswap_zvc_set_single_pass_bytes
 
 extern "C" size_t cswap_zvc_set_single_pass_bytes(size_t bytes)

@@ -148,7 +148,9 @@ int    cswap_zvc_pick_process(size_t n);
  * and one that stages them in LDS and writes whole aligned 1 KB runs with the
  * nontemporal hint; the second is faster for tensors larger than the GPU's
  * memory-side cache and runs for tensors of at least this many bytes (default
- * 192 MiB; 0 = always, SIZE_MAX = never).  Same output either way.  Returns the
+ * 192 MiB; 0 = always, SIZE_MAX = never).  From the same size on cswap_zvc_expand
+ * brings its values in through LDS, and from 5/3 of it the pipeline kernel of
+ * cswap_zvc_compress_fused stores with the hint.  Same output either way.  Returns the
  * previous value.  Process-wide; not meant to be changed while kernels are being launched. */
 size_t cswap_zvc_set_staged_compact_bytes(size_t bytes);
 
